@@ -94,11 +94,13 @@ class HostBuf {
 
 // LBVH in device memory.  Two layouts live side by side: the reference's
 // parity arrays (keys, perm, children, parents) and the traversal layout:
-//   nodes[4*i .. 4*i+3]   one 64-byte record per internal node i:
+//   nodes[4*s .. 4*s+3]   one 64-byte record per internal node, in the slot of
+//       its left child's index s (word >> 2 of its child word):
 //       (L.minx, L.maxx, L.miny, L.maxy) (L.minz, L.maxz, R.minx, R.maxx)
-//       (R.miny, R.maxy, R.minz, R.maxz) (children word, 0, 0, 0)
-//     -- both child boxes next to the child word, so one visit is one
-//        contiguous 64-byte read; a leaf child's slot holds its triangle box.
+//       (R.miny, R.maxy, R.minz, R.maxz) (L's child word, R's, 0, 0)
+//     -- both child boxes and the children's own child words, so one visit is
+//        one contiguous 64-byte read and names the next visit's record and
+//        leaf triangles; a leaf child's slot holds its triangle box, word 0.
 //   tris[3*k .. 3*k+2]   one 48-byte record per sorted triangle k:
 //       (p0.xyz, original id) (e1.xyz, 0) (e2.xyz, 0), e = p - p0.
 struct DeviceBvh {

@@ -499,14 +499,18 @@ struct Box {
     float mnx, mxx, mny, mxy, mnz, mxz;
 };
 
-__device__ __forceinline__ void store_slot(float4* nodes, uint32_t p, bool left, const Box& b) {
-    float4* rec = nodes + 4 * static_cast<size_t>(p);
+// One child's box and word (0 for a leaf) into the record of the node with
+// child word pw.
+__device__ __forceinline__ void store_slot(float4* nodes, uint32_t pw, bool left, const Box& b, uint32_t cw) {
+    float4* rec = nodes + 4 * static_cast<size_t>(pw >> 2);
     if (left) {
         rec[0] = make_float4(b.mnx, b.mxx, b.mny, b.mxy);
         reinterpret_cast<float2*>(rec + 1)[0] = make_float2(b.mnz, b.mxz);
+        reinterpret_cast<uint32_t*>(rec + 3)[0] = cw;
     } else {
         reinterpret_cast<float2*>(rec + 1)[1] = make_float2(b.mnx, b.mxx);
         rec[2] = make_float4(b.mny, b.mxy, b.mnz, b.mxz);
+        reinterpret_cast<uint32_t*>(rec + 3)[1] = cw;
     }
 }
 
@@ -522,14 +526,16 @@ __device__ __forceinline__ Box unite(const Box& a, const Box& b) {
     return o;
 }
 
-// Node p's whole traversal record: both child boxes and the child word, in
-// one 64-byte line.
-__device__ __forceinline__ void store_record(float4* nodes, uint32_t p, const Box& lb, const Box& rb, uint32_t w) {
-    float4* rec = nodes + 4 * static_cast<size_t>(p);
+// The whole traversal record of the node with child word w (slot w >> 2, its
+// left child's index): both child boxes and both children's own words (0 for
+// a leaf), in one 64-byte line.
+__device__ __forceinline__ void store_record(float4* nodes, uint32_t w, const Box& lb, const Box& rb, uint32_t wl,
+                                             uint32_t wr) {
+    float4* rec = nodes + 4 * static_cast<size_t>(w >> 2);
     rec[0] = make_float4(lb.mnx, lb.mxx, lb.mny, lb.mxy);
     rec[1] = make_float4(lb.mnz, lb.mxz, rb.mnx, rb.mxx);
     rec[2] = make_float4(rb.mny, rb.mxy, rb.mnz, rb.mxz);
-    rec[3] = make_float4(__uint_as_float(w), 0.0f, 0.0f, 0.0f);
+    rec[3] = make_float4(__uint_as_float(wl), __uint_as_float(wr), 0.0f, 0.0f);
 }
 
 __device__ __forceinline__ void store_root(float* root_box, const Box& b) {
@@ -576,18 +582,18 @@ __device__ __forceinline__ void refit_level(const uint32_t* __restrict__ childre
                 const uint32_t old = __hip_atomic_fetch_add(counters + p, 1u, __ATOMIC_ACQ_REL,
                                                             __HIP_MEMORY_SCOPE_WORKGROUP);
                 if ((old & kCountMask) == 0u) break;
-                const float4* rec = nodes + 4 * static_cast<size_t>(p);
+                const uint32_t pw = children[p];
+                const float4* rec = nodes + 4 * static_cast<size_t>(pw >> 2);
                 const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
                 const Box lb{r0.x, r0.y, r0.z, r0.w, r1.x, r1.y};
                 const Box rb{r1.z, r1.w, r2.x, r2.y, r2.z, r2.w};
                 const Box b = unite(lb, rb);
-                nodes[4 * static_cast<size_t>(p) + 3] = make_float4(__uint_as_float(children[p]), 0.0f, 0.0f, 0.0f);
                 const uint32_t pp = parents_internal[p];
                 if (pp == kInvalid) {
                     store_root(root_box + 6 * static_cast<size_t>(scene_of[p]), b);
                     break;
                 }
-                store_slot(nodes, pp, (children[pp] >> 2) == p, b);
+                store_slot(nodes, children[pp], (children[pp] >> 2) == p, b, pw);
                 if ((counters[pp] >> kLevelShift) != level) break;
                 p = pp;
             }
@@ -605,7 +611,7 @@ constexpr uint32_t kStageCap = 1024;
 constexpr uint32_t kUpOutside = 0xffffffffu;  // parent handled by a later phase, or none
 
 struct LevelStage {
-    float box[12][kStageCap];  // left child box, then right, in record order
+    float box[14][kStageCap];  // the record: left child box, then right, then their words
     uint32_t node[kStageCap];  // the listed node
     uint32_t word[kStageCap];  // its child word
     uint32_t par[kStageCap];   // its parent (kInvalid at a scene root)
@@ -646,13 +652,14 @@ __device__ __forceinline__ void stage_links(LevelStage& S, uint32_t idx, uint32_
     S.wait[idx] = L.wait;
 }
 
-// A listed node's two child boxes, from its record (stored by earlier phases).
-__device__ __forceinline__ void stage_boxes(LevelStage& S, uint32_t idx, uint32_t s,
+// A listed node's two child boxes and words, from its record (stored by
+// earlier phases); w: its child word.
+__device__ __forceinline__ void stage_boxes(LevelStage& S, uint32_t idx, uint32_t w,
                                             const float4* __restrict__ nodes) {
-    const float4* rec = nodes + 4 * static_cast<size_t>(s);
-    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
-    const float v[12] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w};
-    for (int k = 0; k < 12; ++k) S.box[k][idx] = v[k];
+    const float4* rec = nodes + 4 * static_cast<size_t>(w >> 2);
+    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
+    const float v[14] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w, r3.x, r3.y};
+    for (int k = 0; k < 14; ++k) S.box[k][idx] = v[k];
 }
 
 // The climb over a staged list (after a barrier): every node with no
@@ -669,7 +676,8 @@ __device__ __forceinline__ void climb_staged(LevelStage& S, const uint32_t* __re
             const Box rb{S.box[6][idx], S.box[7][idx], S.box[8][idx], S.box[9][idx], S.box[10][idx], S.box[11][idx]};
             const Box b = unite(lb, rb);
             const uint32_t s = S.node[idx];
-            store_record(nodes, s, lb, rb, S.word[idx]);
+            const uint32_t w = S.word[idx];
+            store_record(nodes, w, lb, rb, __float_as_uint(S.box[12][idx]), __float_as_uint(S.box[13][idx]));
             const uint32_t pp = S.par[idx];
             if (pp == kInvalid) {
                 store_root(root_box + 6 * static_cast<size_t>(scene_of[s]), b);
@@ -677,13 +685,14 @@ __device__ __forceinline__ void climb_staged(LevelStage& S, const uint32_t* __re
             }
             const uint32_t up = S.up[idx];
             if (up == kUpOutside) {
-                store_slot(nodes, pp, (children[pp] >> 2) == s, b);
+                store_slot(nodes, children[pp], (children[pp] >> 2) == s, b, w);
                 break;
             }
             const uint32_t ps = up >> 1;
             const int o = (up & 1u) ? 6 : 0;
             S.box[o + 0][ps] = b.mnx; S.box[o + 1][ps] = b.mxx; S.box[o + 2][ps] = b.mny;
             S.box[o + 3][ps] = b.mxy; S.box[o + 4][ps] = b.mnz; S.box[o + 5][ps] = b.mxz;
+            S.box[12 + (up & 1u)][ps] = __uint_as_float(w);
             const uint32_t old = __hip_atomic_fetch_sub(&S.wait[ps], 1u, __ATOMIC_ACQ_REL,
                                                         __HIP_MEMORY_SCOPE_WORKGROUP);
             if (old != 1u) break;  // the other same-level child completes the parent
@@ -701,7 +710,7 @@ __device__ __forceinline__ void refit_level_staged(LevelStage& S, const uint32_t
                                                    const uint32_t* list, uint32_t count, uint32_t level) {
     for (uint32_t idx = threadIdx.x; idx < count; idx += blockDim.x) {
         const uint32_t s = list[idx];
-        stage_boxes(S, idx, s, nodes);
+        stage_boxes(S, idx, children[s], nodes);
         stage_links(S, idx, s, node_links(s, children, parents_internal, counters, slots, list_start, level));
     }
     __syncthreads();
@@ -856,7 +865,7 @@ __global__ __launch_bounds__(kRefitBlock) void k_refit_local(
     s_leaf.put(tid, b);
     uint32_t p = parents_leaf[k];
     if (!local(p)) {
-        store_slot(nodes, p, (children[p] >> 2) == k, b);  // finished by a later phase
+        store_slot(nodes, children[p], (children[p] >> 2) == k, b, 0u);  // finished by a later phase
         return;
     }
     for (;;) {
@@ -869,14 +878,14 @@ __global__ __launch_bounds__(kRefitBlock) void k_refit_local(
         const Box rb = (w & 2u) ? s_node.get(r - base) : s_leaf.get(r - base);
         b = unite(lb, rb);
         s_node.put(p - base, b);
-        store_record(nodes, p, lb, rb, w);
+        store_record(nodes, w, lb, rb, (w & 1u) ? s_word[l - base] : 0u, (w & 2u) ? s_word[r - base] : 0u);
         const uint32_t pp = s_par[p - base];
         if (pp == kInvalid) {
             store_root(root_box + 6 * static_cast<size_t>(scene_of[p]), b);
             return;
         }
         if (!local(pp)) {  // finished by a later phase, from its record
-            store_slot(nodes, pp, (children[pp] >> 2) == p, b);
+            store_slot(nodes, children[pp], (children[pp] >> 2) == p, b, w);
             return;
         }
         p = pp;
@@ -934,7 +943,7 @@ __global__ __launch_bounds__(1024) void k_refit_mid(const uint32_t* __restrict__
             S.par[idx] = links[1 + 2 * kStageCap + idx];
             S.up[idx] = links[1 + 3 * kStageCap + idx];
             S.wait[idx] = links[1 + 4 * kStageCap + idx];
-            stage_boxes(S, idx, sn, nodes);
+            stage_boxes(S, idx, S.word[idx], nodes);
         }
         __syncthreads();
         climb_staged(S, children, scene_of, nodes, root_box, staged);
@@ -967,7 +976,7 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
             S.par[idx] = top_links[1 + kStageCap + idx];
             S.up[idx] = top_links[1 + 2 * kStageCap + idx];
             S.wait[idx] = top_links[1 + 3 * kStageCap + idx];
-            stage_boxes(S, idx, s, nodes);
+            stage_boxes(S, idx, S.word[idx], nodes);
         }
         __syncthreads();
         climb_staged(S, children, scene_of, nodes, root_box, count);
@@ -1003,7 +1012,7 @@ __global__ __launch_bounds__(256) void k_dump_scene(const float4* __restrict__ n
         for (int k = 0; k < 6; ++k) o[k] = root_box[k];
         return;
     }
-    const float4* rec = nodes + 4 * static_cast<size_t>(pg);
+    const float4* rec = nodes + 4 * static_cast<size_t>(children[pg] >> 2);
     const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
     if ((children[pg] >> 2) == g) {
         o[0] = r0.x; o[1] = r0.z; o[2] = r1.x; o[3] = r0.y; o[4] = r0.w; o[5] = r1.y;

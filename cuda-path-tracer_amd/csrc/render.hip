@@ -47,6 +47,7 @@ struct FrameConst {
     const uint32_t* texels;            // RGBA8 texels of all textures
     const uint4* texinfo;              // per texture: first texel, width, height, 0
     uint32_t* status;                  // the scene's status word (PT_STATUS_* flags)
+    const uint32_t* words;             // child word of each internal node (of a scene's root: words[off])
 };
 
 // Structure-of-arrays queue of rays (origin, direction, path index).
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(kThreads) void k_generate(const FrameConst fc,
 
 // Closest hit for every ray of queue `level` (count on the device): the
 // persistent traversal, rays handed out from the level's ray queue block.
-// Each path traces the scene of its pass (root internal node off[scene]).
+// Each path traces the scene of its pass (root node: word fc.words[off[scene]]).
 template <int LDS>
 __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
                                                             const PassParams* __restrict__ pp,
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
         d = v3(q.dx[i], q.dy[i], q.dz[i]);
         const uint32_t sc = pp[min(q.path[i] / fc.npix, fc.npasses - 1u)].scene;
         const uint32_t b = off[sc], e = off[sc + 1];
-        if (e - b >= 2) return b;
+        if (e - b >= 2) return fc.words[b];
         if (e - b == 1) single = b;
         return kInvalid;
     };
@@ -214,10 +215,11 @@ __device__ __forceinline__ V3 ld3(const float* p) { return v3(p[0], p[1], p[2]);
 // answers the same question and stops at its first hit.
 template <bool LDSS = false>
 __device__ __forceinline__ V3 light_L(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                      uint32_t b, uint32_t e, V3 pos, const pt_dir_light& lt, uint32_t* status,
+                                      const uint32_t* __restrict__ words, uint32_t b, uint32_t e, V3 pos,
+                                      const pt_dir_light& lt, uint32_t* status,
                                       const ShadowStack& ss = ShadowStack{}) {
     const V3 ld = ld3(lt.direction);
-    if (any_hit_in<LDSS>(nodes, tris, b, e, sub(pos, scale(ld, 1e-3f)), neg(ld), status, ss))
+    if (any_hit_in<LDSS>(nodes, tris, words, b, e, sub(pos, scale(ld, 1e-3f)), neg(ld), status, ss))
         return v3(0.0f, 0.0f, 0.0f);
     return scale(ld3(lt.color), lt.intensity);
 }
@@ -327,7 +329,7 @@ __device__ __forceinline__ void bounce_hit(HitShade& hs, V3 d, const FrameConst&
     } else if (LIGHTS) {
         for (uint32_t k = 0; k < fc.nlights; ++k) {
             const V3 ld = ld3(lights[k].direction);
-            L = add(L, scale(light_L<LDSS>(nodes, tris, sb, se, hs.pos, lights[k], fc.status, ss),
+            L = add(L, scale(light_L<LDSS>(nodes, tris, fc.words, sb, se, hs.pos, lights[k], fc.status, ss),
                              gmax(dot(neg(ld), hs.nrm), 0.0f)));
         }
     }
@@ -384,7 +386,7 @@ __device__ __forceinline__ void primary_hit(HitShade& hs, V3 d, const FrameConst
         V3 Lc = v3(0.0f, 0.0f, 0.0f);
         for (uint32_t k = 0; k < fc.nlights; ++k) {
             const V3 ld = ld3(lights[k].direction);
-            Lc = add(Lc, light_L<LDSS>(nodes, tris, sb, se, hs.pos, lights[k], fc.status, ss));
+            Lc = add(Lc, light_L<LDSS>(nodes, tris, fc.words, sb, se, hs.pos, lights[k], fc.status, ss));
             const V3 hw = scale(sub(neg(d), ld), 0.5f);
             acc = add(acc, blinn_phong(Lc, hs.albedo, Lc, v3(0.5f, 0.5f, 0.5f), hs.nrm, neg(ld), hw, hs.spec));
         }
@@ -580,6 +582,12 @@ struct Handout {
 // per workgroup in LDS and added to counters[b] at the end.
 enum : uint32_t { kLaneIdle = 0u, kLaneTrace = 1u, kLaneShade = 2u };
 
+// Groups whose segments have ended shade together once they are at least one
+// in kGroupShade of the wave's groups (1, 2, 4, 8: 5.98, 5.73, 5.73, 5.80 ms
+// for two 1,024 x 1,024 room frames, 2.04, 2.11, 2.09, 2.15 for eight 256 x 256
+// soup frames).
+constexpr uint32_t kGroupShade = 4;
+
 __global__ __launch_bounds__(64) void k_paths_setup(uint32_t* __restrict__ counters, uint32_t* __restrict__ queue,
                                                     uint32_t nlevels) {
     for (uint32_t k = threadIdx.x; k <= nlevels && k < kTrainLevel0Slot; k += blockDim.x) counters[k] = 0u;
@@ -590,16 +598,54 @@ __global__ __launch_bounds__(64) void k_paths_setup(uint32_t* __restrict__ count
     zero_queue(queue, 1u);
 }
 
-// At most 80 VGPRs (6 waves per SIMD): the plain variant fits without
-// spilling, the surface-detail variants too (109 VGPRs uncapped), and the lit
-// variants spill a little in their shading, which costs no more than the
-// waves it buys.
+// Path `slot` (in first-level order) at its primary ray: r.o, r.d, its path
+// index (pass * npix + pixel) and its scene's root word (kInvalid: a scene of
+// fewer than two triangles).
+__device__ __forceinline__ uint32_t start_path(const FrameConst& fc, const PassParams* __restrict__ pp,
+                                               const uint32_t* __restrict__ off, uint32_t slot, RayState& r,
+                                               uint32_t& root) {
+    const uint32_t w = static_cast<uint32_t>(fc.w), h = static_cast<uint32_t>(fc.h);
+    const uint32_t pass = slot / fc.npix;
+    const uint32_t pix = tiled_pixel(slot - pass * fc.npix, w, h);
+    const PassParams& P = pp[pass];
+    const float tx = static_cast<float>(pix % w) / static_cast<float>(fc.w);
+    const float ty = static_cast<float>(pix / w) / static_cast<float>(fc.h);
+    const V3 d00 = v3(P.dirs[0], P.dirs[1], P.dirs[2]);
+    const V3 d10 = v3(P.dirs[3], P.dirs[4], P.dirs[5]);
+    const V3 d11 = v3(P.dirs[6], P.dirs[7], P.dirs[8]);
+    const V3 d01 = v3(P.dirs[9], P.dirs[10], P.dirs[11]);
+    r.o = v3(P.eye[0], P.eye[1], P.eye[2]);
+    r.d = mix(mix(d00, d10, tx), mix(d01, d11, tx), ty);
+    const uint32_t sb = off[P.scene], se = off[P.scene + 1];
+    root = se - sb >= 2 ? fc.words[sb] : kInvalid;
+    return pass * fc.npix + pix;
+}
+
+// The closest hit of a path's segment in a scene of fewer than two triangles.
+__device__ __forceinline__ void answer_single(const FrameConst& fc, const PassParams* __restrict__ pp,
+                                              const uint32_t* __restrict__ off, const float4* __restrict__ tris,
+                                              uint32_t path, RayState& r) {
+    TraceCount cnt{0, 0, 0, 0};
+    const uint32_t sc = pp[path / fc.npix].scene;
+    const TraceHit h = trace_single<false>(tris, off[sc + 1] - off[sc] == 1u ? off[sc] : kInvalid, r.o, r.d, cnt);
+    r.minT = h.t; r.best = h.id; r.bu = h.u; r.bv = h.v;
+}
+
+// At most 96 VGPRs (5 waves per SIMD): the plain and the cache variants fit
+// without spilling.  At 80 (6 waves) they spill inside the visit, and a
+// 1,024 x 1,024 frame of the 871,200-triangle room took 7.2 ms for 2.9; at 4
+// waves it took the same as at 5.
 // CACHE: the pixel paths of a cache frame (one pass, pixel = path), each
 // ending in the cache at its second hit (record_cache_vertex) with its
 // throughput in ps.ar/ag/ab -- the same values the levels k_extend /
 // k_shade<true> leave.
+// lg0 > 0: a frame of few paths, 2^lg0 lanes per path from the start (the
+// grid holds every path; no queue).  Otherwise one lane per path, and once the
+// queue has run dry and kTailLanes paths or fewer are left in a wave, those
+// go on as groups: a frame lasts as long as its longest path's chain of
+// visits, which the groups shorten (traverse.hpp).
 template <int LDS, bool LIGHTS, bool DETAIL, bool CACHE>
-__global__ __launch_bounds__(kPersistThreads, 6) void k_paths(const FrameConst fc, const PassParams* __restrict__ pp,
+__global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst fc, const PassParams* __restrict__ pp,
                                                            const pt_triangle_info* __restrict__ infos,
                                                            const float4* __restrict__ nodes,
                                                            const float4* __restrict__ tris,
@@ -607,13 +653,12 @@ __global__ __launch_bounds__(kPersistThreads, 6) void k_paths(const FrameConst f
                                                            const pt_dir_light* __restrict__ lights, PathState ps,
                                                            uint32_t* __restrict__ counters,
                                                            uint32_t* __restrict__ queue, uint32_t refill,
-                                                           uint32_t pool_large, uint32_t shade_min, CacheIO io) {
+                                                           uint32_t pool_large, uint32_t shade_min, uint32_t lg0,
+                                                           CacheIO io) {
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
     __shared__ uint32_t s_level[kMaxLevels];
     // Plain frames keep each lane's path throughput and radiance in LDS
-    // while it traverses: the registers saved take the kernel to 6 waves per
-    // SIMD.  (With lights or surface detail the kernel stays at 4 waves per
-    // SIMD either way, and the LDS round trips only cost.)
+    // while it traverses alone.
     constexpr bool kCarryLds = !LIGHTS && !DETAIL;
     __shared__ float s_carry[kCarryLds ? 6 : 1][kPersistThreads];
     for (uint32_t k = threadIdx.x; k < kMaxLevels; k += blockDim.x) s_level[k] = 0u;
@@ -621,20 +666,87 @@ __global__ __launch_bounds__(kPersistThreads, 6) void k_paths(const FrameConst f
     const uint32_t npaths = fc.npix * fc.npasses;
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     const int lane = threadIdx.x & 63;
-    // Waves past one per kRayPoolSmall paths skip the loop (but reach the
-    // final barrier).
-    if (wave_id == 0u || static_cast<uint64_t>(wave_id) * kRayPoolSmall < npaths) {
-        uint32_t spill[kStackMax - LDS];
+    uint32_t spill[kStackMax - LDS];
+    keep_in_memory(spill);
+    RayState r;
+    r.o = r.d = r.dinv = v3(0.0f, 0.0f, 0.0f);
+    r.minT = kMinTInit;
+    r.best = kInvalid;
+    r.bu = r.bv = 0.0f;
+    r.word = 0u;
+    r.sp = 0;
+    r.finite = true;
+    uint32_t path = 0, bounce = 0;  // the path's pass and pixel follow from its index
+    uint32_t root = kInvalid;
+    V3 absorbed_r = v3(1.0f, 1.0f, 1.0f), acc_r = v3(0.0f, 0.0f, 0.0f);
+    const int tid = threadIdx.x;
+
+    // The end of a segment: shade its hit and sample the next segment (r.o,
+    // r.d; true), or end the path (false).  `lead`: this lane writes for the
+    // path.  Shadow rays keep their deferred nodes in this lane's (empty)
+    // column of the stack.
+    auto shade = [&](V3& absorbed, V3& acc, bool lead) -> bool {
+        if (lead) atomicAdd(&s_level[bounce], 1u);  // this segment, now complete
+        bool cont = false;
+        if (r.best != kInvalid) {
+            const uint32_t pass = path / fc.npix;
+            const uint32_t pix = path - pass * fc.npix;
+            const PassParams& P = pp[pass];
+            HitShade hs = hit_shade<DETAIL>(fc, infos, r.best, r.minT, r.bu, r.bv, r.o, r.d);
+            const uint32_t sb = off[P.scene], se = off[P.scene + 1];
+            ShadowStack ss;
+            ss.lds = &s_stack[0][threadIdx.x];
+            ss.stride = kPersistThreads;
+            ss.depth = LDS;
+            ss.spill = spill;
+            if (bounce == 0) {
+                primary_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, sb, se, absorbed, acc, ss);
+            } else {
+                bounce_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, sb, se, absorbed, acc, ss);
+            }
+            if (CACHE && bounce == 1 && lead) record_cache_vertex(io, false, pix, path, hs, r.d, absorbed, acc);
+            V3 no{0.0f, 0.0f, 0.0f}, nd{0.0f, 0.0f, 0.0f};
+            const uint32_t limit = CACHE ? 1u : fc.bounces;
+            if (bounce < limit) cont = next_bounce(pix, P.pass, bounce, P.seedw, fc, hs, absorbed, no, nd);
+            if (cont) {
+                ++bounce;
+                r.o = no;
+                r.d = nd;
+            }
+        }
+        if (!cont && lead) {
+            ps.cr[path] = acc.x;
+            ps.cg[path] = acc.y;
+            ps.cb[path] = acc.z;
+            if constexpr (CACHE) {  // the weight of the cache's answer (k_cache_resolve)
+                ps.ar[path] = absorbed.x;
+                ps.ag[path] = absorbed.y;
+                ps.ab[path] = absorbed.z;
+            }
+        }
+        return cont;
+    };
+
+    // What is left to the groups: which lanes hold a path, the groups' stack
+    // sizes (0: a segment that has ended) and lanes per path (log2).
+    bool active = false;
+    uint32_t gsp = 0u, lg = lg0;
+    V3 absorbed = v3(1.0f, 1.0f, 1.0f), acc = v3(0.0f, 0.0f, 0.0f);
+
+    if (lg0 > 0u) {
+        const uint32_t slot = (blockIdx.x * kPersistThreads + threadIdx.x) >> lg0;
+        if (slot < npaths) {
+            path = start_path(fc, pp, off, slot, r, root);
+            active = true;
+            if (root != kInvalid) group_start<LDS>(r, root, gsp, lg, s_stack);
+            else answer_single(fc, pp, off, tris, path, r);
+        }
+    } else if (wave_id == 0u || static_cast<uint64_t>(wave_id) * kRayPoolSmall < npaths) {
+        // (Waves past one per kRayPoolSmall paths have nothing to do.)
         TraceCount cnt{0, 0, 0, 0};
         Handout ho;
         ho.init(queue, npaths, npaths / 4u >= gridDim.x * blockDim.x ? pool_large : kRayPoolSmall, wave_id);
-        RayState r;
         uint32_t state = kLaneIdle;
-        uint32_t path = 0, bounce = 0;  // the path's pass and pixel follow from its index
-        uint32_t root = kInvalid;
-        V3 absorbed_r = v3(1.0f, 1.0f, 1.0f), acc_r = v3(0.0f, 0.0f, 0.0f);
-        const int tid = threadIdx.x;
-        const uint32_t w = static_cast<uint32_t>(fc.w), h = static_cast<uint32_t>(fc.h);
         for (;;) {
             // New paths for idle lanes.
             uint64_t busy = __ballot(state != kLaneIdle);
@@ -649,21 +761,7 @@ __global__ __launch_bounds__(kPersistThreads, 6) void k_paths(const FrameConst f
                     const bool take = ((idle >> lane) & 1ull) && rank < avail;
                     const uint32_t took = min(static_cast<uint32_t>(__popcll(idle)), avail);
                     if (take) {
-                        const uint32_t slot = ho.next + rank;
-                        const uint32_t pass = slot / fc.npix;
-                        const uint32_t pix = tiled_pixel(slot - pass * fc.npix, w, h);
-                        path = pass * fc.npix + pix;
-                        const PassParams& P = pp[pass];
-                        const float tx = static_cast<float>(pix % w) / static_cast<float>(fc.w);
-                        const float ty = static_cast<float>(pix / w) / static_cast<float>(fc.h);
-                        const V3 d00 = v3(P.dirs[0], P.dirs[1], P.dirs[2]);
-                        const V3 d10 = v3(P.dirs[3], P.dirs[4], P.dirs[5]);
-                        const V3 d11 = v3(P.dirs[6], P.dirs[7], P.dirs[8]);
-                        const V3 d01 = v3(P.dirs[9], P.dirs[10], P.dirs[11]);
-                        r.o = v3(P.eye[0], P.eye[1], P.eye[2]);
-                        r.d = mix(mix(d00, d10, tx), mix(d01, d11, tx), ty);
-                        const uint32_t sb = off[P.scene], se = off[P.scene + 1];
-                        root = se - sb >= 2 ? sb : kInvalid;
+                        path = start_path(fc, pp, off, ho.next + rank, r, root);
                         bounce = 0;
                         if constexpr (kCarryLds) {
                             s_carry[0][tid] = 1.0f; s_carry[1][tid] = 1.0f; s_carry[2][tid] = 1.0f;
@@ -680,26 +778,28 @@ __global__ __launch_bounds__(kPersistThreads, 6) void k_paths(const FrameConst f
                 }
             }
             busy = __ballot(state != kLaneIdle);
-            if (busy == 0ull && ho.drained) break;
-            // Count the segments that start this iteration (bounce of each).
-            // (Counted when a lane enters kLaneTrace: at take and at continue.)
+            if (ho.drained) {
+                if (busy == 0ull) break;
+                // The last paths go on as groups, all deferred nodes in LDS.
+                if (static_cast<uint32_t>(__popcll(busy)) <= kTailLanes &&
+                    __ballot(state == kLaneTrace && r.sp >= LDS) == 0ull) {
+                    active = state != kLaneIdle;
+                    if (state == kLaneTrace) {
+                        if (root == kInvalid) {
+                            answer_single(fc, pp, off, tris, path, r);
+                        } else {
+                            s_stack[r.sp][tid] = r.word;
+                            gsp = static_cast<uint32_t>(r.sp) + 1u;
+                        }
+                    }
+                    break;
+                }
+            }
             // One node visit for every traversing lane; a scene with fewer
             // than two triangles answers at once.
             if (state == kLaneTrace) {
                 if (root == kInvalid) {
-                    r.minT = kMinTInit;
-                    r.best = kInvalid;
-                    // A scene of fewer than two triangles: its one triangle, if any.
-                    const uint32_t psc = pp[path / fc.npix].scene;
-                    const uint32_t single = off[psc + 1] - off[psc] == 1u ? off[psc] : kInvalid;
-                    if (single != kInvalid) {
-                        float u = 0.0f, v = 0.0f;
-                        uint32_t id;
-                        const float t = tri_hit(tris, single, r.o, r.d, u, v, id);
-                        if (t <= kMinTInit) {
-                            r.minT = t; r.best = id; r.bu = u; r.bv = v;
-                        }
-                    }
+                    answer_single(fc, pp, off, tris, path, r);
                     state = kLaneShade;
                 } else if (!(r.finite ? visit_step<false, LDS, true>(nodes, tris, r, s_stack, spill, cnt, fc.status)
                                       : visit_step<false, LDS, false>(nodes, tris, r, s_stack, spill, cnt, fc.status))) {
@@ -710,61 +810,61 @@ __global__ __launch_bounds__(kPersistThreads, 6) void k_paths(const FrameConst f
             const uint64_t tracing = __ballot(state == kLaneTrace);
             if (shading != 0ull && (static_cast<uint32_t>(__popcll(shading)) >= shade_min || tracing == 0ull)) {
                 if (state == kLaneShade) {
-                    atomicAdd(&s_level[bounce], 1u);  // this segment, now complete
-                    bool cont = false;
-                    V3 absorbed = absorbed_r, acc = acc_r;
+                    V3 ab = absorbed_r, ac = acc_r;
                     if constexpr (kCarryLds) {
-                        absorbed = v3(s_carry[0][tid], s_carry[1][tid], s_carry[2][tid]);
-                        acc = v3(s_carry[3][tid], s_carry[4][tid], s_carry[5][tid]);
+                        ab = v3(s_carry[0][tid], s_carry[1][tid], s_carry[2][tid]);
+                        ac = v3(s_carry[3][tid], s_carry[4][tid], s_carry[5][tid]);
                     }
-                    if (r.best != kInvalid) {
-                        const uint32_t pass = path / fc.npix;
-                        const uint32_t pix = path - pass * fc.npix;
-                        const PassParams& P = pp[pass];
-                        HitShade hs = hit_shade<DETAIL>(fc, infos, r.best, r.minT, r.bu, r.bv, r.o, r.d);
-                        const uint32_t sb = off[P.scene], se = off[P.scene + 1];
-                        // Shadow rays keep their deferred nodes in this lane's
-                        // (now empty) traversal stack.
-                        ShadowStack ss;
-                        ss.lds = &s_stack[0][threadIdx.x];
-                        ss.stride = kPersistThreads;
-                        ss.depth = LDS;
-                        ss.spill = spill;
-                        if (bounce == 0) {
-                            primary_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, sb, se, absorbed, acc, ss);
+                    if (shade(ab, ac, true)) {
+                        init_ray(r, root);
+                        state = kLaneTrace;
+                        if constexpr (kCarryLds) {
+                            s_carry[0][tid] = ab.x; s_carry[1][tid] = ab.y; s_carry[2][tid] = ab.z;
+                            s_carry[3][tid] = ac.x; s_carry[4][tid] = ac.y; s_carry[5][tid] = ac.z;
                         } else {
-                            bounce_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, sb, se, absorbed, acc, ss);
+                            absorbed_r = ab;
+                            acc_r = ac;
                         }
-                        if (CACHE && bounce == 1) record_cache_vertex(io, false, pix, path, hs, r.d, absorbed, acc);
-                        V3 no{0.0f, 0.0f, 0.0f}, nd{0.0f, 0.0f, 0.0f};
-                        const uint32_t limit = CACHE ? 1u : fc.bounces;
-                        if (bounce < limit) cont = next_bounce(pix, P.pass, bounce, P.seedw, fc, hs, absorbed, no, nd);
-                        if (cont) {
-                            ++bounce;
-                            r.o = no;
-                            r.d = nd;
-                            init_ray(r, root);
-                            state = kLaneTrace;
-                            if constexpr (kCarryLds) {
-                                s_carry[0][tid] = absorbed.x; s_carry[1][tid] = absorbed.y; s_carry[2][tid] = absorbed.z;
-                                s_carry[3][tid] = acc.x; s_carry[4][tid] = acc.y; s_carry[5][tid] = acc.z;
-                            } else {
-                                absorbed_r = absorbed;
-                                acc_r = acc;
-                            }
-                        }
-                    }
-                    if (!cont) {
-                        ps.cr[path] = acc.x;
-                        ps.cg[path] = acc.y;
-                        ps.cb[path] = acc.z;
-                        if constexpr (CACHE) {  // the weight of the cache's answer (k_cache_resolve)
-                            ps.ar[path] = absorbed.x;
-                            ps.ag[path] = absorbed.y;
-                            ps.ab[path] = absorbed.z;
-                        }
+                    } else {
                         state = kLaneIdle;
                     }
+                }
+            }
+        }
+        absorbed = absorbed_r;
+        acc = acc_r;
+        if constexpr (kCarryLds) {
+            absorbed = v3(s_carry[0][tid], s_carry[1][tid], s_carry[2][tid]);
+            acc = v3(s_carry[3][tid], s_carry[4][tid], s_carry[5][tid]);
+        }
+    }
+
+    // Groups: rounds until every path has ended.
+    for (;;) {
+        const uint64_t act = __ballot(active && (lane & ((1 << lg) - 1)) == 0);
+        if (act == 0ull) break;
+        const uint32_t lgn = group_log(static_cast<uint32_t>(__popcll(act)));
+        if (lgn > lg && __ballot(active && gsp > (static_cast<uint32_t>(LDS) << lg)) == 0ull) {
+            const uint32_t own = regroup<LDS>(r, gsp, lg, lgn, act, s_stack);
+            const uint32_t src = own & 63u;
+            path = lane_u32(path, src);
+            bounce = lane_u32(bounce, src);
+            root = lane_u32(root, src);
+            absorbed = lane_v3(absorbed, src);
+            acc = lane_v3(acc, src);
+            active = own < 64u;
+        }
+        group_round<LDS>(nodes, tris, r, gsp, lg, s_stack, spill, fc.status);
+        const uint64_t ended = __ballot(active && gsp == 0u);
+        if (ended != 0ull &&
+            (static_cast<uint32_t>(__popcll(ended)) * kGroupShade >= static_cast<uint32_t>(__popcll(__ballot(active))))) {
+            group_best(r, lg);
+            if (active && gsp == 0u) {
+                const bool lead = (lane & ((1 << lg) - 1)) == 0;
+                active = shade(absorbed, acc, lead);
+                if (active) {
+                    if (root != kInvalid) group_start<LDS>(r, root, gsp, lg, s_stack);
+                    else answer_single(fc, pp, off, tris, path, r);
                 }
             }
         }
@@ -797,6 +897,7 @@ __global__ __launch_bounds__(kSuffixThreads) void k_train_paths(const FrameConst
                                                                 const uint32_t* __restrict__ off) {
     __shared__ uint32_t s_tstack[kTrainLds][kSuffixThreads];
     uint32_t spill[kStackMax - kTrainLds];
+    keep_in_memory(spill);
     const PassParams& P = pp[0];
     const uint32_t seedw = P.seedw ^ kTrainSalt;
     const uint32_t sb = off[P.scene], se = off[P.scene + 1];
@@ -809,8 +910,9 @@ __global__ __launch_bounds__(kSuffixThreads) void k_train_paths(const FrameConst
         atomicAdd(counters + kTrainLevel0Slot, 1u);
         for (uint32_t b = 0;; ++b) {
             TraceHit h;
+            TraceCount cnt{0, 0, 0, 0};
             if (se - sb < 2) {
-                h = trace_ray_in(nodes, tris, sb, se, o, d, fc.status);
+                h = trace_single<false>(tris, se - sb == 1 ? sb : kInvalid, o, d, cnt);
             } else {
                 // The reference-order walk with its first kTrainLds deferred
                 // nodes in LDS (a lone wave per SIMD waits out every stack
@@ -818,8 +920,7 @@ __global__ __launch_bounds__(kSuffixThreads) void k_train_paths(const FrameConst
                 RayState r;
                 r.o = o;
                 r.d = d;
-                init_ray(r, sb);
-                TraceCount cnt{0, 0, 0, 0};
+                init_ray(r, fc.words[sb]);
                 if (r.finite) {
                     while (visit_step<false, kTrainLds, true>(nodes, tris, r, s_tstack, spill, cnt, fc.status)) {
                     }
@@ -1098,14 +1199,15 @@ void launch_frame(Renderer& r, const DeviceScene& scene, const FrameConst& fc, u
     const uint32_t refill = std::min(64u, std::max(1u, tune.refill));
     if (nchains == 0) {  // path-persistent frame
         hipLaunchKernelGGL(k_paths_setup, dim3(1), dim3(64), 0, st, cnt, cnt + 64, nlev);
-        const uint32_t pgrid = std::min(std::max(1u, tune.blocks), grid);
+        const uint32_t lg = launch_group(npaths, static_cast<uint64_t>(std::max(1u, tune.blocks)) * kPersistThreads);
+        const uint32_t pgrid = lg ? grouped_blocks(npaths, lg) : std::min(std::max(1u, tune.blocks), grid);
         const uint32_t pool = pool_for(tune.pool, static_cast<uint32_t>(npaths), pgrid);
         auto kern = tune.lds <= 8 ? paths_kernel<8>(fc) : paths_kernel<16>(fc);
         hipLaunchKernelGGL(kern, dim3(pgrid), dim3(kPersistThreads), 0, st, fc, pp,
                            scene.infos.as<pt_triangle_info>(), scene.bvh.nodes.as<float4>(),
                            scene.bvh.tris.as<float4>(), scene.off.as<uint32_t>(), scene.lights.as<pt_dir_light>(),
                            L.ps, cnt, cnt + 64, refill, pool,
-                           std::min(64u, std::max(1u, render_tuning().shade_min)), CacheIO{});
+                           std::min(64u, std::max(1u, render_tuning().shade_min)), lg, CacheIO{});
         hipLaunchKernelGGL(k_accumulate, dim3(grid_for(fc.npix)), dim3(kThreads), 0, st, fc, L.ps,
                            r.accum.as<double>());
         return;
@@ -1305,6 +1407,7 @@ void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, cons
     fc.stratified = r.settings.stratified;
     fc.nlights = scene.nlights;
     fc.status = scene.status.as<uint32_t>();
+    fc.words = scene.bvh.children.as<uint32_t>();
     set_detail(fc, scene);
 
     const uint32_t nchains = frame_chains(npix * npasses);
@@ -1392,13 +1495,14 @@ void launch_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
     if (paths) {
         // The pixel paths in one path-persistent launch (render.paths), each
         // lane carrying a path from its primary ray to the cache.
-        const uint32_t ppgrid = std::min(std::max(1u, tune.blocks), grid_for(fc.npix));
+        const uint32_t lg = launch_group(fc.npix, static_cast<uint64_t>(std::max(1u, tune.blocks)) * kPersistThreads);
+        const uint32_t ppgrid = lg ? grouped_blocks(fc.npix, lg) : std::min(std::max(1u, tune.blocks), grid_for(fc.npix));
         const uint32_t ppool = pool_for(tune.pool, fc.npix, ppgrid);
         auto kern = tune.lds <= 8 ? cache_paths_kernel<8>(fc) : cache_paths_kernel<16>(fc);
         hipLaunchKernelGGL(kern, dim3(ppgrid), dim3(kPersistThreads), 0, st, fc, pp,
                            scene.infos.as<pt_triangle_info>(), scene.bvh.nodes.as<float4>(),
                            scene.bvh.tris.as<float4>(), scene.off.as<uint32_t>(), scene.lights.as<pt_dir_light>(),
-                           L.ps, cnt, rcnt, refill, ppool, std::min(64u, std::max(1u, render_tuning().shade_min)),
+                           L.ps, cnt, rcnt, refill, ppool, std::min(64u, std::max(1u, render_tuning().shade_min)), lg,
                            io);
     } else {
         // Levels 0 and 1 of the pixel paths (a pixel path ends in the cache at x2).
@@ -1465,6 +1569,7 @@ void render_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
     cf.fc.stratified = r.settings.stratified;
     cf.fc.nlights = scene.nlights;
     cf.fc.status = scene.status.as<uint32_t>();
+    cf.fc.words = scene.bvh.children.as<uint32_t>();
     set_detail(cf.fc, scene);
     cf.steps = cs.train_steps;
     cf.train = (cs.flags & PT_CACHE_TRAIN) != 0;

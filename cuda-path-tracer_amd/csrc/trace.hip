@@ -41,19 +41,17 @@ __device__ __forceinline__ void add_counts(const TraceCount& cnt, unsigned long 
     }
 }
 
+// Closest hit in a scene of at most one triangle (no internal node).
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceThreads) void k_trace(
-    const float4* __restrict__ nodes, const float4* __restrict__ tris, uint32_t ntri,
-    const float* __restrict__ rays, uint32_t nrays, uint32_t* __restrict__ out_id,
-    float* __restrict__ out_t, float2* __restrict__ out_uv,
-    unsigned long long* __restrict__ counters, uint32_t* __restrict__ status) {
+__global__ __launch_bounds__(kTraceThreads) void k_trace_single(
+    const float4* __restrict__ tris, uint32_t ntri, const float* __restrict__ rays, uint32_t nrays,
+    uint32_t* __restrict__ out_id, float* __restrict__ out_t, float2* __restrict__ out_uv,
+    unsigned long long* __restrict__ counters) {
     TraceCount cnt{0, 0, 0, 0};
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nrays; i += stride) {
         const float* r = rays + 6 * static_cast<size_t>(i);
-        const V3 o = v3(r[0], r[1], r[2]);
-        const V3 d = v3(r[3], r[4], r[5]);
-        const TraceHit h = trace_ray<COUNT>(nodes, tris, ntri, o, d, cnt, status);
+        const TraceHit h = trace_single<COUNT>(tris, ntri ? 0u : kInvalid, v3(r[0], r[1], r[2]), v3(r[3], r[4], r[5]), cnt);
         if (out_id) out_id[i] = h.id;
         if (out_t) out_t[i] = h.t;
         if (out_uv) out_uv[i] = make_float2(h.u, h.v);
@@ -65,17 +63,18 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace(
 // the root filter (persistent_trace_filtered), without counting.
 template <bool COUNT, int LDS, bool FILTER>
 __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
-    const float4* __restrict__ nodes, const float4* __restrict__ tris, const float* __restrict__ rays,
-    uint32_t nrays, uint32_t* __restrict__ out_id, float* __restrict__ out_t,
+    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ words,
+    const float* __restrict__ rays, uint32_t nrays, uint32_t* __restrict__ out_id, float* __restrict__ out_t,
     float2* __restrict__ out_uv, uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool,
     unsigned long long* __restrict__ counters, uint32_t* __restrict__ status) {
     static_assert(!(COUNT && FILTER), "the filter's repeated root visit would change the visit counts");
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
+    const uint32_t root = words[0];
     auto load = [&](uint32_t i, V3& o, V3& d, uint32_t&) -> uint32_t {
         const float* rp = rays + 6 * static_cast<size_t>(i);
         o = v3(rp[0], rp[1], rp[2]);
         d = v3(rp[3], rp[4], rp[5]);
-        return 0u;
+        return root;
     };
     auto store = [&](uint32_t i, const TraceHit& h) {
         if (out_id) out_id[i] = h.id;
@@ -95,11 +94,11 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
 }
 
 // Persistent closest hit over rays tagged with a scene of a batch: the ray
-// starts at its scene's root (internal node off[s]).
+// starts at its scene's root (internal node off[s], word words[off[s]]).
 template <int LDS>
 __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
-    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ off,
-    uint32_t nscenes, const float* __restrict__ rays, const uint32_t* __restrict__ scene, uint32_t nrays,
+    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ words,
+    const uint32_t* __restrict__ off, uint32_t nscenes, const float* __restrict__ rays, const uint32_t* __restrict__ scene, uint32_t nrays,
     uint32_t* __restrict__ out_id, float* __restrict__ out_t, float2* __restrict__ out_uv,
     uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool, uint32_t* __restrict__ status) {
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
@@ -113,7 +112,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
             const uint32_t sc = scene[i];
             if (sc >= nscenes) return kInvalid;  // unknown scene: a miss
             const uint32_t b = off[sc], e = off[sc + 1];
-            if (e - b >= 2) return b;
+            if (e - b >= 2) return words[b];
             if (e - b == 1) single = b;
             return kInvalid;
         },
@@ -123,6 +122,53 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
             if (out_uv) out_uv[i] = make_float2(h.u, h.v);
         },
         cnt);
+}
+
+// A launch of few rays: 2^lg lanes per ray from the start (grouped_trace), no
+// queue.  SCENES: rays tagged with a scene of a batch.
+template <int LDS, bool SCENES>
+__global__ __launch_bounds__(kPersistThreads) void k_trace_grouped(
+    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ words,
+    const uint32_t* __restrict__ off, uint32_t nscenes, const float* __restrict__ rays,
+    const uint32_t* __restrict__ scene, uint32_t nrays, uint32_t lg, uint32_t* __restrict__ out_id,
+    float* __restrict__ out_t, float2* __restrict__ out_uv, uint32_t* __restrict__ status) {
+    __shared__ uint32_t s_stack[LDS][kPersistThreads];
+    grouped_trace<LDS>(
+        nodes, tris, nrays, lg, status, s_stack,
+        [&](uint32_t i, V3& o, V3& d, uint32_t& single) -> uint32_t {
+            const float* rp = rays + 6 * static_cast<size_t>(i);
+            o = v3(rp[0], rp[1], rp[2]);
+            d = v3(rp[3], rp[4], rp[5]);
+            if (!SCENES) return words[0];
+            const uint32_t sc = scene[i];
+            if (sc >= nscenes) return kInvalid;  // unknown scene: a miss
+            const uint32_t b = off[sc], e = off[sc + 1];
+            if (e - b >= 2) return words[b];
+            if (e - b == 1) single = b;
+            return kInvalid;
+        },
+        [&](uint32_t i, const TraceHit& h) {
+            if (out_id) out_id[i] = h.id;
+            if (out_t) out_t[i] = h.t;
+            if (out_uv) out_uv[i] = make_float2(h.u, h.v);
+        });
+}
+
+// Whether a launch of n rays runs grouped, and with how many lanes per ray
+// (log2); scene ids may be null (one scene of at least two triangles).
+uint32_t launch_grouped(const DeviceScene& s, const float* d_rays, const uint32_t* d_scene, uint32_t n, uint32_t* d_id,
+                        float* d_t, float* d_uv, hipStream_t st) {
+    const TraceTuning& tune = trace_tuning();
+    const uint32_t lg = launch_group(n, static_cast<uint64_t>(tune.blocks) * kPersistThreads);
+    if (lg == 0) return 0;
+    const uint32_t blocks = grouped_blocks(n, lg);
+    auto kern = d_scene ? (tune.lds <= 8 ? k_trace_grouped<8, true> : k_trace_grouped<16, true>)
+                        : (tune.lds <= 8 ? k_trace_grouped<8, false> : k_trace_grouped<16, false>);
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st, s.bvh.nodes.as<float4>(),
+                       s.bvh.tris.as<float4>(), s.bvh.children.as<uint32_t>(), s.off.as<uint32_t>(), s.nscenes(),
+                       d_rays, d_scene, n, lg, d_id, d_t, reinterpret_cast<float2*>(d_uv), s.status.as<uint32_t>());
+    PT_HIP(hipGetLastError());
+    return lg;
 }
 
 __global__ __launch_bounds__(64) void k_zero_queue(uint32_t* queue) { zero_queue(queue, 1u); }
@@ -135,12 +181,13 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
     if (s.bvh.n < 2) {
         const uint32_t blocks = static_cast<uint32_t>((static_cast<uint64_t>(n) + kTraceThreads - 1) /
                                                       kTraceThreads);
-        hipLaunchKernelGGL(k_trace<COUNT>, dim3(blocks), dim3(kTraceThreads), 0, st,
-                           s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.n, d_rays, n,
-                           d_id, d_t, reinterpret_cast<float2*>(d_uv), d_counters, status);
+        hipLaunchKernelGGL(k_trace_single<COUNT>, dim3(blocks), dim3(kTraceThreads), 0, st,
+                           s.bvh.tris.as<float4>(), s.bvh.n, d_rays, n, d_id, d_t,
+                           reinterpret_cast<float2*>(d_uv), d_counters);
         PT_HIP(hipGetLastError());
         return;
     }
+    if (!COUNT && launch_grouped(s, d_rays, nullptr, n, d_id, d_t, d_uv, st)) return;
     const TraceTuning& tune = trace_tuning();
     hipLaunchKernelGGL(k_zero_queue, dim3(1), dim3(64), 0, st, queue);
     const uint64_t want = (static_cast<uint64_t>(n) + kPersistThreads - 1) / kPersistThreads;
@@ -154,7 +201,7 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
                                         : (tune.lds <= 16 ? k_trace_persistent<COUNT, 16, false>
                                                           : k_trace_persistent<COUNT, 32, false>));
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
-                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), d_rays, n, d_id, d_t,
+                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.children.as<uint32_t>(), d_rays, n, d_id, d_t,
                        reinterpret_cast<float2*>(d_uv), queue, std::min(64u, std::max(1u, tune.refill)),
                        pool_for(tune.pool, n, blocks), d_counters, status);
     PT_HIP(hipGetLastError());
@@ -203,6 +250,7 @@ TraceTuning& trace_tuning() {
 void trace_closest_scenes(const DeviceScene& s, uint32_t* queue, const float* d_rays, const uint32_t* d_scene,
                           uint32_t n, uint32_t* d_id, float* d_t, float* d_uv, hipStream_t st) {
     if (n == 0) return;
+    if (launch_grouped(s, d_rays, d_scene, n, d_id, d_t, d_uv, st)) return;
     const TraceTuning& tune = trace_tuning();
     hipLaunchKernelGGL(k_zero_queue, dim3(1), dim3(64), 0, st, queue);
     const uint64_t want = (static_cast<uint64_t>(n) + kPersistThreads - 1) / kPersistThreads;
@@ -210,8 +258,8 @@ void trace_closest_scenes(const DeviceScene& s, uint32_t* queue, const float* d_
         static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(want, tune.blocks)));
     auto kern = tune.lds <= 8 ? k_trace_scenes<8> : (tune.lds <= 16 ? k_trace_scenes<16> : k_trace_scenes<32>);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
-                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.off.as<uint32_t>(),
-                       s.nscenes(), d_rays, d_scene, n, d_id, d_t, reinterpret_cast<float2*>(d_uv),
+                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.children.as<uint32_t>(),
+                       s.off.as<uint32_t>(), s.nscenes(), d_rays, d_scene, n, d_id, d_t, reinterpret_cast<float2*>(d_uv),
                        queue, std::min(64u, std::max(1u, tune.refill)), pool_for(tune.pool, n, blocks),
                        s.status.as<uint32_t>());
     PT_HIP(hipGetLastError());

@@ -4,6 +4,14 @@
 // a stack.  For the lowest-id tie rule the culling keeps children at exactly
 // the best distance, and a triangle replaces the best hit when nearer, or
 // equally near with a lower original id.
+//
+// A node is known by its child word (left child's index << 2 | left internal
+// | right internal << 1) before it is visited: its record sits in slot
+// word >> 2 and carries its children's words beside their boxes, and its leaf
+// children are triangles word >> 2 and (word >> 2) + 1.  So a visit issues
+// the record's loads and its leaf triangles' loads together, and waits for
+// memory once; with the word inside the record it waited for the record, then
+// for the first triangle, then for the second.
 #pragma once
 
 #include <algorithm>
@@ -43,147 +51,35 @@ __device__ __forceinline__ float child_box(V3 o, V3 dinv, float a, float b, floa
     return FINITE ? slab_test_finite(o, dinv, a, b, c, d, e, f) : slab_test(o, dinv, a, b, c, d, e, f);
 }
 
-__device__ __forceinline__ float tri_hit(const float4* __restrict__ tris, uint32_t k, V3 o, V3 d,
-                                         float& u, float& v, uint32_t& id) {
-    float4 a = tris[3 * static_cast<size_t>(k)];
-    const float4 b = tris[3 * static_cast<size_t>(k) + 1];
-    const float4 c = tris[3 * static_cast<size_t>(k) + 2];
-    // Keep p0's load beside the edges' (the compiler would otherwise sink it
-    // below the determinant test, a second memory round trip).
-    asm volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z));
-    id = __float_as_uint(a.w);
-    return mt_test(o, d, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), v3(c.x, c.y, c.z), u, v);
+// A triangle record in registers: p0 with the original id, and the edges.
+struct TriRec {
+    float4 p;
+    V3 e1, e2;
+};
+
+__device__ __forceinline__ TriRec load_tri(const float4* __restrict__ tris, uint32_t k) {
+    const float4* rec = tris + 3 * static_cast<size_t>(k);
+    const float* e1 = reinterpret_cast<const float*>(rec + 1);
+    const float* e2 = reinterpret_cast<const float*>(rec + 2);
+    return TriRec{rec[0], v3(e1[0], e1[1], e1[2]), v3(e2[0], e2[1], e2[2])};
 }
 
-template <bool COUNT, bool FINITE>
-__device__ __forceinline__ TraceHit traverse_impl(const float4* __restrict__ nodes,
-                                                  const float4* __restrict__ tris, V3 o, V3 d,
-                                                  V3 dinv, TraceCount& cnt, uint32_t* status,
-                                                  uint32_t root = 0) {
-    float minT = kMinTInit;
-    uint32_t best = kInvalid;
-    float bu = 0.0f, bv = 0.0f;
-    uint32_t stack[kStackMax];
-    int sp = 0;
-    uint32_t node = root;
-    for (;;) {
-        for (;;) {
-            const float4* rec = nodes + 4 * static_cast<size_t>(node);
-            const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
-            const uint32_t w = __float_as_uint(r3.x);
-            const uint32_t l = w >> 2;
-            const bool in0 = (w & 1u) != 0, in1 = (w & 2u) != 0;
-            float h0, h1, u0 = 0.0f, v0 = 0.0f, u1 = 0.0f, v1 = 0.0f;
-            uint32_t id0 = kInvalid, id1 = kInvalid;
-            if (COUNT) cnt.iters++;
-            // Both child boxes for every lane (a leaf child's value is
-            // discarded), then the leaf children's triangle tests in one loop.
-            h0 = child_box<COUNT, FINITE>(o, dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
-            h1 = child_box<COUNT, FINITE>(o, dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
-            if (COUNT) cnt.boxes += static_cast<uint32_t>(in0) + static_cast<uint32_t>(in1);
-            const uint32_t nleaf = static_cast<uint32_t>(!in0) + static_cast<uint32_t>(!in1);
-            for (uint32_t j = 0; j < nleaf; ++j) {
-                const bool first = j == 0 && !in0;
-                float u, v;
-                uint32_t id;
-                const float h = tri_hit(tris, first ? l : l + 1, o, d, u, v, id);
-                if (COUNT) cnt.tris++;
-                if (first) {
-                    h0 = h; u0 = u; v0 = v; id0 = id;
-                } else {
-                    h1 = h; u1 = u; v1 = v; id1 = id;
-                }
-            }
-            if (!(h0 <= minT) && !(h1 <= minT)) break;
-            const bool sw = h1 < h0;  // left child wins ties (trace.h:125)
-            const float hc = sw ? h1 : h0, hf = sw ? h0 : h1;
-            const uint32_t cc = sw ? l + 1 : l, cf = sw ? l : l + 1;
-            const bool ic = sw ? in1 : in0, jf = sw ? in0 : in1;
-            const float uc = sw ? u1 : u0, vc = sw ? v1 : v0, uf = sw ? u0 : u1, vf = sw ? v0 : v1;
-            const uint32_t idc = sw ? id1 : id0, idf = sw ? id0 : id1;
-            if (ic) {
-                node = cc;
-                if (hf <= minT) {
-                    if (jf) {
-                        if (sp < kStackMax) {
-                            stack[sp++] = cf;
-                            if (COUNT) cnt.depth = max(cnt.depth, static_cast<uint32_t>(sp));
-                        } else {
-                            raise_status(status, kStatusStackOverflow);
-                        }
-                    } else if (hf < minT || idf < best) {
-                        minT = hf; best = idf; bu = uf; bv = vf;
-                    }
-                }
-                continue;
-            }
-            if (hc < minT || idc < best) {
-                minT = hc; best = idc; bu = uc; bv = vc;
-            }
-            if (hf <= minT) {
-                if (jf) {
-                    node = cf;
-                    continue;
-                }
-                if (hf < minT || idf < best) {
-                    minT = hf; best = idf; bu = uf; bv = vf;
-                }
-            }
-            break;
-        }
-        if (sp == 0) break;
-        node = stack[--sp];
-    }
-    TraceHit hit;
-    hit.id = best;
-    hit.t = best == kInvalid ? kFltMax : minT;
-    hit.u = best == kInvalid ? 0.0f : bu;
-    hit.v = best == kInvalid ? 0.0f : bv;
-    return hit;
+__device__ __forceinline__ float tri_test(const TriRec& c, V3 o, V3 d, float& u, float& v) {
+    return mt_test(o, d, v3(c.p.x, c.p.y, c.p.z), c.e1, c.e2, u, v);
 }
 
-// Entry for one ray over a BVH of ntri triangles.
+// Closest hit of one ray in a scene of fewer than two triangles, which has no
+// internal node: its one triangle `single`, or kInvalid when it is empty.
 template <bool COUNT>
-__device__ __forceinline__ TraceHit trace_ray(const float4* __restrict__ nodes,
-                                              const float4* __restrict__ tris, uint32_t ntri, V3 o,
-                                              V3 d, TraceCount& cnt, uint32_t* status) {
+__device__ __forceinline__ TraceHit trace_single(const float4* __restrict__ tris, uint32_t single, V3 o, V3 d,
+                                                 TraceCount& cnt) {
     TraceHit miss{kFltMax, kInvalid, 0.0f, 0.0f};
-    if (ntri == 0) return miss;
-    if (ntri == 1) {
-        float u = 0.0f, v = 0.0f;
-        uint32_t id;
-        if (COUNT) cnt.tris++;
-        const float h = tri_hit(tris, 0, o, d, u, v, id);
-        if (h <= kMinTInit) return TraceHit{h, id, u, v};
-        return miss;
-    }
-    const V3 dinv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    const bool finite = __builtin_fabsf(dinv.x) <= kFltMax && __builtin_fabsf(dinv.y) <= kFltMax &&
-                        __builtin_fabsf(dinv.z) <= kFltMax;
-    if (finite) return traverse_impl<COUNT, true>(nodes, tris, o, d, dinv, cnt, status);
-    return traverse_impl<COUNT, false>(nodes, tris, o, d, dinv, cnt, status);
-}
-
-// One ray in the scene whose triangles (and internal nodes) occupy slots
-// [b, e) of a batched BVH; a single scene has b = 0.
-__device__ __forceinline__ TraceHit trace_ray_in(const float4* __restrict__ nodes,
-                                                 const float4* __restrict__ tris, uint32_t b, uint32_t e,
-                                                 V3 o, V3 d, uint32_t* status) {
-    TraceHit miss{kFltMax, kInvalid, 0.0f, 0.0f};
-    TraceCount cnt{0, 0, 0, 0};
-    if (e - b == 0) return miss;
-    if (e - b == 1) {
-        float u = 0.0f, v = 0.0f;
-        uint32_t id;
-        const float h = tri_hit(tris, b, o, d, u, v, id);
-        if (h <= kMinTInit) return TraceHit{h, id, u, v};
-        return miss;
-    }
-    const V3 dinv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    const bool finite = __builtin_fabsf(dinv.x) <= kFltMax && __builtin_fabsf(dinv.y) <= kFltMax &&
-                        __builtin_fabsf(dinv.z) <= kFltMax;
-    if (finite) return traverse_impl<false, true>(nodes, tris, o, d, dinv, cnt, status, b);
-    return traverse_impl<false, false>(nodes, tris, o, d, dinv, cnt, status, b);
+    if (single == kInvalid) return miss;
+    float u = 0.0f, v = 0.0f;
+    if (COUNT) cnt.tris++;
+    const TriRec c = load_tri(tris, single);
+    const float h = tri_test(c, o, d, u, v);
+    return h <= kMinTInit ? TraceHit{h, __float_as_uint(c.p.w), u, v} : miss;
 }
 
 // Where a lane keeps a shadow ray's deferred nodes: its column of an LDS
@@ -206,46 +102,49 @@ struct ShadowStack {
 // lends it to its shadow rays) instead of a private array.
 template <bool LDSS = false>
 __device__ __forceinline__ bool any_hit_in(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                          uint32_t b, uint32_t e, V3 o, V3 d, uint32_t* status,
-                                          const ShadowStack& ss = ShadowStack{}) {
+                                          const uint32_t* __restrict__ words, uint32_t b, uint32_t e, V3 o, V3 d,
+                                          uint32_t* status, const ShadowStack& ss = ShadowStack{}) {
     float u, v;
-    uint32_t id;
     if (e - b == 0) return false;
-    if (e - b == 1) return tri_hit(tris, b, o, d, u, v, id) <= kMinTInit;
+    if (e - b == 1) return tri_test(load_tri(tris, b), o, d, u, v) <= kMinTInit;
     const V3 dinv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
     uint32_t stack[LDSS ? 1 : kStackMax];
     int sp = 0;
-    uint32_t node = b;
+    uint32_t word = words[b];
     for (;;) {
-        const float4* rec = nodes + 4 * static_cast<size_t>(node);
-        const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
-        const uint32_t w = __float_as_uint(r3.x);
-        const uint32_t l = w >> 2;
-        const bool in0 = (w & 1u) != 0, in1 = (w & 2u) != 0;
-        const float h0 = in0 ? slab_test(o, dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y)
-                             : tri_hit(tris, l, o, d, u, v, id);
-        const float h1 = in1 ? slab_test(o, dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w)
-                             : tri_hit(tris, l + 1, o, d, u, v, id);
-        if ((!in0 && h0 <= kMinTInit) || (!in1 && h1 <= kMinTInit)) return true;
+        const uint32_t l = word >> 2;
+        const bool in0 = (word & 1u) != 0, in1 = (word & 2u) != 0;
+        const float4* rec = nodes + 4 * static_cast<size_t>(l);
+        const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+        const uint2 cw = *reinterpret_cast<const uint2*>(rec + 3);
+        TriRec ta, tb;
+        if (!in0) ta = load_tri(tris, l);
+        if (!in1) tb = load_tri(tris, l + 1);
+        const float h0 = slab_test(o, dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
+        const float h1 = slab_test(o, dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
+        uint32_t wt = word;
+        asm volatile("" : "+v"(wt));  // keeps the loads above the box tests (see test_children)
+        if ((wt & 1u) == 0u && tri_test(ta, o, d, u, v) <= kMinTInit) return true;
+        if ((wt & 2u) == 0u && tri_test(tb, o, d, u, v) <= kMinTInit) return true;
         const bool go0 = in0 && h0 <= kMinTInit, go1 = in1 && h1 <= kMinTInit;
         if (go0 && go1) {
             if constexpr (LDSS) {
-                if (sp < ss.depth) ss.lds[static_cast<uint32_t>(sp) * ss.stride] = l + 1;
-                else if (sp < kStackMax) ss.spill[sp - ss.depth] = l + 1;
+                if (sp < ss.depth) ss.lds[static_cast<uint32_t>(sp) * ss.stride] = cw.y;
+                else if (sp < kStackMax) ss.spill[sp - ss.depth] = cw.y;
                 else raise_status(status, kStatusStackOverflow);
                 if (sp < kStackMax) ++sp;
             } else {
-                if (sp < kStackMax) stack[sp++] = l + 1;
+                if (sp < kStackMax) stack[sp++] = cw.y;
                 else raise_status(status, kStatusStackOverflow);
             }
-            node = l;
+            word = cw.x;
         } else if (go0 || go1) {
-            node = go0 ? l : l + 1;
+            word = go0 ? cw.x : cw.y;
         } else {
             if (sp == 0) return false;
             --sp;
-            if constexpr (LDSS) node = sp < ss.depth ? ss.lds[static_cast<uint32_t>(sp) * ss.stride] : ss.spill[sp - ss.depth];
-            else node = stack[sp];
+            if constexpr (LDSS) word = sp < ss.depth ? ss.lds[static_cast<uint32_t>(sp) * ss.stride] : ss.spill[sp - ss.depth];
+            else word = stack[sp];
         }
     }
 }
@@ -267,51 +166,116 @@ struct RayState {
     float minT;
     uint32_t best;
     float bu, bv;
-    uint32_t node;
+    uint32_t word;  // the node to visit, as its child word
     int sp;
     bool finite;
 };
+
+__device__ __forceinline__ void init_ray(RayState& r, uint32_t root) {
+    r.dinv = v3(1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z);
+    r.finite = __builtin_fabsf(r.dinv.x) <= kFltMax && __builtin_fabsf(r.dinv.y) <= kFltMax &&
+               __builtin_fabsf(r.dinv.z) <= kFltMax;
+    r.minT = kMinTInit;
+    r.best = kInvalid;
+    r.bu = 0.0f;
+    r.bv = 0.0f;
+    r.word = root;
+    r.sp = 0;
+}
+
+__device__ __forceinline__ TraceHit final_hit(const RayState& r) {
+    TraceHit h;
+    h.id = r.best;
+    h.t = r.best == kInvalid ? kFltMax : r.minT;
+    h.u = r.best == kInvalid ? 0.0f : r.bu;
+    h.v = r.best == kInvalid ? 0.0f : r.bv;
+    return h;
+}
+
+// Keeps a lane's private array of deferred nodes in scratch memory.  The
+// compiler would otherwise hold a short one (the 32 entries past a 32-entry
+// LDS stack) in vector registers: 31 of them in every lane for entries that
+// hardly any ray reaches, 4 waves per SIMD for 6.
+__device__ __forceinline__ void keep_in_memory(uint32_t* spill) { asm volatile("" : : "v"(spill) : "memory"); }
+
+// What a visit finds about the node's two children: their box distances (of
+// internal children; a leaf's slot holds a box too, its value is discarded)
+// and their own words.
+struct Children {
+    float h0, h1;
+    uint32_t w0, w1;
+};
+
+// The tests of one visit.  Leaf children fold into the best hit first.  The
+// reference orders a node's two children by distance and lets a leaf replace
+// the best hit when nearer, or equally near with a lower id (trace.h:125-160):
+// over the leaves of one node that is the lexicographic minimum of (t, id),
+// whatever their order.  Taking it before deciding on the internal children
+// visits the same nodes: an internal child nearer than a leaf stays within
+// the updated best distance, and one farther than a leaf is culled against
+// the distance the leaf set, as in the reference.
+template <bool COUNT, bool FINITE>
+__device__ __forceinline__ Children test_children(const float4* __restrict__ nodes, const float4* __restrict__ tris,
+                                                  RayState& r, TraceCount& cnt) {
+    const uint32_t w = r.word;
+    const uint32_t l = w >> 2;
+    const float4* rec = nodes + 4 * static_cast<size_t>(l);
+    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+    const uint2 cw = *reinterpret_cast<const uint2*>(rec + 3);
+    // The first leaf child (the left one unless it is internal), and the
+    // second of a node with two.
+    TriRec ta, tb;
+    if ((w & 3u) != 3u) {
+        ta = load_tri(tris, (w & 1u) ? l + 1 : l);
+        if ((w & 3u) == 0u) tb = load_tri(tris, l + 1);
+    }
+    if (COUNT) cnt.iters++;
+    Children c;
+    c.h0 = child_box<COUNT, FINITE>(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
+    c.h1 = child_box<COUNT, FINITE>(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
+    c.w0 = cw.x;
+    c.w1 = cw.y;
+    if (COUNT) cnt.boxes += (w & 1u) + ((w >> 1) & 1u);
+    // An opaque copy of the word: with the same condition as above the
+    // compiler would merge the two branches and issue the triangle loads
+    // only after the box tests, a second memory round trip.
+    uint32_t wt = w;
+    asm volatile("" : "+v"(wt));
+    if ((wt & 3u) != 3u) {
+        float u, v;
+        const float t = tri_test(ta, r.o, r.d, u, v);
+        const uint32_t id = __float_as_uint(ta.p.w);
+        if (COUNT) cnt.tris++;
+        if (t < r.minT || (t == r.minT && id < r.best)) {
+            r.minT = t; r.best = id; r.bu = u; r.bv = v;
+        }
+        if ((wt & 3u) == 0u) {
+            float u2, v2;
+            const float t2 = tri_test(tb, r.o, r.d, u2, v2);
+            const uint32_t id2 = __float_as_uint(tb.p.w);
+            if (COUNT) cnt.tris++;
+            if (t2 < r.minT || (t2 == r.minT && id2 < r.best)) {
+                r.minT = t2; r.best = id2; r.bu = u2; r.bv = v2;
+            }
+        }
+    }
+    return c;
+}
 
 template <bool COUNT, int LDS, bool FINITE, int COLS = kPersistThreads>
 __device__ __forceinline__ bool visit_step(const float4* __restrict__ nodes,
                                            const float4* __restrict__ tris, RayState& r,
                                            uint32_t (*s_stack)[COLS],
                                            uint32_t* spill, TraceCount& cnt, uint32_t* status) {
-    const float4* rec = nodes + 4 * static_cast<size_t>(r.node);
-    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
-    const uint32_t w = __float_as_uint(r3.x);
-    const uint32_t l = w >> 2;
-    const bool in0 = (w & 1u) != 0, in1 = (w & 2u) != 0;
-    if (COUNT) cnt.iters++;
-    // Both child boxes in one code path for every lane (a leaf child's slot
-    // holds no box; its value is discarded).
-    const float h0 = child_box<COUNT, FINITE>(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
-    const float h1 = child_box<COUNT, FINITE>(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
-    if (COUNT) cnt.boxes += static_cast<uint32_t>(in0) + static_cast<uint32_t>(in1);
-    // Leaf children first.  The reference orders a node's two children by
-    // distance and lets a leaf replace the best hit when nearer, or equally
-    // near with a lower id (trace.h:125-160): over the leaves of one node
-    // that is the lexicographic minimum of (t, id), whatever their order.
-    // Taking it before deciding on the internal children visits the same
-    // nodes: an internal child nearer than a leaf stays within the updated
-    // best distance, and one farther than a leaf is culled against the
-    // distance the leaf set, as in the reference.
-    const uint32_t nleaf = static_cast<uint32_t>(!in0) + static_cast<uint32_t>(!in1);
-    for (uint32_t j = 0; j < nleaf; ++j) {
-        float u, v;
-        uint32_t id;
-        const float t = tri_hit(tris, (j == 0 && !in0) ? l : l + 1, r.o, r.d, u, v, id);
-        if (COUNT) cnt.tris++;
-        if (t < r.minT || (t == r.minT && id < r.best)) {
-            r.minT = t; r.best = id; r.bu = u; r.bv = v;
-        }
-    }
+    const bool in0 = (r.word & 1u) != 0, in1 = (r.word & 2u) != 0;
+    const Children c = test_children<COUNT, FINITE>(nodes, tris, r, cnt);
+    const float h0 = c.h0, h1 = c.h1;
     const bool g0 = in0 && h0 <= r.minT, g1 = in1 && h1 <= r.minT;
     if (g0 || g1) {
         const bool sw = g1 && (!g0 || h1 < h0);  // left child wins ties (trace.h:125)
-        r.node = sw ? l + 1 : l;
+        r.word = sw ? c.w1 : c.w0;
         if (g0 && g1) {
-            const uint32_t far = sw ? l : l + 1;
+            const uint32_t far = sw ? c.w0 : c.w1;
             const int sp = r.sp;
             if (sp < LDS) {
                 s_stack[sp][threadIdx.x] = far;
@@ -334,9 +298,283 @@ __device__ __forceinline__ bool visit_step(const float4* __restrict__ nodes,
     uint32_t next = s_stack[sp < LDS ? sp : LDS - 1][threadIdx.x];
     asm volatile("" : "+v"(next));
     if (sp >= LDS) next = spill[sp - LDS];
-    r.node = next;
+    r.word = next;
     r.sp = sp;
     return true;
+}
+
+// ---- group traversal -------------------------------------------------------
+//
+// A ray's visits form a chain: each waits for its record's loads (0.5-1 us
+// from the memory side) before it knows the next.  Where a wave has lanes to
+// spare -- a launch of fewer rays than the GPU has lanes, or the end of a
+// persistent loop, when the few longest rays of each wave are left -- 2^lg
+// lanes share one ray: a round takes up to 2^lg nodes off the ray's stack,
+// one per lane, tests them together, and puts their surviving children back,
+// nearer ones on top of farther ones.  The chain shrinks to about a quarter
+// at 8 lanes (longest ray over a 65,536-triangle soup: 282 visits, 44 rounds).
+// The hit is the lexicographic minimum of (t, id) over the tested triangles,
+// whichever lane tests them, as it is for one lane.
+//
+// All lanes of a group hold the ray; r.minT is the group's best distance
+// (agreed on after every round that improved it), and a lane that does not
+// hold a hit at that distance has r.best = kInvalid.  The group's stack is
+// its lanes' columns of the wave's LDS stack, entry e in row e >> lg of column
+// e mod 2^lg, which for lg = 0 is the one-lane layout.  With fewer than
+// kGroupReserve free entries left the group takes one node a round, which
+// is the depth-first walk of one lane: that adds at most 63 entries, and
+// those that do not fit go to the first lane's private array.
+constexpr uint32_t kGroupReserve = 16;
+
+__device__ __forceinline__ uint32_t lane_u32(uint32_t v, uint32_t src) {
+    return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(src << 2), static_cast<int>(v)));
+}
+__device__ __forceinline__ float lane_f32(float v, uint32_t src) {
+    return __uint_as_float(lane_u32(__float_as_uint(v), src));
+}
+__device__ __forceinline__ V3 lane_v3(V3 v, uint32_t src) {
+    return v3(lane_f32(v.x, src), lane_f32(v.y, src), lane_f32(v.z, src));
+}
+
+// The lanes of this lane's group.
+__device__ __forceinline__ uint64_t group_mask(uint32_t lg) {
+    const uint32_t lane = threadIdx.x & 63u;
+    return (~0ull >> (64u - (1u << lg))) << (lane & ~((1u << lg) - 1u));
+}
+
+// Orders the wave's LDS accesses across its lanes (they execute in order; this
+// keeps the compiler from moving them).
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Starts the group's ray at `root`; sp is the group's stack size.
+template <int LDS, int COLS>
+__device__ __forceinline__ void group_start(RayState& r, uint32_t root, uint32_t& sp, uint32_t lg,
+                                            uint32_t (*s_stack)[COLS]) {
+    init_ray(r, root);
+    if ((threadIdx.x & ((1u << lg) - 1u)) == 0u) s_stack[0][threadIdx.x] = root;
+    sp = 1u;
+}
+
+// One round of every group of the wave whose stack is not empty.
+template <int LDS, int COLS>
+__device__ __forceinline__ void group_round(const float4* __restrict__ nodes, const float4* __restrict__ tris,
+                                            RayState& r, uint32_t& sp, uint32_t lg, uint32_t (*s_stack)[COLS],
+                                            uint32_t* spill, uint32_t* status) {
+    constexpr uint32_t kSpill = kStackMax - LDS;
+    const uint32_t G = 1u << lg, j = threadIdx.x & (G - 1u), first = threadIdx.x - j;
+    const uint32_t cap = static_cast<uint32_t>(LDS) << lg;
+    const uint32_t room = sp + kGroupReserve < cap ? cap - kGroupReserve - sp : 1u;
+    const uint32_t k = min(min(sp, G), room);
+    const uint32_t base = sp - k;
+    const bool mine = j < k;
+    const float before = r.minT;
+    Children c{0.0f, 0.0f, 0u, 0u};
+    TraceCount cnt{0, 0, 0, 0};
+    wave_fence();
+    if (mine) {
+        const uint32_t e = base + j;
+        uint32_t word = s_stack[e < cap ? e >> lg : 0u][first + (e & (G - 1u))];
+        asm volatile("" : "+v"(word));  // keeps the LDS and scratch reads apart, as in visit_step
+        if (e >= cap) word = spill[min(e - cap, kSpill - 1u)];
+        r.word = word;
+        c = r.finite ? test_children<false, true>(nodes, tris, r, cnt)
+                     : test_children<false, false>(nodes, tris, r, cnt);
+    }
+    if (__ballot(r.minT < before) != 0ull) {
+        float m = r.minT;
+        for (uint32_t x = 1; x < G; x <<= 1) m = __builtin_fminf(m, __shfl_xor(m, static_cast<int>(x), 64));
+        if (m < r.minT) {
+            r.minT = m;
+            r.best = kInvalid;
+        }
+    }
+    const bool g0 = mine && (r.word & 1u) && c.h0 <= r.minT, g1 = mine && (r.word & 2u) && c.h1 <= r.minT;
+    const uint64_t gm = group_mask(lg), lt = (1ull << (threadIdx.x & 63u)) - 1ull;
+    const uint64_t any = __ballot(g0 || g1) & gm, both = __ballot(g0 && g1) & gm;
+    if (g0 || g1) {
+        const uint32_t p = base + static_cast<uint32_t>(__popcll(any & lt) + __popcll(both & lt));
+        const bool sw = g1 && (!g0 || c.h1 < c.h0);  // left child wins ties (trace.h:125)
+        const uint32_t near_w = sw ? c.w1 : c.w0, far_w = sw ? c.w0 : c.w1;
+        auto put = [&](uint32_t e, uint32_t w) {
+            if (e < cap) s_stack[e >> lg][first + (e & (G - 1u))] = w;
+            else if (e - cap < kSpill) spill[e - cap] = w;
+            else raise_status(status, kStatusStackOverflow);
+        };
+        if (g0 && g1) {
+            put(p, far_w);
+            put(p + 1u, near_w);
+        } else {
+            put(p, near_w);
+        }
+    }
+    sp = base + static_cast<uint32_t>(__popcll(any) + __popcll(both));
+}
+
+// The group's hit on all its lanes (lowest id at the best distance).
+__device__ __forceinline__ void group_best(RayState& r, uint32_t lg) {
+    uint32_t id = r.best;
+    for (uint32_t x = 1; x < (1u << lg); x <<= 1)
+        id = min(id, static_cast<uint32_t>(__shfl_xor(static_cast<int>(id), static_cast<int>(x), 64)));
+    const uint64_t who = __ballot(r.best == id) & group_mask(lg);
+    const uint32_t src = static_cast<uint32_t>(__builtin_ctzll(who));
+    r.best = id;
+    r.bu = lane_f32(r.bu, src);
+    r.bv = lane_f32(r.bv, src);
+}
+
+// Regroups the wave: the groups named by `act` (their first lanes; at most 32)
+// become groups of 2^lgn lanes, in order.  Every named group's stack fits its
+// LDS columns (sp <= LDS << lg).  Returns the first lane of the group this
+// lane's new group was, or 64 when there is none for it; the caller moves its
+// own per-ray values from that lane.
+template <int LDS, int COLS>
+__device__ __forceinline__ uint32_t regroup(RayState& r, uint32_t& sp, uint32_t& lg, uint32_t lgn, uint64_t act,
+                                            uint32_t (*s_stack)[COLS]) {
+    const uint32_t lane = threadIdx.x & 63u, wcol = threadIdx.x - lane;
+    const uint32_t gn = lane >> lgn, jn = lane & ((1u << lgn) - 1u);
+    uint32_t own = 64u, i = 0u;
+    for (uint64_t m = act; m != 0ull; m &= m - 1ull, ++i)
+        if (gn == i) own = static_cast<uint32_t>(__builtin_ctzll(m));
+    const uint32_t src = own < 64u ? own : lane;
+    const uint32_t moved = lane_u32(sp, src);
+    const uint32_t n = own < 64u ? moved : 0u;
+    constexpr int kMove = LDS / 2;  // entries per new lane: LDS << lg over at least 2 << lg lanes
+    uint32_t ent[kMove];
+    wave_fence();
+#pragma unroll
+    for (int q = 0; q < kMove; ++q) {
+        const uint32_t e = jn + (static_cast<uint32_t>(q) << lgn);
+        ent[q] = e < n ? s_stack[e >> lg][wcol + src + (e & ((1u << lg) - 1u))] : 0u;
+    }
+    wave_fence();
+#pragma unroll
+    for (int q = 0; q < kMove; ++q)
+        if (jn + (static_cast<uint32_t>(q) << lgn) < n) s_stack[q][threadIdx.x] = ent[q];
+    wave_fence();
+    // A lane's own best goes with it; the group's further lanes hold none.
+    const uint32_t bsrc = jn < (1u << lg) ? src + jn : src;
+    r.o = lane_v3(r.o, src);
+    r.d = lane_v3(r.d, src);
+    r.dinv = lane_v3(r.dinv, src);
+    r.finite = lane_u32(r.finite ? 1u : 0u, src) != 0u;
+    r.minT = lane_f32(r.minT, src);
+    r.best = lane_u32(r.best, own < 64u ? bsrc : lane);
+    r.bu = lane_f32(r.bu, own < 64u ? bsrc : lane);
+    r.bv = lane_f32(r.bv, own < 64u ? bsrc : lane);
+    if (jn >= (1u << lg)) r.best = kInvalid;
+    sp = n;
+    lg = lgn;
+    return own;
+}
+
+// Lanes per group (log2) that spread `count` rays (1..64) over a wave.
+__device__ __forceinline__ uint32_t group_log(uint32_t count) {
+    return count <= 1u ? 6u : 5u - (31u - static_cast<uint32_t>(__builtin_clz(count - 1u)));
+}
+
+// Traces the wave's groups to their ends: `active` groups with stack size sp
+// (sp <= LDS << lg), the ray's index in `ray` (equal on all lanes of a
+// group).  Once half the groups have ended the rest are given their lanes.
+template <int LDS, int COLS, class Store>
+__device__ __forceinline__ void group_trace(const float4* __restrict__ nodes, const float4* __restrict__ tris,
+                                            RayState& r, uint32_t sp, uint32_t lg, bool active, uint32_t ray,
+                                            uint32_t (*s_stack)[COLS], uint32_t* spill, uint32_t* status,
+                                            Store store) {
+    for (;;) {
+        const bool lead = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
+        const uint64_t act = __ballot(active && lead);
+        if (act == 0ull) return;
+        const uint32_t lgn = group_log(static_cast<uint32_t>(__popcll(act)));
+        if (lgn > lg && __ballot(active && sp > (static_cast<uint32_t>(LDS) << lg)) == 0ull) {
+            const uint32_t own = regroup<LDS>(r, sp, lg, lgn, act, s_stack);
+            ray = lane_u32(ray, own & 63u);
+            active = own < 64u;
+        }
+        group_round<LDS>(nodes, tris, r, sp, lg, s_stack, spill, status);
+        const bool ended = active && sp == 0u;
+        if (__ballot(ended) != 0ull) {
+            RayState f = r;
+            group_best(f, lg);
+            if (ended) {
+                if ((threadIdx.x & ((1u << lg) - 1u)) == 0u) store(ray, final_hit(f));
+                active = false;
+            }
+        }
+    }
+}
+
+// The end of a persistent loop: the wave's active lanes (at most kTailLanes,
+// each with fewer than LDS deferred nodes) go on as groups.  16M shell rays on
+// the 871,200-triangle mesh: 1,236 us without, 932 / 901 / 897 us from 8 / 16 /
+// 32 lanes on; 2M camera rays on the 2.88M-triangle hair ball 1,655 us
+// without, 1,645 / 1,505 / 1,460.
+constexpr uint32_t kTailLanes = 32;
+static_assert(kTailLanes <= 32, "regroup takes at most 32 groups");
+
+template <int LDS, int COLS, class Store>
+__device__ __forceinline__ void group_tail(const float4* __restrict__ nodes, const float4* __restrict__ tris,
+                                           RayState& r, bool active, uint32_t ray, uint32_t (*s_stack)[COLS],
+                                           uint32_t* spill, uint32_t* status, Store store) {
+    if (active) s_stack[r.sp][threadIdx.x] = r.word;
+    group_trace<LDS>(nodes, tris, r, active ? static_cast<uint32_t>(r.sp) + 1u : 0u, 0u, active, ray, s_stack, spill,
+                     status, store);
+}
+
+// A launch of few rays: wave w traces rays [w << (6 - lg), ...) with 2^lg lanes
+// each from the start, without a queue.
+template <int LDS, int COLS, class Load, class Store>
+__device__ __forceinline__ void grouped_trace(const float4* __restrict__ nodes, const float4* __restrict__ tris,
+                                              uint32_t nrays, uint32_t lg, uint32_t* status,
+                                              uint32_t (*s_stack)[COLS], Load load, Store store) {
+    uint32_t spill[kStackMax - LDS];
+    keep_in_memory(spill);
+    const uint32_t ray = (blockIdx.x * static_cast<uint32_t>(COLS) + threadIdx.x) >> lg;
+    const bool lead = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
+    RayState r;
+    r.o = r.d = r.dinv = v3(0.0f, 0.0f, 0.0f);
+    r.finite = true;
+    r.minT = kMinTInit;
+    r.best = kInvalid;
+    r.bu = r.bv = 0.0f;
+    r.word = 0u;
+    r.sp = 0;
+    bool active = false;
+    uint32_t sp = 0u;
+    if (ray < nrays) {
+        uint32_t single = kInvalid;
+        const uint32_t root = load(ray, r.o, r.d, single);
+        if (root == kInvalid) {
+            TraceCount cnt{0, 0, 0, 0};
+            const TraceHit h = trace_single<false>(tris, single, r.o, r.d, cnt);
+            if (lead) store(ray, h);
+        } else {
+            group_start<LDS>(r, root, sp, lg, s_stack);
+            active = true;
+        }
+    }
+    group_trace<LDS>(nodes, tris, r, sp, lg, active, ray, s_stack, spill, status, store);
+}
+
+// Lanes per ray (log2) of a launch of `nrays` rays on `lanes` lanes: as many as
+// there are lanes for, at most 2^kGroupMax; 0: one lane per ray, persistent.
+// Measured: 2,000 rays in a 4,096-triangle soup 89 us with one lane per ray,
+// 23 with up to 8, 19 with up to 16, 18 with up to 32; 131,072 rays (4 lanes)
+// after a rebuild of 2^20 triangles 565 -> 306 us; 65,536-path frames 1,040 ->
+// 260 us.  At 16 the wider rounds already find too few nodes to go further.
+constexpr uint32_t kGroupMax = 4;
+inline uint32_t launch_group(uint64_t nrays, uint64_t lanes) {
+    uint32_t lg = 0;
+    const uint64_t most = lanes < (1ull << 31) ? lanes : 1ull << 31;  // thread indices are 32-bit
+    while (lg < kGroupMax && (nrays << (lg + 1)) <= most) ++lg;
+    return lg;
+}
+// Workgroups of such a launch.
+inline uint32_t grouped_blocks(uint64_t nrays, uint32_t lg) {
+    return static_cast<uint32_t>(((nrays << lg) + kPersistThreads - 1) / kPersistThreads);
 }
 
 // Ray hand-out.  The rays [0, nrays) are split into nq contiguous slices
@@ -379,7 +617,7 @@ __device__ __forceinline__ void zero_queue(uint32_t* __restrict__ queue, uint32_
 // so that a short queue still spreads over every wave.  Idle lanes are
 // refilled when fewer than `refill` (1..64) lanes of the wave are busy.
 // load(i, o, d) fetches ray i; store(i, hit) writes its result.  load returns
-// the ray's root internal node, or kInvalid for a scene without one (fewer
+// the ray's root node's word, or kInvalid for a scene without one (fewer
 // than two triangles); then `single` names its one triangle (or kInvalid) and
 // the ray is answered at once without entering the loop.
 constexpr uint32_t kRayPoolSmall = 64;
@@ -408,6 +646,7 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     if (wave_id > 0u && static_cast<uint64_t>(wave_id) * kRayPoolSmall >= nrays) return;
     uint32_t spill[kStackMax - LDS];
+    keep_in_memory(spill);
     const int lane = threadIdx.x & 63;
     const uint64_t lt = (1ull << lane) - 1ull;
     RayState r;
@@ -460,26 +699,9 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
                     uint32_t single = kInvalid;
                     const uint32_t root = load(ray, r.o, r.d, single);
                     if (root == kInvalid) {
-                        TraceHit h{kFltMax, kInvalid, 0.0f, 0.0f};
-                        if (single != kInvalid) {
-                            float u = 0.0f, v = 0.0f;
-                            uint32_t id;
-                            if (COUNT) cnt.tris++;
-                            const float t = tri_hit(tris, single, r.o, r.d, u, v, id);
-                            if (t <= kMinTInit) h = TraceHit{t, id, u, v};
-                        }
-                        store(ray, h);
+                        store(ray, trace_single<COUNT>(tris, single, r.o, r.d, cnt));
                     } else {
-                        r.dinv = v3(1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z);
-                        r.finite = __builtin_fabsf(r.dinv.x) <= kFltMax &&
-                                   __builtin_fabsf(r.dinv.y) <= kFltMax &&
-                                   __builtin_fabsf(r.dinv.z) <= kFltMax;
-                        r.minT = kMinTInit;
-                        r.best = kInvalid;
-                        r.bu = 0.0f;
-                        r.bv = 0.0f;
-                        r.node = root;
-                        r.sp = 0;
+                        init_ray(r, root);
                         active = true;
                     }
                 }
@@ -511,17 +733,20 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
                 }
             }
         }
-        // With no busy lane the wave stops once no slice has rays left; until
-        // then the next pass probes the slice just chosen.
-        if (__ballot(active) == 0ull && drained) break;
+        // Once no slice has rays left the wave ends with groups (group_trace)
+        // as soon as kTailLanes rays or fewer are left, all with their
+        // deferred nodes in LDS.
+        if (drained) {
+            const uint64_t left = __ballot(active);
+            if (left == 0ull) break;
+            if (!COUNT && static_cast<uint32_t>(__popcll(left)) <= kTailLanes && __ballot(active && r.sp >= LDS) == 0ull) {
+                group_tail<LDS>(nodes, tris, r, active, ray, s_stack, spill, status, store);
+                break;
+            }
+        }
         if (active && !(r.finite ? visit_step<COUNT, LDS, true>(nodes, tris, r, s_stack, spill, cnt, status)
                                  : visit_step<COUNT, LDS, false>(nodes, tris, r, s_stack, spill, cnt, status))) {
-            TraceHit h;
-            h.id = r.best;
-            h.t = r.best == kInvalid ? kFltMax : r.minT;
-            h.u = r.best == kInvalid ? 0.0f : r.bu;
-            h.v = r.best == kInvalid ? 0.0f : r.bv;
-            store(ray, h);
+            store(ray, final_hit(r));
             active = false;
         }
     }
@@ -549,44 +774,10 @@ constexpr uint32_t kSurvCap = 128;  // survivor ring entries per wave
 template <bool FINITE>
 __device__ __forceinline__ bool root_visit(const float4* __restrict__ nodes, const float4* __restrict__ tris,
                                            RayState& r) {
-    const float4* rec = nodes + 4 * static_cast<size_t>(r.node);
-    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
-    const uint32_t w = __float_as_uint(r3.x);
-    const uint32_t l = w >> 2;
-    const bool in0 = (w & 1u) != 0, in1 = (w & 2u) != 0;
-    const float h0 = child_box<false, FINITE>(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
-    const float h1 = child_box<false, FINITE>(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
-    const uint32_t nleaf = static_cast<uint32_t>(!in0) + static_cast<uint32_t>(!in1);
-    for (uint32_t j = 0; j < nleaf; ++j) {
-        float u, v;
-        uint32_t id;
-        const float t = tri_hit(tris, (j == 0 && !in0) ? l : l + 1, r.o, r.d, u, v, id);
-        if (t < r.minT || (t == r.minT && id < r.best)) {
-            r.minT = t; r.best = id; r.bu = u; r.bv = v;
-        }
-    }
-    return (in0 && h0 <= r.minT) || (in1 && h1 <= r.minT);
-}
-
-__device__ __forceinline__ void init_ray(RayState& r, uint32_t root) {
-    r.dinv = v3(1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z);
-    r.finite = __builtin_fabsf(r.dinv.x) <= kFltMax && __builtin_fabsf(r.dinv.y) <= kFltMax &&
-               __builtin_fabsf(r.dinv.z) <= kFltMax;
-    r.minT = kMinTInit;
-    r.best = kInvalid;
-    r.bu = 0.0f;
-    r.bv = 0.0f;
-    r.node = root;
-    r.sp = 0;
-}
-
-__device__ __forceinline__ TraceHit final_hit(const RayState& r) {
-    TraceHit h;
-    h.id = r.best;
-    h.t = r.best == kInvalid ? kFltMax : r.minT;
-    h.u = r.best == kInvalid ? 0.0f : r.bu;
-    h.v = r.best == kInvalid ? 0.0f : r.bv;
-    return h;
+    const bool in0 = (r.word & 1u) != 0, in1 = (r.word & 2u) != 0;
+    TraceCount cnt;
+    const Children c = test_children<false, FINITE>(nodes, tris, r, cnt);
+    return (in0 && c.h0 <= r.minT) || (in1 && c.h1 <= r.minT);
 }
 
 // persistent_trace with the root filter (no counting).  s_surv: this wave's
@@ -603,6 +794,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     if (wave_id > 0u && static_cast<uint64_t>(wave_id) * kRayPoolSmall >= nrays) return;
     uint32_t spill[kStackMax - LDS];
+    keep_in_memory(spill);
     TraceCount cnt{0, 0, 0, 0};
     const int lane = threadIdx.x & 63;
     const uint64_t lt = (1ull << lane) - 1ull;
@@ -666,14 +858,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
                     uint32_t single = kInvalid;
                     const uint32_t root = load(fr, f.o, f.d, single);
                     if (root == kInvalid) {
-                        TraceHit h{kFltMax, kInvalid, 0.0f, 0.0f};
-                        if (single != kInvalid) {
-                            float u = 0.0f, v = 0.0f;
-                            uint32_t id;
-                            const float t = tri_hit(tris, single, f.o, f.d, u, v, id);
-                            if (t <= kMinTInit) h = TraceHit{t, id, u, v};
-                        }
-                        store(fr, h);
+                        store(fr, trace_single<false>(tris, single, f.o, f.d, cnt));
                     } else {
                         init_ray(f, root);
                         surv = f.finite ? root_visit<true>(nodes, tris, f) : root_visit<false>(nodes, tris, f);
@@ -700,7 +885,14 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
             }
             qhead += min(static_cast<uint32_t>(__popcll(idle)), qn);
         }
-        if (__ballot(active) == 0ull && drained && qtail == qhead) break;
+        if (drained && qtail == qhead) {  // as in persistent_trace
+            const uint64_t left = __ballot(active);
+            if (left == 0ull) break;
+            if (static_cast<uint32_t>(__popcll(left)) <= kTailLanes && __ballot(active && r.sp >= LDS) == 0ull) {
+                group_tail<LDS>(nodes, tris, r, active, ray, s_stack, spill, status, store);
+                break;
+            }
+        }
         if (active && !(r.finite ? visit_step<false, LDS, true>(nodes, tris, r, s_stack, spill, cnt, status)
                                  : visit_step<false, LDS, false>(nodes, tris, r, s_stack, spill, cnt, status))) {
             store(ray, final_hit(r));
