@@ -352,7 +352,7 @@ def same_bits(a, b):
 
 
 KNOBS = ("trace.blocks", "trace.refill", "trace.lds_stack", "trace.pool", "trace.filter", "render.paths",
-         "render.chains", "render.shade_min")
+         "render.chains", "render.shade_min", "render.shade_lit", "render.refill")
 
 
 def knob_state():

@@ -693,6 +693,8 @@ uint32_t* tune_slot(const char* name) {
     if (k == "render.chains") return &pt::render_tuning().chains;
     if (k == "render.paths") return &pt::render_tuning().paths;
     if (k == "render.shade_min") return &pt::render_tuning().shade_min;
+    if (k == "render.shade_lit") return &pt::render_tuning().shade_lit;
+    if (k == "render.refill") return &pt::render_tuning().refill;
     return nullptr;
 }
 
@@ -702,7 +704,9 @@ bool tune_valid(const uint32_t* slot, uint32_t v) {
     if (slot == &pt::build_tuning().staged) return v <= 1;
     if (slot == &pt::render_tuning().chains) return v >= 1 && v <= 8;
     if (slot == &pt::render_tuning().paths) return v <= 1;
-    if (slot == &pt::render_tuning().shade_min) return v >= 1 && v <= 64;
+    if (slot == &pt::render_tuning().shade_min || slot == &pt::render_tuning().shade_lit ||
+        slot == &pt::render_tuning().refill)
+        return v >= 1 && v <= 64;
     if (slot == &pt::trace_tuning().lds) return v == 8 || v == 16 || v == 32;
     if (slot == &pt::trace_tuning().pool) return v >= 64 && v <= 4096;
     return v != 0;

@@ -186,6 +186,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
                                                             uint32_t* __restrict__ ray_counters,
                                                             uint32_t level, uint32_t refill, uint32_t pool) {
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
+    __shared__ uint32_t s_pend[kPend][kPersistThreads];
     const uint32_t count = counters[level];
     TraceCount cnt{0, 0, 0, 0};
     auto load = [&](uint32_t i, V3& o, V3& d, uint32_t& single) -> uint32_t {
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
         hq.v[i] = h.v;
     };
     persistent_trace<false, LDS>(nodes, tris, count, ray_counters + level * kQueueWords, fc.status, refill, pool,
-                                 s_stack, load, store, cnt);
+                                 s_stack, s_pend, load, store, cnt);
 }
 
 __device__ __forceinline__ V3 ld3(const float* p) { return v3(p[0], p[1], p[2]); }
@@ -570,7 +571,7 @@ struct Handout {
 // Path-persistent frame (render.paths): one launch traces every path of a
 // frame from its primary ray to its end, one lane per path at a time.  A
 // lane advances its path's current segment by one node visit per loop
-// iteration (persistent_trace's visit); a lane whose segment has ended waits
+// iteration (persistent_trace's walk); a lane whose segment has ended waits
 // until `shade_min` lanes of its wave wait (or none is traversing), then those
 // lanes shade together -- primary_hit / bounce_hit / next_bounce, the
 // wavefront's functions, so every path computes the same bits -- and either
@@ -583,10 +584,11 @@ struct Handout {
 enum : uint32_t { kLaneIdle = 0u, kLaneTrace = 1u, kLaneShade = 2u };
 
 // Groups whose segments have ended shade together once they are at least one
-// in kGroupShade of the wave's groups (1, 2, 4, 8: 5.98, 5.73, 5.73, 5.80 ms
+// in group_shade of the wave's groups (1, 2, 4, 8: 5.98, 5.73, 5.73, 5.80 ms
 // for two 1,024 x 1,024 room frames, 2.04, 2.11, 2.09, 2.15 for eight 256 x 256
-// soup frames).
-constexpr uint32_t kGroupShade = 4;
+// soup frames).  With lights, whose shadow rays make shading the longer part,
+// all of them (a 637 x 359 textured frame under two lights 1.06 -> 0.43 ms).
+constexpr uint32_t group_shade(bool lights) { return lights ? 1u : 4u; }
 
 __global__ __launch_bounds__(64) void k_paths_setup(uint32_t* __restrict__ counters, uint32_t* __restrict__ queue,
                                                     uint32_t nlevels) {
@@ -653,9 +655,9 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                                                            const pt_dir_light* __restrict__ lights, PathState ps,
                                                            uint32_t* __restrict__ counters,
                                                            uint32_t* __restrict__ queue, uint32_t refill,
-                                                           uint32_t pool_large, uint32_t shade_min, uint32_t lg0,
-                                                           CacheIO io) {
+                                                           uint32_t shade_min, uint32_t lg0, CacheIO io) {
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
+    __shared__ uint32_t s_pend[kPend][kPersistThreads];
     __shared__ uint32_t s_level[kMaxLevels];
     // Plain frames keep each lane's path throughput and radiance in LDS
     // while it traverses alone.
@@ -743,10 +745,9 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
         }
     } else if (wave_id == 0u || static_cast<uint64_t>(wave_id) * kRayPoolSmall < npaths) {
         // (Waves past one per kRayPoolSmall paths have nothing to do.)
-        TraceCount cnt{0, 0, 0, 0};
         Handout ho;
-        ho.init(queue, npaths, npaths / 4u >= gridDim.x * blockDim.x ? pool_large : kRayPoolSmall, wave_id);
-        uint32_t state = kLaneIdle;
+        ho.init(queue, npaths, kRayPoolSmall, wave_id);
+        uint32_t state = kLaneIdle, pend = 0;
         for (;;) {
             // New paths for idle lanes.
             uint64_t busy = __ballot(state != kLaneIdle);
@@ -784,10 +785,11 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                 if (static_cast<uint32_t>(__popcll(busy)) <= kTailLanes &&
                     __ballot(state == kLaneTrace && r.sp >= LDS) == 0ull) {
                     active = state != kLaneIdle;
+                    test_pending(tris, r, pend, s_pend);
                     if (state == kLaneTrace) {
                         if (root == kInvalid) {
                             answer_single(fc, pp, off, tris, path, r);
-                        } else {
+                        } else if (r.word != kInvalid) {
                             s_stack[r.sp][tid] = r.word;
                             gsp = static_cast<uint32_t>(r.sp) + 1u;
                         }
@@ -797,15 +799,12 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
             }
             // One node visit for every traversing lane; a scene with fewer
             // than two triangles answers at once.
-            if (state == kLaneTrace) {
-                if (root == kInvalid) {
-                    answer_single(fc, pp, off, tris, path, r);
-                    state = kLaneShade;
-                } else if (!(r.finite ? visit_step<false, LDS, true>(nodes, tris, r, s_stack, spill, cnt, fc.status)
-                                      : visit_step<false, LDS, false>(nodes, tris, r, s_stack, spill, cnt, fc.status))) {
-                    state = kLaneShade;
-                }
+            if (state == kLaneTrace && root == kInvalid) {
+                answer_single(fc, pp, off, tris, path, r);
+                state = kLaneShade;
             }
+            if (walk_wave<LDS>(nodes, tris, r, pend, state == kLaneTrace, s_stack, s_pend, spill, fc.status))
+                state = kLaneShade;
             const uint64_t shading = __ballot(state == kLaneShade);
             const uint64_t tracing = __ballot(state == kLaneTrace);
             if (shading != 0ull && (static_cast<uint32_t>(__popcll(shading)) >= shade_min || tracing == 0ull)) {
@@ -857,7 +856,8 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
         group_round<LDS>(nodes, tris, r, gsp, lg, s_stack, spill, fc.status);
         const uint64_t ended = __ballot(active && gsp == 0u);
         if (ended != 0ull &&
-            (static_cast<uint32_t>(__popcll(ended)) * kGroupShade >= static_cast<uint32_t>(__popcll(__ballot(active))))) {
+            (static_cast<uint32_t>(__popcll(ended)) * group_shade(LIGHTS) >=
+             static_cast<uint32_t>(__popcll(__ballot(active))))) {
             group_best(r, lg);
             if (active && gsp == 0u) {
                 const bool lead = (lane & ((1 << lg) - 1)) == 0;
@@ -1147,7 +1147,7 @@ struct GraphKey {
     const void* accum;
     const void* counters;
     const void* lights;
-    uint32_t blocks, refill, lds, pool, chains, paths, shade_min;
+    uint32_t blocks, refill, lds, pool, chains, paths, shade_min, path_refill;
     hipStream_t stream;
 };
 
@@ -1176,6 +1176,12 @@ void ensure_chain_streams(Renderer& r, uint32_t nchains) {
     }
 }
 
+// Lanes that shade together in a path-persistent frame (render.shade_min, or
+// render.shade_lit where shading traces shadow rays).
+uint32_t shade_batch(const FrameConst& fc) {
+    return std::min(64u, std::max(1u, fc.nlights ? render_tuning().shade_lit : render_tuning().shade_min));
+}
+
 template <int LDS>
 auto paths_kernel(const FrameConst& fc) {
     return fc.detail ? (fc.nlights ? k_paths<LDS, true, true, false> : k_paths<LDS, false, true, false>)
@@ -1201,13 +1207,12 @@ void launch_frame(Renderer& r, const DeviceScene& scene, const FrameConst& fc, u
         hipLaunchKernelGGL(k_paths_setup, dim3(1), dim3(64), 0, st, cnt, cnt + 64, nlev);
         const uint32_t lg = launch_group(npaths, static_cast<uint64_t>(std::max(1u, tune.blocks)) * kPersistThreads);
         const uint32_t pgrid = lg ? grouped_blocks(npaths, lg) : std::min(std::max(1u, tune.blocks), grid);
-        const uint32_t pool = pool_for(tune.pool, static_cast<uint32_t>(npaths), pgrid);
         auto kern = tune.lds <= 8 ? paths_kernel<8>(fc) : paths_kernel<16>(fc);
         hipLaunchKernelGGL(kern, dim3(pgrid), dim3(kPersistThreads), 0, st, fc, pp,
                            scene.infos.as<pt_triangle_info>(), scene.bvh.nodes.as<float4>(),
                            scene.bvh.tris.as<float4>(), scene.off.as<uint32_t>(), scene.lights.as<pt_dir_light>(),
-                           L.ps, cnt, cnt + 64, refill, pool,
-                           std::min(64u, std::max(1u, render_tuning().shade_min)), lg, CacheIO{});
+                           L.ps, cnt, cnt + 64, std::min(64u, std::max(1u, render_tuning().refill)),
+                           shade_batch(fc), lg, CacheIO{});
         hipLaunchKernelGGL(k_accumulate, dim3(grid_for(fc.npix)), dim3(kThreads), 0, st, fc, L.ps,
                            r.accum.as<double>());
         return;
@@ -1434,7 +1439,8 @@ void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, cons
         key.pool = trace_tuning().pool;
         key.chains = nchains;
         key.paths = render_tuning().paths;
-        key.shade_min = render_tuning().shade_min;
+        key.shade_min = shade_batch(fc);
+        key.path_refill = render_tuning().refill;
         key.stream = st;
         replay(r.graph_exec, r.graph_key, key, st,
                [&] { launch_frame(r, scene, fc, nchains, st); });
@@ -1497,12 +1503,11 @@ void launch_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
         // lane carrying a path from its primary ray to the cache.
         const uint32_t lg = launch_group(fc.npix, static_cast<uint64_t>(std::max(1u, tune.blocks)) * kPersistThreads);
         const uint32_t ppgrid = lg ? grouped_blocks(fc.npix, lg) : std::min(std::max(1u, tune.blocks), grid_for(fc.npix));
-        const uint32_t ppool = pool_for(tune.pool, fc.npix, ppgrid);
         auto kern = tune.lds <= 8 ? cache_paths_kernel<8>(fc) : cache_paths_kernel<16>(fc);
         hipLaunchKernelGGL(kern, dim3(ppgrid), dim3(kPersistThreads), 0, st, fc, pp,
                            scene.infos.as<pt_triangle_info>(), scene.bvh.nodes.as<float4>(),
                            scene.bvh.tris.as<float4>(), scene.off.as<uint32_t>(), scene.lights.as<pt_dir_light>(),
-                           L.ps, cnt, rcnt, refill, ppool, std::min(64u, std::max(1u, render_tuning().shade_min)), lg,
+                           L.ps, cnt, rcnt, std::min(64u, std::max(1u, render_tuning().refill)), shade_batch(fc), lg,
                            io);
     } else {
         // Levels 0 and 1 of the pixel paths (a pixel path ends in the cache at x2).
@@ -1538,7 +1543,7 @@ void launch_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
 struct CacheGraphKey {
     FrameConst fc;
     CacheIO io;
-    uint32_t steps, train, blocks, refill, lds, pool, paths, shade_min;
+    uint32_t steps, train, blocks, refill, lds, pool, paths, shade_min, path_refill;
     const void* ptrs[13];
     float box[6], adam[4];
     hipStream_t stream;
@@ -1616,7 +1621,8 @@ void render_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
         key.lds = trace_tuning().lds;
         key.pool = trace_tuning().pool;
         key.paths = render_tuning().paths;
-        key.shade_min = render_tuning().shade_min;
+        key.shade_min = shade_batch(cf.fc);
+        key.path_refill = render_tuning().refill;
         const void* ptrs[13] = {scene.bvh.nodes.as<void>(), scene.bvh.tris.as<void>(), scene.infos.as<void>(),
                                 scene.off.as<void>(),       r.queues.as<void>(),     r.params.as<void>(),
                                 r.accum.as<void>(),         r.counters.as<void>(),   cache.master.as<void>(),

@@ -69,6 +69,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
     unsigned long long* __restrict__ counters, uint32_t* __restrict__ status) {
     static_assert(!(COUNT && FILTER), "the filter's repeated root visit would change the visit counts");
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
+    __shared__ uint32_t s_pend[kPend][kPersistThreads];
     const uint32_t root = words[0];
     auto load = [&](uint32_t i, V3& o, V3& d, uint32_t&) -> uint32_t {
         const float* rp = rays + 6 * static_cast<size_t>(i);
@@ -83,12 +84,12 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
     };
     if constexpr (FILTER) {
         __shared__ uint32_t s_surv[kPersistThreads / 64][kSurvCap];
-        persistent_trace_filtered<LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, s_stack,
+        persistent_trace_filtered<LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, s_stack, s_pend,
                                        s_surv[threadIdx.x / 64], load, store);
     } else {
         TraceCount cnt{0, 0, 0, 0};
-        persistent_trace<COUNT, LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, s_stack, load, store,
-                                     cnt);
+        persistent_trace<COUNT, LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, s_stack, s_pend, load,
+                                     store, cnt);
         if (COUNT) add_counts(cnt, counters);
     }
 }
@@ -102,9 +103,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
     uint32_t* __restrict__ out_id, float* __restrict__ out_t, float2* __restrict__ out_uv,
     uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool, uint32_t* __restrict__ status) {
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
+    __shared__ uint32_t s_pend[kPend][kPersistThreads];
     TraceCount cnt{0, 0, 0, 0};
     persistent_trace<false, LDS>(
-        nodes, tris, nrays, ray_counter, status, refill, pool, s_stack,
+        nodes, tris, nrays, ray_counter, status, refill, pool, s_stack, s_pend,
         [&](uint32_t i, V3& o, V3& d, uint32_t& single) -> uint32_t {
             const float* rp = rays + 6 * static_cast<size_t>(i);
             o = v3(rp[0], rp[1], rp[2]);

@@ -303,6 +303,113 @@ __device__ __forceinline__ bool visit_step(const float4* __restrict__ nodes,
     return true;
 }
 
+// ---- deferred leaf tests ----------------------------------------------------
+//
+// In a wave of lanes walking different rays nearly every visit finds a leaf
+// child on a few lanes (2.8 of 64 on average), and testing those triangles at
+// once costs the whole wave two triangle tests' instructions per visit, more
+// than half of all it issues.  walk_step instead notes a node's leaf children
+// in the lane's column of an LDS list and walks on; the wave tests the noted
+// triangles together (test_pending) once kFlushLanes lanes cannot go on --
+// list full, or nothing left to walk -- or no lane can.  The best distance
+// shrinks a few visits later, so a ray visits somewhat more nodes; its hit is
+// the lexicographic minimum of (t, id) over its triangles in any order.
+// Measured (us; 16M shell rays on the 871,200-triangle mesh, 2M camera rays on
+// the 2.88M-triangle hair ball, two 1,024 x 1,024 room frames): tests at once
+// 897, 1,464, 5,790; four entries and 6 / 12 / 20 / 32 lanes 877 / 863 / 868 /
+// 996, 1,356 / 1,364 / 1,414 / 1,681, 5,630 / 5,490 / 5,505 / 6,630; six entries
+// and 12 lanes 883, 1,366, 5,460.
+constexpr uint32_t kPend = 4;  // list entries per lane
+constexpr uint32_t kFlushLanes = 12;
+
+template <int LDS, bool FINITE, int COLS>
+__device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, RayState& r, uint32_t& pend,
+                                          uint32_t (*s_stack)[COLS], uint32_t (*s_pend)[COLS], uint32_t* spill,
+                                          uint32_t* status) {
+    const uint32_t w = r.word;
+    const uint32_t l = w >> 2;
+    const float4* rec = nodes + 4 * static_cast<size_t>(l);
+    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+    const uint2 cw = *reinterpret_cast<const uint2*>(rec + 3);
+    if ((w & 3u) != 3u) {
+        s_pend[pend][threadIdx.x] = (w & 1u) ? l + 1 : l;
+        if ((w & 3u) == 0u) s_pend[pend + 1][threadIdx.x] = l + 1;
+        pend += (w & 3u) == 0u ? 2u : 1u;
+    }
+    const float h0 = child_box<false, FINITE>(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
+    const float h1 = child_box<false, FINITE>(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
+    const bool g0 = (w & 1u) && h0 <= r.minT, g1 = (w & 2u) && h1 <= r.minT;
+    if (g0 || g1) {
+        const bool sw = g1 && (!g0 || h1 < h0);  // left child wins ties (trace.h:125)
+        r.word = sw ? cw.y : cw.x;
+        if (g0 && g1) {
+            const uint32_t far = sw ? cw.x : cw.y;
+            const int sp = r.sp;
+            if (sp < LDS) {
+                s_stack[sp][threadIdx.x] = far;
+                r.sp = sp + 1;
+            } else if (sp < kStackMax) {
+                spill[sp - LDS] = far;
+                r.sp = sp + 1;
+            } else {
+                raise_status(status, kStatusStackOverflow);
+            }
+        }
+        return;
+    }
+    if (r.sp == 0) {
+        r.word = kInvalid;  // nothing left to walk
+        return;
+    }
+    const int sp = r.sp - 1;
+    uint32_t next = s_stack[sp < LDS ? sp : LDS - 1][threadIdx.x];
+    asm volatile("" : "+v"(next));  // as in visit_step
+    if (sp >= LDS) next = spill[sp - LDS];
+    r.word = next;
+    r.sp = sp;
+}
+
+// Tests every noted triangle of the wave, the next one's record on its way
+// while one is tested.
+template <int COLS>
+__device__ __forceinline__ void test_pending(const float4* __restrict__ tris, RayState& r, uint32_t& pend,
+                                             uint32_t (*s_pend)[COLS]) {
+    TriRec next;
+    if (pend > 0u) next = load_tri(tris, s_pend[0][threadIdx.x]);
+    for (uint32_t k = 0; __ballot(k < pend) != 0ull; ++k) {
+        const TriRec c = next;
+        if (k + 1u < pend) next = load_tri(tris, s_pend[k + 1u][threadIdx.x]);
+        if (k < pend) {
+            float u, v;
+            const float t = tri_test(c, r.o, r.d, u, v);
+            const uint32_t id = __float_as_uint(c.p.w);
+            if (t < r.minT || (t == r.minT && id < r.best)) {
+                r.minT = t; r.best = id; r.bu = u; r.bv = v;
+            }
+        }
+    }
+    pend = 0u;
+}
+
+// One iteration of the wave's walking lanes (`busy`: the lane has a ray), with
+// the pending tests when they are due.  Returns whether the lane's ray has
+// ended.
+template <int LDS, int COLS>
+__device__ __forceinline__ bool walk_wave(const float4* __restrict__ nodes, const float4* __restrict__ tris,
+                                          RayState& r, uint32_t& pend, bool busy, uint32_t (*s_stack)[COLS],
+                                          uint32_t (*s_pend)[COLS], uint32_t* spill, uint32_t* status) {
+    if (busy && r.word != kInvalid && pend <= kPend - 2u) {
+        if (r.finite) walk_step<LDS, true>(nodes, r, pend, s_stack, s_pend, spill, status);
+        else walk_step<LDS, false>(nodes, r, pend, s_stack, s_pend, spill, status);
+    }
+    const bool stuck = busy && ((r.word == kInvalid && pend > 0u) || pend > kPend - 2u);
+    const uint64_t ns = __ballot(stuck);
+    if (ns != 0ull && (static_cast<uint32_t>(__popcll(ns)) >= kFlushLanes ||
+                       __ballot(busy && !stuck && r.word != kInvalid) == 0ull))
+        test_pending(tris, r, pend, s_pend);
+    return busy && r.word == kInvalid && pend == 0u;
+}
+
 // ---- group traversal -------------------------------------------------------
 //
 // A ray's visits form a chain: each waits for its record's loads (0.5-1 us
@@ -517,10 +624,14 @@ static_assert(kTailLanes <= 32, "regroup takes at most 32 groups");
 
 template <int LDS, int COLS, class Store>
 __device__ __forceinline__ void group_tail(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                           RayState& r, bool active, uint32_t ray, uint32_t (*s_stack)[COLS],
-                                           uint32_t* spill, uint32_t* status, Store store) {
-    if (active) s_stack[r.sp][threadIdx.x] = r.word;
-    group_trace<LDS>(nodes, tris, r, active ? static_cast<uint32_t>(r.sp) + 1u : 0u, 0u, active, ray, s_stack, spill,
+                                           RayState& r, uint32_t pend, bool active, uint32_t ray,
+                                           uint32_t (*s_stack)[COLS], uint32_t (*s_pend)[COLS], uint32_t* spill,
+                                           uint32_t* status, Store store) {
+    test_pending(tris, r, pend, s_pend);
+    const bool walking = active && r.word != kInvalid;
+    if (walking) s_stack[r.sp][threadIdx.x] = r.word;
+    if (active && !walking) store(ray, final_hit(r));
+    group_trace<LDS>(nodes, tris, r, walking ? static_cast<uint32_t>(r.sp) + 1u : 0u, 0u, walking, ray, s_stack, spill,
                      status, store);
 }
 
@@ -637,8 +748,9 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
                                                  const float4* __restrict__ tris, uint32_t nrays,
                                                  uint32_t* __restrict__ queue, uint32_t* status,
                                                  uint32_t refill, uint32_t pool_large,
-                                                 uint32_t (*s_stack)[kPersistThreads], Load load,
-                                                 Store store, TraceCount& cnt) {
+                                                 uint32_t (*s_stack)[kPersistThreads],
+                                                 uint32_t (*s_pend)[kPersistThreads], Load load, Store store,
+                                                 TraceCount& cnt) {
     // Waves past one per kRayPoolSmall rays leave at once: every wave that
     // stays drains the queue with the others, and on a short queue (a late
     // render level, a cache frame's training levels) the extra waves would
@@ -651,7 +763,7 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
     const uint64_t lt = (1ull << lane) - 1ull;
     RayState r;
     bool active = false;
-    uint32_t ray = 0;
+    uint32_t ray = 0, pend = 0;
     uint32_t pool_next = 0, pool_end = 0;  // wave-uniform
     bool drained = false;                  // wave-uniform: no rays left to hand out
     const uint32_t pool =
@@ -740,12 +852,18 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
             const uint64_t left = __ballot(active);
             if (left == 0ull) break;
             if (!COUNT && static_cast<uint32_t>(__popcll(left)) <= kTailLanes && __ballot(active && r.sp >= LDS) == 0ull) {
-                group_tail<LDS>(nodes, tris, r, active, ray, s_stack, spill, status, store);
+                group_tail<LDS>(nodes, tris, r, pend, active, ray, s_stack, s_pend, spill, status, store);
                 break;
             }
         }
-        if (active && !(r.finite ? visit_step<COUNT, LDS, true>(nodes, tris, r, s_stack, spill, cnt, status)
-                                 : visit_step<COUNT, LDS, false>(nodes, tris, r, s_stack, spill, cnt, status))) {
+        bool ended;
+        if constexpr (COUNT) {  // the reference's order of visits and tests, which the counts describe
+            ended = active && !(r.finite ? visit_step<true, LDS, true>(nodes, tris, r, s_stack, spill, cnt, status)
+                                         : visit_step<true, LDS, false>(nodes, tris, r, s_stack, spill, cnt, status));
+        } else {
+            ended = walk_wave<LDS>(nodes, tris, r, pend, active, s_stack, s_pend, spill, status);
+        }
+        if (ended) {
             store(ray, final_hit(r));
             active = false;
         }
@@ -790,6 +908,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
                                                           uint32_t* __restrict__ queue, uint32_t* status,
                                                           uint32_t refill, uint32_t pool_large,
                                                           uint32_t (*s_stack)[kPersistThreads],
+                                                          uint32_t (*s_pend)[kPersistThreads],
                                                           uint32_t* __restrict__ s_surv, Load load, Store store) {
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     if (wave_id > 0u && static_cast<uint64_t>(wave_id) * kRayPoolSmall >= nrays) return;
@@ -800,7 +919,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
     const uint64_t lt = (1ull << lane) - 1ull;
     RayState r;
     bool active = false;
-    uint32_t ray = 0;
+    uint32_t ray = 0, pend = 0;
     uint32_t pool_next = 0, pool_end = 0;  // wave-uniform
     bool drained = false;                  // wave-uniform: no rays left to hand out
     uint32_t qhead = 0, qtail = 0;         // wave-uniform: survivor ring positions
@@ -889,12 +1008,11 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
             const uint64_t left = __ballot(active);
             if (left == 0ull) break;
             if (static_cast<uint32_t>(__popcll(left)) <= kTailLanes && __ballot(active && r.sp >= LDS) == 0ull) {
-                group_tail<LDS>(nodes, tris, r, active, ray, s_stack, spill, status, store);
+                group_tail<LDS>(nodes, tris, r, pend, active, ray, s_stack, s_pend, spill, status, store);
                 break;
             }
         }
-        if (active && !(r.finite ? visit_step<false, LDS, true>(nodes, tris, r, s_stack, spill, cnt, status)
-                                 : visit_step<false, LDS, false>(nodes, tris, r, s_stack, spill, cnt, status))) {
+        if (walk_wave<LDS>(nodes, tris, r, pend, active, s_stack, s_pend, spill, status)) {
             store(ray, final_hit(r));
             active = false;
         }

@@ -96,12 +96,13 @@ def render_space(num_cus=256):
 def render_stages(num_cus=256):
     """Staged render search: the frame's structure first (path-persistent,
     or bounce levels in 1, 2 or 4 chains), then how many waiting lanes a
-    path-persistent wave shades together, then the traversal knobs, then the
-    shade batch again (it trades against the lane refill threshold)."""
+    path-persistent wave shades together and when its idle lanes take new
+    paths, then the traversal knobs, then the shade batch again."""
     return [{"render.paths": [1, 0], "render.chains": [1, 2, 4]},
-            {"render.shade_min": [4, 8, 16]},
+            {"render.shade_min": [8, 12, 16], "render.refill": [48, 60]},
+            {"render.shade_lit": [32, 48, 64]},
             render_space(num_cus),
-            {"render.shade_min": [4, 8, 16, 32]}]
+            {"render.shade_min": [4, 8, 12, 16, 24]}]
 
 
 def trace_stages(num_cus=256):

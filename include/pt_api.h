@@ -382,9 +382,14 @@ int pt_device_compute_units(int device, uint32_t* cus);
  *                   ray to its end in one persistent launch (no bounce
  *                   levels), and a cache frame its pixel paths from their
  *                   primary ray to the cache; 0: bounce levels (wavefront)
- *   "render.shade_min" 1..64: in path-persistent frames, the lanes of a
- *                   wave whose segments have ended shade together once this
- *                   many wait (or none is traversing)
+ *   "render.shade_min" 1..64: in path-persistent frames of scenes without
+ *                   directional lights, the lanes of a wave whose segments
+ *                   have ended shade together once this many wait (or none is
+ *                   traversing)
+ *   "render.shade_lit" the same for scenes with directional lights, where
+ *                   shading traces shadow rays
+ *   "render.refill" 1..64: in path-persistent frames, a wave's idle lanes take
+ *                   new paths when fewer than this many are busy
  *   "render.chains" 1..8: with render.paths 0, a plain frame's paths split
  *                   into this many chains of bounce levels on streams of
  *                   their own (at most one per 16,384 paths), so one chain's

@@ -25,7 +25,8 @@ def say(*a):
 
 @pytest.fixture
 def knobs():
-    names = ("trace.blocks", "trace.lds_stack", "trace.filter", "render.paths")
+    names = ("trace.blocks", "trace.lds_stack", "trace.filter", "render.paths", "render.shade_min", "render.shade_lit",
+             "render.refill")
     saved = {k: ptamd.tune_get(k) for k in names}
 
     def set_(**kw):
@@ -151,6 +152,36 @@ def test_frames_of_few_paths(ctx, knobs, lit, blocks):
         acc, spp = ctx.read_accumulator(w, h)
         assert spp == n and o.sum() > 0 and np.array_equal(acc, o)
         assert lit or rays == segs
+    assert ctx.get_status() == 0
+
+
+@pytest.mark.parametrize("shade,refill", [(1, 64), (7, 1), (33, 33), (64, 60)])
+def test_shade_and_refill_thresholds(ctx, knobs, shade, refill):
+    """Persistent frames at the edges of the batch sizes, with and without
+    lights: the accumulator does not depend on them."""
+    from test_oracle_lights import light
+
+    w, h = 41, 29
+    eye, tgt = (0.5, 0.5, -1.5), (0.5, 0.5, 0.0)
+    tris, infos = ptamd.gen_soup(5000, 14)
+    lights = np.array([light((1.0, 0.9, 0.8), (0.3, -1.0, 0.2), 1.5)], np.float32)
+    st = ptamd.Settings(5, 2, 1.0, 1)
+    dirs = ptamd.camera_corners(eye, tgt, (0, 1, 0), 60.0, w / h)
+    b = orc.build(tris, *ptamd.scene_bounds(tris))
+    knobs(trace_blocks=2, render_paths=1, render_shade_min=shade, render_shade_lit=shade, render_refill=refill)
+    for lit in (False, True):
+        say(f"[group] shade {shade}, refill {refill}, lit={lit}")
+        ctx.upload_scene(tris, infos, settings=st, lights=lights if lit else None)
+        ctx.set_primary_rays(dirs, eye)
+        ctx.reset_frames()
+        ctx.render_pass(w, h, 77)
+        acc, _ = ctx.read_accumulator(w, h)
+        o = np.zeros((h, w, 3))
+        if lit:
+            orc.render_pass_lit(tris, b, infos, lights, st, w, h, dirs, eye, 0, 77, o)
+        else:
+            orc.render_pass(tris, b, infos, st, w, h, dirs, eye, 0, 77, o)
+        assert o.sum() > 0 and np.array_equal(acc, o)
     assert ctx.get_status() == 0
 
 
