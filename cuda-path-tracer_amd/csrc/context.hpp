@@ -92,27 +92,25 @@ class HostBuf {
     size_t cap_ = 0;
 };
 
-// LBVH in device memory.  Two layouts live side by side: the reference's
-// parity arrays (keys, perm, children, parents) and the traversal layout:
+// LBVH in device memory: the sorted keys and permutation, and the traversal
+// layout, from which the parity dump derives the reference's arrays:
 //   nodes[4*s .. 4*s+3]   one 64-byte record per internal node, in the slot of
 //       its left child's index s (word >> 2 of its child word):
 //       (L.minx, L.maxx, L.miny, L.maxy) (L.minz, L.maxz, R.minx, R.maxx)
 //       (R.miny, R.maxy, R.minz, R.maxz) (L's child word, R's, 0, 0)
 //     -- both child boxes and the children's own child words, so one visit is
 //        one contiguous 64-byte read and names the next visit's record and
-//        leaf triangles; a leaf child's slot holds its triangle box, word 0.
+//        leaf triangles; a leaf child's slot holds its triangle box, word kInvalid.
 //   tris[3*k .. 3*k+2]   one 48-byte record per sorted triangle k:
 //       (p0.xyz, original id) (e1.xyz, 0) (e2.xyz, 0), e = p - p0.
 struct DeviceBvh {
     uint32_t n = 0;
     DevBuf keys, vals, keys_alt, vals_alt;  // sorted Morton keys, perm (+ ping-pong)
     DevBuf scene_of;                        // scene of each leaf slot
-    DevBuf children, parents_leaf, parents_internal, counters;
-    DevBuf nodes, tris, root_box;
+    DevBuf nodes, tris;
+    DevBuf root_box, root_word;     // per scene: the root's box and child word (kInvalid: one triangle)
     DevBuf tile_hist, digit_total;  // radix sort scratch
-    DevBuf span_list, span_top, span_count;  // refit: per-level node lists
-    DevBuf mid_links, top_links;             // refit: the level-1 and level-2 lists' staged links
-    DevBuf slots;                            // refit: each listed node's position in its list
+    DevBuf open_lists;              // tree: each block's subtrees that the next level goes on with
 };
 
 // One or more scenes: scene s owns triangles [off[s], off[s+1]) and its own
@@ -146,7 +144,7 @@ struct BuildTimes {
     float total = 0.0f;
 };
 
-// LBVH build: Morton keys -> 4-pass LDS radix sort -> radix tree -> refit.
+// LBVH build: Morton keys -> LDS radix sort -> radix tree with its boxes.
 void build_lbvh(DeviceScene& scene, hipStream_t stream);
 // Parity dump of one scene in local indices (device -> host, synchronous).
 void dump_bvh(DeviceScene& scene, uint32_t scene_index, hipStream_t stream, uint32_t* morton,
@@ -155,7 +153,7 @@ void dump_bvh(DeviceScene& scene, uint32_t scene_index, hipStream_t stream, uint
 
 // LBVH build options (tunable).
 struct BuildTuning {
-    uint32_t staged = 1;  // refit the upper levels with their node lists staged in LDS (0: in global memory)
+    uint32_t staged = 1;  // accepted, without effect: the tree has one way to its upper levels
 };
 BuildTuning& build_tuning();
 

@@ -1,10 +1,8 @@
 // LBVH construction on gfx950 (reference: CUDA::BVHBuilder::build,
 // BVHBuilder.cu:207-269, after Karras 2012), for one scene or for a batch of
 // scenes at once.  Scenes are contiguous segments [off[s], off[s+1]) of the
-// triangle array; every array below is indexed by global leaf slot, and the
-// internal nodes of scene s are numbered off[s] + local index (slot
-// off[s+1]-1 is unused), so each node's index lies inside its own leaf range.
-// Child and parent indices are global; the parity dump converts to local.
+// triangle array; every array below is indexed by global leaf slot.  The
+// parity dump derives the reference's node numbers, child and parent words.
 //
 //   k_morton        30-bit Morton key (the scene's box) + index + scene id,
 //                   and the first sort pass's per-tile digit counts
@@ -13,16 +11,12 @@
 //   k_sort_scatter  /  the 30-bit key, then 1-2 over the scene id when
 //                      batched (wave64 ballot match + LDS staging per
 //                      4096-key tile)
-//   k_radix_tree    Karras split per internal node, parents, counter reset,
-//                   list of nodes whose leaf range crosses a refit block
-//   k_refit_local   sorted triangle records + bottom-up AABBs inside each
-//                   1024-leaf block (LDS counters/boxes, workgroup scope);
-//                   extra workgroups stage the level-1 nodes' links
-//   k_refit_mid     nodes inside each 65536-leaf block, one workgroup each;
-//                   one more workgroup stages the level-2 nodes' links
-//   k_refit_top     the remaining nodes, one workgroup
-// Each node's traversal record is written whole by the thread that
-// completes the node's box.
+//   k_tree_leaves   sorted triangle records, then the radix tree and its boxes
+//                   bottom-up inside each 1024-leaf block (LDS, workgroup
+//                   scope); each node's traversal record is written whole by
+//                   the thread that completes it
+//   k_tree_merge    the same over the subtrees that 64 blocks left open, level
+//                   by level until none is
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -39,28 +33,17 @@ constexpr int kSortTile = 4096;                                // keys per sort 
 constexpr int kDigitBits = 10;                                 // 3 passes over a 30-bit key
 constexpr uint32_t kRadix = 1u << kDigitBits;                  // 1024 digits
 constexpr int kScatterThreads = 512;                           // scatter: 8 keys per thread, 8 waves per tile
-// Refit levels.  A node's level is the smallest k whose block of sorted
-// leaves contains the node's whole leaf range:
-//   level 0: inside a 1024-leaf block    -> k_refit_local (LDS, one workgroup per block)
-//   level 1: inside a 65536-leaf block   -> k_refit_mid (one workgroup per block)
-//   level 2: anything larger             -> k_refit_top (one workgroup)
-// A node's children have a level no higher than its own, so each phase only
-// needs the previous phases' boxes.  Levels are kept in bits 30-31 of the
-// node's refit counter.
-constexpr int kRefitBlock = 1024;
-constexpr uint32_t kMidBlock = 65536;
-// Upper-level node lists.  A level-1 node goes to the list of the 1024-leaf
-// block holding the start of its leaf range, a level-2 node to that of the
-// 65536-leaf block; either way its range crosses that block's end, and a
-// boundary is crossed only by the <= 64 ancestors of its two leaves' lowest
-// common ancestor, so a list never holds more than kListCap nodes.  (Lists
-// per small block keep the appends' atomics spread over many counters.)
-// One 65536-leaf block's 64 level-1 lists together hold at most kMidCap.
-constexpr uint32_t kListCap = 64;
-constexpr uint32_t kMidCap = 64 * kListCap;
-constexpr uint32_t kMaxMidBlocks = (1u << 30) / kMidBlock;  // builds hold < 2^30 triangles
-constexpr uint32_t kLevelShift = 30;
-constexpr uint32_t kCountMask = (1u << kLevelShift) - 1u;
+// The tree is built bottom-up, boxes included, in levels: one workgroup per
+// block of kLeafBlock sorted leaves, then one per kFanIn blocks' open subtrees,
+// and so on (see the tree section).
+constexpr uint32_t kLeafBlock = 1024;
+constexpr uint32_t kFanIn = 16;
+// Open subtrees of a block: each hangs off a node whose leaf range crosses the
+// block's first or last boundary, and a boundary is crossed only by the <= 62
+// ancestors of its two leaves' lowest common ancestor.  (About 20 in practice.)
+constexpr uint32_t kOpenCap = 128;
+constexpr uint32_t kMergeCap = kFanIn * kOpenCap;
+constexpr uint32_t kMergeThreads = 512;
 
 // ---- Morton keys ------------------------------------------------------------
 
@@ -98,8 +81,7 @@ __device__ __forceinline__ uint32_t scene_of_slot(const uint32_t* __restrict__ o
 // into the scene's enclosing box with invScale computed on the host
 // (box[6*s..] = min.xyz, invScale.xyz).  One workgroup per 4096-key sort
 // tile, which also counts the tile's first-pass digits (key bits 0-9) into
-// its row of tile_hist -- the first sort pass then starts at the scan.  Also
-// zeroes the refit list counters.
+// its row of tile_hist -- the first sort pass then starts at the scan.
 constexpr int kMortonThreads = 1024;
 
 __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __restrict__ tris, uint32_t n,
@@ -108,13 +90,9 @@ __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __
                                                            uint32_t* __restrict__ keys,
                                                            uint32_t* __restrict__ vals,
                                                            uint32_t* __restrict__ scene_of,
-                                                           uint32_t* __restrict__ tile_hist,
-                                                           uint32_t* __restrict__ span_count,
-                                                           uint32_t n_span_counts) {
+                                                           uint32_t* __restrict__ tile_hist) {
     __shared__ uint32_t h[kRadix];
     const uint32_t tid = threadIdx.x;
-    for (uint32_t i = blockIdx.x * kMortonThreads + tid; i < n_span_counts; i += gridDim.x * kMortonThreads)
-        span_count[i] = 0u;
     for (uint32_t d = tid; d < kRadix; d += kMortonThreads) h[d] = 0u;
     __syncthreads();
     const uint32_t base = blockIdx.x * kSortTile;
@@ -387,132 +365,33 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     }
 }
 
-// ---- radix tree -----------------------------------------------------------------
-
-// delta (BVHBuilder.cu:116-133) of key i and the key x places from it
-// (forward or backward): common prefix length, augmented with the index
-// bits when the keys are equal; -1 outside [0, n).  Indices are 32-bit (a
-// scene holds < 2^30 keys, so an offset clamped to 2^30 is already out of
-// range).
-__device__ __forceinline__ int delta_at(const uint32_t* __restrict__ keys, uint32_t n, uint32_t i, uint32_t ki,
-                                        bool fwd, uint32_t x) {
-    x = min(x, 1u << 30);
-    const int32_t j = fwd ? static_cast<int32_t>(i + x) : static_cast<int32_t>(i) - static_cast<int32_t>(x);
-    if (j < 0 || static_cast<uint32_t>(j) >= n) return -1;
-    const uint32_t kj = keys[j];
-    if (ki == kj) return 32 + __clz(static_cast<int>(i ^ static_cast<uint32_t>(j)));
-    return __clz(static_cast<int>(ki ^ kj));
-}
-
-// radix_tree_construction_kernel (BVHBuilder.cu:135-196), one thread per
-// internal node, on its scene's segment of sorted keys with local indices
-// (the index augmentation of delta uses them, as in a single-scene build).
-// Also initialises the node's refit counter with its refit level (from its
-// global leaf range) and appends level-1 nodes to their 1024-leaf block's
-// list (span_list[block * kListCap ...], count in span_count[block]) and
-// level-2 nodes to their 65536-leaf block's (span_top[...], count in
-// span_count[n_lists1 + block]), with each listed node's list and position
-// in slots[node].  The node's traversal record
-// is written whole by the refit, once its box is known: a 16-byte store into
-// each 64-byte record here would cost a partial-line write per node.
-__global__ __launch_bounds__(256) void k_radix_tree(const uint32_t* __restrict__ keys, uint32_t n,
-                                                    const uint32_t* __restrict__ off,
-                                                    const uint32_t* __restrict__ scene_of,
-                                                    uint32_t* __restrict__ children,
-                                                    uint32_t* __restrict__ parents_leaf,
-                                                    uint32_t* __restrict__ parents_internal,
-                                                    uint32_t* __restrict__ counters,
-                                                    float4* __restrict__ nodes,
-                                                    uint32_t* __restrict__ span_list,
-                                                    uint32_t* __restrict__ span_top,
-                                                    uint32_t* __restrict__ span_count,
-                                                    uint32_t n_lists1,
-                                                    uint32_t* __restrict__ slots,
-                                                    uint32_t* __restrict__ status) {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n) return;
-    const uint32_t sc = scene_of[g];
-    const uint32_t base = off[sc];
-    const int64_t N = off[sc + 1] - base;
-    const int64_t i = g - base;
-    if (i >= N - 1) return;  // unused slot of the scene (or a 1-triangle scene)
-    const uint32_t* sk = keys + base;
-    const uint32_t n_loc = static_cast<uint32_t>(N), il = static_cast<uint32_t>(i);
-    const uint32_t ki = sk[il];
-    // Direction, the range's far end j and the split (Karras 2012, Alg. 2;
-    // the reference's exponential, binary and ceil-halving searches), on
-    // 32-bit offsets from i.
-    const int dp = delta_at(sk, n_loc, il, ki, true, 1), dm = delta_at(sk, n_loc, il, ki, false, 1);
-    const bool fwd = dp > dm;  // never equal: augmented keys are distinct
-    const int dmin = fwd ? dm : dp;
-    uint32_t lmax = 2;
-    while (delta_at(sk, n_loc, il, ki, fwd, lmax) > dmin) lmax *= 2;  // a probe at 2^30 fails: no overflow
-    uint32_t l = 0;
-    while (lmax > 1) {
-        lmax /= 2;
-        if (delta_at(sk, n_loc, il, ki, fwd, l + lmax) > dmin) l += lmax;
-    }
-    const int dnode = delta_at(sk, n_loc, il, ki, fwd, l);
-    uint32_t sx = 0, r = l;
-    while (r > 1) {
-        r = (r + 1) / 2;
-        if (delta_at(sk, n_loc, il, ki, fwd, sx + r) > dnode) sx += r;
-    }
-    const int64_t d = fwd ? 1 : -1;
-    const int64_t j = i + static_cast<int64_t>(l) * d;
-    const int64_t s = i + static_cast<int64_t>(sx) * d + (d < 0 ? d : 0);
-    uint32_t type = 0;
-    if ((i < j ? i : j) != s) {
-        type |= 1u;
-        parents_internal[base + s] = g;
-    } else {
-        parents_leaf[base + s] = g;
-    }
-    if ((i > j ? i : j) != s + 1) {
-        type |= 2u;
-        parents_internal[base + s + 1] = g;
-    } else {
-        parents_leaf[base + s + 1] = g;
-    }
-    children[g] = ((base + static_cast<uint32_t>(s)) << 2) | type;
-    const int64_t lo = base + (i < j ? i : j), hi = base + (i > j ? i : j);
-    uint32_t level = 0;
-    if ((lo / kRefitBlock) != (hi / kRefitBlock)) level = ((lo / kMidBlock) != (hi / kMidBlock)) ? 2u : 1u;
-    counters[g] = level << kLevelShift;
-    if (level != 0) {
-        const uint32_t blk = static_cast<uint32_t>(level == 1 ? lo / kRefitBlock : lo / kMidBlock);
-        const uint32_t slot = atomicAdd(span_count + (level == 1 ? 0u : n_lists1) + blk, 1u);
-        if (slot < kListCap) {
-            (level == 1 ? span_list : span_top)[static_cast<size_t>(blk) * kListCap + slot] = g;
-            // The list within its 65536-leaf block (level 1) or overall (level 2), and the place in it.
-            slots[g] = ((level == 1 ? blk % (kMidBlock / kRefitBlock) : blk) << 6) | slot;
-        } else {
-            raise_status(status, PT_STATUS_REFIT_OVERFLOW);  // bound argued above
-        }
-    }
-    if (i == 0) parents_internal[g] = kInvalid;  // BVHBuilder.cu:224
-}
-
-// ---- refit ------------------------------------------------------------------------
+// ---- tree and boxes -----------------------------------------------------------
+//
+// The radix tree (BVHBuilder.cu:107-201) and its boxes (:39-98) in one
+// bottom-up pass (Apetrei, "Fast and Simple Agglomerative LBVH Construction",
+// 2014).  delta(i) is the length of the common prefix of the adjacent sorted
+// keys i and i + 1, extended by the scene-local index when they are equal
+// (BVHBuilder.cu:116-133), and -1 across a scene's ends.  A finished subtree
+// over leaves [lo, hi] is the left child of its parent, which splits after hi,
+// if delta(hi) > delta(lo - 1), and the right child, split after lo - 1,
+// otherwise (the two differ unless both are -1: the root).  Of the two
+// subtrees meeting at a split the one to arrive second unites them.  So no
+// node searches the keys for its range and split, no separate pass refits the
+// boxes, and the words of both children are at hand where a record is written.
+// The reference's node numbers follow from the splits: a left child split off
+// after s is node s, a right child node s + 1 (see the dump).
+//
+// A workgroup does this in LDS for one block of leaves (hand-offs need only
+// workgroup scope).  Subtrees whose sibling reaches outside the block are
+// written, in leaf order, to the block's open list; the next level's
+// workgroup goes on with the lists of kFanIn blocks as its elements, and so on
+// until one workgroup has them all.  2^20 soup triangles: the separate tree
+// kernel and the refit of three levels took 34 + 57 + 13 + 10 us (the build 194
+// us), these 63 + 13 + 15 + 10 (178 us).
 
 struct Box {
     float mnx, mxx, mny, mxy, mnz, mxz;
 };
-
-// One child's box and word (0 for a leaf) into the record of the node with
-// child word pw.
-__device__ __forceinline__ void store_slot(float4* nodes, uint32_t pw, bool left, const Box& b, uint32_t cw) {
-    float4* rec = nodes + 4 * static_cast<size_t>(pw >> 2);
-    if (left) {
-        rec[0] = make_float4(b.mnx, b.mxx, b.mny, b.mxy);
-        reinterpret_cast<float2*>(rec + 1)[0] = make_float2(b.mnz, b.mxz);
-        reinterpret_cast<uint32_t*>(rec + 3)[0] = cw;
-    } else {
-        reinterpret_cast<float2*>(rec + 1)[1] = make_float2(b.mnx, b.mxx);
-        rec[2] = make_float4(b.mny, b.mxy, b.mnz, b.mxz);
-        reinterpret_cast<uint32_t*>(rec + 3)[1] = cw;
-    }
-}
 
 __device__ __forceinline__ Box unite(const Box& a, const Box& b) {
     // leftBBox.unite(rightBBox) (BVHBuilder.cu:85, BBox.cpp:30-36).
@@ -527,8 +406,8 @@ __device__ __forceinline__ Box unite(const Box& a, const Box& b) {
 }
 
 // The whole traversal record of the node with child word w (slot w >> 2, its
-// left child's index): both child boxes and both children's own words (0 for
-// a leaf), in one 64-byte line.
+// left child's index): both child boxes and both children's own words
+// (kInvalid for a leaf), in one 64-byte line.
 __device__ __forceinline__ void store_record(float4* nodes, uint32_t w, const Box& lb, const Box& rb, uint32_t wl,
                                              uint32_t wr) {
     float4* rec = nodes + 4 * static_cast<size_t>(w >> 2);
@@ -538,487 +417,323 @@ __device__ __forceinline__ void store_record(float4* nodes, uint32_t w, const Bo
     rec[3] = make_float4(__uint_as_float(wl), __uint_as_float(wr), 0.0f, 0.0f);
 }
 
-__device__ __forceinline__ void store_root(float* root_box, const Box& b) {
-    root_box[0] = b.mnx; root_box[1] = b.mny; root_box[2] = b.mnz;
-    root_box[3] = b.mxx; root_box[4] = b.mxy; root_box[5] = b.mxz;
+__device__ __forceinline__ void store_root(float* root_box, uint32_t* root_word, uint32_t scene, const Box& b,
+                                           uint32_t word) {
+    float* o = root_box + 6 * static_cast<size_t>(scene);
+    o[0] = b.mnx; o[1] = b.mny; o[2] = b.mnz;
+    o[3] = b.mxx; o[4] = b.mxy; o[5] = b.mxz;
+    root_word[scene] = word;
 }
 
-// LDS box array in structure-of-arrays form (one float plane per bound).
-struct LdsBoxes {
-    float v[6][kRefitBlock];
-    __device__ __forceinline__ void put(int k, const Box& b) {
-        v[0][k] = b.mnx; v[1][k] = b.mxx; v[2][k] = b.mny;
-        v[3][k] = b.mxy; v[4][k] = b.mnz; v[5][k] = b.mxz;
-    }
-    __device__ __forceinline__ Box get(int k) const {
-        return Box{v[0][k], v[1][k], v[2][k], v[3][k], v[4][k], v[5][k]};
+// A block's open subtrees, in leaf order: last leaf, delta there, child word
+// (kInvalid: one leaf) and box of each.
+struct OpenList {
+    uint32_t count;
+    uint32_t hi[kOpenCap];
+    int32_t delta[kOpenCap];
+    uint32_t word[kOpenCap];
+    float box[6][kOpenCap];
+
+    __device__ __forceinline__ void put(uint32_t k, uint32_t last_leaf, int32_t d, uint32_t w, const Box& b) {
+        hi[k] = last_leaf;
+        delta[k] = d;
+        word[k] = w;
+        box[0][k] = b.mnx; box[1][k] = b.mxx; box[2][k] = b.mny;
+        box[3][k] = b.mxy; box[4][k] = b.mnz; box[5][k] = b.mxz;
     }
 };
 
-// Refit of the level-L nodes listed in `list` (count at *count), all inside
-// one workgroup so the counter hand-off needs only workgroup-scope ordering.
-// Every child box of a node sits in the node's own record: lower-level
-// children were stored by earlier phases, same-level children are stored here
-// before their parent's counter is incremented.  Each lower-level child of a
-// listed node is one "arrival"; the thread completing a node climbs on while
-// the parent is of the same level.
-__device__ __forceinline__ void refit_level(const uint32_t* __restrict__ children,
-                                            const uint32_t* __restrict__ scene_of,
-                                            const uint32_t* __restrict__ parents_internal,
-                                            uint32_t* __restrict__ counters,
-                                            float4* __restrict__ nodes,
-                                            float* __restrict__ root_box,
-                                            const uint32_t* list, uint32_t count, uint32_t level) {
-    for (uint32_t idx = threadIdx.x; idx < count; idx += blockDim.x) {
-        const uint32_t s = list[idx];
-        const uint32_t w = children[s];
-        const uint32_t l = w >> 2, r = l + 1;
-        int arrivals = 0;
-        if (!(w & 1u) || (counters[l] >> kLevelShift) < level) ++arrivals;
-        if (!(w & 2u) || (counters[r] >> kLevelShift) < level) ++arrivals;
-        for (int a = 0; a < arrivals; ++a) {
-            uint32_t p = s;
-            for (;;) {
-                const uint32_t old = __hip_atomic_fetch_add(counters + p, 1u, __ATOMIC_ACQ_REL,
-                                                            __HIP_MEMORY_SCOPE_WORKGROUP);
-                if ((old & kCountMask) == 0u) break;
-                const uint32_t pw = children[p];
-                const float4* rec = nodes + 4 * static_cast<size_t>(pw >> 2);
-                const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
-                const Box lb{r0.x, r0.y, r0.z, r0.w, r1.x, r1.y};
-                const Box rb{r1.z, r1.w, r2.x, r2.y, r2.z, r2.w};
-                const Box b = unite(lb, rb);
-                const uint32_t pp = parents_internal[p];
-                if (pp == kInvalid) {
-                    store_root(root_box + 6 * static_cast<size_t>(scene_of[p]), b);
-                    break;
-                }
-                store_slot(nodes, children[pp], (children[pp] >> 2) == p, b, pw);
-                if ((counters[pp] >> kLevelShift) != level) break;
-                p = pp;
-            }
-        }
+// The elements of one workgroup (leaves or open subtrees) and the subtrees
+// waiting for their siblings.  Boundary x lies before element x (boundary CAP
+// at most: after the last).  A subtree over elements [e0, e1] waits in slot e1
+// as a left child and in slot e0 as a right child, facing its sibling; before
+// that the slot belonged to one of its own parts.  Whole waves issue a step's
+// instructions until their last lane stops, and those bound the leaf kernel,
+// so a step has no branch but its exits and moves a slot as two 16-byte
+// accesses.
+template <uint32_t CAP>
+struct TreeStage {
+    float4 lo[CAP];            // min.x, max.x, min.y, max.y
+    float4 hi[CAP];            // min.z, max.z, child word, the far end and the delta beyond it (far_word)
+    int32_t delta[CAP + 1];    // across boundary x
+    uint32_t at[CAP + 1];      // arrivals at boundary x: 1 from the left, 16 from the right
+    uint32_t open[CAP];        // slot of an open subtree: 1 a left child, 2 a right child
+
+    static __device__ __forceinline__ uint32_t far_word(uint32_t far, int32_t d) {
+        return far | static_cast<uint32_t>(d + 1) << 16;
     }
-}
-
-// The same refit with the list staged in LDS (lists of up to kStageCap
-// nodes): every listed node's record (the child boxes the earlier phases
-// stored), its parent and its count of same-level children are gathered
-// first, so the climb itself touches only LDS.  Each completed node's
-// record is written whole; a box whose parent belongs to a later phase also
-// goes into that parent's record.
-constexpr uint32_t kStageCap = 1024;
-constexpr uint32_t kUpOutside = 0xffffffffu;  // parent handled by a later phase, or none
-
-struct LevelStage {
-    float box[14][kStageCap];  // the record: left child box, then right, then their words
-    uint32_t node[kStageCap];  // the listed node
-    uint32_t word[kStageCap];  // its child word
-    uint32_t par[kStageCap];   // its parent (kInvalid at a scene root)
-    uint32_t up[kStageCap];    // parent's slot << 1 | right side, or kUpOutside
-    uint32_t wait[kStageCap];  // same-level children not yet complete
+    __device__ __forceinline__ void put(uint32_t k, const Box& b, uint32_t word, uint32_t fw) {
+        lo[k] = make_float4(b.mnx, b.mxx, b.mny, b.mxy);
+        hi[k] = make_float4(b.mnz, b.mxz, __uint_as_float(word), __uint_as_float(fw));
+    }
+    __device__ __forceinline__ Box get(uint32_t k, uint32_t& word, uint32_t& fw) const {
+        const float4 l = lo[k], h = hi[k];
+        word = __float_as_uint(h.z);
+        fw = __float_as_uint(h.w);
+        return Box{l.x, l.y, l.z, l.w, h.x, h.y};
+    }
 };
+static_assert(kMergeCap <= 65536, "a slot's far end takes 16 bits");
 
-// A listed node's links: its child word, parent, the parent's slot in the
-// same list (or kUpOutside) and its number of same-level children.
-struct Links {
-    uint32_t word, par, up, wait;
-};
-
-__device__ __forceinline__ Links node_links(uint32_t s, const uint32_t* __restrict__ children,
-                                            const uint32_t* __restrict__ parents_internal,
-                                            const uint32_t* __restrict__ counters,
-                                            const uint32_t* __restrict__ slots, const uint32_t* list_start,
-                                            uint32_t level) {
-    Links L;
-    L.word = children[s];
-    const uint32_t l = L.word >> 2, r = l + 1;
-    L.wait = static_cast<uint32_t>((L.word & 1u) && (counters[l] >> kLevelShift) == level) +
-             static_cast<uint32_t>((L.word & 2u) && (counters[r] >> kLevelShift) == level);
-    L.par = parents_internal[s];
-    L.up = kUpOutside;
-    if (L.par != kInvalid && (counters[L.par] >> kLevelShift) == level) {
-        const uint32_t sl = slots[L.par];
-        L.up = ((list_start[sl >> 6] + (sl & 63u)) << 1) | static_cast<uint32_t>((children[L.par] >> 2) != s);
+// Element e's climb.  last_leaf(e): the last leaf of element e.
+template <uint32_t CAP, class LastLeaf>
+__device__ __forceinline__ void climb(TreeStage<CAP>& S, uint32_t e, Box b, uint32_t word, float4* __restrict__ nodes,
+                                      float* __restrict__ root_box, uint32_t* __restrict__ root_word,
+                                      const uint32_t* __restrict__ scene_of, LastLeaf last_leaf) {
+    uint32_t e0 = e, e1 = e;
+    int32_t dl = S.delta[e], dr = S.delta[e + 1u];
+    while ((dl & dr) >= 0) {  // until the subtree is a whole scene (both -1)
+        const uint32_t left = dr > dl ? 1u : 0u;
+        const uint32_t x = left ? e1 + 1u : e0;  // the boundary its sibling lies beyond
+        S.put(x - left, b, word, TreeStage<CAP>::far_word(left ? e0 : e1, left ? dl : dr));
+        // A wave's LDS accesses are carried out in order, so the slot is written
+        // before the arrival counts and read after it without waiting in
+        // between; the fences keep the compiler to that order.  At the outer
+        // boundaries nobody else arrives.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        const uint32_t before = __hip_atomic_fetch_add(&S.at[x], left ? 1u : 16u, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (before == 0u) return;
+        uint32_t sw, sf;
+        const Box sb = S.get(x - 1u + left, sw, sf);
+        const uint32_t far = sf & 0xffffu;
+        const int32_t fard = static_cast<int32_t>(sf >> 16) - 1;
+        e0 = left ? e0 : far;
+        e1 = left ? far : e1;
+        dl = left ? dl : fard;
+        dr = left ? fard : dr;
+        const Box lb{left ? b.mnx : sb.mnx, left ? b.mxx : sb.mxx, left ? b.mny : sb.mny,
+                     left ? b.mxy : sb.mxy, left ? b.mnz : sb.mnz, left ? b.mxz : sb.mxz};
+        const Box rb{left ? sb.mnx : b.mnx, left ? sb.mxx : b.mxx, left ? sb.mny : b.mny,
+                     left ? sb.mxy : b.mxy, left ? sb.mnz : b.mnz, left ? sb.mxz : b.mxz};
+        const uint32_t wl = left ? word : sw, wr = left ? sw : word;
+        word = (last_leaf(x - 1u) << 2) | (wl != kInvalid ? 1u : 0u) | (wr != kInvalid ? 2u : 0u);
+        store_record(nodes, word, lb, rb, wl, wr);
+        b = unite(lb, rb);
     }
-    return L;
+    store_root(root_box, root_word, scene_of ? scene_of[last_leaf(e1)] : 0u, b, word);
 }
 
-__device__ __forceinline__ void stage_links(LevelStage& S, uint32_t idx, uint32_t s, const Links& L) {
-    S.node[idx] = s;
-    S.word[idx] = L.word;
-    S.par[idx] = L.par;
-    S.up[idx] = L.up;
-    S.wait[idx] = L.wait;
-}
-
-// A listed node's two child boxes and words, from its record (stored by
-// earlier phases); w: its child word.
-__device__ __forceinline__ void stage_boxes(LevelStage& S, uint32_t idx, uint32_t w,
-                                            const float4* __restrict__ nodes) {
-    const float4* rec = nodes + 4 * static_cast<size_t>(w >> 2);
-    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
-    const float v[14] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w, r3.x, r3.y};
-    for (int k = 0; k < 14; ++k) S.box[k][idx] = v[k];
-}
-
-// The climb over a staged list (after a barrier): every node with no
-// same-level child starts one; the thread completing a node's second
-// same-level child goes on to the node.
-__device__ __forceinline__ void climb_staged(LevelStage& S, const uint32_t* __restrict__ children,
-                                             const uint32_t* __restrict__ scene_of, float4* __restrict__ nodes,
-                                             float* __restrict__ root_box, uint32_t count) {
-    for (uint32_t first = threadIdx.x; first < count; first += blockDim.x) {
-        if (S.wait[first] != 0u) continue;
-        uint32_t idx = first;
-        for (;;) {
-            const Box lb{S.box[0][idx], S.box[1][idx], S.box[2][idx], S.box[3][idx], S.box[4][idx], S.box[5][idx]};
-            const Box rb{S.box[6][idx], S.box[7][idx], S.box[8][idx], S.box[9][idx], S.box[10][idx], S.box[11][idx]};
-            const Box b = unite(lb, rb);
-            const uint32_t s = S.node[idx];
-            const uint32_t w = S.word[idx];
-            store_record(nodes, w, lb, rb, __float_as_uint(S.box[12][idx]), __float_as_uint(S.box[13][idx]));
-            const uint32_t pp = S.par[idx];
-            if (pp == kInvalid) {
-                store_root(root_box + 6 * static_cast<size_t>(scene_of[s]), b);
-                break;
-            }
-            const uint32_t up = S.up[idx];
-            if (up == kUpOutside) {
-                store_slot(nodes, children[pp], (children[pp] >> 2) == s, b, w);
-                break;
-            }
-            const uint32_t ps = up >> 1;
-            const int o = (up & 1u) ? 6 : 0;
-            S.box[o + 0][ps] = b.mnx; S.box[o + 1][ps] = b.mxx; S.box[o + 2][ps] = b.mny;
-            S.box[o + 3][ps] = b.mxy; S.box[o + 4][ps] = b.mnz; S.box[o + 5][ps] = b.mxz;
-            S.box[12 + (up & 1u)][ps] = __uint_as_float(w);
-            const uint32_t old = __hip_atomic_fetch_sub(&S.wait[ps], 1u, __ATOMIC_ACQ_REL,
-                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (old != 1u) break;  // the other same-level child completes the parent
-            idx = ps;
-        }
-    }
-}
-
-__device__ __forceinline__ void refit_level_staged(LevelStage& S, const uint32_t* __restrict__ children,
-                                                   const uint32_t* __restrict__ scene_of,
-                                                   const uint32_t* __restrict__ parents_internal,
-                                                   const uint32_t* __restrict__ counters,
-                                                   const uint32_t* __restrict__ slots, const uint32_t* list_start,
-                                                   float4* __restrict__ nodes, float* __restrict__ root_box,
-                                                   const uint32_t* list, uint32_t count, uint32_t level) {
-    for (uint32_t idx = threadIdx.x; idx < count; idx += blockDim.x) {
-        const uint32_t s = list[idx];
-        stage_boxes(S, idx, children[s], nodes);
-        stage_links(S, idx, s, node_links(s, children, parents_internal, counters, slots, list_start, level));
+// After a barrier: the subtrees left waiting for a sibling outside.
+template <uint32_t CAP>
+__device__ __forceinline__ void mark_open(TreeStage<CAP>& S, uint32_t count) {
+    for (uint32_t x = threadIdx.x; x <= count; x += blockDim.x) {
+        const uint32_t a = S.at[x];
+        if (a == 1u) S.open[x - 1u] = 1u;
+        else if (a == 16u) S.open[x] = 2u;
     }
     __syncthreads();
-    climb_staged(S, children, scene_of, nodes, root_box, count);
 }
 
-// The lists of one level, concatenated in LDS-held order: list k starts at
-// start[k] (exclusive prefix of the counts, one thread per list).
-__device__ __forceinline__ uint32_t concat_lists(const uint32_t* __restrict__ counts, uint32_t nlists,
-                                                 const uint32_t* __restrict__ lists, uint32_t* start,
-                                                 uint32_t* out, uint32_t* status) {
-    __shared__ uint32_t s_carry;
+// One workgroup per kLeafBlock sorted leaves, one thread per leaf: the leaf's
+// triangle is gathered through the sort permutation into its 48-byte record
+// (the reference instead permutes the 40-byte triangles inside the sort), then
+// climbs.  2^20 soup triangles take 63 us: without the climb (gather, a random
+// 40-byte read per leaf, and triangle records) 36, the record stores add 14,
+// the climb's steps the rest; with the triangles already in order 50.
+__global__ __launch_bounds__(kLeafBlock) void k_tree_leaves(
+    const pt_triangle* __restrict__ in_tris, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ perm,
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ scene_of, uint32_t n,
+    float4* __restrict__ nodes, float4* __restrict__ tri_recs, float* __restrict__ root_box,
+    uint32_t* __restrict__ root_word, OpenList* __restrict__ lists, uint32_t* __restrict__ status) {
+    __shared__ TreeStage<kLeafBlock> S;
     __shared__ uint32_t s_w[16];
-    if (threadIdx.x == 0) s_carry = 0u;
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t b0 = 0; b0 < nlists; b0 += blockDim.x) {
-        const uint32_t k = b0 + threadIdx.x;
-        uint32_t c = 0;
-        if (k < nlists) {
-            c = counts[k];
-            if (c > kListCap) {  // counted past a full list (flagged by the append)
-                raise_status(status, PT_STATUS_REFIT_OVERFLOW);
-                c = kListCap;
-            }
+    const uint32_t tid = threadIdx.x;
+    const uint32_t base = blockIdx.x * kLeafBlock;
+    const uint32_t count = min(kLeafBlock, n - base);
+    const uint32_t k = base + tid;
+    S.at[tid] = 0u;
+    if (tid == 0u) S.at[kLeafBlock] = 0u;
+    S.open[tid] = 0u;
+    Box b{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    // delta between leaves i and i + 1 (scene_of null: one scene).
+    auto delta_after = [&](uint32_t i) -> int32_t {
+        if (i + 1u >= n) return -1;
+        uint32_t first = 0u;
+        if (scene_of) {
+            const uint32_t sc = scene_of[i];
+            if (scene_of[i + 1u] != sc) return -1;
+            first = off[sc];
         }
+        const uint32_t ka = keys[i], kb = keys[i + 1u];
+        if (ka == kb) return 32 + __clz(static_cast<int>((i - first) ^ (i + 1u - first)));
+        return __clz(static_cast<int>(ka ^ kb));
+    };
+    if (tid < count) {
+        const pt_triangle* t = in_tris + perm[k];
+        const V3 v0 = v3(t->v0[0], t->v0[1], t->v0[2]);
+        const V3 v1 = v3(t->v1[0], t->v1[1], t->v1[2]);
+        const V3 v2 = v3(t->v2[0], t->v2[1], t->v2[2]);
+        const uint32_t id = t->id;
+        S.delta[tid + 1u] = delta_after(k);
+        if (tid == 0u) S.delta[0] = base > 0u ? delta_after(base - 1u) : -1;
+        const V3 e1 = sub(v1, v0), e2 = sub(v2, v0);
+        tri_recs[3 * static_cast<size_t>(k) + 0] = make_float4(v0.x, v0.y, v0.z, __uint_as_float(id));
+        tri_recs[3 * static_cast<size_t>(k) + 1] = make_float4(e1.x, e1.y, e1.z, 0.0f);
+        tri_recs[3 * static_cast<size_t>(k) + 2] = make_float4(e2.x, e2.y, e2.z, 0.0f);
+        // BBox() then unite({v0, v1, v2}) (BBox.cpp:4-6, 14-24).
+        b.mnx = gmin(gmin(gmin(kFltMax, v0.x), v1.x), v2.x);
+        b.mny = gmin(gmin(gmin(kFltMax, v0.y), v1.y), v2.y);
+        b.mnz = gmin(gmin(gmin(kFltMax, v0.z), v1.z), v2.z);
+        b.mxx = gmax(gmax(gmax(-kFltMax, v0.x), v1.x), v2.x);
+        b.mxy = gmax(gmax(gmax(-kFltMax, v0.y), v1.y), v2.y);
+        b.mxz = gmax(gmax(gmax(-kFltMax, v0.z), v1.z), v2.z);
+    }
+    __syncthreads();
+    if (tid < count)
+        climb(S, tid, b, kInvalid, nodes, root_box, root_word, scene_of, [&](uint32_t e) { return base + e; });
+    __syncthreads();
+    mark_open(S, count);
+    const uint32_t o = tid < count ? S.open[tid] : 0u;
+    uint32_t total;
+    const uint32_t pos = block_excl_scan<kLeafBlock / 64>(o ? 1u : 0u, s_w, total);
+    OpenList& L = lists[blockIdx.x];
+    if (tid == 0u) {
+        L.count = min(total, kOpenCap);
+        if (total > kOpenCap) raise_status(status, PT_STATUS_REFIT_OVERFLOW);  // bound argued above
+    }
+    if (o && pos < kOpenCap) {
+        uint32_t word, fw;
+        const Box ob = S.get(tid, word, fw);
+        const uint32_t end = o == 1u ? tid : fw & 0xffffu;
+        L.put(pos, base + end, S.delta[end + 1u], word, ob);
+    }
+}
+
+// One workgroup per kFanIn lists of the level below: their open subtrees as
+// elements, in order, climb on; what is still open goes to this level's list.
+// Bound by the longest chain of climb steps (19 in a 16-block part of the
+// 2^20-triangle soup), each a few LDS round trips, so the fan-in is of little
+// weight: 2^20 triangles build in 183 / 178 / 178 / 179 us at 8 / 16 / 32 / 64,
+// 2.88M in 376 / 363 / 372 / 379.
+__global__ __launch_bounds__(kMergeThreads) void k_tree_merge(const OpenList* __restrict__ in, uint32_t nlists,
+                                                              const uint32_t* __restrict__ scene_of,
+                                                              float4* __restrict__ nodes,
+                                                              float* __restrict__ root_box,
+                                                              uint32_t* __restrict__ root_word,
+                                                              OpenList* __restrict__ out,
+                                                              uint32_t* __restrict__ status) {
+    constexpr uint32_t kPer = kMergeCap / kMergeThreads;
+    __shared__ TreeStage<kMergeCap> S;
+    __shared__ uint32_t s_last[kMergeCap];  // last leaf of element e
+    __shared__ uint32_t s_start[kFanIn + 1];
+    __shared__ uint32_t s_w[kMergeThreads / 64];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t k0 = blockIdx.x * kFanIn;
+    if (tid < 64u) {  // the lists' places: an exclusive scan of their counts
+        const uint32_t c = tid < kFanIn && k0 + tid < nlists ? in[k0 + tid].count : 0u;
         uint32_t x = c;
+#pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
+            if (tid >= static_cast<uint32_t>(o)) x += y;
         }
-        if (lane == 63) s_w[wave] = x;
-        __syncthreads();
-        uint32_t pre = s_carry;
-        for (int w = 0; w < wave; ++w) pre += s_w[w];
-        if (k < nlists) start[k] = pre + x - c;
-        __syncthreads();
-        if (threadIdx.x == blockDim.x - 1) s_carry = pre + x;
-        __syncthreads();
-    }
-    const uint32_t total = s_carry;
-    if (threadIdx.x == 0) start[nlists] = total;
-    __syncthreads();
-    for (uint32_t e = threadIdx.x; e < nlists * kListCap; e += blockDim.x) {
-        const uint32_t k = e / kListCap, j = e % kListCap;
-        if (j < start[k + 1] - start[k]) out[start[k] + j] = lists[static_cast<size_t>(k) * kListCap + j];
+        if (tid < kFanIn) s_start[tid + 1u] = x;
+        if (tid == 0u) s_start[0] = 0u;
+    } else if (tid == 64u) {  // before the first list: the level's previous element, or a scene's start
+        const uint32_t c = k0 > 0u ? in[k0 - 1u].count : 0u;
+        S.delta[0] = c > 0u ? in[k0 - 1u].delta[c - 1u] : -1;
+        S.at[0] = 0u;
     }
     __syncthreads();
-    return total;
-}
-
-// Level-1 links prepared by k_refit_local's last workgroups, per 65536-leaf
-// block: [0] the block's list length, then per listed node the node, its
-// child word, parent, parent's slot and same-level child count (kStageCap
-// each).
-constexpr uint32_t kMidLinksWords = 1 + 5 * kStageCap;
-static_assert(sizeof(LdsBoxes) >= 4 * kMidCap, "level-1 list staging fits in a box array");
-
-// Refit, phase 1 (compute_internal_node_bbox_kernel, BVHBuilder.cu:54-91):
-// one thread per sorted leaf, one workgroup per block of kRefitBlock leaves.
-// The leaf writes its sorted triangle record (the reference instead permutes
-// the 40-byte triangles inside the sort), then climbs: the first thread to
-// reach a node stops, the second unites the two child boxes.  Every node
-// below the spanning ones has its whole leaf range -- hence both children --
-// inside the block, so counters and boxes live in LDS and the hand-off needs
-// only workgroup-scope ordering.  The thread completing a node writes the
-// node's whole traversal record (both child boxes, leaves' included, and the
-// child word); a box whose parent is finished by a later phase is also
-// stored into that parent's record.  A node inside the block has its index
-// inside its leaf range, so the block's nodes are the indices [base, base +
-// kRefitBlock): their child words, parents and levels are loaded into LDS
-// once, coalesced, and the climb reads no global memory.  The launch's last
-// mid_blocks workgroups instead concatenate each 65536-leaf block's level-1
-// lists and stage their links (children, parents, counters and slots, none
-// of which this launch writes) into mid_links for k_refit_mid.
-__global__ __launch_bounds__(kRefitBlock) void k_refit_local(
-    const pt_triangle* __restrict__ in_tris, const uint32_t* __restrict__ perm,
-    const uint32_t* __restrict__ off, const uint32_t* __restrict__ scene_of,
-    const uint32_t* __restrict__ children, uint32_t* __restrict__ parents_leaf,
-    const uint32_t* __restrict__ parents_internal, const uint32_t* __restrict__ counters,
-    float4* __restrict__ nodes, float4* __restrict__ tri_recs, float* __restrict__ root_box,
-    uint32_t n, const uint32_t* __restrict__ span_list, const uint32_t* __restrict__ span_count,
-    const uint32_t* __restrict__ slots, uint32_t stage_max, uint32_t* __restrict__ mid_links,
-    uint32_t* __restrict__ status) {
-    __shared__ uint32_t s_cnt[kRefitBlock];
-    __shared__ uint32_t s_word[kRefitBlock];   // child word of node base + j
-    __shared__ uint32_t s_par[kRefitBlock];    // its parent
-    __shared__ uint32_t s_local[kRefitBlock];  // 1: refit here (level 0)
-    __shared__ LdsBoxes s_leaf;
-    __shared__ LdsBoxes s_node;
-    const int tid = threadIdx.x;
-    const uint32_t n_lists1 = (n + kRefitBlock - 1) / kRefitBlock;
-    if (blockIdx.x >= n_lists1) {  // level-1 link staging for 65536-leaf block m
-        constexpr uint32_t kLists = kMidBlock / kRefitBlock;
-        const uint32_t m = blockIdx.x - n_lists1;
-        uint32_t* s_list = reinterpret_cast<uint32_t*>(&s_leaf);   // kMidCap words
-        uint32_t* s_start = reinterpret_cast<uint32_t*>(&s_node);  // kLists + 1 words
-        const uint32_t k0 = m * kLists;
-        const uint32_t count = concat_lists(span_count + k0, min(kLists, n_lists1 - k0),
-                                            span_list + static_cast<size_t>(k0) * kListCap, s_start, s_list, status);
-        uint32_t* out = mid_links + static_cast<size_t>(m) * kMidLinksWords;
-        if (tid == 0) out[0] = count;
-        if (count > stage_max) return;
-        for (uint32_t idx = tid; idx < count; idx += kRefitBlock) {
-            const uint32_t sn = s_list[idx];
-            const Links L = node_links(sn, children, parents_internal, counters, slots, s_start, 1u);
-            out[1 + idx] = sn;
-            out[1 + kStageCap + idx] = L.word;
-            out[1 + 2 * kStageCap + idx] = L.par;
-            out[1 + 3 * kStageCap + idx] = L.up;
-            out[1 + 4 * kStageCap + idx] = L.wait;
-        }
-        return;
-    }
-    const uint32_t base = blockIdx.x * kRefitBlock;
-    const uint32_t k = base + tid;
-    s_cnt[tid] = 0u;
-    if (k < n) {
-        s_word[tid] = children[k];
-        s_par[tid] = parents_internal[k];
-        s_local[tid] = (counters[k] >> kLevelShift) == 0u ? 1u : 0u;
-    } else {
-        s_local[tid] = 0u;
+    const uint32_t count = s_start[kFanIn];
+    Box b[kPer];
+    uint32_t w[kPer];
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; ++q) {
+        const uint32_t e = tid + q * kMergeThreads;
+        if (e >= count) continue;
+        uint32_t l = 0u;  // the last list that starts at or before e
+#pragma unroll
+        for (uint32_t h = kFanIn / 2; h > 0u; h >>= 1)
+            if (s_start[l + h] <= e) l += h;
+        const OpenList& L = in[k0 + l];
+        const uint32_t j = e - s_start[l];
+        b[q] = Box{L.box[0][j], L.box[1][j], L.box[2][j], L.box[3][j], L.box[4][j], L.box[5][j]};
+        w[q] = L.word[j];
+        s_last[e] = L.hi[j];
+        S.delta[e + 1u] = L.delta[j];
+        S.at[e + 1u] = 0u;
+        S.open[e] = 0u;
     }
     __syncthreads();
-    if (k >= n) return;
-    // Node q is refit by this block: inside [base, base + kRefitBlock) and of level 0.
-    auto local = [&](uint32_t q) { return q - base < static_cast<uint32_t>(kRefitBlock) && s_local[q - base]; };
-    const pt_triangle* t = in_tris + perm[k];
-    const V3 v0 = v3(t->v0[0], t->v0[1], t->v0[2]);
-    const V3 v1 = v3(t->v1[0], t->v1[1], t->v1[2]);
-    const V3 v2 = v3(t->v2[0], t->v2[1], t->v2[2]);
-    const uint32_t id = t->id;
-    const V3 e1 = sub(v1, v0), e2 = sub(v2, v0);
-    tri_recs[3 * static_cast<size_t>(k) + 0] = make_float4(v0.x, v0.y, v0.z, __uint_as_float(id));
-    tri_recs[3 * static_cast<size_t>(k) + 1] = make_float4(e1.x, e1.y, e1.z, 0.0f);
-    tri_recs[3 * static_cast<size_t>(k) + 2] = make_float4(e2.x, e2.y, e2.z, 0.0f);
-    // BBox() then unite({v0, v1, v2}) (BBox.cpp:4-6, 14-24).
-    Box b;
-    b.mnx = gmin(gmin(gmin(kFltMax, v0.x), v1.x), v2.x);
-    b.mny = gmin(gmin(gmin(kFltMax, v0.y), v1.y), v2.y);
-    b.mnz = gmin(gmin(gmin(kFltMax, v0.z), v1.z), v2.z);
-    b.mxx = gmax(gmax(gmax(-kFltMax, v0.x), v1.x), v2.x);
-    b.mxy = gmax(gmax(gmax(-kFltMax, v0.y), v1.y), v2.y);
-    b.mxz = gmax(gmax(gmax(-kFltMax, v0.z), v1.z), v2.z);
-    const uint32_t sc = scene_of[k];
-    if (off[sc + 1] - off[sc] == 1) {  // one-triangle scene: no internal node
-        parents_leaf[k] = kInvalid;
-        store_root(root_box + 6 * static_cast<size_t>(sc), b);
-        return;
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; ++q) {
+        const uint32_t e = tid + q * kMergeThreads;
+        if (e < count) climb(S, e, b[q], w[q], nodes, root_box, root_word, scene_of, [&](uint32_t x) { return s_last[x]; });
     }
-    s_leaf.put(tid, b);
-    uint32_t p = parents_leaf[k];
-    if (!local(p)) {
-        store_slot(nodes, children[p], (children[p] >> 2) == k, b, 0u);  // finished by a later phase
-        return;
+    __syncthreads();
+    mark_open(S, count);
+    OpenList& L = out[blockIdx.x];
+    uint32_t kept = 0u;
+    for (uint32_t e0 = 0u; e0 < count; e0 += kMergeThreads) {
+        const uint32_t e = e0 + tid;
+        const uint32_t o = e < count ? S.open[e] : 0u;
+        uint32_t total;
+        const uint32_t pos = kept + block_excl_scan<kMergeThreads / 64>(o ? 1u : 0u, s_w, total);
+        if (o && pos < kOpenCap) {
+            uint32_t word, fw;
+            const Box ob = S.get(e, word, fw);
+            const uint32_t end = o == 1u ? e : fw & 0xffffu;
+            L.put(pos, s_last[end], S.delta[end + 1u], word, ob);
+        }
+        kept += total;
     }
-    for (;;) {
-        const uint32_t old = __hip_atomic_fetch_add(s_cnt + (p - base), 1u, __ATOMIC_ACQ_REL,
-                                                    __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (old == 0u) return;
-        const uint32_t w = s_word[p - base];
-        const uint32_t l = w >> 2, r = l + 1;
-        const Box lb = (w & 1u) ? s_node.get(l - base) : s_leaf.get(l - base);
-        const Box rb = (w & 2u) ? s_node.get(r - base) : s_leaf.get(r - base);
-        b = unite(lb, rb);
-        s_node.put(p - base, b);
-        store_record(nodes, w, lb, rb, (w & 1u) ? s_word[l - base] : 0u, (w & 2u) ? s_word[r - base] : 0u);
-        const uint32_t pp = s_par[p - base];
-        if (pp == kInvalid) {
-            store_root(root_box + 6 * static_cast<size_t>(scene_of[p]), b);
-            return;
-        }
-        if (!local(pp)) {  // finished by a later phase, from its record
-            store_slot(nodes, children[pp], (children[pp] >> 2) == p, b, w);
-            return;
-        }
-        p = pp;
+    if (tid == 0u) {
+        L.count = min(kept, kOpenCap);
+        if (kept > kOpenCap) raise_status(status, PT_STATUS_REFIT_OVERFLOW);  // bound argued above
     }
 }
 
-// The level-2 stage prepared by k_refit_mid's last workgroup for k_refit_top:
-// [0] the list's length, then per listed node its child word, parent,
-// parent's slot and same-level child count (kStageCap each).
-constexpr uint32_t kTopLinksWords = 1 + 4 * kStageCap;
-
-// Level-1 nodes: one workgroup per 65536-leaf block (its 64 lists).  With
-// level-2 nodes present, one more workgroup concatenates their lists into
-// top_list and stages their links (children, parents, counters and slots,
-// none of which this launch writes) into top_links, so that k_refit_top
-// only has to gather the child boxes.
-__global__ __launch_bounds__(1024) void k_refit_mid(const uint32_t* __restrict__ children,
-                                                    const uint32_t* __restrict__ scene_of,
-                                                    const uint32_t* __restrict__ parents_internal,
-                                                    uint32_t* __restrict__ counters,
-                                                    float4* __restrict__ nodes,
-                                                    float* __restrict__ root_box,
-                                                    const uint32_t* __restrict__ span_list,
-                                                    const uint32_t* __restrict__ span_count, uint32_t n_lists1,
-                                                    const uint32_t* __restrict__ span_top, uint32_t n_lists2,
-                                                    uint32_t* __restrict__ top_list, uint32_t* __restrict__ top_links,
-                                                    const uint32_t* __restrict__ mid_links,
-                                                    const uint32_t* __restrict__ slots, uint32_t stage_max,
-                                                    uint32_t* __restrict__ status) {
-    constexpr uint32_t kLists = kMidBlock / kRefitBlock;
-    __shared__ LevelStage S;
-    __shared__ uint32_t s_buf[kMaxMidBlocks + 1 > kMidCap + kLists + 1 ? kMaxMidBlocks + 1 : kMidCap + kLists + 1];
-    const uint32_t n_mid = (n_lists1 + kLists - 1) / kLists;
-    if (blockIdx.x == n_mid) {  // the level-2 preparation
-        uint32_t* s_start = s_buf;
-        const uint32_t count = concat_lists(span_count + n_lists1, n_lists2, span_top, s_start, top_list, status);
-        if (threadIdx.x == 0) top_links[0] = count;
-        if (count > stage_max) return;
-        for (uint32_t idx = threadIdx.x; idx < count; idx += blockDim.x) {
-            const Links L = node_links(top_list[idx], children, parents_internal, counters, slots, s_start, 2u);
-            top_links[1 + idx] = L.word;
-            top_links[1 + kStageCap + idx] = L.par;
-            top_links[1 + 2 * kStageCap + idx] = L.up;
-            top_links[1 + 3 * kStageCap + idx] = L.wait;
-        }
-        return;
+// Parity dump of scene [base, base + n): the reference's arrays in local
+// indices, from the records.  The record of the node that splits after leaf s
+// sits in slot s; its left child, if internal, is node s, its right child node
+// s + 1, and the root is node 0.  First each node's child word and box (min.xyz,
+// max.xyz) from its parent's record, and owner[s]: the number of the node that
+// splits after s.
+__global__ __launch_bounds__(256) void k_dump_nodes(const float4* __restrict__ nodes,
+                                                    const uint32_t* __restrict__ root_word,
+                                                    const float* __restrict__ root_box, uint32_t base, uint32_t n,
+                                                    float* __restrict__ out_boxes, uint32_t* __restrict__ out_children,
+                                                    uint32_t* __restrict__ owner) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s + 1 >= n) return;
+    const uint32_t lb = base << 2;
+    if (s == 0) {
+        const uint32_t w = root_word[0] - lb;
+        out_children[0] = w;
+        owner[w >> 2] = 0u;
+        for (int k = 0; k < 6; ++k) out_boxes[k] = root_box[k];
     }
-    const uint32_t* links = mid_links + static_cast<size_t>(blockIdx.x) * kMidLinksWords;
-    const uint32_t staged = links[0];
-    if (staged <= stage_max) {
-        for (uint32_t idx = threadIdx.x; idx < staged; idx += blockDim.x) {
-            const uint32_t sn = links[1 + idx];
-            S.node[idx] = sn;
-            S.word[idx] = links[1 + kStageCap + idx];
-            S.par[idx] = links[1 + 2 * kStageCap + idx];
-            S.up[idx] = links[1 + 3 * kStageCap + idx];
-            S.wait[idx] = links[1 + 4 * kStageCap + idx];
-            stage_boxes(S, idx, S.word[idx], nodes);
-        }
-        __syncthreads();
-        climb_staged(S, children, scene_of, nodes, root_box, staged);
-        return;
-    }
-    uint32_t* s_list = s_buf;
-    uint32_t* s_start = s_buf + kMidCap;
-    const uint32_t k0 = blockIdx.x * kLists;
-    const uint32_t count = concat_lists(span_count + k0, min(kLists, n_lists1 - k0),
-                                        span_list + static_cast<size_t>(k0) * kListCap, s_start, s_list, status);
-    refit_level(children, scene_of, parents_internal, counters, nodes, root_box, s_list, count, 1u);
-}
-
-// Level-2 nodes: one workgroup, over the list and links k_refit_mid prepared.
-__global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__ children,
-                                                    const uint32_t* __restrict__ scene_of,
-                                                    const uint32_t* __restrict__ parents_internal,
-                                                    uint32_t* __restrict__ counters,
-                                                    float4* __restrict__ nodes,
-                                                    float* __restrict__ root_box,
-                                                    const uint32_t* __restrict__ top_list,
-                                                    const uint32_t* __restrict__ top_links, uint32_t stage_max) {
-    __shared__ LevelStage S;
-    const uint32_t count = top_links[0];
-    if (count <= stage_max) {
-        for (uint32_t idx = threadIdx.x; idx < count; idx += blockDim.x) {
-            const uint32_t s = top_list[idx];
-            S.node[idx] = s;
-            S.word[idx] = top_links[1 + idx];
-            S.par[idx] = top_links[1 + kStageCap + idx];
-            S.up[idx] = top_links[1 + 2 * kStageCap + idx];
-            S.wait[idx] = top_links[1 + 3 * kStageCap + idx];
-            stage_boxes(S, idx, S.word[idx], nodes);
-        }
-        __syncthreads();
-        climb_staged(S, children, scene_of, nodes, root_box, count);
-    } else {
-        refit_level(children, scene_of, parents_internal, counters, nodes, root_box, top_list, count, 2u);
-    }
-}
-
-// Parity dump of scene [base, base + n): internal node boxes in the
-// reference's BBox layout (min.xyz, max.xyz), read back from the parents'
-// records, plus the child and parent words converted to local indices.
-__global__ __launch_bounds__(256) void k_dump_scene(const float4* __restrict__ nodes,
-                                                    const uint32_t* __restrict__ children,
-                                                    const uint32_t* __restrict__ parents_leaf,
-                                                    const uint32_t* __restrict__ parents_internal,
-                                                    const float* __restrict__ root_box, uint32_t base,
-                                                    uint32_t n, float* __restrict__ out_boxes,
-                                                    uint32_t* __restrict__ out_children,
-                                                    uint32_t* __restrict__ out_pl,
-                                                    uint32_t* __restrict__ out_pi) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n) {
-        const uint32_t p = parents_leaf[base + c];
-        out_pl[c] = p == kInvalid ? kInvalid : p - base;
-    }
-    if (c + 1 >= n) return;
-    const uint32_t g = base + c;
-    out_children[c] = children[g] - (base << 2);
-    const uint32_t pg = parents_internal[g];
-    out_pi[c] = pg == kInvalid ? kInvalid : pg - base;
-    float* o = out_boxes + 6 * static_cast<size_t>(c);
-    if (pg == kInvalid) {
-        for (int k = 0; k < 6; ++k) o[k] = root_box[k];
-        return;
-    }
-    const float4* rec = nodes + 4 * static_cast<size_t>(children[pg] >> 2);
-    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
-    if ((children[pg] >> 2) == g) {
+    const float4* rec = nodes + 4 * static_cast<size_t>(base + s);
+    const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
+    const uint32_t wl = __float_as_uint(r3.x), wr = __float_as_uint(r3.y);
+    if (wl != kInvalid) {
+        out_children[s] = wl - lb;
+        owner[(wl - lb) >> 2] = s;
+        float* o = out_boxes + 6 * static_cast<size_t>(s);
         o[0] = r0.x; o[1] = r0.z; o[2] = r1.x; o[3] = r0.y; o[4] = r0.w; o[5] = r1.y;
-    } else {
+    }
+    if (wr != kInvalid) {
+        out_children[s + 1] = wr - lb;
+        owner[(wr - lb) >> 2] = s + 1;
+        float* o = out_boxes + 6 * static_cast<size_t>(s + 1);
         o[0] = r1.z; o[1] = r2.x; o[2] = r2.z; o[3] = r1.w; o[4] = r2.y; o[5] = r2.w;
     }
+}
+
+// Then the parents.
+__global__ __launch_bounds__(256) void k_dump_parents(const float4* __restrict__ nodes,
+                                                      const uint32_t* __restrict__ owner, uint32_t base, uint32_t n,
+                                                      uint32_t* __restrict__ out_pl, uint32_t* __restrict__ out_pi) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) (n == 1 ? out_pl : out_pi)[0] = kInvalid;  // BVHBuilder.cu:224
+    if (s + 1 >= n) return;
+    const uint2 w = *reinterpret_cast<const uint2*>(nodes + 4 * static_cast<size_t>(base + s) + 3);
+    const uint32_t p = owner[s];
+    (w.x != kInvalid ? out_pi : out_pl)[s] = p;
+    (w.y != kInvalid ? out_pi : out_pl)[s + 1] = p;
 }
 
 __global__ __launch_bounds__(256) void k_sub_u32(const uint32_t* __restrict__ in, uint32_t sub,
@@ -1049,31 +764,24 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     b.keys_alt.reserve(n4);
     b.vals_alt.reserve(n4);
     b.scene_of.reserve(n4);
-    b.children.reserve(n4);
-    b.parents_leaf.reserve(n4);
-    b.parents_internal.reserve(n4);
-    b.counters.reserve(n4);
     b.nodes.reserve(static_cast<size_t>(n) * 64);
     b.tris.reserve(static_cast<size_t>(n) * 48);
     b.root_box.reserve(static_cast<size_t>(nscenes) * 6 * sizeof(float));
+    b.root_word.reserve(static_cast<size_t>(nscenes) * 4);
     const uint32_t num_tiles = div_up(n, kSortTile);
     b.tile_hist.reserve(static_cast<size_t>(num_tiles) * kRadix * 4);
     b.digit_total.reserve(kRadix * 4);
-    const uint32_t mid_blocks = div_up(n, kMidBlock);
-    const uint32_t n_lists1 = div_up(n, kRefitBlock);
-    b.span_list.reserve(static_cast<size_t>(n_lists1) * kListCap * 4);
-    b.span_top.reserve(static_cast<size_t>(mid_blocks) * kListCap * 4 * 2);  // lists, then their concatenation
-    b.span_count.reserve((static_cast<size_t>(n_lists1) + mid_blocks) * 4);
-    b.top_links.reserve(kTopLinksWords * 4);
-    b.mid_links.reserve(static_cast<size_t>(mid_blocks) * kMidLinksWords * 4);
-    b.slots.reserve(n4);
+    // Open lists of every level, one after the other.
+    const uint32_t blocks = div_up(n, kLeafBlock);
+    size_t nlists = blocks;
+    for (uint32_t m = blocks; m > 1; m = div_up(m, kFanIn)) nlists += div_up(m, kFanIn);
+    b.open_lists.reserve(nlists * sizeof(OpenList));
 
     uint32_t* kin = b.keys.as<uint32_t>();
     uint32_t* vin = b.vals.as<uint32_t>();
     hipLaunchKernelGGL(k_morton, dim3(num_tiles), dim3(kMortonThreads), 0, st, s.tris.as<pt_triangle>(), n,
                        s.off.as<uint32_t>(), nscenes, s.morton_box.as<float>(), kin, vin,
-                       b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>(), b.span_count.as<uint32_t>(),
-                       n_lists1 + mid_blocks);
+                       b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>());
     PT_HIP(hipGetLastError());
 
     if (n >= 2) {
@@ -1116,40 +824,19 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
             swap(b.vals, b.vals_alt);
         }
         PT_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_radix_tree, dim3(div_up(n, 256)), dim3(256), 0, st, b.keys.as<uint32_t>(), n,
-                           s.off.as<uint32_t>(), b.scene_of.as<uint32_t>(), b.children.as<uint32_t>(),
-                           b.parents_leaf.as<uint32_t>(), b.parents_internal.as<uint32_t>(),
-                           b.counters.as<uint32_t>(), b.nodes.as<float4>(), b.span_list.as<uint32_t>(),
-                           b.span_top.as<uint32_t>(), b.span_count.as<uint32_t>(), n_lists1,
-                           b.slots.as<uint32_t>(), s.status.as<uint32_t>());
-        PT_HIP(hipGetLastError());
     }
-    const uint32_t stage_max = build_tuning().staged ? kStageCap : 0u;
-    // With level-1 nodes present, mid_blocks more workgroups stage their links.
-    const uint32_t mid_prep = n > static_cast<uint32_t>(kRefitBlock) ? mid_blocks : 0u;
-    hipLaunchKernelGGL(k_refit_local, dim3(n_lists1 + mid_prep), dim3(kRefitBlock), 0, st,
-                       s.tris.as<pt_triangle>(), b.vals.as<uint32_t>(), s.off.as<uint32_t>(),
-                       b.scene_of.as<uint32_t>(), b.children.as<uint32_t>(),
-                       b.parents_leaf.as<uint32_t>(), b.parents_internal.as<uint32_t>(),
-                       b.counters.as<uint32_t>(), b.nodes.as<float4>(), b.tris.as<float4>(),
-                       b.root_box.as<float>(), n, b.span_list.as<uint32_t>(), b.span_count.as<uint32_t>(),
-                       b.slots.as<uint32_t>(), stage_max, b.mid_links.as<uint32_t>(), s.status.as<uint32_t>());
-    if (n > static_cast<uint32_t>(kRefitBlock)) {
-        // One more workgroup prepares the level-2 refit when there is one.
-        const uint32_t top = n > kMidBlock ? 1u : 0u;
-        uint32_t* top_list = b.span_top.as<uint32_t>() + static_cast<size_t>(mid_blocks) * kListCap;
-        hipLaunchKernelGGL(k_refit_mid, dim3(mid_blocks + top), dim3(1024), 0, st, b.children.as<uint32_t>(),
-                           b.scene_of.as<uint32_t>(), b.parents_internal.as<uint32_t>(),
-                           b.counters.as<uint32_t>(), b.nodes.as<float4>(), b.root_box.as<float>(),
-                           b.span_list.as<uint32_t>(), b.span_count.as<uint32_t>(), n_lists1,
-                           b.span_top.as<uint32_t>(), mid_blocks, top_list, b.top_links.as<uint32_t>(),
-                           b.mid_links.as<uint32_t>(), b.slots.as<uint32_t>(), stage_max, s.status.as<uint32_t>());
-        if (top) {
-            hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(1024), 0, st, b.children.as<uint32_t>(),
-                               b.scene_of.as<uint32_t>(), b.parents_internal.as<uint32_t>(),
-                               b.counters.as<uint32_t>(), b.nodes.as<float4>(), b.root_box.as<float>(), top_list,
-                               b.top_links.as<uint32_t>(), stage_max);
-        }
+    const uint32_t* scene_of = nscenes > 1 ? b.scene_of.as<uint32_t>() : nullptr;
+    OpenList* lists = b.open_lists.as<OpenList>();
+    hipLaunchKernelGGL(k_tree_leaves, dim3(blocks), dim3(kLeafBlock), 0, st, s.tris.as<pt_triangle>(),
+                       b.keys.as<uint32_t>(), b.vals.as<uint32_t>(), s.off.as<uint32_t>(), scene_of, n,
+                       b.nodes.as<float4>(), b.tris.as<float4>(), b.root_box.as<float>(), b.root_word.as<uint32_t>(),
+                       lists, s.status.as<uint32_t>());
+    for (uint32_t m = blocks; m > 1;) {
+        const uint32_t next = div_up(m, kFanIn);
+        hipLaunchKernelGGL(k_tree_merge, dim3(next), dim3(kMergeThreads), 0, st, lists, m, scene_of, b.nodes.as<float4>(),
+                           b.root_box.as<float>(), b.root_word.as<uint32_t>(), lists + m, s.status.as<uint32_t>());
+        lists += m;
+        m = next;
     }
     PT_HIP(hipGetLastError());
 }
@@ -1164,20 +851,24 @@ void dump_bvh(DeviceScene& s, uint32_t scene, hipStream_t st, uint32_t* morton, 
     if (n == 0) return;
     const size_t m = n - 1;
     DevBuf tmp;
-    tmp.reserve(static_cast<size_t>(n) * 4 * 4 + m * 24 + 256);
+    tmp.reserve(static_cast<size_t>(n) * 5 * 4 + m * 24 + 256);
     uint32_t* t_perm = tmp.as<uint32_t>();
     uint32_t* t_ch = t_perm + n;
     uint32_t* t_pl = t_ch + n;
     uint32_t* t_pi = t_pl + n;
-    float* t_box = reinterpret_cast<float*>(t_pi + n);
+    uint32_t* t_owner = t_pi + n;
+    float* t_box = reinterpret_cast<float*>(t_owner + n);
     if (morton)
         PT_HIP(hipMemcpyAsync(morton, b.keys.as<uint32_t>() + base, n * 4ull, hipMemcpyDeviceToHost, st));
     hipLaunchKernelGGL(k_sub_u32, dim3(div_up(n, 256)), dim3(256), 0, st, b.vals.as<uint32_t>() + base,
                        base, n, t_perm);
-    hipLaunchKernelGGL(k_dump_scene, dim3(div_up(n, 256)), dim3(256), 0, st, b.nodes.as<float4>(),
-                       b.children.as<uint32_t>(), b.parents_leaf.as<uint32_t>(),
-                       b.parents_internal.as<uint32_t>(), b.root_box.as<float>() + 6 * static_cast<size_t>(scene),
-                       base, n, t_box, t_ch, t_pl, t_pi);
+    if (n > 1) {
+        hipLaunchKernelGGL(k_dump_nodes, dim3(div_up(n, 256)), dim3(256), 0, st, b.nodes.as<float4>(),
+                           b.root_word.as<uint32_t>() + scene, b.root_box.as<float>() + 6 * static_cast<size_t>(scene),
+                           base, n, t_box, t_ch, t_owner);
+    }
+    hipLaunchKernelGGL(k_dump_parents, dim3(div_up(n, 256)), dim3(256), 0, st, b.nodes.as<float4>(), t_owner, base, n,
+                       t_pl, t_pi);
     PT_HIP(hipGetLastError());
     if (perm) PT_HIP(hipMemcpyAsync(perm, t_perm, n * 4ull, hipMemcpyDeviceToHost, st));
     if (parents_leaf) PT_HIP(hipMemcpyAsync(parents_leaf, t_pl, n * 4ull, hipMemcpyDeviceToHost, st));

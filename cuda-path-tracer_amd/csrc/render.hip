@@ -47,7 +47,7 @@ struct FrameConst {
     const uint32_t* texels;            // RGBA8 texels of all textures
     const uint4* texinfo;              // per texture: first texel, width, height, 0
     uint32_t* status;                  // the scene's status word (PT_STATUS_* flags)
-    const uint32_t* words;             // child word of each internal node (of a scene's root: words[off])
+    const uint32_t* roots;             // child word of each scene's root (two triangles or more)
 };
 
 // Structure-of-arrays queue of rays (origin, direction, path index).
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kThreads) void k_generate(const FrameConst fc,
 
 // Closest hit for every ray of queue `level` (count on the device): the
 // persistent traversal, rays handed out from the level's ray queue block.
-// Each path traces the scene of its pass (root node: word fc.words[off[scene]]).
+// Each path traces the scene of its pass (root node: word fc.roots[scene]).
 template <int LDS>
 __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
                                                             const PassParams* __restrict__ pp,
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
         d = v3(q.dx[i], q.dy[i], q.dz[i]);
         const uint32_t sc = pp[min(q.path[i] / fc.npix, fc.npasses - 1u)].scene;
         const uint32_t b = off[sc], e = off[sc + 1];
-        if (e - b >= 2) return fc.words[b];
+        if (e - b >= 2) return fc.roots[sc];
         if (e - b == 1) single = b;
         return kInvalid;
     };
@@ -216,11 +216,11 @@ __device__ __forceinline__ V3 ld3(const float* p) { return v3(p[0], p[1], p[2]);
 // answers the same question and stops at its first hit.
 template <bool LDSS = false>
 __device__ __forceinline__ V3 light_L(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                      const uint32_t* __restrict__ words, uint32_t b, uint32_t e, V3 pos,
+                                      uint32_t root, uint32_t b, uint32_t e, V3 pos,
                                       const pt_dir_light& lt, uint32_t* status,
                                       const ShadowStack& ss = ShadowStack{}) {
     const V3 ld = ld3(lt.direction);
-    if (any_hit_in<LDSS>(nodes, tris, words, b, e, sub(pos, scale(ld, 1e-3f)), neg(ld), status, ss))
+    if (any_hit_in<LDSS>(nodes, tris, root, b, e, sub(pos, scale(ld, 1e-3f)), neg(ld), status, ss))
         return v3(0.0f, 0.0f, 0.0f);
     return scale(ld3(lt.color), lt.intensity);
 }
@@ -320,7 +320,7 @@ template <bool LIGHTS, bool LDSS = false>
 __device__ __forceinline__ void bounce_hit(HitShade& hs, V3 d, const FrameConst& fc,
                                            const pt_dir_light* __restrict__ lights,
                                            const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                           uint32_t sb, uint32_t se, V3& absorbed, V3& acc,
+                                           uint32_t root, uint32_t sb, uint32_t se, V3& absorbed, V3& acc,
                                            const ShadowStack& ss = ShadowStack{}) {
     V3 L = v3(0.0f, 0.0f, 0.0f);
     if (hs.emissive) {
@@ -330,7 +330,7 @@ __device__ __forceinline__ void bounce_hit(HitShade& hs, V3 d, const FrameConst&
     } else if (LIGHTS) {
         for (uint32_t k = 0; k < fc.nlights; ++k) {
             const V3 ld = ld3(lights[k].direction);
-            L = add(L, scale(light_L<LDSS>(nodes, tris, fc.words, sb, se, hs.pos, lights[k], fc.status, ss),
+            L = add(L, scale(light_L<LDSS>(nodes, tris, root, sb, se, hs.pos, lights[k], fc.status, ss),
                              gmax(dot(neg(ld), hs.nrm), 0.0f)));
         }
     }
@@ -377,7 +377,7 @@ template <bool LIGHTS, bool LDSS = false>
 __device__ __forceinline__ void primary_hit(HitShade& hs, V3 d, const FrameConst& fc,
                                             const pt_dir_light* __restrict__ lights,
                                             const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                            uint32_t sb, uint32_t se, V3& absorbed, V3& acc,
+                                            uint32_t root, uint32_t sb, uint32_t se, V3& absorbed, V3& acc,
                                             const ShadowStack& ss = ShadowStack{}) {
     acc = v3(0.0f, 0.0f, 0.0f);
     if (hs.emissive) {
@@ -387,7 +387,7 @@ __device__ __forceinline__ void primary_hit(HitShade& hs, V3 d, const FrameConst
         V3 Lc = v3(0.0f, 0.0f, 0.0f);
         for (uint32_t k = 0; k < fc.nlights; ++k) {
             const V3 ld = ld3(lights[k].direction);
-            Lc = add(Lc, light_L<LDSS>(nodes, tris, fc.words, sb, se, hs.pos, lights[k], fc.status, ss));
+            Lc = add(Lc, light_L<LDSS>(nodes, tris, root, sb, se, hs.pos, lights[k], fc.status, ss));
             const V3 hw = scale(sub(neg(d), ld), 0.5f);
             acc = add(acc, blinn_phong(Lc, hs.albedo, Lc, v3(0.5f, 0.5f, 0.5f), hs.nrm, neg(ld), hw, hs.spec));
         }
@@ -454,11 +454,11 @@ __global__ __launch_bounds__(kShadeThreads) void k_shade(const FrameConst fc,
             const uint32_t sb = off[P.scene], se = off[P.scene + 1];
             V3 absorbed, acc;
             if (level == 0) {
-                primary_hit<LIGHTS>(hs, d, fc, lights, nodes, tris, sb, se, absorbed, acc);
+                primary_hit<LIGHTS>(hs, d, fc, lights, nodes, tris, fc.roots[P.scene], sb, se, absorbed, acc);
             } else {
                 absorbed = v3(ps.ar[path], ps.ag[path], ps.ab[path]);
                 acc = v3(ps.cr[path], ps.cg[path], ps.cb[path]);
-                bounce_hit<LIGHTS>(hs, d, fc, lights, nodes, tris, sb, se, absorbed, acc);
+                bounce_hit<LIGHTS>(hs, d, fc, lights, nodes, tris, fc.roots[P.scene], sb, se, absorbed, acc);
             }
             if (CACHE && level == 1) record_cache_vertex(io, train, pix, path, hs, d, absorbed, acc);
             // Next bounce index = level (bounce loop, cuda_path_tracer.cu:267).
@@ -619,7 +619,7 @@ __device__ __forceinline__ uint32_t start_path(const FrameConst& fc, const PassP
     r.o = v3(P.eye[0], P.eye[1], P.eye[2]);
     r.d = mix(mix(d00, d10, tx), mix(d01, d11, tx), ty);
     const uint32_t sb = off[P.scene], se = off[P.scene + 1];
-    root = se - sb >= 2 ? fc.words[sb] : kInvalid;
+    root = se - sb >= 2 ? fc.roots[P.scene] : kInvalid;
     return pass * fc.npix + pix;
 }
 
@@ -702,9 +702,9 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
             ss.depth = LDS;
             ss.spill = spill;
             if (bounce == 0) {
-                primary_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, sb, se, absorbed, acc, ss);
+                primary_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, root, sb, se, absorbed, acc, ss);
             } else {
-                bounce_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, sb, se, absorbed, acc, ss);
+                bounce_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, root, sb, se, absorbed, acc, ss);
             }
             if (CACHE && bounce == 1 && lead) record_cache_vertex(io, false, pix, path, hs, r.d, absorbed, acc);
             V3 no{0.0f, 0.0f, 0.0f}, nd{0.0f, 0.0f, 0.0f};
@@ -920,7 +920,7 @@ __global__ __launch_bounds__(kSuffixThreads) void k_train_paths(const FrameConst
                 RayState r;
                 r.o = o;
                 r.d = d;
-                init_ray(r, fc.words[sb]);
+                init_ray(r, fc.roots[P.scene]);
                 if (r.finite) {
                     while (visit_step<false, kTrainLds, true>(nodes, tris, r, s_tstack, spill, cnt, fc.status)) {
                     }
@@ -934,13 +934,13 @@ __global__ __launch_bounds__(kSuffixThreads) void k_train_paths(const FrameConst
             HitShade hs = hit_shade<DETAIL>(fc, infos, h.id, h.t, h.u, h.v, o, d);
             if (b == 0) {
                 if (fc.nlights)
-                    primary_hit<true>(hs, d, fc, lights, nodes, tris, sb, se, absorbed, acc);
+                    primary_hit<true>(hs, d, fc, lights, nodes, tris, fc.roots[P.scene], sb, se, absorbed, acc);
                 else
-                    primary_hit<false>(hs, d, fc, lights, nodes, tris, sb, se, absorbed, acc);
+                    primary_hit<false>(hs, d, fc, lights, nodes, tris, fc.roots[P.scene], sb, se, absorbed, acc);
             } else if (fc.nlights) {
-                bounce_hit<true>(hs, d, fc, lights, nodes, tris, sb, se, absorbed, acc);
+                bounce_hit<true>(hs, d, fc, lights, nodes, tris, fc.roots[P.scene], sb, se, absorbed, acc);
             } else {
-                bounce_hit<false>(hs, d, fc, lights, nodes, tris, sb, se, absorbed, acc);
+                bounce_hit<false>(hs, d, fc, lights, nodes, tris, fc.roots[P.scene], sb, se, absorbed, acc);
             }
             if (b == 1) record_cache_vertex(io, true, key, path, hs, d, absorbed, acc);
             if (!(b < io.train_levels - 1u)) break;
@@ -1412,7 +1412,7 @@ void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, cons
     fc.stratified = r.settings.stratified;
     fc.nlights = scene.nlights;
     fc.status = scene.status.as<uint32_t>();
-    fc.words = scene.bvh.children.as<uint32_t>();
+    fc.roots = scene.bvh.root_word.as<uint32_t>();
     set_detail(fc, scene);
 
     const uint32_t nchains = frame_chains(npix * npasses);
@@ -1574,7 +1574,7 @@ void render_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
     cf.fc.stratified = r.settings.stratified;
     cf.fc.nlights = scene.nlights;
     cf.fc.status = scene.status.as<uint32_t>();
-    cf.fc.words = scene.bvh.children.as<uint32_t>();
+    cf.fc.roots = scene.bvh.root_word.as<uint32_t>();
     set_detail(cf.fc, scene);
     cf.steps = cs.train_steps;
     cf.train = (cs.flags & PT_CACHE_TRAIN) != 0;

@@ -63,14 +63,14 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_single(
 // the root filter (persistent_trace_filtered), without counting.
 template <bool COUNT, int LDS, bool FILTER>
 __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
-    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ words,
+    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ roots,
     const float* __restrict__ rays, uint32_t nrays, uint32_t* __restrict__ out_id, float* __restrict__ out_t,
     float2* __restrict__ out_uv, uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool,
     unsigned long long* __restrict__ counters, uint32_t* __restrict__ status) {
     static_assert(!(COUNT && FILTER), "the filter's repeated root visit would change the visit counts");
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
     __shared__ uint32_t s_pend[kPend][kPersistThreads];
-    const uint32_t root = words[0];
+    const uint32_t root = roots[0];
     auto load = [&](uint32_t i, V3& o, V3& d, uint32_t&) -> uint32_t {
         const float* rp = rays + 6 * static_cast<size_t>(i);
         o = v3(rp[0], rp[1], rp[2]);
@@ -95,10 +95,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
 }
 
 // Persistent closest hit over rays tagged with a scene of a batch: the ray
-// starts at its scene's root (internal node off[s], word words[off[s]]).
+// starts at its scene's root (word roots[s]).
 template <int LDS>
 __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
-    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ words,
+    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ roots,
     const uint32_t* __restrict__ off, uint32_t nscenes, const float* __restrict__ rays, const uint32_t* __restrict__ scene, uint32_t nrays,
     uint32_t* __restrict__ out_id, float* __restrict__ out_t, float2* __restrict__ out_uv,
     uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool, uint32_t* __restrict__ status) {
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
             const uint32_t sc = scene[i];
             if (sc >= nscenes) return kInvalid;  // unknown scene: a miss
             const uint32_t b = off[sc], e = off[sc + 1];
-            if (e - b >= 2) return words[b];
+            if (e - b >= 2) return roots[sc];
             if (e - b == 1) single = b;
             return kInvalid;
         },
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
 // queue.  SCENES: rays tagged with a scene of a batch.
 template <int LDS, bool SCENES>
 __global__ __launch_bounds__(kPersistThreads) void k_trace_grouped(
-    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ words,
+    const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ roots,
     const uint32_t* __restrict__ off, uint32_t nscenes, const float* __restrict__ rays,
     const uint32_t* __restrict__ scene, uint32_t nrays, uint32_t lg, uint32_t* __restrict__ out_id,
     float* __restrict__ out_t, float2* __restrict__ out_uv, uint32_t* __restrict__ status) {
@@ -141,11 +141,11 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_grouped(
             const float* rp = rays + 6 * static_cast<size_t>(i);
             o = v3(rp[0], rp[1], rp[2]);
             d = v3(rp[3], rp[4], rp[5]);
-            if (!SCENES) return words[0];
+            if (!SCENES) return roots[0];
             const uint32_t sc = scene[i];
             if (sc >= nscenes) return kInvalid;  // unknown scene: a miss
             const uint32_t b = off[sc], e = off[sc + 1];
-            if (e - b >= 2) return words[b];
+            if (e - b >= 2) return roots[sc];
             if (e - b == 1) single = b;
             return kInvalid;
         },
@@ -167,7 +167,7 @@ uint32_t launch_grouped(const DeviceScene& s, const float* d_rays, const uint32_
     auto kern = d_scene ? (tune.lds <= 8 ? k_trace_grouped<8, true> : k_trace_grouped<16, true>)
                         : (tune.lds <= 8 ? k_trace_grouped<8, false> : k_trace_grouped<16, false>);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st, s.bvh.nodes.as<float4>(),
-                       s.bvh.tris.as<float4>(), s.bvh.children.as<uint32_t>(), s.off.as<uint32_t>(), s.nscenes(),
+                       s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(), s.off.as<uint32_t>(), s.nscenes(),
                        d_rays, d_scene, n, lg, d_id, d_t, reinterpret_cast<float2*>(d_uv), s.status.as<uint32_t>());
     PT_HIP(hipGetLastError());
     return lg;
@@ -203,7 +203,7 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
                                         : (tune.lds <= 16 ? k_trace_persistent<COUNT, 16, false>
                                                           : k_trace_persistent<COUNT, 32, false>));
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
-                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.children.as<uint32_t>(), d_rays, n, d_id, d_t,
+                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(), d_rays, n, d_id, d_t,
                        reinterpret_cast<float2*>(d_uv), queue, std::min(64u, std::max(1u, tune.refill)),
                        pool_for(tune.pool, n, blocks), d_counters, status);
     PT_HIP(hipGetLastError());
@@ -260,7 +260,7 @@ void trace_closest_scenes(const DeviceScene& s, uint32_t* queue, const float* d_
         static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(want, tune.blocks)));
     auto kern = tune.lds <= 8 ? k_trace_scenes<8> : (tune.lds <= 16 ? k_trace_scenes<16> : k_trace_scenes<32>);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
-                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.children.as<uint32_t>(),
+                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(),
                        s.off.as<uint32_t>(), s.nscenes(), d_rays, d_scene, n, d_id, d_t, reinterpret_cast<float2*>(d_uv),
                        queue, std::min(64u, std::max(1u, tune.refill)), pool_for(tune.pool, n, blocks),
                        s.status.as<uint32_t>());

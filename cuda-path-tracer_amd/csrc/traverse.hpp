@@ -92,7 +92,7 @@ struct ShadowStack {
     uint32_t* spill = nullptr;
 };
 
-// Whether a ray hits any triangle of the scene in [b, e) that the closest-hit
+// Whether a ray hits any triangle of the scene in [b, e) (root word `root`) that the closest-hit
 // search would accept (the shadow-ray question of computeL,
 // LightAlgorithms.h:12-20: closest-hit t < FLT_MAX).  Until its first hit
 // the closest-hit search culls nothing (its bound is still the initial
@@ -102,15 +102,15 @@ struct ShadowStack {
 // lends it to its shadow rays) instead of a private array.
 template <bool LDSS = false>
 __device__ __forceinline__ bool any_hit_in(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                          const uint32_t* __restrict__ words, uint32_t b, uint32_t e, V3 o, V3 d,
-                                          uint32_t* status, const ShadowStack& ss = ShadowStack{}) {
+                                          uint32_t root, uint32_t b, uint32_t e, V3 o, V3 d, uint32_t* status,
+                                          const ShadowStack& ss = ShadowStack{}) {
     float u, v;
     if (e - b == 0) return false;
     if (e - b == 1) return tri_test(load_tri(tris, b), o, d, u, v) <= kMinTInit;
     const V3 dinv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
     uint32_t stack[LDSS ? 1 : kStackMax];
     int sp = 0;
-    uint32_t word = words[b];
+    uint32_t word = root;
     for (;;) {
         const uint32_t l = word >> 2;
         const bool in0 = (word & 1u) != 0, in1 = (word & 2u) != 0;

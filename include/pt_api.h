@@ -48,7 +48,7 @@ extern "C" {
  * pt_read_accumulator) returns PT_E_INTERNAL and clears it. */
 #define PT_STATUS_STACK_OVERFLOW 1u /* deferred-node stack deeper than 64 (reference: */
                                     /* MAX_TRAVERSAL_STACK_SIZE 64, cuda_defs.h:21, unchecked) */
-#define PT_STATUS_REFIT_OVERFLOW 2u /* refit level list over its capacity */
+#define PT_STATUS_REFIT_OVERFLOW 2u /* a build level's open list over its capacity */
 
 /* Triangle as the caller hands it over: three fp32 vertices plus the caller's
  * triangle id (reference: CUDA::Triangle, geometry.h:20-30 -- v0, v1, v2,
@@ -363,10 +363,8 @@ int pt_device_compute_units(int device, uint32_t* cus);
 /* ---- launch tuning (no reference counterpart) -------------------------------
  * Process-wide launch-shape knobs read by the kernels' host launchers; results
  * do not depend on them (tests check this).  Names:
- *   "build.staged"  1: the LBVH refit's upper levels (nodes whose leaves span
- *                   more than one 1024-leaf block) run with each block's
- *                   node list staged in LDS when it holds at most 1024
- *                   nodes; 0: always from global memory
+ *   "build.staged"  0 or 1: accepted, without effect (the tree's upper levels
+ *                   are built one way)
  *   "trace.blocks"  persistent closest-hit workgroups (256 threads each)
  *   "trace.refill"  refill idle lanes when fewer than this many of 64 are busy
  *   "trace.lds_stack" traversal stack entries per lane kept in LDS (8, 16 or
