@@ -152,55 +152,95 @@ __global__ __launch_bounds__(kThreads) void k_mlp_pack(const float* __restrict__
 }
 
 __device__ __forceinline__ half4 to_half4(floatx4 v) {
-    half4 h;
-    h.x = static_cast<_Float16>(v.x);
-    h.y = static_cast<_Float16>(v.y);
-    h.z = static_cast<_Float16>(v.z);
-    h.w = static_cast<_Float16>(v.w);
-    return h;
+    return __builtin_convertvector(v, half4);
+}
+
+// ReLU of the rounded values: max(x, 0) commutes with rounding to fp16, and
+// on halves it takes one instruction per pair.
+__device__ __forceinline__ half4 relu_half4(floatx4 v) {
+    return __builtin_elementwise_max(to_half4(v), half4{0, 0, 0, 0});
 }
 
 struct SceneBox {
     float mn[3], inv_ext[3];
 };
 
-// Input features idx and idx + 1 (idx even, 0..94) of one sample from its
-// 12 raw floats: below 72 the (sin, cos) pair of 2^k pi p for one axis and
-// frequency -- sin/cos(2^k pi p) = sin/cos(2 pi frac(2^(k-1) p)), the
-// hardware sine and cosine taking revolutions -- then the normal, incoming
-// direction and albedo, then zero padding.
-__device__ __forceinline__ void feature_pair(int idx, const float* p01, const float* raw, float& f0, float& f1) {
-    if (idx < 72) {
-        const int a = idx / 24, k = (idx % 24) / 2;
-        const float rev = ldexpf(p01[a], k - 1);
-        const float fr = rev - floorf(rev);
-        f0 = __builtin_amdgcn_sinf(fr);
-        f1 = __builtin_amdgcn_cosf(fr);
+// Input features 16 F + 4 g + {0, 1, 2, 3} of one sample (g: the lane's group
+// of 16).  Features below 72 are (sin, cos) pairs of 2^k pi p, 12 frequencies
+// for each axis -- sin/cos(2^k pi p) = sin/cos(2 pi frac(2^(k-1) p)), the
+// hardware sine and cosine taking revolutions -- then come the normal, incoming
+// direction and albedo (raw[3..11]), then zero padding.  F fixes the axis (in
+// F = 1 up to the group) and what else a lane may hold, so nothing is indexed
+// at run time: with arrays indexed by feature the 12 raw floats and positions
+// lived in scratch memory.
+template <int F>
+__device__ __forceinline__ floatx4 features(int g, const float* p01, floatx4 rest) {
+    floatx4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (F < 5) {
+        float p;
+        int k;  // frequency of the first pair
+        if constexpr (F == 0) { p = p01[0]; k = 2 * g; }
+        if constexpr (F == 1) { p = g >= 2 ? p01[1] : p01[0]; k = 2 * g + (g >= 2 ? -4 : 8); }
+        if constexpr (F == 2) { p = p01[1]; k = 2 * g + 4; }
+        if constexpr (F == 3) { p = p01[2]; k = 2 * g; }
+        if constexpr (F == 4) { p = p01[2]; k = 2 * g + 8; }
+        // Powers of two: exact, and a lane's factor is the same for every sample.
+        const float r0 = p * __uint_as_float(static_cast<uint32_t>(126 + k) << 23), r1 = r0 + r0;
+        const float f0 = r0 - floorf(r0), f1 = r1 - floorf(r1);
+        v.x = __builtin_amdgcn_sinf(f0);
+        v.y = __builtin_amdgcn_cosf(f0);
+        v.z = __builtin_amdgcn_sinf(f1);
+        v.w = __builtin_amdgcn_cosf(f1);
+        if constexpr (F == 4) {
+            v.x = g < 2 ? v.x : rest.x;
+            v.y = g < 2 ? v.y : rest.y;
+            v.z = g < 2 ? v.z : rest.z;
+            v.w = g < 2 ? v.w : rest.w;
+        }
     } else {
-        f0 = idx < 81 ? raw[3 + idx - 72] : 0.0f;
-        f1 = idx + 1 < 81 ? raw[3 + idx + 1 - 72] : 0.0f;
+        v.x = g == 0 ? rest.w : 0.0f;
     }
+    return v;
+}
+
+// What a lane reads of one sample (zeros past the batch): the position, and of
+// the other nine floats the four that its group's features hold -- raw[3..6]
+// (group 2), raw[7..10] (group 3) or, as the last, raw[11] (group 0).  Two
+// loads that need no more than the floats' own alignment.
+struct Sample {
+    float x, y, z;
+    floatx4 rest;
+};
+__device__ __forceinline__ Sample load_sample(const float* __restrict__ raw, uint32_t n, uint32_t s) {
+    typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+    const int g = (threadIdx.x & 63) / 16;
+    Sample v = {0.0f, 0.0f, 0.0f, {0.0f, 0.0f, 0.0f, 0.0f}};
+    if (s < n) {
+        const float* p = raw + 12 * static_cast<size_t>(s);
+        v.rest = *reinterpret_cast<const floatx4u*>(p + (g == 2 ? 3 : (g == 3 ? 7 : 8)));
+        v.x = p[0];
+        v.y = p[1];
+        v.z = p[2];
+    }
+    return v;
+}
+__device__ __forceinline__ void in_box(const Sample& v, const SceneBox& box, float* p01) {
+    p01[0] = (v.x - box.mn[0]) * box.inv_ext[0];
+    p01[1] = (v.y - box.mn[1]) * box.inv_ext[1];
+    p01[2] = (v.z - box.mn[2]) * box.inv_ext[2];
 }
 
 // Lane's view of one 16-sample block: the input fragments X[f] (k-block f).
-__device__ __forceinline__ void encode_block(const float* __restrict__ raw, uint32_t n, uint32_t s,
-                                             const SceneBox& box, half4* X) {
-    const int lane = threadIdx.x & 63;
-    float rw[12];
-    if (s < n) {
-        for (int k = 0; k < 12; ++k) rw[k] = raw[12 * static_cast<size_t>(s) + k];
-    } else {
-        for (int k = 0; k < 12; ++k) rw[k] = 0.0f;
-    }
+__device__ __forceinline__ void encode_block(const Sample& v, const SceneBox& box, half4* X) {
+    const int g = (threadIdx.x & 63) / 16;
     float p01[3];
-    for (int a = 0; a < 3; ++a) p01[a] = (rw[a] - box.mn[a]) * box.inv_ext[a];
-#pragma unroll
-    for (int f = 0; f < fb(0); ++f) {
-        float a, b, c, d;
-        feature_pair(16 * f + 4 * (lane / 16) + 0, p01, rw, a, b);
-        feature_pair(16 * f + 4 * (lane / 16) + 2, p01, rw, c, d);
-        X[f] = to_half4(floatx4{a, b, c, d});
-    }
+    in_box(v, box, p01);
+    X[0] = to_half4(features<0>(g, p01, v.rest));
+    X[1] = to_half4(features<1>(g, p01, v.rest));
+    X[2] = to_half4(features<2>(g, p01, v.rest));
+    X[3] = to_half4(features<3>(g, p01, v.rest));
+    X[4] = to_half4(features<4>(g, p01, v.rest));
+    X[5] = to_half4(features<5>(g, p01, v.rest));
 }
 
 __device__ __forceinline__ half4 lds_frag(const uint2* __restrict__ frags, int idx) {
@@ -210,100 +250,34 @@ __device__ __forceinline__ half4 lds_frag(const uint2* __restrict__ frags, int i
     return h;
 }
 
-__device__ __forceinline__ floatx4 bias4(const float* __restrict__ b, int r, int nvalid) {
-    const int lane = threadIdx.x & 63;
-    floatx4 v;
-    const int o = 16 * r + 4 * (lane / 16);
-    v.x = o + 0 < nvalid ? b[o + 0] : 0.0f;
-    v.y = o + 1 < nvalid ? b[o + 1] : 0.0f;
-    v.z = o + 2 < nvalid ? b[o + 2] : 0.0f;
-    v.w = o + 3 < nvalid ? b[o + 3] : 0.0f;
-    return v;
+// Biases of a lane's four rows of row block r, from LDS (zeros past the layer).
+__device__ __forceinline__ floatx4 bias4(const float* b, int r) {
+    const int o = 16 * r + 4 * ((threadIdx.x & 63) / 16);
+    return floatx4{b[o + 0], b[o + 1], b[o + 2], b[o + 3]};
 }
 
-__device__ __forceinline__ floatx4 relu4(floatx4 v) {
-    v.x = v.x > 0.0f ? v.x : 0.0f;
-    v.y = v.y > 0.0f ? v.y : 0.0f;
-    v.z = v.z > 0.0f ? v.z : 0.0f;
-    v.w = v.w > 0.0f ? v.w : 0.0f;
-    return v;
-}
-
-// Forward of one block.  H[l][r] = fp16 input fragments of layer l (l = 1..4);
-// returns the output pre-activation fragment (rows 0..2 valid on lanes 0..15).
-__device__ __forceinline__ floatx4 forward_block(const uint2* __restrict__ frags,
-                                                 const float* __restrict__ master, const half4* X,
-                                                 half4 (*H)[4]) {
-    // The four row blocks' accumulators advance together (independent MFMA
-    // chains); each still sums its k-blocks in order.
-    {
-        floatx4 acc[4];
+// Global -> LDS copy of BYTES bytes (a multiple of 1,024; both 16-byte aligned)
+// by the workgroup's waves, 1,024 bytes an instruction straight into LDS, all
+// in flight at once.  Barrier-ready once stage_wait has returned.
+template <uint32_t BYTES>
+__device__ __forceinline__ void stage(void* dst, const void* __restrict__ src) {
+    static_assert(BYTES % 1024u == 0u, "whole wave copies");
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), lane = threadIdx.x & 63u;
+    const char* s = static_cast<const char*>(src) + lane * 16u;
+    char* d = static_cast<char*>(dst);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] = bias4(master + b_off(0), r, kHid);
-#pragma unroll
-        for (int f = 0; f < fb(0); ++f)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] = mfma(lds_frag(frags, fwd_base(0) + r * fb(0) + f), X[f], acc[r]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) H[1][r] = to_half4(relu4(acc[r]));
-    }
-#pragma unroll
-    for (int l = 1; l < 4; ++l) {
-        floatx4 acc[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] = bias4(master + b_off(l), r, kHid);
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] = mfma(lds_frag(frags, fwd_base(l) + r * 4 + f), H[l][f], acc[r]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) H[l + 1][r] = to_half4(relu4(acc[r]));
-    }
-    floatx4 z = bias4(master + b_off(4), 0, kOut);
-#pragma unroll
-    for (int f = 0; f < 4; ++f) z = mfma(lds_frag(frags, fwd_base(4) + f), H[4][f], z);
-    return z;
-}
-
-// Global -> LDS copy of `count` elements by the workgroup, eight loads in
-// flight per thread before their stores (a load-store loop would wait out
-// one memory round trip per element).
-template <class T>
-__device__ __forceinline__ void stage(T* dst, const T* __restrict__ src, int count) {
-    constexpr int kBatch = 8;
-    const int step = static_cast<int>(blockDim.x);
-    for (int base = static_cast<int>(threadIdx.x); base < count; base += kBatch * step) {
-        T v[kBatch];
-#pragma unroll
-        for (int j = 0; j < kBatch; ++j) {
-            const int k = base + j * step;
-            if (k < count) v[j] = src[k];
-        }
-#pragma unroll
-        for (int j = 0; j < kBatch; ++j) {
-            const int k = base + j * step;
-            if (k < count) dst[k] = v[j];
+    for (uint32_t k = 0; k < (BYTES / 1024u + kThreads / 64u - 1u) / (kThreads / 64u); ++k) {
+        const uint32_t piece = k * (kThreads / 64u) + wave;
+        if (piece < BYTES / 1024u) {
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)(s + piece * 1024u),
+                (__attribute__((address_space(3))) void*)(d + piece * 1024u), 16, 0, 0);
         }
     }
 }
-
-__device__ __forceinline__ void stage_frags(uint2* dst, const uint2* __restrict__ src, int nfrags) {
-    stage(dst, src, nfrags * 64);
+__device__ __forceinline__ void stage_wait() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-}
-
-// Input features kperm(q, g, 0..7) of one sample for the 16x16x32 B operand
-// (lane group g): pairs kperm(q, g, j), +1 for even j.
-__device__ __forceinline__ half8 encode32(int q, int g, const float* p01, const float* raw) {
-    half8 x;
-#pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-        float f0, f1;
-        feature_pair(kperm(q, g, j), p01, raw, f0, f1);
-        x[j] = static_cast<_Float16>(f0);
-        x[j + 1] = static_cast<_Float16>(f1);
-    }
-    return x;
 }
 
 __device__ __forceinline__ half8 lds_frag32(const uint4* __restrict__ frags, int idx) {
@@ -313,52 +287,39 @@ __device__ __forceinline__ half8 lds_frag32(const uint4* __restrict__ frags, int
     return h;
 }
 
+__device__ __forceinline__ half8 join(half4 a, half4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+
 // Next layer's B operand for k-block q from the D fragments of row blocks
 // 2q and 2q + 1 (ReLU, fp16).
-__device__ __forceinline__ half8 join_relu(floatx4 a, floatx4 b) {
-    half8 h;
-    h[0] = static_cast<_Float16>(a.x > 0.0f ? a.x : 0.0f);
-    h[1] = static_cast<_Float16>(a.y > 0.0f ? a.y : 0.0f);
-    h[2] = static_cast<_Float16>(a.z > 0.0f ? a.z : 0.0f);
-    h[3] = static_cast<_Float16>(a.w > 0.0f ? a.w : 0.0f);
-    h[4] = static_cast<_Float16>(b.x > 0.0f ? b.x : 0.0f);
-    h[5] = static_cast<_Float16>(b.y > 0.0f ? b.y : 0.0f);
-    h[6] = static_cast<_Float16>(b.z > 0.0f ? b.z : 0.0f);
-    h[7] = static_cast<_Float16>(b.w > 0.0f ? b.w : 0.0f);
-    return h;
-}
+__device__ __forceinline__ half8 join_relu(floatx4 a, floatx4 b) { return join(relu_half4(a), relu_half4(b)); }
 
 // Inference: out[3s + c] = exp(z_c).  A wave runs kInferBlocks 16-sample
 // blocks at a time so each weight fragment read from LDS feeds kInferBlocks
-// MFMAs.
+// MFMAs.  2,073,600 samples take 76 us (152 with inputs indexed through
+// scratch, MFMA results in accumulation registers and 16 lanes finishing one
+// block's outputs): of a SIMD's 197,000 cycles its matrix core is busy 77,000,
+// its vector instructions issue for 96,000, and 25,000 of these coincide.
+// Prefetching the next samples (142 registers, three waves) changed nothing;
+// what memory and staging alone take is 31 us.
 constexpr int kInferBlocks = 4;
 
 __global__ __launch_bounds__(kThreads) void k_mlp_infer(const uint4* __restrict__ f32,
                                                         const float* __restrict__ master,
                                                         const float* __restrict__ raw, uint32_t n,
                                                         SceneBox box, float* __restrict__ out) {
-    __shared__ uint4 s_frag[kF32Frags * 64];
+    __shared__ __align__(16) uint4 s_frag[kF32Frags * 64];
     __shared__ float s_bias[kLayers][kHid];
-    stage(s_frag, f32, kF32Frags * 64);
+    stage<kF32Frags * 1024u>(s_frag, f32);
     for (int k = threadIdx.x; k < kLayers * kHid; k += blockDim.x) {
         const int l = k / kHid, o = k % kHid;
         s_bias[l][o] = o < dim(l + 1) ? master[b_off(l) + o] : 0.0f;
     }
-    __syncthreads();
+    stage_wait();
     const int lane = threadIdx.x & 63, g = lane / 16;
     const uint32_t wave = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
     const uint32_t nwaves = gridDim.x * (blockDim.x / 64);
-    auto bias = [&](int l, int r) {
-        const int o = 16 * r + 4 * g;
-        floatx4 v;
-        v.x = s_bias[l][o + 0];
-        v.y = s_bias[l][o + 1];
-        v.z = s_bias[l][o + 2];
-        v.w = s_bias[l][o + 3];
-        return v;
-    };
+    auto bias = [&](int l, int r) { return bias4(s_bias[l], r); };
     constexpr uint32_t kSpan = 16 * kInferBlocks;
-    const bool aligned = (reinterpret_cast<uintptr_t>(raw) & 15u) == 0u;  // 48-byte samples, 16-byte loads
     for (uint32_t base = wave * kSpan; base < n; base += nwaves * kSpan) {
         // Weight fragments are read from LDS where used: kept from one
         // iteration to the next they would take 152 VGPRs (one wave per SIMD).
@@ -366,25 +327,16 @@ __global__ __launch_bounds__(kThreads) void k_mlp_infer(const uint4* __restrict_
         half8 X[kInferBlocks][3];
 #pragma unroll
         for (int b = 0; b < kInferBlocks; ++b) {
-            const uint32_t s = base + 16 * b + lane % 16;
-            float rw[12];
-            if (s < n && aligned) {
-                const float4* rp = reinterpret_cast<const float4*>(raw + 12 * static_cast<size_t>(s));
-                const float4 r0 = rp[0], r1 = rp[1], r2 = rp[2];
-                rw[0] = r0.x; rw[1] = r0.y; rw[2] = r0.z; rw[3] = r0.w;
-                rw[4] = r1.x; rw[5] = r1.y; rw[6] = r1.z; rw[7] = r1.w;
-                rw[8] = r2.x; rw[9] = r2.y; rw[10] = r2.z; rw[11] = r2.w;
-            } else if (s < n) {
-                for (int k = 0; k < 12; ++k) rw[k] = raw[12 * static_cast<size_t>(s) + k];
-            } else {
-                for (int k = 0; k < 12; ++k) rw[k] = 0.0f;
-            }
-            float p01[3];
-            for (int a = 0; a < 3; ++a) p01[a] = (rw[a] - box.mn[a]) * box.inv_ext[a];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) X[b][q] = encode32(q, g, p01, rw);
+            half4 x[fb(0)];
+            encode_block(load_sample(raw, n, base + 16 * b + lane % 16), box, x);
+            X[b][0] = join(x[0], x[1]);
+            X[b][1] = join(x[2], x[3]);
+            X[b][2] = join(x[4], x[5]);
         }
-        // Layer 0: 96 -> 64.
+        // Layer 0: 96 -> 64.  Waves in their layers issue before waves that
+        // encode, whose vector instructions fill the matrix cores' cycles
+        // (77.2 us against 78.4).
+        __builtin_amdgcn_s_setprio(1);
         half8 H[kInferBlocks][2];
 #pragma unroll
         for (int rp = 0; rp < 2; ++rp) {
@@ -432,42 +384,49 @@ __global__ __launch_bounds__(kThreads) void k_mlp_infer(const uint4* __restrict_
                 H[b][1] = Hn[b][1];
             }
         }
-        // Layer 4: 64 -> 3 (rows 0..2 of the first row block), exp.
+        // Layer 4: 64 -> 3, exp.  Every fourth row takes the weights of rows
+        // 0..3, so each lane group holds the three outputs of every block and
+        // finishes one block: 64 samples' exponentials and stores at once.
         floatx4 z[kInferBlocks];
-        const floatx4 b4 = bias(4, 0);
+        const floatx4 b4 = {s_bias[4][0], s_bias[4][1], s_bias[4][2], 0.0f};
 #pragma unroll
         for (int b = 0; b < kInferBlocks; ++b) z[b] = b4;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            const half8 a = lds_frag32(s_frag, f32_base(4) + q);
+            half8 a;
+            __builtin_memcpy(&a, &s_frag[(f32_base(4) + q) * 64 + (lane & ~12)], sizeof a);
 #pragma unroll
             for (int b = 0; b < kInferBlocks; ++b) z[b] = mfma32(a, H[b][q], z[b]);
         }
-#pragma unroll
-        for (int b = 0; b < kInferBlocks; ++b) {
-            const uint32_t s = base + 16 * b + lane % 16;
-            if (lane < 16 && s < n) {
-                out[3 * static_cast<size_t>(s) + 0] = expf(z[b].x);
-                out[3 * static_cast<size_t>(s) + 1] = expf(z[b].y);
-                out[3 * static_cast<size_t>(s) + 2] = expf(z[b].z);
-            }
+        __builtin_amdgcn_s_setprio(0);
+        static_assert(kInferBlocks == 4, "one lane group for each block's outputs");
+        const floatx4 zl = g < 2 ? (g == 0 ? z[0] : z[1]) : (g == 2 ? z[2] : z[3]);
+        const uint32_t s = base + lane;
+        if (s < n) {
+            out[3 * static_cast<size_t>(s) + 0] = expf(zl.x);
+            out[3 * static_cast<size_t>(s) + 1] = expf(zl.y);
+            out[3 * static_cast<size_t>(s) + 2] = expf(zl.z);
         }
     }
 }
 
 // Training rounds: 64 samples per workgroup round, one 16-sample block per
-// wave.  Layer inputs act_l (act0: 96 rows, act1..4: 64) and deltas
-// delta_l = dL/dz_l scaled by n (delta0..3: 64 rows, delta4: 16 rows with
-// rows 3..15 zero) go to LDS feature-major, [row][sample] with a padded row.
+// wave.  A sample's layer inputs act_l (96 + 4 x 64 halves) and deltas delta_l
+// = dL/dz_l scaled by n (4 x 64, then 16 of which 3 are used) are a row each of
+// two LDS arrays: a lane stores the four features of its fragment in one
+// 8-byte write, and gfx950's transposing LDS read returns them feature by
+// feature, four samples to a lane, as the operands of the weight gradients.
+// Row strides of 8 x an odd number of banks: the transposing read's eight rows
+// of 32 bytes fall in different banks.
 constexpr int kTrainChunk = 64;
-constexpr int kActRows = kIn + 4 * kHid;   // 352
-constexpr int kDelRows = 4 * kHid + 16;    // 272
-constexpr int kRowLd = kTrainChunk + 4;    // 68 halves: rows 34 banks apart
-__host__ __device__ constexpr int act_row(int l) { return l == 0 ? 0 : kIn + kHid * (l - 1); }
-__host__ __device__ constexpr int del_row(int l) { return kHid * l; }
-constexpr int kWTiles = fwd_base(kLayers);  // 76 weight tiles (16 x 16), 19 per wave
-constexpr int kTilesPerWave = kWTiles / 4;
-static_assert(kWTiles % 4 == 0, "weight tiles split evenly over four waves");
+constexpr int kActLd = 8 * 46;             // 352 halves used
+constexpr int kDelLd = 8 * 34;             // 272 halves
+static_assert(kActLd >= kIn + 4 * kHid && kActLd / 2 % 16 == 8, "activation rows");
+static_assert(kDelLd >= 4 * kHid + 16 && kDelLd / 2 % 16 == 8, "delta rows");
+__host__ __device__ constexpr int act_col(int l) { return l == 0 ? 0 : kIn + kHid * (l - 1); }
+__host__ __device__ constexpr int del_col(int l) { return kHid * l; }
+constexpr int kTilesPerWave = fwd_base(kLayers) / 4;  // 76 weight tiles (16 x 16)
+static_assert(kTilesPerWave == 19, "weight tiles of a wave: 6 + 3 x 4 + 1");
 constexpr uint32_t kMaxTrainBlocks = 256;  // workgroups (gradient partials) of one step
 
 // Deltas are gradients of n * loss (a static loss scale of n keeps them well
@@ -478,32 +437,34 @@ __device__ __forceinline__ float sat(float x) {
     return x > kHalfMax ? kHalfMax : (x < -kHalfMax ? -kHalfMax : x);
 }
 
+// Deltas d through the ReLU whose outputs are h (never negative): clamped as
+// halves (rounding first gives the same: what rounds past the largest half
+// becomes infinite and is clamped; NaN stays NaN), zero where h is zero.
 __device__ __forceinline__ half4 mask4(floatx4 d, half4 h) {
-    floatx4 m;
-    m.x = h.x > static_cast<_Float16>(0.0f) ? sat(d.x) : 0.0f;
-    m.y = h.y > static_cast<_Float16>(0.0f) ? sat(d.y) : 0.0f;
-    m.z = h.z > static_cast<_Float16>(0.0f) ? sat(d.z) : 0.0f;
-    m.w = h.w > static_cast<_Float16>(0.0f) ? sat(d.w) : 0.0f;
-    return to_half4(m);
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    const half4 hi = static_cast<half4>(static_cast<_Float16>(kHalfMax));
+    const half4 x = __builtin_elementwise_minimum(__builtin_elementwise_maximum(to_half4(d), -hi), hi);
+    const short4v on = (static_cast<short4v>(0) - __builtin_bit_cast(short4v, h)) >> 15;
+    return __builtin_bit_cast(half4, static_cast<short4v>(__builtin_bit_cast(short4v, x) & on));
 }
 
-// A 16x16 D-layout fragment (lane: rows 4(l/16)+e, column = sample l%16) into
-// LDS rows row0 .. row0+15, columns col0 .. col0+15.
-__device__ __forceinline__ void lds_put(_Float16 (*rows)[kRowLd], int row0, int col0, half4 v) {
-    const int lane = threadIdx.x & 63;
-    const int r = row0 + 4 * (lane / 16), c = col0 + lane % 16;
-    rows[r + 0][c] = v.x;
-    rows[r + 1][c] = v.y;
-    rows[r + 2][c] = v.z;
-    rows[r + 3][c] = v.w;
+// A lane's four features (row0 + 4(l/16) + e) of its sample (column l%16 of
+// the wave's block): its place in the sample's LDS row.
+__device__ __forceinline__ half4* lds_cell(_Float16* sample, int row0) {
+    return reinterpret_cast<half4*>(sample + row0 + 4 * ((threadIdx.x & 63) / 16));
 }
 
-// MFMA operand from LDS: lane l reads row row0 + l%16, samples k0 + 4(l/16) .. +3.
-__device__ __forceinline__ half4 lds_get(const _Float16 (*rows)[kRowLd], int row0, int k0) {
-    const int lane = threadIdx.x & 63;
-    half4 h;
-    __builtin_memcpy(&h, &rows[row0 + lane % 16][k0 + 4 * (lane / 16)], sizeof h);
-    return h;
+// MFMA operand: lane l gets feature l%16 of the 16 at `tile` (+ the lane's own
+// offset tr_off, see there) for samples 4(l/16) .. +3 of the tile's 16.
+__device__ __forceinline__ half4 lds_get(const _Float16* tile) {
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                         (__attribute__((address_space(3))) short4v*)(tile)));
+}
+// Where lane l reads for lds_get: 8 bytes of sample 4(l/16) + (l%16)/4.
+__device__ __forceinline__ int tr_off(int ld) {
+    const int l = threadIdx.x & 63;
+    return (4 * (l / 16) + l % 16 / 4) * ld + 4 * (l % 4);
 }
 
 // One training step's gradient partials.  Workgroup b handles rounds b,
@@ -512,137 +473,201 @@ __device__ __forceinline__ half4 lds_get(const _Float16 (*rows)[kRowLd], int row
 // whose first target channel is NaN is masked: zero loss, zero deltas (it
 // still counts in the mean's n).  Thread 0 of workgroup 0 advances the Adam
 // step counter by `advance` (read by k_mlp_adam_pack after this launch).
+//
+// Up to 16,384 samples a workgroup has one round and a SIMD one wave, so the
+// kernel lasts as long as one round's chain of dependent steps, and code that
+// runs once comes from memory as it is needed: the middle layers are loops
+// (11 KB of code; unrolled, with the tiles' places worked out one by one, it
+// was 25 KB), the samples and targets are loaded before the weights are
+// staged.  A wave's tiles share operands: layer 0's six have one block of
+// deltas, a middle layer's four one block of inputs.  A gradient of
+// 16,384 samples takes 22.7 us of which this is 17; it took 42.5.
 __global__ __launch_bounds__(kThreads) void k_mlp_train(
     const uint2* __restrict__ fwd, const uint2* __restrict__ bwd, const float* __restrict__ master,
     const float* __restrict__ raw, const float* __restrict__ target, uint32_t n, SceneBox box,
     float* __restrict__ part, float* __restrict__ loss, uint32_t* __restrict__ step, uint32_t advance) {
-    __shared__ uint2 s_fwd[kFwdFrags * 64];
-    __shared__ uint2 s_bwd[kBwdFrags * 64];
-    __shared__ _Float16 s_act[kActRows][kRowLd];
-    __shared__ _Float16 s_del[kDelRows][kRowLd];
+    __shared__ __align__(16) uint2 s_fwd[kFwdFrags * 64];
+    __shared__ __align__(16) uint2 s_bwd[kBwdFrags * 64];
+    __shared__ __align__(16) _Float16 s_act[kTrainChunk][kActLd];
+    __shared__ __align__(16) _Float16 s_del[kTrainChunk][kDelLd];
+    __shared__ __align__(16) float s_bias[kLayers][kHid];
+    const int lane = threadIdx.x & 63, g = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int col = 16 * wave + lane % 16;  // the lane's sample of a round
+    // Lane groups 0..2 hold a sample's three target channels, `first` the
+    // first (NaN: masked) in all of them.
+    float t = 0.0f, first = 0.0f;
+    Sample in;
+    auto load = [&](uint32_t round) {
+        const uint32_t s = round * kTrainChunk + col;
+        in = load_sample(raw, n, s);
+        if (s < n) {
+            first = target[3 * static_cast<size_t>(s)];
+            t = target[3 * static_cast<size_t>(s) + (g < kOut ? g : 0)];
+        }
+    };
+    load(blockIdx.x);
+    stage<kFwdFrags * 512u>(s_fwd, fwd);
+    stage<kBwdFrags * 512u>(s_bwd, bwd);
+    for (int k = threadIdx.x; k < kLayers * kHid; k += kThreads) {
+        const int l = k / kHid, o = k % kHid;
+        s_bias[l][o] = o < dim(l + 1) ? master[b_off(l) + o] : 0.0f;
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0 && advance) step[0] += advance;
-    stage(s_bwd, bwd, kBwdFrags * 64);
-    stage_frags(s_fwd, fwd, kFwdFrags);
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x / 64;
+    stage_wait();
     floatx4 acc[kTilesPerWave];
 #pragma unroll
-    for (int t = 0; t < kTilesPerWave; ++t) acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    // This wave's dW tiles: LDS rows of their layer inputs and deltas
-    // (wave-uniform, computed once).
-    uint32_t arow[kTilesPerWave], drow[kTilesPerWave];
-#pragma unroll
-    for (int t = 0; t < kTilesPerWave; ++t) {
-        const int task = wave + 4 * t;
-        int l = 0;
-        while (l + 1 < kLayers && task >= fwd_base(l + 1)) ++l;
-        const int k = task - fwd_base(l);
-        const int ri = k % fb(l), co = k / fb(l);
-        arow[t] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(act_row(l) + 16 * ri));
-        drow[t] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>((l == 4 ? kHid * 4 : del_row(l)) + 16 * co));
-    }
-    // Bias sums: thread t owns delta row t (layers 0..3) and, for t < 3,
-    // output bias t (delta4 row t).
+    for (int k = 0; k < kTilesPerWave; ++k) acc[k] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    // Bias sums: thread t owns delta column t (layers 0..3) and, for t < 3,
+    // output bias t (delta 4's column t).
     float bsum = 0.0f, bsum4 = 0.0f;
     for (uint32_t round = blockIdx.x; round * kTrainChunk < n; round += gridDim.x) {
-        const uint32_t s = round * kTrainChunk + 16 * wave + lane % 16;
-        const int col0 = 16 * wave;
-        half4 X[fb(0)];
-        half4 H[5][4];
-        encode_block(raw, n, s, box, X);
-        const floatx4 z = forward_block(s_fwd, master, X, H);
-        for (int f = 0; f < fb(0); ++f) lds_put(s_act, act_row(0) + 16 * f, col0, X[f]);
-        for (int l = 1; l < 5; ++l)
-            for (int r = 0; r < 4; ++r) lds_put(s_act, act_row(l) + 16 * r, col0, H[l][r]);
-        // Output delta: d/dz of (e^z - t)^2 / (sg(e^z)^2 + eps), per sample.
-        floatx4 d4 = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (lane < 16 && s < n && target[3 * static_cast<size_t>(s)] == target[3 * static_cast<size_t>(s)]) {
-            float lsum = 0.0f;
-            float zz[3] = {z.x, z.y, z.z};
-            float dd[3];
-            for (int c = 0; c < 3; ++c) {
-                const float y = expf(zz[c]);
-                const float t = target[3 * static_cast<size_t>(s) + c];
-                const float den = y * y + kRelEps;
-                lsum += (y - t) * (y - t) / den;
-                const float g = 2.0f * (y - t) / den * y;
-                dd[c] = g == g ? sat(g) : 0.0f;  // NaN (inf/inf) -> no update
-            }
-            d4.x = dd[0];
-            d4.y = dd[1];
-            d4.z = dd[2];
-            if (loss) loss[s] = lsum;
-        } else if (lane < 16 && s < n && loss) {
-            loss[s] = 0.0f;
-        }
-        const half4 D4 = to_half4(d4);
-        lds_put(s_del, del_row(4), col0, D4);
-        // delta_3 = W4 delta_4 (masked by ReLU of layer 3's output = H[4]).
-        half4 Dn[4];
-        for (int r = 0; r < 4; ++r) {
-            floatx4 a = {0.0f, 0.0f, 0.0f, 0.0f};
-            a = mfma(lds_frag(s_bwd, bwd_base(4) + r), D4, a);
-            Dn[r] = mask4(a, H[4][r]);
-            lds_put(s_del, del_row(3) + 16 * r, col0, Dn[r]);
-        }
-        for (int l = 3; l >= 1; --l) {
-            floatx4 a[4];
+        if (round != blockIdx.x) load(round);
+        const uint32_t s = round * kTrainChunk + col;
+        _Float16* act = s_act[col];
+        _Float16* del = s_del[col];
+        // Forward.
+        half4 H[4];
+        {
+            half4 X[fb(0)];
+            encode_block(in, box, X);
+            floatx4 z[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) a[r] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int r = 0; r < 4; ++r) z[r] = bias4(s_bias[0], r);
+#pragma unroll
+            for (int f = 0; f < fb(0); ++f) {
+                *lds_cell(act, 16 * f) = X[f];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[r] = mfma(lds_frag(s_fwd, r * fb(0) + f), X[f], z[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                H[r] = relu_half4(z[r]);
+                *lds_cell(act, act_col(1) + 16 * r) = H[r];
+            }
+        }
+#pragma unroll 1
+        for (int l = 1; l < 4; ++l) {
+            const uint2* frags = s_fwd + (fwd_base(1) + 16 * (l - 1)) * 64;
+            floatx4 z[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) z[r] = bias4(s_bias[l], r);
 #pragma unroll
             for (int f = 0; f < 4; ++f)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) a[r] = mfma(lds_frag(s_bwd, bwd_base(l) + r * 4 + f), Dn[f], a[r]);
+                for (int r = 0; r < 4; ++r) z[r] = mfma(lds_frag(frags, 4 * r + f), H[f], z[r]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                Dn[r] = mask4(a[r], H[l][r]);
-                lds_put(s_del, del_row(l - 1) + 16 * r, col0, Dn[r]);
+                H[r] = relu_half4(z[r]);
+                *lds_cell(act, act_col(1) + kHid * l + 16 * r) = H[r];
+            }
+        }
+        // Outputs: as in inference, every lane group gets all three.
+        floatx4 z = {s_bias[4][0], s_bias[4][1], s_bias[4][2], 0.0f};
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            half4 a;
+            __builtin_memcpy(&a, &s_fwd[(fwd_base(4) + f) * 64 + (lane & ~12)], sizeof a);
+            z = mfma(a, H[f], z);
+        }
+        // Output delta: d/dz of (e^z - t)^2 / (sg(e^z)^2 + eps), lane group c
+        // computing channel c of its samples.
+        const bool live = s < n && first == first;
+        const float y = expf(g == 0 ? z.x : (g == 1 ? z.y : z.z));
+        const float den = y * y + kRelEps;
+        const float lc = (y - t) * (y - t) / den;
+        const float gr = 2.0f * (y - t) / den * y;
+        const float dd = live && gr == gr ? sat(gr) : 0.0f;  // NaN (inf/inf) -> no update
+        const int c0 = lane % 16;
+        const float l1 = __shfl(lc, c0 + 16), l2 = __shfl(lc, c0 + 32);
+        const float d1 = __shfl(dd, c0 + 16), d2 = __shfl(dd, c0 + 32);
+        if (lane < 16 && s < n && loss) loss[s] = live ? (lc + l1) + l2 : 0.0f;
+        const floatx4 d4 = {dd, d1, d2, 0.0f};
+        const half4 D4 = lane < 16 ? to_half4(d4) : half4{0, 0, 0, 0};
+        *lds_cell(del, del_col(4)) = D4;
+        // delta_3 = W4 delta_4 (masked by ReLU of layer 3's output).
+        half4 D[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            floatx4 a = {0.0f, 0.0f, 0.0f, 0.0f};
+            a = mfma(lds_frag(s_bwd, bwd_base(4) + r), D4, a);
+            D[r] = mask4(a, H[r]);
+            *lds_cell(del, del_col(3) + 16 * r) = D[r];
+        }
+#pragma unroll 1
+        for (int l = 3; l >= 1; --l) {
+            const uint2* frags = s_bwd + 16 * (l - 1) * 64;
+            half4 h[4];  // layer l's inputs, as this lane stored them
+            floatx4 a[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                h[r] = *lds_cell(act, act_col(1) + kHid * (l - 1) + 16 * r);
+                a[r] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+#pragma unroll
+            for (int f = 0; f < 4; ++f)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[r] = mfma(lds_frag(frags, 4 * r + f), D[f], a[r]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                D[r] = mask4(a[r], h[r]);
+                *lds_cell(del, kHid * (l - 1) + 16 * r) = D[r];
             }
         }
         __syncthreads();
-        // dW tiles of this wave over the round's 64 samples (K = 4 x 16).
+        // dW tiles of this wave over the round's 64 samples (K = 4 x 16):
+        // layer 0 inputs 16 f .. by outputs 16 wave .., layers 1..3 inputs
+        // 16 wave .. by outputs 16 r .., layer 4 inputs 16 wave ...
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) {
+            const _Float16* a0 = s_act[16 * kb] + tr_off(kActLd);
+            const _Float16* d0 = s_del[16 * kb] + tr_off(kDelLd);
+            {
+                const half4 d = lds_get(d0 + 16 * wave);
 #pragma unroll
-            for (int t = 0; t < kTilesPerWave; ++t) {
-                const half4 a = lds_get(s_act, static_cast<int>(arow[t]), 16 * kb);
-                const half4 b = lds_get(s_del, static_cast<int>(drow[t]), 16 * kb);
-                acc[t] = mfma(a, b, acc[t]);
+                for (int f = 0; f < fb(0); ++f) acc[f] = mfma(lds_get(a0 + 16 * f), d, acc[f]);
             }
+#pragma unroll
+            for (int l = 1; l < 4; ++l) {
+                const half4 a = lds_get(a0 + act_col(l) + 16 * wave);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    acc[2 + 4 * l + r] = mfma(a, lds_get(d0 + del_col(l) + 16 * r), acc[2 + 4 * l + r]);
+            }
+            acc[18] = mfma(lds_get(a0 + act_col(4) + 16 * wave), lds_get(d0 + del_col(4)), acc[18]);
         }
         {
-            const int t = threadIdx.x;
-            float a = 0.0f, a4 = 0.0f;
-            for (int j = 0; j < kTrainChunk; ++j) {
-                a += static_cast<float>(s_del[t][j]);
-                if (t < kOut) a4 += static_cast<float>(s_del[kHid * 4 + t][j]);
-            }
+            const int c = threadIdx.x;
+            float a = 0.0f;
+#pragma unroll 16
+            for (int j = 0; j < kTrainChunk; ++j) a += static_cast<float>(s_del[j][c]);
             bsum += a;
-            bsum4 += a4;
+            if (c < kOut) {
+                float a4 = 0.0f;
+#pragma unroll 16
+                for (int j = 0; j < kTrainChunk; ++j) a4 += static_cast<float>(s_del[j][del_col(4) + c]);
+                bsum4 += a4;
+            }
         }
         __syncthreads();  // the next round rewrites the LDS rows
     }
+    // D lane: column (output) lane%16 of the tile, rows (inputs) 4(lane/16) + e.
     float* out = part + static_cast<size_t>(blockIdx.x) * kParams;
+    const int in0 = 4 * g, o = lane % 16;
 #pragma unroll
-    for (int t = 0; t < kTilesPerWave; ++t) {
-        const int task = wave + 4 * t;
-        int l = 0;
-        while (l + 1 < kLayers && task >= fwd_base(l + 1)) ++l;
-        const int k = task - fwd_base(l);
-        const int ri = k % fb(l), co = k / fb(l);
-        const int ni = dim(l), no = dim(l + 1);
-        // D lane: column (output) 16co + lane%16, rows (inputs) 16ri + 4(lane/16) + e.
-        const int o = 16 * co + lane % 16;
-        for (int e = 0; e < 4; ++e) {
-            const int i = 16 * ri + 4 * (lane / 16) + e;
-            if (i < ni && o < no) out[w_off(l) + i * no + o] = acc[t][e];
-        }
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int f = 0; f < fb(0); ++f) out[(16 * f + in0 + e) * kHid + 16 * wave + o] = acc[f][e];
+#pragma unroll
+        for (int l = 1; l < 4; ++l)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                out[w_off(l) + (16 * wave + in0 + e) * kHid + 16 * r + o] = acc[2 + 4 * l + r][e];
+        if (o < kOut) out[w_off(4) + (16 * wave + in0 + e) * kOut + o] = acc[18][e];
     }
-    {
-        const int t = threadIdx.x;
-        out[b_off(t / kHid) + t % kHid] = bsum;
-        if (t < kOut) out[b_off(4) + t] = bsum4;
-    }
+    const int c = threadIdx.x;
+    out[b_off(c / kHid) + c % kHid] = bsum;
+    if (c < kOut) out[b_off(4) + c] = bsum4;
 }
 
 // Adam (Kingma & Ba 2015) on the fp32 masters, one thread per parameter; the
@@ -672,7 +697,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_adam_pack(float* __restrict__ 
     float acc = 0.0f;
     if (p < kParams) {
         uint32_t s = static_cast<uint32_t>(wave);
-#pragma unroll 8
+#pragma unroll 16
         for (; s < nparts; s += kWaves) acc += part[static_cast<size_t>(s) * kParams + p];
     }
     s_sum[wave][lane] = acc;
@@ -784,7 +809,10 @@ void RadianceCache::infer(const float* d_raw, uint32_t n, float* d_out, hipStrea
         b.mn[k] = box_min[k];
         b.inv_ext[k] = box_inv[k];
     }
-    const uint32_t blocks = std::min<uint32_t>(blocks_for(n, 4 * 16 * kInferBlocks), 2048);
+    // At most what is resident at once (four workgroups a CU by LDS and
+    // registers): the weights are staged once (2,048 blocks: a single call of
+    // 2,073,600 samples 91.1 us, 89.6 with 1,024).
+    const uint32_t blocks = std::min<uint32_t>(blocks_for(n, 4 * 16 * kInferBlocks), 1024);
     hipLaunchKernelGGL(k_mlp_infer, dim3(blocks), dim3(kThreads), 0, st, f32.as<uint4>(), master.as<float>(),
                        d_raw, n, b, d_out);
     PT_HIP(hipGetLastError());
