@@ -214,6 +214,7 @@ void upload_scenes(pt_context* ctx, const pt_triangle* tris, const uint32_t* off
     PT_HIP(hipMemcpyAsync(s.off.as<void>(), offs, (nscenes + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, st));
     PT_HIP(hipMemcpyAsync(s.morton_box.as<void>(), mbox.data(), mbox.size() * sizeof(float),
                           hipMemcpyHostToDevice, st));
+    pt::plan_sort(s, st);
     if (n) {
         s.tris.reserve(sizeof(pt_triangle) * static_cast<size_t>(n));
         PT_HIP(hipMemcpyAsync(s.tris.as<void>(), tris, sizeof(pt_triangle) * static_cast<size_t>(n),

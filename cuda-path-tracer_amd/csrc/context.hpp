@@ -122,6 +122,12 @@ struct DeviceScene {
     std::vector<float> box_host;           // per scene: min.xyz, max.xyz
     DevBuf off;                            // device copy of off_host
     DevBuf morton_box;                     // per scene: min.xyz, 1/(max-min).xyz
+    // The build's sort (plan_sort): whether each scene is a segment, its tiles,
+    // the segments that need a scan, and with segments the tables of both.
+    bool sort_segmented = false;
+    uint32_t sort_tiles = 0, sort_scans = 0;
+    std::vector<uint32_t> sort_plan_host;
+    DevBuf sort_plan;
     DevBuf tris;                           // pt_triangle[n] as uploaded
     DevBuf infos;                          // pt_triangle_info[ninfos]
     DevBuf lights;                         // pt_dir_light[nlights] (all scenes)
@@ -144,6 +150,8 @@ struct BuildTimes {
     float total = 0.0f;
 };
 
+// Sort tiles of the scenes in off_host, planned once per upload.
+void plan_sort(DeviceScene& scene, hipStream_t stream);
 // LBVH build: Morton keys -> LDS radix sort -> radix tree with its boxes.
 void build_lbvh(DeviceScene& scene, hipStream_t stream);
 // Parity dump of one scene in local indices (device -> host, synchronous).

@@ -8,14 +8,15 @@
 //                   and the first sort pass's per-tile digit counts
 //   k_sort_hist     \
 //   k_sort_rowscan   } LSD radix sort, 10-bit digits, stable: 3 passes over
-//   k_sort_scatter  /  the 30-bit key, then 1-2 over the scene id when
-//                      batched (wave64 ballot match + LDS staging per
-//                      4096-key tile)
+//   k_sort_scatter  /  the 30-bit key, each scene of a batch on its own or,
+//                      with many small ones, all together and then 1-2
+//                      passes over the scene id (wave64 ballot match + LDS
+//                      staging per 4096-key tile)
 //   k_tree_leaves   sorted triangle records, then the radix tree and its boxes
 //                   bottom-up inside each 1024-leaf block (LDS, workgroup
 //                   scope); each node's traversal record is written whole by
 //                   the thread that completes it
-//   k_tree_merge    the same over the subtrees that 64 blocks left open, level
+//   k_tree_merge    the same over the subtrees that 16 blocks left open, level
 //                   by level until none is
 #include <hip/hip_runtime.h>
 
@@ -33,6 +34,18 @@ constexpr int kSortTile = 4096;                                // keys per sort 
 constexpr int kDigitBits = 10;                                 // 3 passes over a 30-bit key
 constexpr uint32_t kRadix = 1u << kDigitBits;                  // 1024 digits
 constexpr int kScatterThreads = 512;                           // scatter: 8 keys per thread, 8 waves per tile
+// A segment (see there) of at most this many tiles needs no scan launch: its
+// scatter workgroups add up the tiles' counts themselves, all loads in flight
+// together.  Soups of 17 / 25 / 32 / 64 tiles build in 87.6 / 91.9 / 94.1 / 111.3
+// us so, in 94.1 / 97.9 / 97.4 / 105.3 with the scan.
+constexpr uint32_t kFewTiles = 32;
+// Scenes of a batch are sorted as segments of their own, which saves the passes
+// over the scene id, unless that takes too many half-empty tiles: at most
+// kSpareTiles + 4 per tile of an unsegmented sort.  64 scenes of 100 triangles
+// build in 54 us (78 by scene passes), 1,000 in 91 (109), 2,000 in 137 (138),
+// 4,000 in 237 (160); 2,000 scenes of 500 in 192 (209), 1,000 of 2,500 in 280
+// (463), 64 of 1,024 .. 262,144 in 345 (447).
+constexpr uint32_t kSpareTiles = 1536;
 // The tree is built bottom-up, boxes included, in levels: one workgroup per
 // block of kLeafBlock sorted leaves, then one per kFanIn blocks' open subtrees,
 // and so on (see the tree section).
@@ -65,6 +78,25 @@ __device__ __forceinline__ uint32_t quantize1024(float x) {
     return static_cast<uint32_t>(static_cast<int32_t>(s));
 }
 
+// Sort tiles.  A segment is a range of slots sorted on its own: each scene
+// (table: an entry for every tile), or all slots (no table).
+struct Segment {
+    uint32_t start, end;  // slots
+    uint32_t id;          // scene
+    uint32_t first_tile;
+};
+__device__ __forceinline__ Segment segment_of_tile(const uint4* __restrict__ table, uint32_t n, uint32_t tile) {
+    if (table == nullptr) return Segment{0u, n, 0u, 0u};
+    const uint4 t = table[tile];
+    return Segment{t.x, t.y, t.z, t.w};
+}
+__device__ __forceinline__ uint32_t tile_base(const Segment& s, uint32_t tile) {
+    return s.start + (tile - s.first_tile) * kSortTile;
+}
+__device__ __forceinline__ uint32_t tile_count(const Segment& s) {
+    return (s.end - s.start + kSortTile - 1u) / kSortTile;
+}
+
 // Scene of leaf slot i: the last s with off[s] <= i (off has nscenes + 1 entries).
 __device__ __forceinline__ uint32_t scene_of_slot(const uint32_t* __restrict__ off, uint32_t nscenes,
                                                   uint32_t i) {
@@ -79,14 +111,14 @@ __device__ __forceinline__ uint32_t scene_of_slot(const uint32_t* __restrict__ o
 
 // morton_encoder (BVHBuilder.cu:12-32): centroid ((v0 + v1) + v2) / 3, mapped
 // into the scene's enclosing box with invScale computed on the host
-// (box[6*s..] = min.xyz, invScale.xyz).  One workgroup per 4096-key sort
-// tile, which also counts the tile's first-pass digits (key bits 0-9) into
+// (box[6*s..] = min.xyz, invScale.xyz).  One workgroup per sort tile, which also counts the tile's first-pass digits (key bits 0-9) into
 // its row of tile_hist -- the first sort pass then starts at the scan.
 constexpr int kMortonThreads = 1024;
 
 __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __restrict__ tris, uint32_t n,
                                                            const uint32_t* __restrict__ off, uint32_t nscenes,
                                                            const float* __restrict__ box,
+                                                           const uint4* __restrict__ table,
                                                            uint32_t* __restrict__ keys,
                                                            uint32_t* __restrict__ vals,
                                                            uint32_t* __restrict__ scene_of,
@@ -95,12 +127,13 @@ __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __
     const uint32_t tid = threadIdx.x;
     for (uint32_t d = tid; d < kRadix; d += kMortonThreads) h[d] = 0u;
     __syncthreads();
-    const uint32_t base = blockIdx.x * kSortTile;
+    const Segment seg = segment_of_tile(table, n, blockIdx.x);
+    const uint32_t base = tile_base(seg, blockIdx.x);
 #pragma unroll
     for (int r = 0; r < kSortTile / kMortonThreads; ++r) {
         const uint32_t i = base + r * kMortonThreads + tid;
-        if (i >= n) break;
-        const uint32_t sc = scene_of_slot(off, nscenes, i);
+        if (i >= seg.end) break;
+        const uint32_t sc = table != nullptr ? seg.id : scene_of_slot(off, nscenes, i);
         const float* bx = box + 6 * static_cast<size_t>(sc);
         const float* t = reinterpret_cast<const float*>(tris + i);
         float cx = ((t[0] + t[3]) + t[6]) / 3.0f;
@@ -138,26 +171,30 @@ template <bool BY_SCENE>
 __global__ __launch_bounds__(kHistThreads) void k_sort_hist(const uint32_t* __restrict__ keys,
                                                             const uint32_t* __restrict__ vals,
                                                             const uint32_t* __restrict__ scene_of,
+                                                            const uint4* __restrict__ table,
                                                             uint32_t n, int shift,
-                                                            uint32_t num_tiles,
                                                             uint32_t* __restrict__ tile_hist) {
     __shared__ uint32_t h[kRadix];
     const int tid = threadIdx.x;
     for (int d = tid; d < static_cast<int>(kRadix); d += kHistThreads) h[d] = 0;
     __syncthreads();
-    const uint32_t base = blockIdx.x * kSortTile;
+    const Segment seg = segment_of_tile(table, n, blockIdx.x);
+    const uint32_t base = tile_base(seg, blockIdx.x);
 #pragma unroll
     for (int r = 0; r < kSortTile / kHistThreads; ++r) {
         uint32_t i = base + r * kHistThreads + tid;
-        if (i < n) atomicAdd(&h[sort_digit<BY_SCENE>(keys[i], BY_SCENE ? vals[i] : 0u, scene_of, shift)], 1u);
+        if (i < seg.end) atomicAdd(&h[sort_digit<BY_SCENE>(keys[i], BY_SCENE ? vals[i] : 0u, scene_of, shift)], 1u);
     }
     __syncthreads();
     for (int d = tid; d < static_cast<int>(kRadix); d += kHistThreads)
         tile_hist[static_cast<size_t>(blockIdx.x) * kRadix + d] = h[d];
 }
 
-// Exclusive scan of each digit's counts over the tiles (in place) and the
-// digit's total.  One workgroup per 64 digits: lane = digit, so every load
+// Exclusive scan of each digit's counts over a segment's tiles (in place) and
+// the digit's total, for segments of more than kFewTiles tiles (scans: first and
+// past-last tile of each; none: all tiles).  Their totals' row is first_tile /
+// (kFewTiles + 1), which no two of them share.  One workgroup per segment and 64
+// digits: lane = digit, so every load
 // and store of a tile's 64 counts is one contiguous 256-byte access; the 16
 // waves split the tiles into 16 ranges, and each wave's range starts at the
 // sum of the earlier ranges.
@@ -166,13 +203,17 @@ constexpr int kScanWaves = 16;
 
 __global__ __launch_bounds__(kScanWaves * 64) void k_sort_rowscan(uint32_t* __restrict__ tile_hist,
                                                                   uint32_t num_tiles,
+                                                                  const uint2* __restrict__ scans,
                                                                   uint32_t* __restrict__ digit_total) {
     __shared__ uint32_t s_part[kScanWaves][kScanDigits];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const uint32_t d = blockIdx.x * kScanDigits + lane;
-    const uint32_t per = (num_tiles + kScanWaves - 1) / kScanWaves;
-    const uint32_t t0 = min(num_tiles, wave * per), t1 = min(num_tiles, t0 + per);
+    const uint32_t seg = blockIdx.x / (kRadix / kScanDigits);
+    const uint32_t d = blockIdx.x % (kRadix / kScanDigits) * kScanDigits + lane;
+    const uint32_t first = scans != nullptr ? scans[seg].x : 0u;
+    const uint32_t last = scans != nullptr ? scans[seg].y : num_tiles;
+    const uint32_t per = (last - first + kScanWaves - 1) / kScanWaves;
+    const uint32_t t0 = min(last, first + wave * per), t1 = min(last, t0 + per);
     // Loads in batches of kScanBatch, issued together (the counts come from
     // other XCDs' writes: each load is a far round trip).  The first batch
     // stays in registers for the second sweep (up to 256 tiles, 2^20 keys,
@@ -213,7 +254,7 @@ __global__ __launch_bounds__(kScanWaves * 64) void k_sort_rowscan(uint32_t* __re
             run += v[k];
         }
     }
-    if (wave == kScanWaves - 1) digit_total[d] = run;
+    if (wave == kScanWaves - 1) digit_total[static_cast<size_t>(first / (kFewTiles + 1u)) * kRadix + d] = run;
 }
 
 // Block-wide exclusive scan of one value per thread over WAVES waves;
@@ -253,9 +294,8 @@ template <bool BY_SCENE, int THREADS>
 __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
-    const uint32_t* __restrict__ scene_of, uint32_t n, int shift,
-    uint32_t num_tiles, const uint32_t* __restrict__ tile_hist,
-    const uint32_t* __restrict__ digit_total) {
+    const uint32_t* __restrict__ scene_of, const uint4* __restrict__ table, uint32_t n, int shift,
+    const uint32_t* __restrict__ tile_hist, const uint32_t* __restrict__ digit_total) {
     constexpr int WAVES = THREADS / 64;
     constexpr int KPT = kSortTile / THREADS;  // keys per thread
     constexpr int DPT = kRadix / THREADS;     // digits per thread
@@ -277,8 +317,9 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     __syncthreads();
 
     const uint32_t tile = blockIdx.x;
-    const uint32_t base = tile * kSortTile;
-    const uint32_t count = min(static_cast<uint32_t>(kSortTile), n - base);
+    const Segment seg = segment_of_tile(table, n, tile);
+    const uint32_t base = tile_base(seg, tile);
+    const uint32_t count = min(static_cast<uint32_t>(kSortTile), seg.end - base);
     const uint64_t lt = (1ull << lane) - 1ull;
 
     uint32_t key[KPT], val[KPT], rk[KPT];
@@ -289,6 +330,32 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
         const bool valid = li < count;
         key[r] = valid ? keys_in[base + li] : 0u;
         val[r] = valid ? vals_in[base + li] : 0u;
+    }
+    // This thread's digits: the segment's totals, and those of the tiles before
+    // (up to kFewTiles tiles, tile_hist still holds each tile's own counts).
+    static_assert(DPT == 2, "a thread's two digits are one load");
+    uint32_t gt[DPT], before[DPT];
+    const uint32_t tiles = tile_count(seg);
+    if (tiles <= kFewTiles) {
+        const uint2* row = reinterpret_cast<const uint2*>(tile_hist + static_cast<size_t>(seg.first_tile) * kRadix) + tid;
+        const uint32_t mine = tile - seg.first_tile;
+        gt[0] = gt[1] = before[0] = before[1] = 0u;
+#pragma unroll 4
+        for (uint32_t t = 0; t < tiles; ++t) {
+            const uint2 c = row[static_cast<size_t>(t) * (kRadix / 2)];
+            gt[0] += c.x;
+            gt[1] += c.y;
+            before[0] += t < mine ? c.x : 0u;
+            before[1] += t < mine ? c.y : 0u;
+        }
+    } else {
+        const uint2 g2 = reinterpret_cast<const uint2*>(
+            digit_total + static_cast<size_t>(seg.first_tile / (kFewTiles + 1u)) * kRadix)[tid];
+        const uint2 b2 = reinterpret_cast<const uint2*>(tile_hist + static_cast<size_t>(tile) * kRadix)[tid];
+        gt[0] = g2.x;
+        gt[1] = g2.y;
+        before[0] = b2.x;
+        before[1] = b2.y;
     }
 #pragma unroll
     for (int r = 0; r < KPT; ++r) {
@@ -314,7 +381,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     __syncthreads();
 
     // Digits DPT*t ..: offsets of each wave's run, tile-local start, global base.
-    uint32_t tot[DPT], gt[DPT];
+    uint32_t tot[DPT];
     uint32_t tsum = 0, gsum = 0;
 #pragma unroll
     for (int j = 0; j < DPT; ++j) {
@@ -327,18 +394,17 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
             run += c;
         }
         tot[j] = run;
-        gt[j] = digit_total[d];
         tsum += tot[j];
         gsum += gt[j];
     }
     uint32_t tmp;
     uint32_t dstart = block_excl_scan<WAVES>(tsum, s_w, tmp);
-    uint32_t gpre = block_excl_scan<WAVES>(gsum, s_w, tmp);
+    uint32_t gpre = seg.start + block_excl_scan<WAVES>(gsum, s_w, tmp);
 #pragma unroll
     for (int j = 0; j < DPT; ++j) {
         const int d = DPT * tid + j;
         s_dstart[d] = dstart;
-        s_gbase[d] = gpre + tile_hist[static_cast<size_t>(tile) * kRadix + d];
+        s_gbase[d] = gpre + before[j];
         dstart += tot[j];
         gpre += gt[j];
     }
@@ -751,6 +817,38 @@ BuildTuning& build_tuning() {
     return t;
 }
 
+void plan_sort(DeviceScene& s, hipStream_t st) {
+    const uint32_t nscenes = s.nscenes();
+    const uint32_t plain = div_up(s.n, kSortTile);
+    uint64_t tiles = 0;
+    for (uint32_t k = 0; k < nscenes; ++k) tiles += div_up(s.off_host[k + 1] - s.off_host[k], kSortTile);
+    s.sort_plan_host.clear();
+    s.sort_segmented = nscenes > 1 && tiles <= kSpareTiles + 4ull * plain;
+    if (!s.sort_segmented) {
+        s.sort_tiles = plain;
+        s.sort_scans = plain > kFewTiles ? 1u : 0u;
+        return;
+    }
+    // An entry per tile, then first and past-last tile of each segment to scan.
+    s.sort_tiles = static_cast<uint32_t>(tiles);
+    s.sort_scans = 0;
+    std::vector<uint32_t>& plan = s.sort_plan_host;
+    plan.reserve(4 * tiles);
+    std::vector<uint32_t> scans;
+    uint32_t t = 0;
+    for (uint32_t k = 0; k < nscenes; ++k) {
+        const uint32_t a = s.off_host[k], b = s.off_host[k + 1], first = t;
+        for (const uint32_t last = first + div_up(b - a, kSortTile); t < last; ++t) plan.insert(plan.end(), {a, b, k, first});
+        if (t - first > kFewTiles) {
+            scans.insert(scans.end(), {first, t});
+            ++s.sort_scans;
+        }
+    }
+    plan.insert(plan.end(), scans.begin(), scans.end());
+    s.sort_plan.reserve(plan.size() * 4);
+    PT_HIP(hipMemcpyAsync(s.sort_plan.as<void>(), plan.data(), plan.size() * 4, hipMemcpyHostToDevice, st));
+}
+
 void build_lbvh(DeviceScene& s, hipStream_t st) {
     DeviceBvh& b = s.bvh;
     const uint32_t n = s.n;
@@ -768,9 +866,11 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     b.tris.reserve(static_cast<size_t>(n) * 48);
     b.root_box.reserve(static_cast<size_t>(nscenes) * 6 * sizeof(float));
     b.root_word.reserve(static_cast<size_t>(nscenes) * 4);
-    const uint32_t num_tiles = div_up(n, kSortTile);
+    const uint32_t num_tiles = s.sort_tiles;
+    const uint4* table = s.sort_segmented ? s.sort_plan.as<uint4>() : nullptr;
+    const uint2* scans = table ? reinterpret_cast<const uint2*>(table + num_tiles) : nullptr;
     b.tile_hist.reserve(static_cast<size_t>(num_tiles) * kRadix * 4);
-    b.digit_total.reserve(kRadix * 4);
+    b.digit_total.reserve(static_cast<size_t>(num_tiles / (kFewTiles + 1) + 1) * kRadix * 4);
     // Open lists of every level, one after the other.
     const uint32_t blocks = div_up(n, kLeafBlock);
     size_t nlists = blocks;
@@ -780,41 +880,39 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     uint32_t* kin = b.keys.as<uint32_t>();
     uint32_t* vin = b.vals.as<uint32_t>();
     hipLaunchKernelGGL(k_morton, dim3(num_tiles), dim3(kMortonThreads), 0, st, s.tris.as<pt_triangle>(), n,
-                       s.off.as<uint32_t>(), nscenes, s.morton_box.as<float>(), kin, vin,
+                       s.off.as<uint32_t>(), nscenes, s.morton_box.as<float>(), table, kin, vin,
                        b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>());
     PT_HIP(hipGetLastError());
 
     if (n >= 2) {
         uint32_t* kout = b.keys_alt.as<uint32_t>();
         uint32_t* vout = b.vals_alt.as<uint32_t>();
-        // 3 passes over the 30-bit keys, then the scene id's 10-bit digits
-        // (stable: each scene keeps its key order, ties in input order).
+        // 3 passes over the 30-bit keys; unless the scenes are segments, then the
+        // scene id's 10-bit digits (stable: each scene keeps its key order, ties
+        // in input order).
         constexpr int kKeyPasses = (30 + kDigitBits - 1) / kDigitBits;
         int scene_passes = 0;
-        for (uint32_t v = nscenes - 1; v != 0; v >>= kDigitBits) ++scene_passes;
+        if (!s.sort_segmented)
+            for (uint32_t v = nscenes - 1; v != 0; v >>= kDigitBits) ++scene_passes;
         const int passes = kKeyPasses + scene_passes;
+        const uint32_t* sc = b.scene_of.as<uint32_t>();
+        uint32_t* hist = b.tile_hist.as<uint32_t>();
+        uint32_t* totals = b.digit_total.as<uint32_t>();
         for (int pass = 0; pass < passes; ++pass) {
             const bool by_scene = pass >= kKeyPasses;
             const int shift = kDigitBits * (by_scene ? pass - kKeyPasses : pass);
             // The first pass's counts come from k_morton.
-            if (by_scene) {
-                hipLaunchKernelGGL(k_sort_hist<true>, dim3(num_tiles), dim3(kHistThreads), 0, st, kin, vin,
-                                   b.scene_of.as<uint32_t>(), n, shift, num_tiles, b.tile_hist.as<uint32_t>());
-            } else if (pass > 0) {
-                hipLaunchKernelGGL(k_sort_hist<false>, dim3(num_tiles), dim3(kHistThreads), 0, st, kin, vin,
-                                   b.scene_of.as<uint32_t>(), n, shift, num_tiles, b.tile_hist.as<uint32_t>());
+            if (pass > 0) {
+                hipLaunchKernelGGL(by_scene ? k_sort_hist<true> : k_sort_hist<false>, dim3(num_tiles), dim3(kHistThreads),
+                                   0, st, kin, vin, sc, table, n, shift, hist);
             }
-            hipLaunchKernelGGL(k_sort_rowscan, dim3(kRadix / kScanDigits), dim3(kScanWaves * 64), 0, st,
-                               b.tile_hist.as<uint32_t>(), num_tiles, b.digit_total.as<uint32_t>());
-            if (by_scene) {
-                hipLaunchKernelGGL((k_sort_scatter<true, kScatterThreads>), dim3(num_tiles), dim3(kScatterThreads), 0, st, kin, vin,
-                                   kout, vout, b.scene_of.as<uint32_t>(), n, shift, num_tiles,
-                                   b.tile_hist.as<uint32_t>(), b.digit_total.as<uint32_t>());
-            } else {
-                hipLaunchKernelGGL((k_sort_scatter<false, kScatterThreads>), dim3(num_tiles), dim3(kScatterThreads), 0, st, kin, vin,
-                                   kout, vout, b.scene_of.as<uint32_t>(), n, shift, num_tiles,
-                                   b.tile_hist.as<uint32_t>(), b.digit_total.as<uint32_t>());
+            if (s.sort_scans > 0) {
+                hipLaunchKernelGGL(k_sort_rowscan, dim3(s.sort_scans * (kRadix / kScanDigits)), dim3(kScanWaves * 64), 0, st,
+                                   hist, num_tiles, scans, totals);
             }
+            const auto scatter = by_scene ? k_sort_scatter<true, kScatterThreads> : k_sort_scatter<false, kScatterThreads>;
+            hipLaunchKernelGGL(scatter, dim3(num_tiles), dim3(kScatterThreads), 0, st, kin, vin, kout, vout, sc, table, n,
+                               shift, hist, totals);
             std::swap(kin, kout);
             std::swap(vin, vout);
         }
