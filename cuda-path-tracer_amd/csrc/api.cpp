@@ -19,7 +19,7 @@ namespace {
 thread_local std::string g_last_error;
 
 template <class F>
-int guarded(pt_context* ctx, F&& f) {
+int guarded_frame(pt_context* ctx, F&& f) {
     try {
         if (ctx) PT_HIP(hipSetDevice(ctx->device));
         f();
@@ -37,6 +37,13 @@ int guarded(pt_context* ctx, F&& f) {
         g_last_error = "unknown error";
         return PT_E_INTERNAL;
     }
+}
+
+// Any other call: frames that follow are ordered after its work.
+template <class F>
+int guarded(pt_context* ctx, F&& f) {
+    if (ctx) ctx->renderer.other_work = true;
+    return guarded_frame(ctx, std::forward<F>(f));
 }
 
 void require(bool cond, const char* msg) {
@@ -566,7 +573,7 @@ int pt_set_screen_buffer(pt_context* ctx, void* d_rgba, uint32_t w, uint32_t h, 
 int pt_read_image_device(pt_context* ctx, void* d_rgba, uint32_t w, uint32_t h, size_t row_pitch,
                          void* stream) {
     if (!ctx || !d_rgba) return PT_E_INVALID_ARG;
-    return guarded(ctx, [&] {
+    return guarded_frame(ctx, [&] {
         require(row_pitch >= static_cast<size_t>(w) * 16 && row_pitch % 16 == 0,
                 "row pitch must hold w float4 texels and be a multiple of 16 bytes");
         require(reinterpret_cast<uintptr_t>(d_rgba) % 16 == 0, "image buffer must be 16-byte aligned");
@@ -576,7 +583,7 @@ int pt_read_image_device(pt_context* ctx, void* d_rgba, uint32_t w, uint32_t h, 
 
 int pt_set_primary_rays(pt_context* ctx, const float* dirs, const float* eye) {
     if (!ctx || !dirs || !eye) return PT_E_INVALID_ARG;
-    return guarded(ctx, [&] {
+    return guarded_frame(ctx, [&] {
         std::memcpy(ctx->renderer.dirs, dirs, sizeof ctx->renderer.dirs);
         std::memcpy(ctx->renderer.eye, eye, sizeof ctx->renderer.eye);
     });
@@ -584,7 +591,7 @@ int pt_set_primary_rays(pt_context* ctx, const float* dirs, const float* eye) {
 
 int pt_render_pass(pt_context* ctx, int w, int h, uint64_t pass_seed) {
     if (!ctx) return PT_E_INVALID_ARG;
-    return guarded(ctx, [&] {
+    return guarded_frame(ctx, [&] {
         if (!ctx->scene.ready) throw pt::Error(PT_E_NO_SCENE, "no scene uploaded");
         hipStream_t st = ctx->stream;
         pt::render_resize(ctx->renderer, w, h, st);
@@ -600,7 +607,7 @@ int pt_render_pass(pt_context* ctx, int w, int h, uint64_t pass_seed) {
 int pt_render_passes(pt_context* ctx, int w, int h, uint32_t npasses, const float* dirs,
                      const uint64_t* seeds, const uint32_t* scenes) {
     if (!ctx || !seeds) return PT_E_INVALID_ARG;
-    return guarded(ctx, [&] {
+    return guarded_frame(ctx, [&] {
         if (!ctx->scene.ready) throw pt::Error(PT_E_NO_SCENE, "no scene uploaded");
         hipStream_t st = ctx->stream;
         pt::render_resize(ctx->renderer, w, h, st);
@@ -621,7 +628,7 @@ int pt_last_frame_rays(pt_context* ctx, uint64_t* rays) {
 
 int pt_reset_frames(pt_context* ctx) {
     if (!ctx) return PT_E_INVALID_ARG;
-    return guarded(ctx, [&] { pt::render_reset(ctx->renderer, ctx->stream); });
+    return guarded_frame(ctx, [&] { pt::render_reset(ctx->renderer, ctx->stream); });
 }
 
 int pt_read_accumulator(pt_context* ctx, double* rgb_sum, uint32_t* spp) {

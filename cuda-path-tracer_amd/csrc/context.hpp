@@ -210,6 +210,7 @@ struct PassParams {
     uint32_t scene;  // scene of a batch traced by this pass
 };
 constexpr uint32_t kMaxPasses = 1024;  // passes per frame
+constexpr int kFrameSlots = 3;       // frames traced beside the last one
 constexpr int kParamRing = 4;        // pinned PassParams slots in flight
 
 // Progressive renderer state (wavefront queues + FP64 accumulator).
@@ -229,6 +230,22 @@ struct Renderer {
     int ring_next = 0;
     void* graph_exec = nullptr;   // hipGraphExec_t of the last captured frame
     alignas(8) char graph_key[256] = {};
+    // Frames that follow one another while the last is still at work trace their
+    // paths on streams of their own (render_passes): slot k's stream, path
+    // state, counters and pass block; `traced` after its paths, `added` after
+    // their sum into the accumulator, which the frames' own stream does in order.
+    struct FrameSlot {
+        hipStream_t st = nullptr;
+        hipEvent_t traced = nullptr, added = nullptr;
+        DevBuf state, counters, params;
+    };
+    FrameSlot slots[kFrameSlots];
+    int slot_next = 0;
+    hipEvent_t frame_ev = nullptr;   // after the last frame
+    bool frame_sent = false;
+    hipEvent_t base_ev = nullptr;    // before the first frame since other_work
+    bool other_work = true;          // a call other than a frame's came in between
+    const uint32_t* last_counters = nullptr;  // of the last frame
     bool timed = false;   // a pass has been bracketed by the context events
     uint32_t last_levels = 0;  // queue levels of the last frame
     uint32_t last_chains = 1;  // level chains of the last frame

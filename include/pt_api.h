@@ -255,7 +255,10 @@ int pt_trace_closest_counted(pt_context* ctx, const float* d_rays, uint32_t n,
 int pt_set_primary_rays(pt_context* ctx, const float* dirs, const float* eye);
 /* CUDAPathTracer::raytrace (cuda_path_tracer.cu:423-464): one 1-spp pass over
  * w x h pixels, added to the FP64 accumulator.  The accumulator is reset when
- * w/h change.  pass_seed replaces the per-pass host random seed. */
+ * w/h change.  pass_seed replaces the per-pass host random seed.  Asynchronous
+ * on the context's stream, like pt_render_passes; a frame of up to 2^22 paths
+ * sent while the one before is at work traces its paths beside it (at most
+ * three such frames, each with 24 bytes of memory per path). */
 int pt_render_pass(pt_context* ctx, int w, int h, uint64_t pass_seed);
 /* Several passes in one frame (no reference counterpart; the reference
  * launches one pass per frame): the accumulator ends up exactly as after
@@ -303,7 +306,8 @@ int pt_set_stop_frame(pt_context* ctx, uint32_t frames);
  * after the last reset to the render call that found the limit reached, or -1
  * while it has not been reached. */
 int pt_generation_time(pt_context* ctx, double* seconds);
-/* Wall time in ms of the last pt_render_pass (HIP events). */
+/* Wall time in ms of the last pt_render_pass (HIP events); of one sent while the
+ * frame before was at work, the time the context's stream spent on it. */
 int pt_last_render_ms(pt_context* ctx, float* ms);
 
 /* ---- learned radiance cache (no reference counterpart) -----------------------
