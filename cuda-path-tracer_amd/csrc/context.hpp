@@ -105,7 +105,7 @@ class HostBuf {
 //       (p0.xyz, original id) (e1.xyz, 0) (e2.xyz, 0), e = p - p0.
 struct DeviceBvh {
     uint32_t n = 0;
-    DevBuf keys, vals, keys_alt, vals_alt;  // sorted Morton keys, perm (+ ping-pong)
+    DevBuf pairs, pairs_alt;                // sorted (Morton key, perm) (+ ping-pong)
     DevBuf scene_of;                        // scene of each leaf slot
     DevBuf nodes, tris;
     DevBuf root_box, root_word;     // per scene: the root's box and child word (kInvalid: one triangle)

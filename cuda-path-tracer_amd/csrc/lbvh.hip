@@ -119,8 +119,7 @@ __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __
                                                            const uint32_t* __restrict__ off, uint32_t nscenes,
                                                            const float* __restrict__ box,
                                                            const uint4* __restrict__ table,
-                                                           uint32_t* __restrict__ keys,
-                                                           uint32_t* __restrict__ vals,
+                                                           uint2* __restrict__ pairs,
                                                            uint32_t* __restrict__ scene_of,
                                                            uint32_t* __restrict__ tile_hist) {
     __shared__ uint32_t h[kRadix];
@@ -143,8 +142,7 @@ __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __
         uint32_t qy = quantize1024((cy - bx[1]) * bx[4]);
         uint32_t qz = quantize1024((cz - bx[2]) * bx[5]);
         const uint32_t key = spread10(qx) | (spread10(qy) << 1) | (spread10(qz) << 2);
-        keys[i] = key;
-        vals[i] = i;
+        pairs[i] = make_uint2(key, i);
         scene_of[i] = sc;
         atomicAdd(&h[key & (kRadix - 1u)], 1u);
     }
@@ -168,8 +166,7 @@ __device__ __forceinline__ uint32_t sort_digit(uint32_t k, uint32_t v,
 constexpr int kHistThreads = 1024;
 
 template <bool BY_SCENE>
-__global__ __launch_bounds__(kHistThreads) void k_sort_hist(const uint32_t* __restrict__ keys,
-                                                            const uint32_t* __restrict__ vals,
+__global__ __launch_bounds__(kHistThreads) void k_sort_hist(const uint2* __restrict__ pairs,
                                                             const uint32_t* __restrict__ scene_of,
                                                             const uint4* __restrict__ table,
                                                             uint32_t n, int shift,
@@ -183,7 +180,10 @@ __global__ __launch_bounds__(kHistThreads) void k_sort_hist(const uint32_t* __re
 #pragma unroll
     for (int r = 0; r < kSortTile / kHistThreads; ++r) {
         uint32_t i = base + r * kHistThreads + tid;
-        if (i < seg.end) atomicAdd(&h[sort_digit<BY_SCENE>(keys[i], BY_SCENE ? vals[i] : 0u, scene_of, shift)], 1u);
+        if (i < seg.end) {
+            const uint2 p = pairs[i];
+            atomicAdd(&h[sort_digit<BY_SCENE>(p.x, p.y, scene_of, shift)], 1u);
+        }
     }
     __syncthreads();
     for (int d = tid; d < static_cast<int>(kRadix); d += kHistThreads)
@@ -292,8 +292,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_w, u
 // scans.
 template <bool BY_SCENE, int THREADS>
 __global__ __launch_bounds__(THREADS) void k_sort_scatter(
-    const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
-    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
+    const uint2* __restrict__ pairs_in, uint2* __restrict__ pairs_out,
     const uint32_t* __restrict__ scene_of, const uint4* __restrict__ table, uint32_t n, int shift,
     const uint32_t* __restrict__ tile_hist, const uint32_t* __restrict__ digit_total) {
     constexpr int WAVES = THREADS / 64;
@@ -303,8 +302,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     __shared__ uint32_t s_wc[WAVES][kRadix];
     __shared__ uint32_t s_dstart[kRadix];
     __shared__ uint32_t s_gbase[kRadix];
-    __shared__ uint32_t s_keys[kSortTile];
-    __shared__ uint32_t s_vals[kSortTile];
+    __shared__ uint2 s_pairs[kSortTile];
     __shared__ uint32_t s_w[WAVES];
 
     const int tid = threadIdx.x;
@@ -322,14 +320,14 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     const uint32_t count = min(static_cast<uint32_t>(kSortTile), seg.end - base);
     const uint64_t lt = (1ull << lane) - 1ull;
 
-    uint32_t key[KPT], val[KPT], rk[KPT];
+    uint2 pair[KPT];
+    uint32_t rk[KPT];
     uint32_t dig[KPT];
 #pragma unroll
     for (int r = 0; r < KPT; ++r) {
         const uint32_t li = wave * (KPT * 64) + r * 64 + lane;
         const bool valid = li < count;
-        key[r] = valid ? keys_in[base + li] : 0u;
-        val[r] = valid ? vals_in[base + li] : 0u;
+        pair[r] = valid ? pairs_in[base + li] : make_uint2(0u, 0u);
     }
     // This thread's digits: the segment's totals, and those of the tiles before
     // (up to kFewTiles tiles, tile_hist still holds each tile's own counts).
@@ -361,7 +359,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     for (int r = 0; r < KPT; ++r) {
         const uint32_t li = wave * (KPT * 64) + r * 64 + lane;
         const bool valid = li < count;
-        const uint32_t d = valid ? sort_digit<BY_SCENE>(key[r], val[r], scene_of, shift) : 0u;
+        const uint32_t d = valid ? sort_digit<BY_SCENE>(pair[r].x, pair[r].y, scene_of, shift) : 0u;
         uint64_t peers = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < kDigitBits; ++b) {
@@ -416,18 +414,15 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
         if (li < count) {
             const uint32_t d = dig[r];
             const uint32_t pos = s_dstart[d] + s_wc[wave][d] + rk[r];
-            s_keys[pos] = key[r];
-            s_vals[pos] = val[r];
+            s_pairs[pos] = pair[r];
         }
     }
     __syncthreads();
     for (uint32_t i = tid; i < count; i += THREADS) {
-        const uint32_t k = s_keys[i];
-        const uint32_t v = s_vals[i];
-        const uint32_t d = sort_digit<BY_SCENE>(k, v, scene_of, shift);
+        const uint2 p = s_pairs[i];
+        const uint32_t d = sort_digit<BY_SCENE>(p.x, p.y, scene_of, shift);
         const uint32_t g = s_gbase[d] + (i - s_dstart[d]);
-        keys_out[g] = k;
-        vals_out[g] = v;
+        pairs_out[g] = p;
     }
 }
 
@@ -599,7 +594,7 @@ __device__ __forceinline__ void mark_open(TreeStage<CAP>& S, uint32_t count) {
 // 40-byte read per leaf, and triangle records) 36, the record stores add 14,
 // the climb's steps the rest; with the triangles already in order 50.
 __global__ __launch_bounds__(kLeafBlock) void k_tree_leaves(
-    const pt_triangle* __restrict__ in_tris, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ perm,
+    const pt_triangle* __restrict__ in_tris, const uint2* __restrict__ pairs,
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ scene_of, uint32_t n,
     float4* __restrict__ nodes, float4* __restrict__ tri_recs, float* __restrict__ root_box,
     uint32_t* __restrict__ root_word, OpenList* __restrict__ lists, uint32_t* __restrict__ status) {
@@ -622,12 +617,12 @@ __global__ __launch_bounds__(kLeafBlock) void k_tree_leaves(
             if (scene_of[i + 1u] != sc) return -1;
             first = off[sc];
         }
-        const uint32_t ka = keys[i], kb = keys[i + 1u];
+        const uint32_t ka = pairs[i].x, kb = pairs[i + 1u].x;
         if (ka == kb) return 32 + __clz(static_cast<int>((i - first) ^ (i + 1u - first)));
         return __clz(static_cast<int>(ka ^ kb));
     };
     if (tid < count) {
-        const pt_triangle* t = in_tris + perm[k];
+        const pt_triangle* t = in_tris + pairs[k].y;
         const V3 v0 = v3(t->v0[0], t->v0[1], t->v0[2]);
         const V3 v1 = v3(t->v1[0], t->v1[1], t->v1[2]);
         const V3 v2 = v3(t->v2[0], t->v2[1], t->v2[2]);
@@ -802,10 +797,14 @@ __global__ __launch_bounds__(256) void k_dump_parents(const float4* __restrict__
     (w.y != kInvalid ? out_pi : out_pl)[s + 1] = p;
 }
 
-__global__ __launch_bounds__(256) void k_sub_u32(const uint32_t* __restrict__ in, uint32_t sub,
-                                                 uint32_t n, uint32_t* __restrict__ out) {
+// Sorted keys, and the permutation in local indices.
+__global__ __launch_bounds__(256) void k_dump_pairs(const uint2* __restrict__ pairs, uint32_t base, uint32_t n,
+                                                    uint32_t* __restrict__ out_keys, uint32_t* __restrict__ out_perm) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = in[i] - sub;
+    if (i >= n) return;
+    const uint2 p = pairs[base + i];
+    out_keys[i] = p.x;
+    out_perm[i] = p.y - base;
 }
 
 inline uint32_t div_up(uint64_t a, uint64_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
@@ -857,10 +856,8 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     if (n == 0) return;
     if (n >= (1u << 30)) throw Error(PT_E_INVALID_ARG, "LBVH supports fewer than 2^30 triangles");
     const size_t n4 = static_cast<size_t>(n) * 4;
-    b.keys.reserve(n4);
-    b.vals.reserve(n4);
-    b.keys_alt.reserve(n4);
-    b.vals_alt.reserve(n4);
+    b.pairs.reserve(2 * n4);
+    b.pairs_alt.reserve(2 * n4);
     b.scene_of.reserve(n4);
     b.nodes.reserve(static_cast<size_t>(n) * 64);
     b.tris.reserve(static_cast<size_t>(n) * 48);
@@ -877,16 +874,14 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     for (uint32_t m = blocks; m > 1; m = div_up(m, kFanIn)) nlists += div_up(m, kFanIn);
     b.open_lists.reserve(nlists * sizeof(OpenList));
 
-    uint32_t* kin = b.keys.as<uint32_t>();
-    uint32_t* vin = b.vals.as<uint32_t>();
+    uint2* in = b.pairs.as<uint2>();
     hipLaunchKernelGGL(k_morton, dim3(num_tiles), dim3(kMortonThreads), 0, st, s.tris.as<pt_triangle>(), n,
-                       s.off.as<uint32_t>(), nscenes, s.morton_box.as<float>(), table, kin, vin,
+                       s.off.as<uint32_t>(), nscenes, s.morton_box.as<float>(), table, in,
                        b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>());
     PT_HIP(hipGetLastError());
 
     if (n >= 2) {
-        uint32_t* kout = b.keys_alt.as<uint32_t>();
-        uint32_t* vout = b.vals_alt.as<uint32_t>();
+        uint2* out = b.pairs_alt.as<uint2>();
         // 3 passes over the 30-bit keys; unless the scenes are segments, then the
         // scene id's 10-bit digits (stable: each scene keeps its key order, ties
         // in input order).
@@ -904,29 +899,27 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
             // The first pass's counts come from k_morton.
             if (pass > 0) {
                 hipLaunchKernelGGL(by_scene ? k_sort_hist<true> : k_sort_hist<false>, dim3(num_tiles), dim3(kHistThreads),
-                                   0, st, kin, vin, sc, table, n, shift, hist);
+                                   0, st, in, sc, table, n, shift, hist);
             }
             if (s.sort_scans > 0) {
                 hipLaunchKernelGGL(k_sort_rowscan, dim3(s.sort_scans * (kRadix / kScanDigits)), dim3(kScanWaves * 64), 0, st,
                                    hist, num_tiles, scans, totals);
             }
             const auto scatter = by_scene ? k_sort_scatter<true, kScatterThreads> : k_sort_scatter<false, kScatterThreads>;
-            hipLaunchKernelGGL(scatter, dim3(num_tiles), dim3(kScatterThreads), 0, st, kin, vin, kout, vout, sc, table, n,
+            hipLaunchKernelGGL(scatter, dim3(num_tiles), dim3(kScatterThreads), 0, st, in, out, sc, table, n,
                                shift, hist, totals);
-            std::swap(kin, kout);
-            std::swap(vin, vout);
+            std::swap(in, out);
         }
         if (passes % 2) {
             // Odd pass count: the result sits in the alternate buffers.
-            swap(b.keys, b.keys_alt);
-            swap(b.vals, b.vals_alt);
+            swap(b.pairs, b.pairs_alt);
         }
         PT_HIP(hipGetLastError());
     }
     const uint32_t* scene_of = nscenes > 1 ? b.scene_of.as<uint32_t>() : nullptr;
     OpenList* lists = b.open_lists.as<OpenList>();
     hipLaunchKernelGGL(k_tree_leaves, dim3(blocks), dim3(kLeafBlock), 0, st, s.tris.as<pt_triangle>(),
-                       b.keys.as<uint32_t>(), b.vals.as<uint32_t>(), s.off.as<uint32_t>(), scene_of, n,
+                       b.pairs.as<uint2>(), s.off.as<uint32_t>(), scene_of, n,
                        b.nodes.as<float4>(), b.tris.as<float4>(), b.root_box.as<float>(), b.root_word.as<uint32_t>(),
                        lists, s.status.as<uint32_t>());
     for (uint32_t m = blocks; m > 1;) {
@@ -949,17 +942,15 @@ void dump_bvh(DeviceScene& s, uint32_t scene, hipStream_t st, uint32_t* morton, 
     if (n == 0) return;
     const size_t m = n - 1;
     DevBuf tmp;
-    tmp.reserve(static_cast<size_t>(n) * 5 * 4 + m * 24 + 256);
+    tmp.reserve(static_cast<size_t>(n) * 6 * 4 + m * 24 + 256);
     uint32_t* t_perm = tmp.as<uint32_t>();
     uint32_t* t_ch = t_perm + n;
     uint32_t* t_pl = t_ch + n;
     uint32_t* t_pi = t_pl + n;
     uint32_t* t_owner = t_pi + n;
-    float* t_box = reinterpret_cast<float*>(t_owner + n);
-    if (morton)
-        PT_HIP(hipMemcpyAsync(morton, b.keys.as<uint32_t>() + base, n * 4ull, hipMemcpyDeviceToHost, st));
-    hipLaunchKernelGGL(k_sub_u32, dim3(div_up(n, 256)), dim3(256), 0, st, b.vals.as<uint32_t>() + base,
-                       base, n, t_perm);
+    uint32_t* t_keys = t_owner + n;
+    float* t_box = reinterpret_cast<float*>(t_keys + n);
+    hipLaunchKernelGGL(k_dump_pairs, dim3(div_up(n, 256)), dim3(256), 0, st, b.pairs.as<uint2>(), base, n, t_keys, t_perm);
     if (n > 1) {
         hipLaunchKernelGGL(k_dump_nodes, dim3(div_up(n, 256)), dim3(256), 0, st, b.nodes.as<float4>(),
                            b.root_word.as<uint32_t>() + scene, b.root_box.as<float>() + 6 * static_cast<size_t>(scene),
@@ -968,6 +959,7 @@ void dump_bvh(DeviceScene& s, uint32_t scene, hipStream_t st, uint32_t* morton, 
     hipLaunchKernelGGL(k_dump_parents, dim3(div_up(n, 256)), dim3(256), 0, st, b.nodes.as<float4>(), t_owner, base, n,
                        t_pl, t_pi);
     PT_HIP(hipGetLastError());
+    if (morton) PT_HIP(hipMemcpyAsync(morton, t_keys, n * 4ull, hipMemcpyDeviceToHost, st));
     if (perm) PT_HIP(hipMemcpyAsync(perm, t_perm, n * 4ull, hipMemcpyDeviceToHost, st));
     if (parents_leaf) PT_HIP(hipMemcpyAsync(parents_leaf, t_pl, n * 4ull, hipMemcpyDeviceToHost, st));
     if (m > 0) {

@@ -1418,12 +1418,8 @@ namespace {
 bool frame_in_flight(Renderer& r) {
     if (!r.frame_sent) return false;
     const hipError_t e = hipEventQuery(r.frame_ev);
-    if (e == hipErrorNotReady) {
-        (void)hipGetLastError();
-        return true;
-    }
-    PT_HIP(e);
-    return false;
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipErrorNotReady;
 }
 
 // The next slot, ready for npaths paths, or none if memory does not allow it.
