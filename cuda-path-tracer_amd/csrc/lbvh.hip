@@ -299,10 +299,12 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
     constexpr int KPT = kSortTile / THREADS;  // keys per thread
     constexpr int DPT = kRadix / THREADS;     // digits per thread
     static_assert(KPT * THREADS == kSortTile && DPT * THREADS == static_cast<int>(kRadix), "tile shape");
-    __shared__ uint32_t s_wc[WAVES][kRadix];
+    // The waves' digit counters, then (once every key has its place) the keys.
+    __shared__ uint2 s_pairs[kSortTile];
+    static_assert(WAVES * kRadix <= 2 * kSortTile, "the counters fit the keys' memory");
+    uint32_t (*s_wc)[kRadix] = reinterpret_cast<uint32_t (*)[kRadix]>(s_pairs);
     __shared__ uint32_t s_dstart[kRadix];
     __shared__ uint32_t s_gbase[kRadix];
-    __shared__ uint2 s_pairs[kSortTile];
     __shared__ uint32_t s_w[WAVES];
 
     const int tid = threadIdx.x;
@@ -411,11 +413,13 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(
 #pragma unroll
     for (int r = 0; r < KPT; ++r) {
         const uint32_t li = wave * (KPT * 64) + r * 64 + lane;
-        if (li < count) {
-            const uint32_t d = dig[r];
-            const uint32_t pos = s_dstart[d] + s_wc[wave][d] + rk[r];
-            s_pairs[pos] = pair[r];
-        }
+        if (li < count) rk[r] += s_dstart[dig[r]] + s_wc[wave][dig[r]];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+        const uint32_t li = wave * (KPT * 64) + r * 64 + lane;
+        if (li < count) s_pairs[rk[r]] = pair[r];
     }
     __syncthreads();
     for (uint32_t i = tid; i < count; i += THREADS) {
