@@ -511,15 +511,21 @@ __global__ __launch_bounds__(kShadeThreads) void k_shade(const FrameConst fc,
 // non-empty pool in [next, end) or sets `drained` once every slice is used
 // up; each call either takes a pool or adds a used-up slice to `seen`, so
 // it returns after at most nq + 1 atomics.
+// FIRST: slots [0, nfirst) come before the queue's, which follow them: wave w
+// takes them from 64 w on, 64 at a time, every 64 times the grid's waves.
+template <bool FIRST>
 struct Handout {
     uint32_t* queue;
     uint32_t nq, per, extra, pool, q;
     uint64_t seen;
     uint32_t next, end;
+    uint32_t first, nfirst;
     bool drained;
 
-    __device__ __forceinline__ void init(uint32_t* qb, uint32_t n, uint32_t pool_size, uint32_t wave_id) {
+    __device__ __forceinline__ void init(uint32_t* qb, uint32_t n, uint32_t pool_size, uint32_t wave_id, uint32_t nf) {
         queue = qb;
+        first = wave_id * 64u;
+        nfirst = nf;
         nq = queue_slices(n);
         per = n / nq;
         extra = n % nq;
@@ -528,12 +534,17 @@ struct Handout {
         const uint64_t all = nq == 64u ? ~0ull : (1ull << nq) - 1ull;
         seen = ~all;
         next = end = 0;
-        drained = n == 0;
+        drained = n == 0 && (!FIRST || first >= nfirst);
     }
 
     __device__ __forceinline__ void next_pool() {
         const int lane = threadIdx.x & 63;
         uint64_t* mask = reinterpret_cast<uint64_t*>(queue + kQueueMask);
+        if (FIRST && next >= end && first < nfirst) {
+            next = first;
+            end = min(first + 64u, nfirst);
+            first += gridDim.x * (blockDim.x / 64u) * 64u;
+        }
         while (!drained && next >= end) {
             const uint32_t beg = q * per + min(q, extra);
             const uint32_t len = per + (q < extra ? 1u : 0u);
@@ -544,8 +555,8 @@ struct Handout {
             }
             base = __builtin_amdgcn_readfirstlane(base);
             if (base < len) {
-                next = beg + base;
-                end = beg + base + min(pool, len - base);
+                next = (FIRST ? nfirst : 0u) + beg + base;
+                end = next + min(pool, len - base);
                 return;
             }
             seen |= 1ull << q;
@@ -603,15 +614,10 @@ __global__ __launch_bounds__(64) void k_paths_setup(uint32_t* __restrict__ count
 // Path `slot` (in first-level order) at its primary ray: r.o, r.d, its path
 // index (pass * npix + pixel) and its scene's root word (kInvalid: a scene of
 // fewer than two triangles).
-__device__ __forceinline__ uint32_t start_path(const FrameConst& fc, const PassParams* __restrict__ pp,
-                                               const uint32_t* __restrict__ off, uint32_t slot, RayState& r,
-                                               uint32_t& root) {
-    const uint32_t w = static_cast<uint32_t>(fc.w), h = static_cast<uint32_t>(fc.h);
-    const uint32_t pass = slot / fc.npix;
-    const uint32_t pix = tiled_pixel(slot - pass * fc.npix, w, h);
-    const PassParams& P = pp[pass];
-    const float tx = static_cast<float>(pix % w) / static_cast<float>(fc.w);
-    const float ty = static_cast<float>(pix / w) / static_cast<float>(fc.h);
+__device__ __forceinline__ void start_at(const FrameConst& fc, const PassParams& P, const uint32_t* __restrict__ off,
+                                         uint32_t x, uint32_t y, RayState& r, uint32_t& root) {
+    const float tx = static_cast<float>(x) / static_cast<float>(fc.w);
+    const float ty = static_cast<float>(y) / static_cast<float>(fc.h);
     const V3 d00 = v3(P.dirs[0], P.dirs[1], P.dirs[2]);
     const V3 d10 = v3(P.dirs[3], P.dirs[4], P.dirs[5]);
     const V3 d11 = v3(P.dirs[6], P.dirs[7], P.dirs[8]);
@@ -620,15 +626,38 @@ __device__ __forceinline__ uint32_t start_path(const FrameConst& fc, const PassP
     r.d = mix(mix(d00, d10, tx), mix(d01, d11, tx), ty);
     const uint32_t sb = off[P.scene], se = off[P.scene + 1];
     root = se - sb >= 2 ? fc.roots[P.scene] : kInvalid;
+}
+__device__ __forceinline__ uint32_t start_path(const FrameConst& fc, const PassParams* __restrict__ pp,
+                                               const uint32_t* __restrict__ off, uint32_t slot, RayState& r,
+                                               uint32_t& root) {
+    const uint32_t w = static_cast<uint32_t>(fc.w), h = static_cast<uint32_t>(fc.h);
+    const uint32_t pass = slot / fc.npix;
+    const uint32_t pix = tiled_pixel(slot - pass * fc.npix, w, h);
+    start_at(fc, pp[pass], off, pix % w, pix / w, r, root);
     return pass * fc.npix + pix;
 }
 
+// Training path `key` of a cache frame likewise: on one cell of every 4x4 pixel
+// block, the cell stepping through all 16 with the pass index; path k takes
+// block floor(k * nblocks / ntrain), so the paths spread evenly over the image.
+__device__ __forceinline__ void train_cell(const FrameConst& fc, const PassParams& P, uint32_t ntrain, uint32_t key,
+                                           uint32_t& x, uint32_t& y) {
+    const uint32_t w = static_cast<uint32_t>(fc.w), h = static_cast<uint32_t>(fc.h);
+    const uint32_t ox = min(P.pass % 4u, w - 1u), oy = min((P.pass / 4u) % 4u, h - 1u);
+    const uint32_t cw = (w - ox + 3u) / 4u, ch = (h - oy + 3u) / 4u;
+    const uint64_t ncell = static_cast<uint64_t>(cw) * ch;
+    const uint32_t c = static_cast<uint32_t>((static_cast<uint64_t>(key) * ncell) / ntrain);
+    x = ox + 4u * (c % cw);
+    y = oy + 4u * (c / cw);
+}
+
 // The closest hit of a path's segment in a scene of fewer than two triangles.
+template <bool CACHE>
 __device__ __forceinline__ void answer_single(const FrameConst& fc, const PassParams* __restrict__ pp,
                                               const uint32_t* __restrict__ off, const float4* __restrict__ tris,
                                               uint32_t path, RayState& r) {
     TraceCount cnt{0, 0, 0, 0};
-    const uint32_t sc = pp[path / fc.npix].scene;
+    const uint32_t sc = pp[CACHE ? 0u : path / fc.npix].scene;
     const TraceHit h = trace_single<false>(tris, off[sc + 1] - off[sc] == 1u ? off[sc] : kInvalid, r.o, r.d, cnt);
     r.minT = h.t; r.best = h.id; r.bu = h.u; r.bv = h.v;
 }
@@ -637,10 +666,16 @@ __device__ __forceinline__ void answer_single(const FrameConst& fc, const PassPa
 // without spilling.  At 80 (6 waves) they spill inside the visit, and a
 // 1,024 x 1,024 frame of the 871,200-triangle room took 7.2 ms for 2.9; at 4
 // waves it took the same as at 5.
-// CACHE: the pixel paths of a cache frame (one pass, pixel = path), each
-// ending in the cache at its second hit (record_cache_vertex) with its
-// throughput in ps.ar/ag/ab -- the same values the levels k_extend /
-// k_shade<true> leave.
+// CACHE: a cache frame (one pass).  Its pixel paths (pixel = path) end in the
+// cache at their second hit (record_cache_vertex) with their throughput in
+// ps.ar/ag/ab, its training paths (path npix + key) after train_levels - 1
+// bounces -- the same values k_extend / k_shade<true> and k_train_paths leave.
+// The training paths are the longest by far (ten bounces against one), so they
+// come first: 64 for each of the first waves, which then go on with pixels.  On
+// a stream of their own, one wave per SIMD, they went on for 960 us after the
+// pixel paths of a 1,920 x 1,080 frame with 65,536 of them: two such frames take
+// 3,880 us so, 4,175 apart; 640 x 360 with 16,384 1,290 against 2,260; with 256
+// training paths at 1,920 x 1,080 3,565 against 3,615.
 // lg0 > 0: a frame of few paths, 2^lg0 lanes per path from the start (the
 // grid holds every path; no queue).  Otherwise one lane per path, and once the
 // queue has run dry and kTailLanes paths or fewer are left in a wave, those
@@ -665,7 +700,8 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
     __shared__ float s_carry[kCarryLds ? 6 : 1][kPersistThreads];
     for (uint32_t k = threadIdx.x; k < kMaxLevels; k += blockDim.x) s_level[k] = 0u;
     __syncthreads();
-    const uint32_t npaths = fc.npix * fc.npasses;
+    const uint32_t npix = fc.npix * fc.npasses, ntrain = CACHE ? io.ntrain : 0u;
+    const uint32_t npaths = npix + ntrain;
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     const int lane = threadIdx.x & 63;
     uint32_t spill[kStackMax - LDS];
@@ -683,16 +719,31 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
     V3 absorbed_r = v3(1.0f, 1.0f, 1.0f), acc_r = v3(0.0f, 0.0f, 0.0f);
     const int tid = threadIdx.x;
 
+    // Path `slot`: a training path below ntrain, else a pixel's.
+    auto start = [&](uint32_t slot) {
+        if (CACHE && slot < ntrain) {
+            uint32_t x, y;
+            train_cell(fc, pp[0], ntrain, slot, x, y);
+            start_at(fc, pp[0], off, x, y, r, root);
+            io.tvalid[slot] = 0u;
+            path = npix + slot;
+        } else {
+            path = start_path(fc, pp, off, slot - ntrain, r, root);
+            if (CACHE) io.qvalid[path] = 0u;
+        }
+    };
     // The end of a segment: shade its hit and sample the next segment (r.o,
     // r.d; true), or end the path (false).  `lead`: this lane writes for the
     // path.  Shadow rays keep their deferred nodes in this lane's (empty)
     // column of the stack.
     auto shade = [&](V3& absorbed, V3& acc, bool lead) -> bool {
-        if (lead) atomicAdd(&s_level[bounce], 1u);  // this segment, now complete
+        const bool train = CACHE && path >= npix;
+        // This segment, now complete.
+        if (lead) atomicAdd(&s_level[train && bounce < 2u ? kTrainLevel0Slot + bounce : bounce], 1u);
         bool cont = false;
         if (r.best != kInvalid) {
-            const uint32_t pass = path / fc.npix;
-            const uint32_t pix = path - pass * fc.npix;
+            const uint32_t pass = CACHE ? 0u : path / fc.npix;
+            const uint32_t pix = CACHE ? (train ? path - npix : path) : path - pass * fc.npix;
             const PassParams& P = pp[pass];
             HitShade hs = hit_shade<DETAIL>(fc, infos, r.best, r.minT, r.bu, r.bv, r.o, r.d);
             const uint32_t sb = off[P.scene], se = off[P.scene + 1];
@@ -706,10 +757,17 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
             } else {
                 bounce_hit<LIGHTS, true>(hs, r.d, fc, lights, nodes, tris, root, sb, se, absorbed, acc, ss);
             }
-            if (CACHE && bounce == 1 && lead) record_cache_vertex(io, false, pix, path, hs, r.d, absorbed, acc);
+            if (CACHE && bounce == 1) {
+                if (lead) record_cache_vertex(io, train, pix, path, hs, r.d, absorbed, acc);
+                if (train) {  // on all of the path's lanes
+                    absorbed = v3(1.0f, 1.0f, 1.0f);
+                    acc = v3(0.0f, 0.0f, 0.0f);
+                }
+            }
             V3 no{0.0f, 0.0f, 0.0f}, nd{0.0f, 0.0f, 0.0f};
-            const uint32_t limit = CACHE ? 1u : fc.bounces;
-            if (bounce < limit) cont = next_bounce(pix, P.pass, bounce, P.seedw, fc, hs, absorbed, no, nd);
+            const uint32_t limit = CACHE ? (train ? io.train_levels - 1u : 1u) : fc.bounces;
+            const uint32_t seedw = train ? P.seedw ^ kTrainSalt : P.seedw;
+            if (bounce < limit) cont = next_bounce(pix, P.pass, bounce, seedw, fc, hs, absorbed, no, nd);
             if (cont) {
                 ++bounce;
                 r.o = no;
@@ -738,15 +796,15 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
     if (lg0 > 0u) {
         const uint32_t slot = (blockIdx.x * kPersistThreads + threadIdx.x) >> lg0;
         if (slot < npaths) {
-            path = start_path(fc, pp, off, slot, r, root);
+            start(slot);
             active = true;
             if (root != kInvalid) group_start<LDS>(r, root, gsp, lg, s_stack);
-            else answer_single(fc, pp, off, tris, path, r);
+            else answer_single<CACHE>(fc, pp, off, tris, path, r);
         }
     } else if (wave_id == 0u || static_cast<uint64_t>(wave_id) * kRayPoolSmall < npaths) {
         // (Waves past one per kRayPoolSmall paths have nothing to do.)
-        Handout ho;
-        ho.init(queue, npaths, kRayPoolSmall, wave_id);
+        Handout<CACHE> ho;
+        ho.init(queue, npix, kRayPoolSmall, wave_id, ntrain);
         uint32_t state = kLaneIdle, pend = 0;
         for (;;) {
             // New paths for idle lanes.
@@ -762,7 +820,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                     const bool take = ((idle >> lane) & 1ull) && rank < avail;
                     const uint32_t took = min(static_cast<uint32_t>(__popcll(idle)), avail);
                     if (take) {
-                        path = start_path(fc, pp, off, ho.next + rank, r, root);
+                        start(ho.next + rank);
                         bounce = 0;
                         if constexpr (kCarryLds) {
                             s_carry[0][tid] = 1.0f; s_carry[1][tid] = 1.0f; s_carry[2][tid] = 1.0f;
@@ -788,7 +846,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                     test_pending(tris, r, pend, s_pend);
                     if (state == kLaneTrace) {
                         if (root == kInvalid) {
-                            answer_single(fc, pp, off, tris, path, r);
+                            answer_single<CACHE>(fc, pp, off, tris, path, r);
                         } else if (r.word != kInvalid) {
                             s_stack[r.sp][tid] = r.word;
                             gsp = static_cast<uint32_t>(r.sp) + 1u;
@@ -800,7 +858,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
             // One node visit for every traversing lane; a scene with fewer
             // than two triangles answers at once.
             if (state == kLaneTrace && root == kInvalid) {
-                answer_single(fc, pp, off, tris, path, r);
+                answer_single<CACHE>(fc, pp, off, tris, path, r);
                 state = kLaneShade;
             }
             if (walk_wave<LDS>(nodes, tris, r, pend, state == kLaneTrace, s_stack, s_pend, spill, fc.status))
@@ -864,22 +922,21 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                 active = shade(absorbed, acc, lead);
                 if (active) {
                     if (root != kInvalid) group_start<LDS>(r, root, gsp, lg, s_stack);
-                    else answer_single(fc, pp, off, tris, path, r);
+                    else answer_single<CACHE>(fc, pp, off, tris, path, r);
                 }
             }
         }
     }
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < kMaxLevels && k < kTrainLevel0Slot; k += blockDim.x)
+    for (uint32_t k = threadIdx.x; k < kMaxLevels; k += blockDim.x)
         if (s_level[k]) atomicAdd(counters + k, s_level[k]);
 }
 
-// Cache frames: the training paths, one lane per path from its primary ray
-// to its end, on a stream of their own beside the pixel paths' two levels,
-// the inference and the resolve (the per-level launches of a few thousand
-// rays are latency bound -- each level waits for its slowest ray -- and one
-// lane per path waits only for the slowest path).  Traversal, shading and
-// sampling are k_extend / k_shade's (primary_hit, bounce_hit,
+// Cache frames with bounce levels (render.paths 0): the training paths, one
+// lane per path from its primary ray to its end, on a stream of their own
+// beside the pixel paths' two levels, the inference and the resolve (the
+// per-level launches of a few thousand rays are latency bound).  Traversal,
+// shading and sampling are k_extend / k_shade's (primary_hit, bounce_hit,
 // record_cache_vertex, next_bounce), so the training batches are the same
 // bits as when these paths ran through the levels.
 constexpr int kSuffixThreads = 64;
@@ -979,34 +1036,27 @@ __global__ __launch_bounds__(kThreads) void k_accumulate(const FrameConst fc, Pa
     }
 }
 
-// Cache frame: pixel paths (0 .. npix) as k_generate with one pass, then
-// training paths on one cell of every 4x4 pixel block, the cell (ox, oy)
-// stepping through all 16 with the pass index; training path k takes block
-// floor(k * nblocks / ntrain), so the paths spread evenly over the image.
+// Cache frame with bounce levels: pixel paths (0 .. npix) as k_generate with one
+// pass, then training paths (train_cell).
 __global__ __launch_bounds__(kThreads) void k_generate_cache(const FrameConst fc,
                                                              const PassParams* __restrict__ pp,
                                                              RayQueue q, PathState ps,
                                                              uint32_t* __restrict__ counters,
                                                              uint32_t* __restrict__ ray_counters,
-                                                             uint32_t nlevels, CacheIO io, uint32_t count0) {
+                                                             uint32_t nlevels, CacheIO io) {
     const uint32_t npaths = fc.npix + io.ntrain;
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid == 0) {
-        // The pixel paths' first-level count: npix when the levels trace
-        // them, 0 when a path-persistent launch does and counts its own
-        // segments; the training paths' rays (slots npix ..) are read by
-        // k_train_paths.
-        counters[0] = count0;
+        // The pixel paths' first-level count; the training paths' rays (slots
+        // npix ..) are read by k_train_paths.
+        counters[0] = fc.npix;
         for (uint32_t k = 1; k <= nlevels; ++k) counters[k] = 0u;
         counters[kTrainLevel0Slot] = 0u;
         counters[kTrainLevel1Slot] = 0u;
     }
     if (blockIdx.x == 0) zero_queue(ray_counters, nlevels);
     const PassParams& P = pp[0];
-    const uint32_t w = static_cast<uint32_t>(fc.w), h = static_cast<uint32_t>(fc.h);
-    const uint32_t ox = min(P.pass % 4u, w - 1u), oy = min((P.pass / 4u) % 4u, h - 1u);
-    const uint32_t cw = (w - ox + 3u) / 4u, ch = (h - oy + 3u) / 4u;
-    const uint64_t ncell = static_cast<uint64_t>(cw) * ch;
+    const uint32_t w = static_cast<uint32_t>(fc.w);
     for (uint32_t p = gid; p < npaths; p += gridDim.x * blockDim.x) {
         uint32_t x, y;
         if (p < fc.npix) {
@@ -1014,11 +1064,8 @@ __global__ __launch_bounds__(kThreads) void k_generate_cache(const FrameConst fc
             y = p / w;
             io.qvalid[p] = 0u;
         } else {
-            const uint32_t k = p - fc.npix;
-            const uint32_t c = static_cast<uint32_t>((static_cast<uint64_t>(k) * ncell) / io.ntrain);
-            x = ox + 4u * (c % cw);
-            y = oy + 4u * (c / cw);
-            io.tvalid[k] = 0u;
+            train_cell(fc, P, io.ntrain, p - fc.npix, x, y);
+            io.tvalid[p - fc.npix] = 0u;
         }
         const float tx = static_cast<float>(x) / static_cast<float>(fc.w);
         const float ty = static_cast<float>(y) / static_cast<float>(fc.h);
@@ -1569,30 +1616,11 @@ void launch_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
                            : (fc.nlights ? k_shade<true, true, false> : k_shade<true, false, false>);
     auto train_paths = fc.detail ? k_train_paths<true> : k_train_paths<false>;
     const bool paths = render_tuning().paths != 0;
-    hipLaunchKernelGGL(k_generate_cache, dim3(grid), dim3(kThreads), 0, st, fc, pp, L.q[0], L.ps, cnt, rcnt,
-                       nlev, io, paths ? 0u : fc.npix);
-    // The training paths run on the side stream from here, beside the pixel
-    // paths (two levels, or one path-persistent launch), inference, resolve
-    // and accumulation: they read the first level's queue slots from npix on
-    // and write only training-path state, the training batch and counter
-    // slots the pixel paths do not read.
-    // The join comes before the training targets and the Adam steps, which
-    // change the weights the inference reads.
-    if (io.ntrain) {
-        PT_HIP(hipEventRecord(r.fork_ev, st));
-        PT_HIP(hipStreamWaitEvent(r.side, r.fork_ev, 0));
-        const uint32_t sgrid = std::max(1u, std::min(4096u, (io.ntrain + kSuffixThreads - 1) / kSuffixThreads));
-        hipLaunchKernelGGL(train_paths, dim3(sgrid), dim3(kSuffixThreads), 0, r.side, fc, pp,
-                           scene.infos.as<pt_triangle_info>(), L.q[0], L.ps, cnt, io,
-                           scene.lights.as<pt_dir_light>(), scene.bvh.nodes.as<float4>(),
-                           scene.bvh.tris.as<float4>(), scene.off.as<uint32_t>());
-        PT_HIP(hipEventRecord(r.join_ev, r.side));
-    }
     if (paths) {
-        // The pixel paths in one path-persistent launch (render.paths), each
-        // lane carrying a path from its primary ray to the cache.
-        const uint32_t lg = launch_group(fc.npix, static_cast<uint64_t>(std::max(1u, tune.blocks)) * kPersistThreads);
-        const uint32_t ppgrid = lg ? grouped_blocks(fc.npix, lg) : std::min(std::max(1u, tune.blocks), grid_for(fc.npix));
+        // Training and pixel paths in one path-persistent launch (render.paths).
+        hipLaunchKernelGGL(k_paths_setup, dim3(1), dim3(64), 0, st, cnt, rcnt, nlev);
+        const uint32_t lg = launch_group(npaths, static_cast<uint64_t>(std::max(1u, tune.blocks)) * kPersistThreads);
+        const uint32_t ppgrid = lg ? grouped_blocks(npaths, lg) : pgrid;
         auto kern = tune.lds <= 8 ? cache_paths_kernel<8>(fc) : cache_paths_kernel<16>(fc);
         hipLaunchKernelGGL(kern, dim3(ppgrid), dim3(kPersistThreads), 0, st, fc, pp,
                            scene.infos.as<pt_triangle_info>(), scene.bvh.nodes.as<float4>(),
@@ -1600,6 +1628,23 @@ void launch_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
                            L.ps, cnt, rcnt, std::min(64u, std::max(1u, render_tuning().refill)), shade_batch(fc), lg,
                            io);
     } else {
+        hipLaunchKernelGGL(k_generate_cache, dim3(grid), dim3(kThreads), 0, st, fc, pp, L.q[0], L.ps, cnt, rcnt, nlev, io);
+        // The training paths run on the side stream from here, beside the pixel
+        // paths' two levels, inference, resolve and accumulation: they read the
+        // first level's queue slots from npix on and write only training-path
+        // state, the training batch and counter slots the pixel paths do not
+        // read.  The join comes before the training targets and the Adam steps,
+        // which change the weights the inference reads.
+        if (io.ntrain) {
+            PT_HIP(hipEventRecord(r.fork_ev, st));
+            PT_HIP(hipStreamWaitEvent(r.side, r.fork_ev, 0));
+            const uint32_t sgrid = std::max(1u, std::min(4096u, (io.ntrain + kSuffixThreads - 1) / kSuffixThreads));
+            hipLaunchKernelGGL(train_paths, dim3(sgrid), dim3(kSuffixThreads), 0, r.side, fc, pp,
+                               scene.infos.as<pt_triangle_info>(), L.q[0], L.ps, cnt, io,
+                               scene.lights.as<pt_dir_light>(), scene.bvh.nodes.as<float4>(),
+                               scene.bvh.tris.as<float4>(), scene.off.as<uint32_t>());
+            PT_HIP(hipEventRecord(r.join_ev, r.side));
+        }
         // Levels 0 and 1 of the pixel paths (a pixel path ends in the cache at x2).
         for (uint32_t lvl = 0; lvl < 2; ++lvl) {
             hipLaunchKernelGGL(extend, dim3(pgrid), dim3(kPersistThreads), 0, st, fc, pp,
@@ -1616,7 +1661,7 @@ void launch_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
     hipLaunchKernelGGL(k_cache_resolve, dim3(grid_for(fc.npix)), dim3(kThreads), 0, st, fc, io, L.ps);
     hipLaunchKernelGGL(k_accumulate, dim3(grid_for(fc.npix)), dim3(kThreads), 0, st, fc, L.ps,
                        r.accum.as<double>());
-    if (io.ntrain) PT_HIP(hipStreamWaitEvent(st, r.join_ev, 0));
+    if (io.ntrain && !paths) PT_HIP(hipStreamWaitEvent(st, r.join_ev, 0));
     if (io.ntrain) {
         hipLaunchKernelGGL(k_train_targets, dim3(grid_for(io.ntrain)), dim3(kThreads), 0, st, fc, io, L.ps);
         if (cf.train) {

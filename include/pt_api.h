@@ -383,7 +383,8 @@ int pt_device_compute_units(int device, uint32_t* cus);
  *   "render.paths"  1: a plain frame traces every path from its primary
  *                   ray to its end in one persistent launch (no bounce
  *                   levels), and a cache frame its pixel paths from their
- *                   primary ray to the cache; 0: bounce levels (wavefront)
+ *                   primary ray to the cache and its training paths;
+ *                   0: bounce levels (wavefront), training paths beside them
  *   "render.shade_min" 1..64: in path-persistent frames of scenes without
  *                   directional lights, the lanes of a wave whose segments
  *                   have ended shade together once this many wait (or none is
