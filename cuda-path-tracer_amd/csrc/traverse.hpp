@@ -885,6 +885,14 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
 // as the full traversal would, and a survivor is traced in full.
 
 constexpr uint32_t kSurvCap = 128;  // survivor ring entries per wave
+// Lanes are refilled from the ring already when fewer than this many are busy:
+// with a survivor ready for every idle lane, or no more rays to filter, that
+// costs no filter round.  (Filter rounds wait for the launch's `refill`: with 48
+// for both, 16M shell rays, which mostly end in the filter, took 1 % longer.)
+// 2.88M-triangle hair ball, 2,073,600 camera rays: 1,344 us without, 1,275 / 1,245
+// / 1,220 at 40 / 48 / 56, 10^6 rays 930 and 770 / 764 / 760; 4M camera rays on
+// the 871,200-triangle mesh 654 and 640 / 628 / 613; 16M shell rays 867 each.
+constexpr uint32_t kReadyRefill = 56;
 
 // The root visit alone (visit_step's decisions without the stack): leaf
 // children fold into the best hit; returns whether an internal child is to
@@ -933,7 +941,8 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
     uint64_t seen = ~all;
     for (;;) {
         const uint32_t nbusy = static_cast<uint32_t>(__popcll(__ballot(active)));
-        if (nbusy < refill && (!drained || qtail != qhead)) {
+        const uint32_t ready = qtail - qhead;
+        if (nbusy < (ready + nbusy >= 64u || drained ? max(refill, kReadyRefill) : refill) && (!drained || ready != 0u)) {
             // Filter rounds until the ring can fill every idle lane (or the
             // rays run out).  Each pass either consumes pool rays, takes a
             // new pool, or finds a slice used up (at most nq times).
