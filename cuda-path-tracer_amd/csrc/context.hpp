@@ -138,7 +138,7 @@ struct DeviceScene {
     uint32_t ndetail = 0, ntex = 0;
     uint32_t max_id = 0;                   // largest triangle id of the upload
     // Status word the kernels OR PT_STATUS_* flags into (a violated bound:
-    // traversal stack, refit list); sticky until pt_get_status reads it.
+    // traversal stack, open list); sticky until pt_get_status reads it.
     DevBuf status;
     DeviceBvh bvh;
     bool ready = false;

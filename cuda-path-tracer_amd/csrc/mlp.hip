@@ -17,10 +17,11 @@
 // Training step (deterministic: no floating-point atomics), two launches:
 //   k_mlp_train      per workgroup, 64-sample rounds (one 16-sample block per
 //                    wave): forward, relative-L2 loss, backward deltas, then
-//                    the layer inputs and deltas go to LDS feature-major and
-//                    the four waves accumulate dW = act^T delta (MFMA, K =
-//                    samples) and db = sum delta over the workgroup's
-//                    samples; one fp32 partial per workgroup
+//                    the layer inputs and deltas go to LDS, a row per sample,
+//                    and the four waves accumulate dW = act^T delta (MFMA,
+//                    K = samples, operands through the transposing LDS read)
+//                    and db = sum delta over the workgroup's samples; one fp32
+//                    partial per workgroup
 //   k_mlp_adam_pack  sums the partials in workgroup order, Adam on the fp32
 //                    masters, and writes each updated weight into its fp16
 //                    fragments (forward, backward and inference layouts)

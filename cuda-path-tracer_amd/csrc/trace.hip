@@ -205,7 +205,7 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
                        s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(), d_rays, n, d_id, d_t,
                        reinterpret_cast<float2*>(d_uv), queue, std::min(64u, std::max(1u, tune.refill)),
-                       pool_for(tune.pool, n, blocks), d_counters, status);
+                       pool_for(tune.pool), d_counters, status);
     PT_HIP(hipGetLastError());
 }
 
@@ -262,7 +262,7 @@ void trace_closest_scenes(const DeviceScene& s, uint32_t* queue, const float* d_
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
                        s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(),
                        s.off.as<uint32_t>(), s.nscenes(), d_rays, d_scene, n, d_id, d_t, reinterpret_cast<float2*>(d_uv),
-                       queue, std::min(64u, std::max(1u, tune.refill)), pool_for(tune.pool, n, blocks),
+                       queue, std::min(64u, std::max(1u, tune.refill)), pool_for(tune.pool),
                        s.status.as<uint32_t>());
     PT_HIP(hipGetLastError());
 }
