@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdint>
 #include <map>
@@ -108,13 +109,13 @@ struct DeviceBvh {
     DevBuf pairs, pairs_alt;                // sorted (Morton key, perm) (+ ping-pong)
     DevBuf scene_of;                        // scene of each leaf slot
     DevBuf nodes, tris;
-    DevBuf root_box, root_word;     // per scene: the root's box and child word (kInvalid: one triangle)
+    DevBuf root_box, root_word;     // per scene: the root's box and child word (kInvalid: no internal node)
     DevBuf tile_hist, digit_total;  // radix sort scratch
     DevBuf open_lists;              // tree: each block's subtrees that the next level goes on with
 };
 
 // One or more scenes: scene s owns triangles [off[s], off[s+1]) and its own
-// LBVH over them (internal node off[s] is its root).
+// LBVH over them (its root is root_word[s]).
 struct DeviceScene {
     uint32_t n = 0;
     uint32_t ninfos = 0;
@@ -143,6 +144,12 @@ struct DeviceScene {
     DeviceBvh bvh;
     bool ready = false;
     uint32_t nscenes() const { return static_cast<uint32_t>(off_host.size()) - 1; }
+    // The first scene that has triangles (0 when none has): a trace without
+    // scene ids is traced there.
+    uint32_t first_scene() const {
+        const auto it = std::upper_bound(off_host.begin(), off_host.end(), 0u);
+        return it == off_host.end() ? 0u : static_cast<uint32_t>(it - off_host.begin()) - 1u;
+    }
 };
 
 // Builder timings (ms) of the last build, from HIP events.

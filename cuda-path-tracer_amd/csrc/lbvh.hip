@@ -111,8 +111,10 @@ __device__ __forceinline__ uint32_t scene_of_slot(const uint32_t* __restrict__ o
 
 // morton_encoder (BVHBuilder.cu:12-32): centroid ((v0 + v1) + v2) / 3, mapped
 // into the scene's enclosing box with invScale computed on the host
-// (box[6*s..] = min.xyz, invScale.xyz).  One workgroup per sort tile, which also counts the tile's first-pass digits (key bits 0-9) into
-// its row of tile_hist -- the first sort pass then starts at the scan.
+// (box[6*s..] = min.xyz, invScale.xyz).  One workgroup per sort tile, which also
+// counts the tile's first-pass digits (key bits 0-9) into its row of tile_hist --
+// the first sort pass then starts at the scan.  Also sets every scene's root word
+// to kInvalid, for the scenes whose tree writes none.
 constexpr int kMortonThreads = 1024;
 
 __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __restrict__ tris, uint32_t n,
@@ -121,9 +123,11 @@ __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __
                                                            const uint4* __restrict__ table,
                                                            uint2* __restrict__ pairs,
                                                            uint32_t* __restrict__ scene_of,
-                                                           uint32_t* __restrict__ tile_hist) {
+                                                           uint32_t* __restrict__ tile_hist,
+                                                           uint32_t* __restrict__ root_word) {
     __shared__ uint32_t h[kRadix];
     const uint32_t tid = threadIdx.x;
+    for (uint32_t s = blockIdx.x * kMortonThreads + tid; s < nscenes; s += gridDim.x * kMortonThreads) root_word[s] = kInvalid;
     for (uint32_t d = tid; d < kRadix; d += kMortonThreads) h[d] = 0u;
     __syncthreads();
     const Segment seg = segment_of_tile(table, n, blockIdx.x);
@@ -881,7 +885,7 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     uint2* in = b.pairs.as<uint2>();
     hipLaunchKernelGGL(k_morton, dim3(num_tiles), dim3(kMortonThreads), 0, st, s.tris.as<pt_triangle>(), n,
                        s.off.as<uint32_t>(), nscenes, s.morton_box.as<float>(), table, in,
-                       b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>());
+                       b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>(), b.root_word.as<uint32_t>());
     PT_HIP(hipGetLastError());
 
     if (n >= 2) {

@@ -59,7 +59,8 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_single(
     if (COUNT) add_counts(cnt, counters);
 }
 
-// Persistent closest-hit kernel over an AoS ray batch (ntri >= 2); FILTER:
+// Persistent closest-hit kernel over an AoS ray batch in the scene with root word
+// *roots (two triangles or more); FILTER:
 // the root filter (persistent_trace_filtered), without counting.
 template <bool COUNT, int LDS, bool FILTER>
 __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
     static_assert(!(COUNT && FILTER), "the filter's repeated root visit would change the visit counts");
     __shared__ uint32_t s_stack[LDS][kPersistThreads];
     __shared__ uint32_t s_pend[kPend][kPersistThreads];
-    const uint32_t root = roots[0];
+    const uint32_t root = *roots;
     auto load = [&](uint32_t i, V3& o, V3& d, uint32_t&) -> uint32_t {
         const float* rp = rays + 6 * static_cast<size_t>(i);
         o = v3(rp[0], rp[1], rp[2]);
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_grouped(
             const float* rp = rays + 6 * static_cast<size_t>(i);
             o = v3(rp[0], rp[1], rp[2]);
             d = v3(rp[3], rp[4], rp[5]);
-            if (!SCENES) return roots[0];
+            if (!SCENES) return *roots;
             const uint32_t sc = scene[i];
             if (sc >= nscenes) return kInvalid;  // unknown scene: a miss
             const uint32_t b = off[sc], e = off[sc + 1];
@@ -157,8 +158,9 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_grouped(
 }
 
 // Whether a launch of n rays runs grouped, and with how many lanes per ray
-// (log2); scene ids may be null (one scene of at least two triangles).
-uint32_t launch_grouped(const DeviceScene& s, const float* d_rays, const uint32_t* d_scene, uint32_t n, uint32_t* d_id,
+// (log2); scene ids may be null (all rays in scene `first`, of at least two
+// triangles).
+uint32_t launch_grouped(const DeviceScene& s, uint32_t first, const float* d_rays, const uint32_t* d_scene, uint32_t n, uint32_t* d_id,
                         float* d_t, float* d_uv, hipStream_t st) {
     const TraceTuning& tune = trace_tuning();
     const uint32_t lg = launch_group(n, static_cast<uint64_t>(tune.blocks) * kPersistThreads);
@@ -167,7 +169,7 @@ uint32_t launch_grouped(const DeviceScene& s, const float* d_rays, const uint32_
     auto kern = d_scene ? (tune.lds <= 8 ? k_trace_grouped<8, true> : k_trace_grouped<16, true>)
                         : (tune.lds <= 8 ? k_trace_grouped<8, false> : k_trace_grouped<16, false>);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st, s.bvh.nodes.as<float4>(),
-                       s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(), s.off.as<uint32_t>(), s.nscenes(),
+                       s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>() + first, s.off.as<uint32_t>(), s.nscenes(),
                        d_rays, d_scene, n, lg, d_id, d_t, reinterpret_cast<float2*>(d_uv), s.status.as<uint32_t>());
     PT_HIP(hipGetLastError());
     return lg;
@@ -180,16 +182,20 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
                   float* d_t, float* d_uv, unsigned long long* d_counters, hipStream_t st) {
     if (n == 0) return;
     uint32_t* status = s.status.as<uint32_t>();
-    if (s.bvh.n < 2) {
+    // Rays without scene ids go to the first scene that has triangles.  The scenes
+    // before it are empty, so its one triangle, if it has no more, is triangle 0.
+    const uint32_t first = s.first_scene();
+    const uint32_t ntri = s.off_host[first + 1] - s.off_host[first];
+    if (ntri < 2) {
         const uint32_t blocks = static_cast<uint32_t>((static_cast<uint64_t>(n) + kTraceThreads - 1) /
                                                       kTraceThreads);
         hipLaunchKernelGGL(k_trace_single<COUNT>, dim3(blocks), dim3(kTraceThreads), 0, st,
-                           s.bvh.tris.as<float4>(), s.bvh.n, d_rays, n, d_id, d_t,
+                           s.bvh.tris.as<float4>(), ntri, d_rays, n, d_id, d_t,
                            reinterpret_cast<float2*>(d_uv), d_counters);
         PT_HIP(hipGetLastError());
         return;
     }
-    if (!COUNT && launch_grouped(s, d_rays, nullptr, n, d_id, d_t, d_uv, st)) return;
+    if (!COUNT && launch_grouped(s, first, d_rays, nullptr, n, d_id, d_t, d_uv, st)) return;
     const TraceTuning& tune = trace_tuning();
     hipLaunchKernelGGL(k_zero_queue, dim3(1), dim3(64), 0, st, queue);
     const uint64_t want = (static_cast<uint64_t>(n) + kPersistThreads - 1) / kPersistThreads;
@@ -203,8 +209,8 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
                                         : (tune.lds <= 16 ? k_trace_persistent<COUNT, 16, false>
                                                           : k_trace_persistent<COUNT, 32, false>));
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
-                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(), d_rays, n, d_id, d_t,
-                       reinterpret_cast<float2*>(d_uv), queue, std::min(64u, std::max(1u, tune.refill)),
+                       s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>() + first, d_rays,
+                       n, d_id, d_t, reinterpret_cast<float2*>(d_uv), queue, std::min(64u, std::max(1u, tune.refill)),
                        pool_for(tune.pool), d_counters, status);
     PT_HIP(hipGetLastError());
 }
@@ -252,7 +258,7 @@ TraceTuning& trace_tuning() {
 void trace_closest_scenes(const DeviceScene& s, uint32_t* queue, const float* d_rays, const uint32_t* d_scene,
                           uint32_t n, uint32_t* d_id, float* d_t, float* d_uv, hipStream_t st) {
     if (n == 0) return;
-    if (launch_grouped(s, d_rays, d_scene, n, d_id, d_t, d_uv, st)) return;
+    if (launch_grouped(s, 0u, d_rays, d_scene, n, d_id, d_t, d_uv, st)) return;
     const TraceTuning& tune = trace_tuning();
     hipLaunchKernelGGL(k_zero_queue, dim3(1), dim3(64), 0, st, queue);
     const uint64_t want = (static_cast<uint64_t>(n) + kPersistThreads - 1) / kPersistThreads;

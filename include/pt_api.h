@@ -219,7 +219,9 @@ int pt_verify_bvh(pt_context* ctx, uint32_t* bad_scenes);
  * the context's last upload or build (unless the stream is being captured
  * into a graph: then the caller orders it).  Each stream has its own ray
  * queue, allocated on its first trace, so traces on different streams may
- * overlap. */
+ * overlap.
+ * In a batch (pt_upload_scenes) these trace the first scene that has triangles;
+ * pt_trace_closest_scenes_device names each ray's scene. */
 int pt_trace_closest(pt_context* ctx, const float* rays, uint32_t n,
                      uint32_t* id, float* t, float* uv);
 int pt_trace_closest_device(pt_context* ctx, const float* d_rays, uint32_t n,
