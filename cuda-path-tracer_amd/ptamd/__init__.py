@@ -187,6 +187,19 @@ def _f32(x, n=None):
     return a
 
 
+def _light_rows(lights):
+    """Directional lights as rows of pt_dir_light: color, direction, intensity
+    (7 floats); of rows of 6 floats the intensity is 1."""
+    a = np.ascontiguousarray(lights, np.float32)
+    if a.size == 0:
+        return a.reshape(0, 7)
+    if a.size == 6 * len(a):
+        a = np.concatenate([a.reshape(-1, 6), np.ones((len(a), 1), np.float32)], axis=1)
+    if a.size != 7 * len(a):
+        raise ValueError(f"a light is 7 floats (color, direction, intensity), got an array of shape {a.shape}")
+    return a.reshape(-1, 7)
+
+
 def _check(rc, ctx=None):
     if rc < 0:
         buf = ctypes.create_string_buffer(512)
@@ -428,8 +441,8 @@ class Context:
         bmin_a = None if bmin is None else _f32(bmin, 3)
         bmax_a = None if bmax is None else _f32(bmax, 3)
         st = None if settings is None else ctypes.byref(settings)
-        nl = 0 if lights is None else len(lights)
-        la = None if lights is None else np.ascontiguousarray(lights, np.float32)
+        la = None if lights is None else _light_rows(lights)
+        nl = 0 if la is None else len(la)
         self._c(_lib.pt_upload_scene(self._h, _ptr(tris), len(tris), _ptr(infos), len(infos),
                                      _ptr(la), nl, _ptr(bmin_a), _ptr(bmax_a), st))
         self.n = len(tris)
