@@ -29,14 +29,15 @@ def test_other_shapes_are_refused(shape):
 def test_six_floats_render_as_intensity_one(ctx):
     """Lit cache frames and plain frames: the same bits as seven floats give, and
     light arrives."""
-    tris, infos = ptamd.gen_sphere(24, 6)
+    tris, infos = ptamd.gen_soup(20000, 4)
+    eye = (0.5, 0.5, -1.5)
     w, h = 96, 64
-    dirs = ptamd.camera_corners((0.1, 0.2, 2.4), (0, 0, 0), (0, 1, 0), 60.0, w / h, 0.4, 0.2)
+    dirs = ptamd.camera_corners(eye, (0.5, 0.5, 0.0), (0, 1, 0), 60.0, w / h, 0.4, 0.2)
     six = np.array([[2.0, 1.9, 1.8, 0.28, -0.94, -0.19]], np.float32)
     got = []
     for lights in (None, six, np.concatenate([six, np.ones((1, 1), np.float32)], axis=1)):
         ctx.upload_scene(tris, infos, settings=ptamd.Settings(2, 3, 1.0, 1), lights=lights)
-        ctx.set_primary_rays(dirs, (0.1, 0.2, 2.4))
+        ctx.set_primary_rays(dirs, eye)
         ctx.cache_init(2, np.full(3, -4, np.float32), np.full(3, 4, np.float32))
         ctx.reset_frames()
         ctx.render_pass(w, h, 3)
