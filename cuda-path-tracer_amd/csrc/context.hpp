@@ -110,6 +110,7 @@ struct DeviceBvh {
     DevBuf scene_of;                        // scene of each leaf slot
     DevBuf nodes, tris;
     DevBuf root_box, root_word;     // per scene: the root's box and child word (kInvalid: no internal node)
+    DevBuf strict;                  // 1: a triangle's box is NaN, rays walk in the reference's order only
     DevBuf tile_hist, digit_total;  // radix sort scratch
     DevBuf open_lists;              // tree: each block's subtrees that the next level goes on with
 };

@@ -114,7 +114,7 @@ __device__ __forceinline__ uint32_t scene_of_slot(const uint32_t* __restrict__ o
 // (box[6*s..] = min.xyz, invScale.xyz).  One workgroup per sort tile, which also
 // counts the tile's first-pass digits (key bits 0-9) into its row of tile_hist --
 // the first sort pass then starts at the scan.  Also sets every scene's root word
-// to kInvalid, for the scenes whose tree writes none.
+// to kInvalid, for the scenes whose tree writes none, and clears `strict`.
 constexpr int kMortonThreads = 1024;
 
 __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __restrict__ tris, uint32_t n,
@@ -124,9 +124,11 @@ __global__ __launch_bounds__(kMortonThreads) void k_morton(const pt_triangle* __
                                                            uint2* __restrict__ pairs,
                                                            uint32_t* __restrict__ scene_of,
                                                            uint32_t* __restrict__ tile_hist,
-                                                           uint32_t* __restrict__ root_word) {
+                                                           uint32_t* __restrict__ root_word,
+                                                           uint32_t* __restrict__ strict) {
     __shared__ uint32_t h[kRadix];
     const uint32_t tid = threadIdx.x;
+    if (blockIdx.x == 0 && tid == 0) *strict = 0u;
     for (uint32_t s = blockIdx.x * kMortonThreads + tid; s < nscenes; s += gridDim.x * kMortonThreads) root_word[s] = kInvalid;
     for (uint32_t d = tid; d < kRadix; d += kMortonThreads) h[d] = 0u;
     __syncthreads();
@@ -605,7 +607,8 @@ __global__ __launch_bounds__(kLeafBlock) void k_tree_leaves(
     const pt_triangle* __restrict__ in_tris, const uint2* __restrict__ pairs,
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ scene_of, uint32_t n,
     float4* __restrict__ nodes, float4* __restrict__ tri_recs, float* __restrict__ root_box,
-    uint32_t* __restrict__ root_word, OpenList* __restrict__ lists, uint32_t* __restrict__ status) {
+    uint32_t* __restrict__ root_word, uint32_t* __restrict__ strict, OpenList* __restrict__ lists,
+    uint32_t* __restrict__ status) {
     __shared__ TreeStage<kLeafBlock> S;
     __shared__ uint32_t s_w[16];
     const uint32_t tid = threadIdx.x;
@@ -648,6 +651,9 @@ __global__ __launch_bounds__(kLeafBlock) void k_tree_leaves(
         b.mxx = gmax(gmax(gmax(-kFltMax, v0.x), v1.x), v2.x);
         b.mxy = gmax(gmax(gmax(-kFltMax, v0.y), v1.y), v2.y);
         b.mxz = gmax(gmax(gmax(-kFltMax, v0.z), v1.z), v2.z);
+        if (__builtin_isunordered(b.mnx, b.mxx) || __builtin_isunordered(b.mny, b.mxy) ||
+            __builtin_isunordered(b.mnz, b.mxz))
+            atomicOr(strict, 1u);
     }
     __syncthreads();
     if (tid < count)
@@ -861,7 +867,11 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     const uint32_t n = s.n;
     const uint32_t nscenes = static_cast<uint32_t>(s.off_host.size()) - 1;
     b.n = n;
-    if (n == 0) return;
+    b.strict.reserve(sizeof(uint32_t));
+    if (n == 0) {
+        PT_HIP(hipMemsetAsync(b.strict.as<void>(), 0, sizeof(uint32_t), st));
+        return;
+    }
     if (n >= (1u << 30)) throw Error(PT_E_INVALID_ARG, "LBVH supports fewer than 2^30 triangles");
     const size_t n4 = static_cast<size_t>(n) * 4;
     b.pairs.reserve(2 * n4);
@@ -885,7 +895,8 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     uint2* in = b.pairs.as<uint2>();
     hipLaunchKernelGGL(k_morton, dim3(num_tiles), dim3(kMortonThreads), 0, st, s.tris.as<pt_triangle>(), n,
                        s.off.as<uint32_t>(), nscenes, s.morton_box.as<float>(), table, in,
-                       b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>(), b.root_word.as<uint32_t>());
+                       b.scene_of.as<uint32_t>(), b.tile_hist.as<uint32_t>(), b.root_word.as<uint32_t>(),
+                       b.strict.as<uint32_t>());
     PT_HIP(hipGetLastError());
 
     if (n >= 2) {
@@ -929,7 +940,7 @@ void build_lbvh(DeviceScene& s, hipStream_t st) {
     hipLaunchKernelGGL(k_tree_leaves, dim3(blocks), dim3(kLeafBlock), 0, st, s.tris.as<pt_triangle>(),
                        b.pairs.as<uint2>(), s.off.as<uint32_t>(), scene_of, n,
                        b.nodes.as<float4>(), b.tris.as<float4>(), b.root_box.as<float>(), b.root_word.as<uint32_t>(),
-                       lists, s.status.as<uint32_t>());
+                       b.strict.as<uint32_t>(), lists, s.status.as<uint32_t>());
     for (uint32_t m = blocks; m > 1;) {
         const uint32_t next = div_up(m, kFanIn);
         hipLaunchKernelGGL(k_tree_merge, dim3(next), dim3(kMergeThreads), 0, st, lists, m, scene_of, b.nodes.as<float4>(),

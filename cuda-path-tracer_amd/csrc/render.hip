@@ -48,6 +48,7 @@ struct FrameConst {
     const uint4* texinfo;              // per texture: first texel, width, height, 0
     uint32_t* status;                  // the scene's status word (PT_STATUS_* flags)
     const uint32_t* roots;             // child word of each scene's root (two triangles or more)
+    const uint32_t* strict;            // whether all rays walk in the reference's order (DeviceBvh)
 };
 
 // Structure-of-arrays queue of rays (origin, direction, path index).
@@ -185,8 +186,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
                                                             const uint32_t* __restrict__ counters,
                                                             uint32_t* __restrict__ ray_counters,
                                                             uint32_t level, uint32_t refill, uint32_t pool) {
-    __shared__ uint32_t s_stack[LDS][kPersistThreads];
-    __shared__ uint32_t s_pend[kPend][kPersistThreads];
+    __shared__ uint32_t s_ray[kRayRows<LDS>][kPersistThreads];
     const uint32_t count = counters[level];
     TraceCount cnt{0, 0, 0, 0};
     auto load = [&](uint32_t i, V3& o, V3& d, uint32_t& single) -> uint32_t {
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_extend(const FrameConst fc,
         hq.v[i] = h.v;
     };
     persistent_trace<false, LDS>(nodes, tris, count, ray_counters + level * kQueueWords, fc.status, refill, pool,
-                                 s_stack, s_pend, load, store, cnt);
+                                 *fc.strict ? kRayExact : 0u, s_ray, load, store, cnt);
 }
 
 __device__ __forceinline__ V3 ld3(const float* p) { return v3(p[0], p[1], p[2]); }
@@ -664,6 +664,8 @@ __device__ __forceinline__ void answer_single(const FrameConst& fc, const PassPa
     const uint32_t sc = pp[CACHE ? 0u : path / fc.npix].scene;
     const TraceHit h = trace_single<false>(tris, off[sc + 1] - off[sc] == 1u ? off[sc] : kInvalid, r.o, r.d, cnt);
     r.minT = h.t; r.best = h.id; r.bu = h.u; r.bv = h.v;
+    r.bound = h.t;
+    r.flags = 0u;
 }
 
 // At most 96 VGPRs (5 waves per SIMD): the plain and the cache variants fit
@@ -695,8 +697,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                                                            uint32_t* __restrict__ counters,
                                                            uint32_t* __restrict__ queue, uint32_t refill,
                                                            uint32_t shade_min, uint32_t lg0, CacheIO io) {
-    __shared__ uint32_t s_stack[LDS][kPersistThreads];
-    __shared__ uint32_t s_pend[kPend][kPersistThreads];
+    __shared__ uint32_t s_ray[kRayRows<LDS>][kPersistThreads];
     __shared__ uint32_t s_level[kMaxLevels];
     // Plain frames keep each lane's path throughput and radiance in LDS
     // while it traverses alone.
@@ -708,16 +709,12 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
     const uint32_t npaths = npix + ntrain;
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     const int lane = threadIdx.x & 63;
-    uint32_t spill[kStackMax - LDS];
+    const uint32_t strict = *fc.strict ? kRayExact : 0u;
+    uint32_t spill[kSpillMax<LDS>];
     keep_in_memory(spill);
     RayState r;
-    r.o = r.d = r.dinv = v3(0.0f, 0.0f, 0.0f);
-    r.minT = kMinTInit;
-    r.best = kInvalid;
-    r.bu = r.bv = 0.0f;
-    r.word = 0u;
-    r.sp = 0;
-    r.finite = true;
+    r.o = r.d = v3(0.0f, 0.0f, 0.0f);
+    init_ray(r, 0u, 0u);
     uint32_t path = 0, bounce = 0;  // the path's pass and pixel follow from its index
     uint32_t root = kInvalid;
     V3 absorbed_r = v3(1.0f, 1.0f, 1.0f), acc_r = v3(0.0f, 0.0f, 0.0f);
@@ -752,7 +749,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
             HitShade hs = hit_shade<DETAIL>(fc, infos, r.best, r.minT, r.bu, r.bv, r.o, r.d);
             const uint32_t sb = off[P.scene], se = off[P.scene + 1];
             ShadowStack ss;
-            ss.lds = &s_stack[0][threadIdx.x];
+            ss.lds = &s_ray[0][threadIdx.x];
             ss.stride = kPersistThreads;
             ss.depth = LDS;
             ss.spill = spill;
@@ -791,10 +788,10 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
         return cont;
     };
 
-    // What is left to the groups: which lanes hold a path, the groups' stack
-    // sizes (0: a segment that has ended) and lanes per path (log2).
+    // What is left to the groups: which lanes hold a path, and the groups
+    // (stack size 0: a segment that has ended).
     bool active = false;
-    uint32_t gsp = 0u, lg = lg0;
+    Group g{0u, lg0, kInvalid, kMinTInit};
     V3 absorbed = v3(1.0f, 1.0f, 1.0f), acc = v3(0.0f, 0.0f, 0.0f);
 
     if (lg0 > 0u) {
@@ -802,7 +799,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
         if (slot < npaths) {
             start(slot);
             active = true;
-            if (root != kInvalid) group_start<LDS>(r, root, gsp, lg, s_stack);
+            if (root != kInvalid) group_start<LDS>(r, root, strict, g, s_ray);
             else answer_single<CACHE>(fc, pp, off, tris, path, r);
         }
     } else if (wave_id == 0u || static_cast<uint64_t>(wave_id) * kRayPoolSmall < npaths) {
@@ -833,7 +830,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                             absorbed_r = v3(1.0f, 1.0f, 1.0f);
                             acc_r = v3(0.0f, 0.0f, 0.0f);
                         }
-                        init_ray(r, root);
+                        init_ray(r, root, strict);
                         state = kLaneTrace;
                     }
                     ho.next += took;
@@ -847,13 +844,17 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                 if (static_cast<uint32_t>(__popcll(busy)) <= kTailLanes &&
                     __ballot(state == kLaneTrace && r.sp >= LDS) == 0ull) {
                     active = state != kLaneIdle;
-                    test_pending(tris, r, pend, s_pend);
+                    test_pending<LDS>(tris, r, pend, s_ray);
                     if (state == kLaneTrace) {
                         if (root == kInvalid) {
                             answer_single<CACHE>(fc, pp, off, tris, path, r);
-                        } else if (r.word != kInvalid) {
-                            s_stack[r.sp][tid] = r.word;
-                            gsp = static_cast<uint32_t>(r.sp) + 1u;
+                        } else {
+                            if (r.flags & kRayTie) init_ray(r, root, kRayExact);
+                            r.flags &= ~kRayTested;  // the group visits the node anew
+                            if (r.word != kInvalid) {
+                                s_ray[r.sp][tid] = r.word;
+                                g.sp = static_cast<uint32_t>(r.sp) + 1u;
+                            }
                         }
                     }
                     break;
@@ -865,8 +866,10 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                 answer_single<CACHE>(fc, pp, off, tris, path, r);
                 state = kLaneShade;
             }
-            if (walk_wave<LDS>(nodes, tris, r, pend, state == kLaneTrace, s_stack, s_pend, spill, fc.status))
-                state = kLaneShade;
+            if (walk_wave<LDS>(nodes, tris, r, pend, state == kLaneTrace, s_ray, spill, fc.status)) {
+                if (r.flags & kRayTie) init_ray(r, root, kRayExact);
+                else state = kLaneShade;
+            }
             const uint64_t shading = __ballot(state == kLaneShade);
             const uint64_t tracing = __ballot(state == kLaneTrace);
             if (shading != 0ull && (static_cast<uint32_t>(__popcll(shading)) >= shade_min || tracing == 0ull)) {
@@ -877,7 +880,7 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                         ac = v3(s_carry[3][tid], s_carry[4][tid], s_carry[5][tid]);
                     }
                     if (shade(ab, ac, true)) {
-                        init_ray(r, root);
+                        init_ray(r, root, strict);
                         state = kLaneTrace;
                         if constexpr (kCarryLds) {
                             s_carry[0][tid] = ab.x; s_carry[1][tid] = ab.y; s_carry[2][tid] = ab.z;
@@ -902,11 +905,11 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
 
     // Groups: rounds until every path has ended.
     for (;;) {
-        const uint64_t act = __ballot(active && (lane & ((1 << lg) - 1)) == 0);
+        const uint64_t act = __ballot(active && (lane & ((1 << g.lg) - 1)) == 0);
         if (act == 0ull) break;
         const uint32_t lgn = group_log(static_cast<uint32_t>(__popcll(act)));
-        if (lgn > lg && __ballot(active && gsp > (static_cast<uint32_t>(LDS) << lg)) == 0ull) {
-            const uint32_t own = regroup<LDS>(r, gsp, lg, lgn, act, s_stack);
+        if (lgn > g.lg && __ballot(active && !group_movable<LDS>(g)) == 0ull) {
+            const uint32_t own = regroup<LDS>(r, g, lgn, act, s_ray);
             const uint32_t src = own & 63u;
             path = lane_u32(path, src);
             bounce = lane_u32(bounce, src);
@@ -915,17 +918,19 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
             acc = lane_v3(acc, src);
             active = own < 64u;
         }
-        group_round<LDS>(nodes, tris, r, gsp, lg, s_stack, spill, fc.status);
-        const uint64_t ended = __ballot(active && gsp == 0u);
+        group_round<LDS>(nodes, tris, r, g, s_ray, spill, fc.status);
+        const uint64_t ended = __ballot(active && g.sp == 0u);
         if (ended != 0ull &&
             (static_cast<uint32_t>(__popcll(ended)) * group_shade(LIGHTS) >=
              static_cast<uint32_t>(__popcll(__ballot(active))))) {
-            group_best(r, lg);
-            if (active && gsp == 0u) {
-                const bool lead = (lane & ((1 << lg) - 1)) == 0;
-                active = shade(absorbed, acc, lead);
+            RayState f = r;
+            const bool tie = group_best(f, g.lg);
+            if (active && g.sp == 0u) {
+                const bool lead = (lane & ((1 << g.lg) - 1)) == 0;
+                r = f;
+                if (!tie) active = shade(absorbed, acc, lead);
                 if (active) {
-                    if (root != kInvalid) group_start<LDS>(r, root, gsp, lg, s_stack);
+                    if (root != kInvalid) group_start<LDS>(r, root, tie ? kRayExact : strict, g, s_ray);
                     else answer_single<CACHE>(fc, pp, off, tris, path, r);
                 }
             }
@@ -981,7 +986,7 @@ __global__ __launch_bounds__(kSuffixThreads) void k_train_paths(const FrameConst
                 RayState r;
                 r.o = o;
                 r.d = d;
-                init_ray(r, fc.roots[P.scene]);
+                init_ray(r, fc.roots[P.scene], 0u);
                 if (r.finite) {
                     while (visit_step<false, kTrainLds, true>(nodes, tris, r, s_tstack, spill, cnt, fc.status)) {
                     }
@@ -1525,6 +1530,7 @@ void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, cons
     fc.nlights = scene.nlights;
     fc.status = scene.status.as<uint32_t>();
     fc.roots = scene.bvh.root_word.as<uint32_t>();
+    fc.strict = scene.bvh.strict.as<uint32_t>();
     set_detail(fc, scene);
 
     const uint32_t nchains = frame_chains(npix * npasses);
@@ -1714,6 +1720,7 @@ void render_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
     cf.fc.nlights = scene.nlights;
     cf.fc.status = scene.status.as<uint32_t>();
     cf.fc.roots = scene.bvh.root_word.as<uint32_t>();
+    cf.fc.strict = scene.bvh.strict.as<uint32_t>();
     set_detail(cf.fc, scene);
     cf.steps = cs.train_steps;
     cf.train = (cs.flags & PT_CACHE_TRAIN) != 0;

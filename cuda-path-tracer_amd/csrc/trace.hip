@@ -67,11 +67,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
     const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ roots,
     const float* __restrict__ rays, uint32_t nrays, uint32_t* __restrict__ out_id, float* __restrict__ out_t,
     float2* __restrict__ out_uv, uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool,
-    unsigned long long* __restrict__ counters, uint32_t* __restrict__ status) {
+    const uint32_t* __restrict__ strict, unsigned long long* __restrict__ counters, uint32_t* __restrict__ status) {
     static_assert(!(COUNT && FILTER), "the filter's repeated root visit would change the visit counts");
-    __shared__ uint32_t s_stack[LDS][kPersistThreads];
-    __shared__ uint32_t s_pend[kPend][kPersistThreads];
-    const uint32_t root = *roots;
+    __shared__ uint32_t s_ray[kRayRows<LDS>][kPersistThreads];
+    const uint32_t root = *roots, flags = *strict ? kRayExact : 0u;
     auto load = [&](uint32_t i, V3& o, V3& d, uint32_t&) -> uint32_t {
         const float* rp = rays + 6 * static_cast<size_t>(i);
         o = v3(rp[0], rp[1], rp[2]);
@@ -85,12 +84,12 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_persistent(
     };
     if constexpr (FILTER) {
         __shared__ uint32_t s_surv[kPersistThreads / 64][kSurvCap];
-        persistent_trace_filtered<LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, s_stack, s_pend,
+        persistent_trace_filtered<LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, flags, s_ray,
                                        s_surv[threadIdx.x / 64], load, store);
     } else {
         TraceCount cnt{0, 0, 0, 0};
-        persistent_trace<COUNT, LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, s_stack, s_pend, load,
-                                     store, cnt);
+        persistent_trace<COUNT, LDS>(nodes, tris, nrays, ray_counter, status, refill, pool, flags, s_ray, load, store,
+                                     cnt);
         if (COUNT) add_counts(cnt, counters);
     }
 }
@@ -102,12 +101,12 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_scenes(
     const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ roots,
     const uint32_t* __restrict__ off, uint32_t nscenes, const float* __restrict__ rays, const uint32_t* __restrict__ scene, uint32_t nrays,
     uint32_t* __restrict__ out_id, float* __restrict__ out_t, float2* __restrict__ out_uv,
-    uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool, uint32_t* __restrict__ status) {
-    __shared__ uint32_t s_stack[LDS][kPersistThreads];
-    __shared__ uint32_t s_pend[kPend][kPersistThreads];
+    uint32_t* __restrict__ ray_counter, uint32_t refill, uint32_t pool, const uint32_t* __restrict__ strict,
+    uint32_t* __restrict__ status) {
+    __shared__ uint32_t s_ray[kRayRows<LDS>][kPersistThreads];
     TraceCount cnt{0, 0, 0, 0};
     persistent_trace<false, LDS>(
-        nodes, tris, nrays, ray_counter, status, refill, pool, s_stack, s_pend,
+        nodes, tris, nrays, ray_counter, status, refill, pool, *strict ? kRayExact : 0u, s_ray,
         [&](uint32_t i, V3& o, V3& d, uint32_t& single) -> uint32_t {
             const float* rp = rays + 6 * static_cast<size_t>(i);
             o = v3(rp[0], rp[1], rp[2]);
@@ -134,10 +133,11 @@ __global__ __launch_bounds__(kPersistThreads) void k_trace_grouped(
     const float4* __restrict__ nodes, const float4* __restrict__ tris, const uint32_t* __restrict__ roots,
     const uint32_t* __restrict__ off, uint32_t nscenes, const float* __restrict__ rays,
     const uint32_t* __restrict__ scene, uint32_t nrays, uint32_t lg, uint32_t* __restrict__ out_id,
-    float* __restrict__ out_t, float2* __restrict__ out_uv, uint32_t* __restrict__ status) {
-    __shared__ uint32_t s_stack[LDS][kPersistThreads];
+    float* __restrict__ out_t, float2* __restrict__ out_uv, const uint32_t* __restrict__ strict,
+    uint32_t* __restrict__ status) {
+    __shared__ uint32_t s_ray[kRayRows<LDS>][kPersistThreads];
     grouped_trace<LDS>(
-        nodes, tris, nrays, lg, status, s_stack,
+        nodes, tris, nrays, lg, *strict ? kRayExact : 0u, status, s_ray,
         [&](uint32_t i, V3& o, V3& d, uint32_t& single) -> uint32_t {
             const float* rp = rays + 6 * static_cast<size_t>(i);
             o = v3(rp[0], rp[1], rp[2]);
@@ -170,7 +170,8 @@ uint32_t launch_grouped(const DeviceScene& s, uint32_t first, const float* d_ray
                         : (tune.lds <= 8 ? k_trace_grouped<8, false> : k_trace_grouped<16, false>);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st, s.bvh.nodes.as<float4>(),
                        s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>() + first, s.off.as<uint32_t>(), s.nscenes(),
-                       d_rays, d_scene, n, lg, d_id, d_t, reinterpret_cast<float2*>(d_uv), s.status.as<uint32_t>());
+                       d_rays, d_scene, n, lg, d_id, d_t, reinterpret_cast<float2*>(d_uv), s.bvh.strict.as<uint32_t>(),
+                       s.status.as<uint32_t>());
     PT_HIP(hipGetLastError());
     return lg;
 }
@@ -211,7 +212,7 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kPersistThreads), 0, st,
                        s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>() + first, d_rays,
                        n, d_id, d_t, reinterpret_cast<float2*>(d_uv), queue, std::min(64u, std::max(1u, tune.refill)),
-                       pool_for(tune.pool), d_counters, status);
+                       pool_for(tune.pool), s.bvh.strict.as<uint32_t>(), d_counters, status);
     PT_HIP(hipGetLastError());
 }
 
@@ -269,7 +270,7 @@ void trace_closest_scenes(const DeviceScene& s, uint32_t* queue, const float* d_
                        s.bvh.nodes.as<float4>(), s.bvh.tris.as<float4>(), s.bvh.root_word.as<uint32_t>(),
                        s.off.as<uint32_t>(), s.nscenes(), d_rays, d_scene, n, d_id, d_t, reinterpret_cast<float2*>(d_uv),
                        queue, std::min(64u, std::max(1u, tune.refill)), pool_for(tune.pool),
-                       s.status.as<uint32_t>());
+                       s.bvh.strict.as<uint32_t>(), s.status.as<uint32_t>());
     PT_HIP(hipGetLastError());
 }
 

@@ -3,7 +3,9 @@
 // descend into the nearer (left on ties), defer the farther internal child on
 // a stack.  For the lowest-id tie rule the culling keeps children at exactly
 // the best distance, and a triangle replaces the best hit when nearer, or
-// equally near with a lower original id.
+// equally near with a lower original id.  Loops that test triangles later or
+// several nodes at once give the same hit: see "the reference's hit from other
+// visiting orders".
 //
 // A node is known by its child word (left child's index << 2 | left internal
 // | right internal << 1) before it is visited: its record sits in slot
@@ -154,11 +156,9 @@ __device__ __forceinline__ bool any_hit_in(const float4* __restrict__ nodes, con
 // One lane = one ray at a time, advanced one node visit per loop iteration;
 // a lane whose ray has finished takes the next ray from its wave's pool, so
 // long rays do not hold a whole wave's lanes idle.  The visiting order per ray
-// is exactly traverse_impl's.  The deferred-node stack keeps its first
-// kLdsStack entries in LDS ([depth][thread] so a wave's lanes hit distinct
+// is the reference's.  The deferred-node stack keeps its first LDS entries (8,
+// 16 or 32, tuned) in LDS ([depth][thread] so a wave's lanes hit distinct
 // banks) and the rest in a private array (scratch), touched only by deep rays.
-
-constexpr int kLdsStack = 16;  // default LDS depth (tuned: 8, 16 or 32 entries)
 constexpr int kPersistThreads = 256;
 
 struct RayState {
@@ -166,21 +166,84 @@ struct RayState {
     float minT;
     uint32_t best;
     float bu, bv;
+    float bound;    // culling distance of the loops that defer or group (see there)
+    uint32_t flags; // kRayExact ...
     uint32_t word;  // the node to visit, as its child word
     int sp;
     bool finite;
 };
+enum : uint32_t {
+    kRayExact = 1u,   // walks in the reference's order
+    kRayTested = 2u,  // ... and the current node's leaf children are tested
+    kRayTie = 4u,     // the hit may depend on the order: to be walked again with kRayExact
+};
 
-__device__ __forceinline__ void init_ray(RayState& r, uint32_t root) {
+__device__ __forceinline__ void init_ray(RayState& r, uint32_t root, uint32_t flags) {
     r.dinv = v3(1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z);
-    r.finite = __builtin_fabsf(r.dinv.x) <= kFltMax && __builtin_fabsf(r.dinv.y) <= kFltMax &&
-               __builtin_fabsf(r.dinv.z) <= kFltMax;
+    auto normal = [](float x) { return __builtin_fabsf(x) <= kFltMax && x != 0.0f; };
+    r.finite = normal(r.dinv.x) && normal(r.dinv.y) && normal(r.dinv.z);
     r.minT = kMinTInit;
     r.best = kInvalid;
     r.bu = 0.0f;
     r.bv = 0.0f;
+    r.bound = kMinTInit;
+    r.flags = flags;
     r.word = root;
     r.sp = 0;
+}
+
+// ---- the reference's hit from other visiting orders ---------------------------
+//
+// The reference culls a box with h <= (best distance so far), h from the slab
+// test and the distance from Moller-Trumbore, which round independently: a
+// triangle's t may lie an ulp or more below the h of a box that holds it (flat
+// boxes, grazing rays).  Then which triangles are tested, and with equal or
+// nearly equal distances which one wins, depends on the order of the tests.  The
+// loops below test triangles later than the reference, or many nodes at once,
+// and still return its hit:
+//
+//  - They visit every node that the reference visits.  A node's children are
+//    culled with a bound, the minimum of max(t, h of the triangle's own box)
+//    over some of the triangles that come before the node in the reference's
+//    depth-first order.  Boxes are exact minima and maxima and every step of the
+//    slab test is monotonic, so that h is no less than the h of any box around
+//    the triangle; and a triangle the reference did not test lies in a box that
+//    it had culled, with h above its best distance then, which only falls.  So
+//    the bound is never below the reference's best distance at that node.
+//  - Of all triangles they test, the lexicographic minimum W of (t, id) is the
+//    reference's hit if the reference tested it, and it did unless another
+//    triangle's t is below max(t, h) of W: up to W its best distance was no less
+//    than the other triangles' minimum, so it culled no box around W.
+//  - Where another t is below (kRayTie: overlapping or repeated triangles in a
+//    plane along the axes, rays through shared edges), the ray is walked again in
+//    the reference's order (kRayExact).  On a model of these loops, 0 of 40,000
+//    rays are in soups and rooms, 7 % at the edges of a wall of 3,200 triangles,
+//    9 % on two tessellations of one wall, 83 % on 4,000 overlapping decals.
+//  - The slab test is monotonic unless a product is NaN: a ray with an infinite
+//    dinv component is a tie when one arises, and where a triangle's box is NaN
+//    (strict, from the build) every ray walks in the reference's order.
+
+// One tested triangle: its distance t (+inf: missed) and the h of its own box
+// (0 for kRayExact rays, whose bound is the best distance itself).  Returns
+// max(t, h).
+__device__ __forceinline__ float take_hit(RayState& r, float t, uint32_t id, float u, float v, float h) {
+    const float c = __builtin_fmaxf(t, h);
+    const bool better = t < r.minT || (t == r.minT && id < r.best);
+    const float other = __builtin_fmaxf(t, r.minT);  // of the two, not the best
+    r.bound = better ? c : r.bound;  // lower, unless it is a tie
+    if (better) {
+        r.minT = t; r.best = id; r.bu = u; r.bv = v;
+    }
+    if (other < r.bound) r.flags |= kRayTie;
+    return c;
+}
+
+// Whether a product of the slab test of a box is NaN.
+__device__ __forceinline__ bool slab_nan(V3 o, V3 dinv, float minx, float maxx, float miny, float maxy, float minz,
+                                         float maxz) {
+    return __builtin_isunordered((minx - o.x) * dinv.x, (maxx - o.x) * dinv.x) ||
+           __builtin_isunordered((miny - o.y) * dinv.y, (maxy - o.y) * dinv.y) ||
+           __builtin_isunordered((minz - o.z) * dinv.z, (maxz - o.z) * dinv.z);
 }
 
 __device__ __forceinline__ TraceHit final_hit(const RayState& r) {
@@ -206,7 +269,7 @@ struct Children {
     uint32_t w0, w1;
 };
 
-// The tests of one visit.  Leaf children fold into the best hit first.  The
+// The tests of one visit, in the reference's order.  Leaf children fold into the best hit first.  The
 // reference orders a node's two children by distance and lets a leaf replace
 // the best hit when nearer, or equally near with a lower id (trace.h:125-160):
 // over the leaves of one node that is the lexicographic minimum of (t, id),
@@ -214,9 +277,11 @@ struct Children {
 // visits the same nodes: an internal child nearer than a leaf stays within
 // the updated best distance, and one farther than a leaf is culled against
 // the distance the leaf set, as in the reference.
-template <bool COUNT, bool FINITE>
+// ORDERED false: for a group's lane (take_hit); `reach` is lowered to the leaf
+// children's max(t, h).
+template <bool COUNT, bool FINITE, bool ORDERED = true>
 __device__ __forceinline__ Children test_children(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                                  RayState& r, TraceCount& cnt) {
+                                                  RayState& r, TraceCount& cnt, float* reach = nullptr) {
     const uint32_t w = r.word;
     const uint32_t l = w >> 2;
     const float4* rec = nodes + 4 * static_cast<size_t>(l);
@@ -236,6 +301,11 @@ __device__ __forceinline__ Children test_children(const float4* __restrict__ nod
     c.w0 = cw.x;
     c.w1 = cw.y;
     if (COUNT) cnt.boxes += (w & 1u) + ((w >> 1) & 1u);
+    if constexpr (!ORDERED && !FINITE) {
+        if (!(r.flags & kRayExact) && (slab_nan(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y) ||
+                                       slab_nan(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w)))
+            r.flags |= kRayTie;
+    }
     // An opaque copy of the word: with the same condition as above the
     // compiler would merge the two branches and issue the triangle loads
     // only after the box tests, a second memory round trip.
@@ -246,7 +316,9 @@ __device__ __forceinline__ Children test_children(const float4* __restrict__ nod
         const float t = tri_test(ta, r.o, r.d, u, v);
         const uint32_t id = __float_as_uint(ta.p.w);
         if (COUNT) cnt.tris++;
-        if (t < r.minT || (t == r.minT && id < r.best)) {
+        if constexpr (!ORDERED) {
+            *reach = __builtin_fminf(*reach, take_hit(r, t, id, u, v, (r.flags & kRayExact) ? 0.0f : ((wt & 1u) ? c.h1 : c.h0)));
+        } else if (t < r.minT || (t == r.minT && id < r.best)) {
             r.minT = t; r.best = id; r.bu = u; r.bv = v;
         }
         if ((wt & 3u) == 0u) {
@@ -254,7 +326,9 @@ __device__ __forceinline__ Children test_children(const float4* __restrict__ nod
             const float t2 = tri_test(tb, r.o, r.d, u2, v2);
             const uint32_t id2 = __float_as_uint(tb.p.w);
             if (COUNT) cnt.tris++;
-            if (t2 < r.minT || (t2 == r.minT && id2 < r.best)) {
+            if constexpr (!ORDERED) {
+                *reach = __builtin_fminf(*reach, take_hit(r, t2, id2, u2, v2, (r.flags & kRayExact) ? 0.0f : c.h1));
+            } else if (t2 < r.minT || (t2 == r.minT && id2 < r.best)) {
                 r.minT = t2; r.best = id2; r.bu = u2; r.bv = v2;
             }
         }
@@ -309,11 +383,13 @@ __device__ __forceinline__ bool visit_step(const float4* __restrict__ nodes,
 // child on a few lanes (2.8 of 64 on average), and testing those triangles at
 // once costs the whole wave two triangle tests' instructions per visit, more
 // than half of all it issues.  walk_step instead notes a node's leaf children
-// in the lane's column of an LDS list and walks on; the wave tests the noted
-// triangles together (test_pending) once kFlushLanes lanes cannot go on --
-// list full, or nothing left to walk -- or no lane can.  The best distance
-// shrinks a few visits later, so a ray visits somewhat more nodes; its hit is
-// the lexicographic minimum of (t, id) over its triangles in any order.
+// in the lane's column of an LDS list, with the distances of their boxes, and
+// walks on; the wave tests all noted triangles together (test_pending) once
+// kFlushLanes lanes cannot go on -- list full, or nothing left to walk -- or no
+// lane can.  The bound shrinks a few visits later, so a ray visits somewhat more
+// nodes; its hit is the reference's (see above).  A kRayExact lane cannot go on
+// while it has noted triangles, and culls the other child of their node only
+// after they are tested.
 // Measured (us; 16M shell rays on the 871,200-triangle mesh, 2M camera rays on
 // the 2.88M-triangle hair ball, two 1,024 x 1,024 room frames): tests at once
 // 897, 1,464, 5,790; four entries and 6 / 12 / 20 / 32 lanes 877 / 863 / 868 /
@@ -321,24 +397,50 @@ __device__ __forceinline__ bool visit_step(const float4* __restrict__ nodes,
 // and 12 lanes 883, 1,366, 5,460.
 constexpr uint32_t kPend = 4;  // list entries per lane
 constexpr uint32_t kFlushLanes = 12;
+// LDS words per lane: its stack, then its list (triangles, then distances).
+template <int LDS>
+constexpr int kRayRows = LDS + 2 * static_cast<int>(kPend);
 
 template <int LDS, bool FINITE, int COLS>
 __device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, RayState& r, uint32_t& pend,
-                                          uint32_t (*s_stack)[COLS], uint32_t (*s_pend)[COLS], uint32_t* spill,
-                                          uint32_t* status) {
+                                          uint32_t (*s_ray)[COLS], uint32_t* spill, uint32_t* status) {
     const uint32_t w = r.word;
     const uint32_t l = w >> 2;
     const float4* rec = nodes + 4 * static_cast<size_t>(l);
     const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
     const uint2 cw = *reinterpret_cast<const uint2*>(rec + 3);
-    if ((w & 3u) != 3u) {
-        s_pend[pend][threadIdx.x] = (w & 1u) ? l + 1 : l;
-        if ((w & 3u) == 0u) s_pend[pend + 1][threadIdx.x] = l + 1;
-        pend += (w & 3u) == 0u ? 2u : 1u;
-    }
     const float h0 = child_box<false, FINITE>(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
     const float h1 = child_box<false, FINITE>(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
-    const bool g0 = (w & 1u) && h0 <= r.minT, g1 = (w & 2u) && h1 <= r.minT;
+    if constexpr (!FINITE) {
+        if (!(r.flags & kRayExact) && (slab_nan(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y) ||
+                                       slab_nan(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w)))
+            r.flags |= kRayTie;
+    }
+    if ((w & 3u) != 3u) {
+        uint32_t (*s_pend)[COLS] = s_ray + LDS;
+        const uint32_t one = (w & 1u) ? l + 1 : l;
+        if (!(r.flags & kRayExact)) {
+            s_pend[pend][threadIdx.x] = one;
+            s_pend[kPend + pend][threadIdx.x] = __float_as_uint((w & 1u) ? h1 : h0);
+            if ((w & 3u) == 0u) {
+                s_pend[pend + 1u][threadIdx.x] = l + 1;
+                s_pend[kPend + pend + 1u][threadIdx.x] = __float_as_uint(h1);
+            }
+            pend += (w & 3u) == 0u ? 2u : 1u;
+        } else if (!(r.flags & kRayTested)) {
+            // A full list, the triangles twice: the lane stops until they are tested.
+            for (uint32_t k = 0; k < kPend; ++k) {
+                s_pend[k][threadIdx.x] = (k & 1u) && (w & 3u) == 0u ? l + 1 : one;
+                s_pend[kPend + k][threadIdx.x] = 0u;
+            }
+            pend = kPend;
+            r.flags |= kRayTested;
+            return;
+        } else {
+            r.flags &= ~kRayTested;
+        }
+    }
+    const bool g0 = (w & 1u) && h0 <= r.bound, g1 = (w & 2u) && h1 <= r.bound;
     if (g0 || g1) {
         const bool sw = g1 && (!g0 || h1 < h0);  // left child wins ties (trace.h:125)
         r.word = sw ? cw.y : cw.x;
@@ -346,7 +448,7 @@ __device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, RayS
             const uint32_t far = sw ? cw.x : cw.y;
             const int sp = r.sp;
             if (sp < LDS) {
-                s_stack[sp][threadIdx.x] = far;
+                s_ray[sp][threadIdx.x] = far;
                 r.sp = sp + 1;
             } else if (sp < kStackMax) {
                 spill[sp - LDS] = far;
@@ -362,7 +464,7 @@ __device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, RayS
         return;
     }
     const int sp = r.sp - 1;
-    uint32_t next = s_stack[sp < LDS ? sp : LDS - 1][threadIdx.x];
+    uint32_t next = s_ray[sp < LDS ? sp : LDS - 1][threadIdx.x];
     asm volatile("" : "+v"(next));  // as in visit_step
     if (sp >= LDS) next = spill[sp - LDS];
     r.word = next;
@@ -370,10 +472,11 @@ __device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, RayS
 }
 
 // Tests every noted triangle of the wave, the next one's record on its way
-// while one is tested.
-template <int COLS>
+// while one is tested.  A ray that has become a tie ends its walk.
+template <int LDS, int COLS>
 __device__ __forceinline__ void test_pending(const float4* __restrict__ tris, RayState& r, uint32_t& pend,
-                                             uint32_t (*s_pend)[COLS]) {
+                                             uint32_t (*s_ray)[COLS]) {
+    uint32_t (*s_pend)[COLS] = s_ray + LDS;
     TriRec next;
     if (pend > 0u) next = load_tri(tris, s_pend[0][threadIdx.x]);
     for (uint32_t k = 0; __ballot(k < pend) != 0ull; ++k) {
@@ -382,31 +485,32 @@ __device__ __forceinline__ void test_pending(const float4* __restrict__ tris, Ra
         if (k < pend) {
             float u, v;
             const float t = tri_test(c, r.o, r.d, u, v);
-            const uint32_t id = __float_as_uint(c.p.w);
-            if (t < r.minT || (t == r.minT && id < r.best)) {
-                r.minT = t; r.best = id; r.bu = u; r.bv = v;
-            }
+            take_hit(r, t, __float_as_uint(c.p.w), u, v, __uint_as_float(s_pend[kPend + k][threadIdx.x]));
         }
     }
     pend = 0u;
+    if (r.flags & kRayTie) {
+        r.word = kInvalid;
+        r.sp = 0;
+    }
 }
 
 // One iteration of the wave's walking lanes (`busy`: the lane has a ray), with
 // the pending tests when they are due.  Returns whether the lane's ray has
-// ended.
+// ended: with kRayTie, to be started again with kRayExact.
 template <int LDS, int COLS>
 __device__ __forceinline__ bool walk_wave(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                          RayState& r, uint32_t& pend, bool busy, uint32_t (*s_stack)[COLS],
-                                          uint32_t (*s_pend)[COLS], uint32_t* spill, uint32_t* status) {
+                                          RayState& r, uint32_t& pend, bool busy, uint32_t (*s_ray)[COLS],
+                                          uint32_t* spill, uint32_t* status) {
     if (busy && r.word != kInvalid && pend <= kPend - 2u) {
-        if (r.finite) walk_step<LDS, true>(nodes, r, pend, s_stack, s_pend, spill, status);
-        else walk_step<LDS, false>(nodes, r, pend, s_stack, s_pend, spill, status);
+        if (r.finite) walk_step<LDS, true>(nodes, r, pend, s_ray, spill, status);
+        else walk_step<LDS, false>(nodes, r, pend, s_ray, spill, status);
     }
     const bool stuck = busy && ((r.word == kInvalid && pend > 0u) || pend > kPend - 2u);
     const uint64_t ns = __ballot(stuck);
     if (ns != 0ull && (static_cast<uint32_t>(__popcll(ns)) >= kFlushLanes ||
                        __ballot(busy && !stuck && r.word != kInvalid) == 0ull))
-        test_pending(tris, r, pend, s_pend);
+        test_pending<LDS>(tris, r, pend, s_ray);
     return busy && r.word == kInvalid && pend == 0u;
 }
 
@@ -420,18 +524,52 @@ __device__ __forceinline__ bool walk_wave(const float4* __restrict__ nodes, cons
 // one per lane, tests them together, and puts their surviving children back,
 // nearer ones on top of farther ones.  The chain shrinks to about a quarter
 // at 8 lanes (longest ray over a 65,536-triangle soup: 282 visits, 44 rounds).
-// The hit is the lexicographic minimum of (t, id) over the tested triangles,
-// whichever lane tests them, as it is for one lane.
 //
-// All lanes of a group hold the ray; r.minT is the group's best distance
-// (agreed on after every round that improved it), and a lane that does not
-// hold a hit at that distance has r.best = kInvalid.  The group's stack is
-// its lanes' columns of the wave's LDS stack, entry e in row e >> lg of column
-// e mod 2^lg, which for lg = 0 is the one-lane layout.  With fewer than
-// kGroupReserve free entries left the group takes one node a round, which
-// is the depth-first walk of one lane: that adds at most 63 entries, and
-// those that do not fit go to the first lane's private array.
-constexpr uint32_t kGroupReserve = 16;
+// All lanes of a group hold the ray; each keeps the best of the triangles that
+// it tested itself (group_best makes the group's hit of them at the end).  The
+// stack is in the reference's order from the top down, so what a lane finds
+// comes before the nodes of the lanes below it and before the rest of the
+// stack, but not before the nodes above: entries are (word, bound) pairs.  A
+// round lowers each lane's bound to the minimum over the lanes from it to the
+// top, gives that to the children it puts back, and the whole round's minimum to
+// the entry below the round's nodes; that entry hands it on when its turn comes.
+// (With one bound for the whole group, 27 % of rays on overlapping coplanar
+// triangles got another hit than the reference's; on soups and rooms the rounds
+// rise by 0.3 %.)  A kRayExact group takes one node a round, which is the
+// reference's walk.
+//
+// The group's stack takes its lanes' columns of the wave's LDS, stacks and leaf
+// lists together: words in the first half of the rows, bounds in the second,
+// entry e in row e >> lg of column e mod 2^lg.  (As 8-byte pairs a wave's rows
+// would overlap those of the workgroup's other waves, which may still walk.)
+// With fewer than kGroupReserve free
+// entries left the group takes one node a round, which is the depth-first walk of
+// one lane: that adds at most 63 entries, and those that do not fit go, as words,
+// to the first lane's private array.  One-node rounds pop them with the last
+// round's bound (`run`), as everything tested since they were put there comes
+// before them.
+constexpr uint32_t kGroupReserve = 2 * kPend;
+constexpr uint32_t kGroupSpill = kStackMax - kGroupReserve;
+static_assert(kGroupReserve + kGroupSpill >= 63, "a one-lane walk from a full group stack");
+template <int LDS>
+constexpr uint32_t kGroupRows = kRayRows<LDS> / 2;
+// Private entries of a lane that walks alone or in a group.
+template <int LDS>
+constexpr uint32_t kSpillMax = std::max(static_cast<uint32_t>(kStackMax - LDS), kGroupSpill);
+
+// A group's stack size, lanes per group (log2), where the last round's nodes
+// began (kInvalid: unknown) and its bound.
+struct Group {
+    uint32_t sp, lg, from;
+    float run;
+};
+
+// Whether the group can be given more lanes: its stack is in LDS, or it is a lane
+// that walked alone, with at most LDS words.
+template <int LDS>
+__device__ __forceinline__ bool group_movable(const Group& g) {
+    return g.sp <= (g.lg == 0u ? static_cast<uint32_t>(LDS) : kGroupRows<LDS> << g.lg);
+}
 
 __device__ __forceinline__ uint32_t lane_u32(uint32_t v, uint32_t src) {
     return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(src << 2), static_cast<int>(v)));
@@ -441,6 +579,56 @@ __device__ __forceinline__ float lane_f32(float v, uint32_t src) {
 }
 __device__ __forceinline__ V3 lane_v3(V3 v, uint32_t src) {
     return v3(lane_f32(v.x, src), lane_f32(v.y, src), lane_f32(v.z, src));
+}
+
+// Lane operations on rows of 16 lanes without the LDS unit's latency.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v, uint32_t old) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(old), static_cast<int>(v), CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ uint32_t bits(uint32_t v) { return v; }
+__device__ __forceinline__ uint32_t bits(float v) { return __float_as_uint(v); }
+__device__ __forceinline__ void set_bits(uint32_t& v, uint32_t b) { v = b; }
+__device__ __forceinline__ void set_bits(float& v, uint32_t b) { v = __uint_as_float(b); }
+
+// The minimum over the lane's group of 2^lg lanes, on all of them.
+template <class T, class Min>
+__device__ __forceinline__ T group_min(T x, uint32_t lg, Min min2) {
+    auto with = [&](uint32_t other) {
+        T y;
+        set_bits(y, other);
+        x = min2(x, y);
+    };
+    if (lg > 0u) with(dpp<0xB1>(bits(x), bits(x)));   // quad_perm 1,0,3,2
+    if (lg > 1u) with(dpp<0x4E>(bits(x), bits(x)));   // quad_perm 2,3,0,1
+    if (lg > 2u) with(dpp<0x141>(bits(x), bits(x)));  // row_half_mirror
+    if (lg > 3u) with(dpp<0x140>(bits(x), bits(x)));  // row_mirror
+    if (lg > 4u) with(lane_u32(bits(x), (threadIdx.x & 63u) ^ 16u));
+    if (lg > 5u) with(lane_u32(bits(x), (threadIdx.x & 63u) ^ 32u));
+    return x;
+}
+
+// The minimum over the lanes of the group from this one, its j-th, to the last.
+__device__ __forceinline__ float min_from_here(float x, uint32_t lg, uint32_t j) {
+    const uint32_t G = 1u << lg, none = __float_as_uint(__builtin_huge_valf());
+    auto with = [&](uint32_t up, uint32_t by) {
+        if (j + by < G) x = __builtin_fminf(x, __uint_as_float(up));
+    };
+    const uint32_t lane = threadIdx.x & 63u;
+    with(dpp<0x101>(__float_as_uint(x), none), 1u);  // row_shl: from the lane above
+    if (lg > 1u) with(dpp<0x102>(__float_as_uint(x), none), 2u);
+    if (lg > 2u) with(dpp<0x104>(__float_as_uint(x), none), 4u);
+    if (lg > 3u) with(dpp<0x108>(__float_as_uint(x), none), 8u);
+    // Of a larger group each row's minimum is in its first lane now.
+    if (lg > 4u) {
+        float rows = __builtin_huge_valf();
+        for (uint32_t k = 16u; k < G; k += 16u) {
+            const float row = lane_f32(x, lane - j + k);
+            if (k > j) rows = __builtin_fminf(rows, row);
+        }
+        x = __builtin_fminf(x, rows);
+    }
+    return x;
 }
 
 // The lanes of this lane's group.
@@ -457,49 +645,69 @@ __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Starts the group's ray at `root`; sp is the group's stack size.
+// A group stack's entry: word and bound.
 template <int LDS, int COLS>
-__device__ __forceinline__ void group_start(RayState& r, uint32_t root, uint32_t& sp, uint32_t lg,
-                                            uint32_t (*s_stack)[COLS]) {
-    init_ray(r, root);
-    if ((threadIdx.x & ((1u << lg) - 1u)) == 0u) s_stack[0][threadIdx.x] = root;
-    sp = 1u;
+__device__ __forceinline__ uint2 get_entry(uint32_t (*s_ray)[COLS], uint32_t row, uint32_t col) {
+    return make_uint2(s_ray[row][col], s_ray[kGroupRows<LDS> + row][col]);
+}
+template <int LDS, int COLS>
+__device__ __forceinline__ void put_entry(uint32_t (*s_ray)[COLS], uint32_t row, uint32_t col, uint32_t word, float bound) {
+    s_ray[row][col] = word;
+    s_ray[kGroupRows<LDS> + row][col] = __float_as_uint(bound);
+}
+
+// Starts the group's ray at `root`.
+template <int LDS, int COLS>
+__device__ __forceinline__ void group_start(RayState& r, uint32_t root, uint32_t flags, Group& g,
+                                            uint32_t (*s_ray)[COLS]) {
+    init_ray(r, root, flags);
+    if ((threadIdx.x & ((1u << g.lg) - 1u)) == 0u)
+        put_entry<LDS>(s_ray, 0u, threadIdx.x, root, kMinTInit);
+    g.sp = 1u;
+    g.from = kInvalid;
+    g.run = kMinTInit;
 }
 
 // One round of every group of the wave whose stack is not empty.
 template <int LDS, int COLS>
 __device__ __forceinline__ void group_round(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                            RayState& r, uint32_t& sp, uint32_t lg, uint32_t (*s_stack)[COLS],
-                                            uint32_t* spill, uint32_t* status) {
-    constexpr uint32_t kSpill = kStackMax - LDS;
+                                            RayState& r, Group& gr, uint32_t (*s_ray)[COLS], uint32_t* spill,
+                                            uint32_t* status) {
+    const uint32_t lg = gr.lg, sp = gr.sp;
     const uint32_t G = 1u << lg, j = threadIdx.x & (G - 1u), first = threadIdx.x - j;
-    const uint32_t cap = static_cast<uint32_t>(LDS) << lg;
-    const uint32_t room = sp + kGroupReserve < cap ? cap - kGroupReserve - sp : 1u;
+    const uint32_t cap = kGroupRows<LDS> << lg;
+    uint32_t (*s_bound)[COLS] = s_ray + kGroupRows<LDS>;
+    const uint32_t room =
+        !(r.flags & kRayExact) && sp + kGroupReserve < cap ? cap - kGroupReserve - sp : 1u;
     const uint32_t k = min(min(sp, G), room);
     const uint32_t base = sp - k;
     const bool mine = j < k;
-    const float before = r.minT;
+    const bool hands_on = j == 0u && base > 0u && base <= cap;  // to the entry below, base - 1
     Children c{0.0f, 0.0f, 0u, 0u};
     TraceCount cnt{0, 0, 0, 0};
+    float bound = __builtin_huge_valf(), reach = __builtin_huge_valf(), below = 0.0f;
     wave_fence();
+    if (hands_on) below = __uint_as_float(s_bound[(base - 1u) >> lg][first + ((base - 1u) & (G - 1u))]);
     if (mine) {
         const uint32_t e = base + j;
-        uint32_t word = s_stack[e < cap ? e >> lg : 0u][first + (e & (G - 1u))];
+        const uint2 pair = get_entry<LDS>(s_ray, e < cap ? e >> lg : 0u, first + (e & (G - 1u)));
+        uint32_t word = pair.x;
         asm volatile("" : "+v"(word));  // keeps the LDS and scratch reads apart, as in visit_step
-        if (e >= cap) word = spill[min(e - cap, kSpill - 1u)];
-        r.word = word;
-        c = r.finite ? test_children<false, true>(nodes, tris, r, cnt)
-                     : test_children<false, false>(nodes, tris, r, cnt);
-    }
-    if (__ballot(r.minT < before) != 0ull) {
-        float m = r.minT;
-        for (uint32_t x = 1; x < G; x <<= 1) m = __builtin_fminf(m, __shfl_xor(m, static_cast<int>(x), 64));
-        if (m < r.minT) {
-            r.minT = m;
-            r.best = kInvalid;
+        bound = __uint_as_float(pair.y);
+        if (e >= cap) {
+            word = spill[min(e - cap, kGroupSpill - 1u)];
+            bound = gr.run;
         }
+        r.word = word;
+        c = r.finite ? test_children<false, true, false>(nodes, tris, r, cnt, &reach)
+                     : test_children<false, false, false>(nodes, tris, r, cnt, &reach);
     }
-    const bool g0 = mine && (r.word & 1u) && c.h0 <= r.minT, g1 = mine && (r.word & 2u) && c.h1 <= r.minT;
+    // Bounds of a round's nodes fall from the top down already unless one of them
+    // found a hit or lies below the entry that the last round's minimum went to.
+    const bool scan = __ballot((mine && reach < bound) || (mine && base + 1u < gr.from)) != 0ull;
+    bound = __builtin_fminf(bound, reach);
+    if (scan) bound = min_from_here(bound, lg, j);
+    const bool g0 = mine && (r.word & 1u) && c.h0 <= bound, g1 = mine && (r.word & 2u) && c.h1 <= bound;
     const uint64_t gm = group_mask(lg), lt = (1ull << (threadIdx.x & 63u)) - 1ull;
     const uint64_t any = __ballot(g0 || g1) & gm, both = __ballot(g0 && g1) & gm;
     if (g0 || g1) {
@@ -507,9 +715,13 @@ __device__ __forceinline__ void group_round(const float4* __restrict__ nodes, co
         const bool sw = g1 && (!g0 || c.h1 < c.h0);  // left child wins ties (trace.h:125)
         const uint32_t near_w = sw ? c.w1 : c.w0, far_w = sw ? c.w0 : c.w1;
         auto put = [&](uint32_t e, uint32_t w) {
-            if (e < cap) s_stack[e >> lg][first + (e & (G - 1u))] = w;
-            else if (e - cap < kSpill) spill[e - cap] = w;
-            else raise_status(status, kStatusStackOverflow);
+            if (e < cap) {
+                put_entry<LDS>(s_ray, e >> lg, first + (e & (G - 1u)), w, bound);
+            } else if (e - cap < kGroupSpill) {
+                spill[e - cap] = w;
+            } else {
+                raise_status(status, kStatusStackOverflow);
+            }
         };
         if (g0 && g1) {
             put(p, far_w);
@@ -518,63 +730,97 @@ __device__ __forceinline__ void group_round(const float4* __restrict__ nodes, co
             put(p, near_w);
         }
     }
-    sp = base + static_cast<uint32_t>(__popcll(any) + __popcll(both));
+    if (hands_on && bound < below)
+        s_bound[(base - 1u) >> lg][first + ((base - 1u) & (G - 1u))] = __float_as_uint(bound);
+    gr.sp = base + static_cast<uint32_t>(__popcll(any) + __popcll(both));
+    gr.from = base;
+    gr.run = bound;
+    // A tie ends the group's walk (group_best reports it).
+    if (__ballot((r.flags & kRayTie) != 0u) & gm) gr.sp = 0u;
 }
 
-// The group's hit on all its lanes (lowest id at the best distance).
-__device__ __forceinline__ void group_best(RayState& r, uint32_t lg) {
-    uint32_t id = r.best;
-    for (uint32_t x = 1; x < (1u << lg); x <<= 1)
-        id = min(id, static_cast<uint32_t>(__shfl_xor(static_cast<int>(id), static_cast<int>(x), 64)));
-    const uint64_t who = __ballot(r.best == id) & group_mask(lg);
+// The group's hit on all its lanes (lowest id at the best distance).  Returns
+// whether it is a tie.
+__device__ __forceinline__ bool group_best(RayState& r, uint32_t lg) {
+    const float t = group_min(r.minT, lg, [](float a, float b) { return __builtin_fminf(a, b); });
+    const uint32_t id = group_min(r.minT == t ? r.best : kInvalid, lg, [](uint32_t a, uint32_t b) { return min(a, b); });
+    const uint64_t gm = group_mask(lg);
+    const uint64_t who = __ballot(r.minT == t && r.best == id) & gm;
     const uint32_t src = static_cast<uint32_t>(__builtin_ctzll(who));
+    const float reach = lane_f32(r.bound, src);
+    const bool other = (threadIdx.x & 63u) != src && r.best != kInvalid && r.minT < reach;
+    const bool tie = (__ballot(other || (r.flags & kRayTie) != 0u) & gm) != 0ull;
+    r.minT = t;
     r.best = id;
     r.bu = lane_f32(r.bu, src);
     r.bv = lane_f32(r.bv, src);
+    return tie;
 }
 
 // Regroups the wave: the groups named by `act` (their first lanes; at most 32)
-// become groups of 2^lgn lanes, in order.  Every named group's stack fits its
-// LDS columns (sp <= LDS << lg).  Returns the first lane of the group this
-// lane's new group was, or 64 when there is none for it; the caller moves its
-// own per-ray values from that lane.
+// become groups of 2^lgn lanes, in order.  Every named group is movable (a lane
+// that walked alone has no bounds in its stack: all that it tested comes before
+// all of it).  Returns the first lane of the group this lane's new group was, or 64 when there is none
+// for it; the caller moves its own per-ray values from that lane.
 template <int LDS, int COLS>
-__device__ __forceinline__ uint32_t regroup(RayState& r, uint32_t& sp, uint32_t& lg, uint32_t lgn, uint64_t act,
-                                            uint32_t (*s_stack)[COLS]) {
+__device__ __forceinline__ uint32_t regroup(RayState& r, Group& g, uint32_t lgn, uint64_t act,
+                                            uint32_t (*s_ray)[COLS]) {
+    constexpr uint32_t R = kGroupRows<LDS>;
+    const uint32_t lg = g.lg;
     const uint32_t lane = threadIdx.x & 63u, wcol = threadIdx.x - lane;
     const uint32_t gn = lane >> lgn, jn = lane & ((1u << lgn) - 1u);
     uint32_t own = 64u, i = 0u;
     for (uint64_t m = act; m != 0ull; m &= m - 1ull, ++i)
         if (gn == i) own = static_cast<uint32_t>(__builtin_ctzll(m));
     const uint32_t src = own < 64u ? own : lane;
-    const uint32_t moved = lane_u32(sp, src);
+    const uint32_t moved = lane_u32(g.sp, src);
     const uint32_t n = own < 64u ? moved : 0u;
-    constexpr int kMove = LDS / 2;  // entries per new lane: LDS << lg over at least 2 << lg lanes
-    uint32_t ent[kMove];
-    wave_fence();
+    const float alone = lane_f32(r.bound, src);
+    // A new lane gets at most M of the entries: LDS words, or R << lg pairs, over
+    // at least 2 << lg lanes.
+    auto move = [&](auto& ent, auto read, auto word, auto bound) {
+        constexpr int M = sizeof ent / sizeof ent[0];
+        static_assert(M <= static_cast<int>(R), "the entries fit");
+        wave_fence();
 #pragma unroll
-    for (int q = 0; q < kMove; ++q) {
-        const uint32_t e = jn + (static_cast<uint32_t>(q) << lgn);
-        ent[q] = e < n ? s_stack[e >> lg][wcol + src + (e & ((1u << lg) - 1u))] : 0u;
+        for (int q = 0; q < M; ++q) {
+            const uint32_t e = jn + (static_cast<uint32_t>(q) << lgn);
+            if (e < n) ent[q] = read(e);
+        }
+        wave_fence();
+#pragma unroll
+        for (int q = 0; q < M; ++q)
+            if (jn + (static_cast<uint32_t>(q) << lgn) < n) put_entry<LDS>(s_ray, q, threadIdx.x, word(ent[q]), bound(ent[q]));
+        wave_fence();
+    };
+    if (lg == 0u) {
+        uint32_t ent[LDS / 2];
+        move(ent, [&](uint32_t e) { return s_ray[e][wcol + src]; }, [](uint32_t w) { return w; }, [&](uint32_t) { return alone; });
+    } else {
+        uint2 ent[R / 2];
+        move(ent, [&](uint32_t e) { return get_entry<LDS>(s_ray, e >> lg, wcol + src + (e & ((1u << lg) - 1u))); },
+             [](uint2 p) { return p.x; }, [](uint2 p) { return __uint_as_float(p.y); });
     }
-    wave_fence();
-#pragma unroll
-    for (int q = 0; q < kMove; ++q)
-        if (jn + (static_cast<uint32_t>(q) << lgn) < n) s_stack[q][threadIdx.x] = ent[q];
-    wave_fence();
     // A lane's own best goes with it; the group's further lanes hold none.
-    const uint32_t bsrc = jn < (1u << lg) ? src + jn : src;
+    const uint32_t bsrc = own < 64u ? (jn < (1u << lg) ? src + jn : src) : lane;
     r.o = lane_v3(r.o, src);
     r.d = lane_v3(r.d, src);
     r.dinv = lane_v3(r.dinv, src);
     r.finite = lane_u32(r.finite ? 1u : 0u, src) != 0u;
-    r.minT = lane_f32(r.minT, src);
-    r.best = lane_u32(r.best, own < 64u ? bsrc : lane);
-    r.bu = lane_f32(r.bu, own < 64u ? bsrc : lane);
-    r.bv = lane_f32(r.bv, own < 64u ? bsrc : lane);
-    if (jn >= (1u << lg)) r.best = kInvalid;
-    sp = n;
-    lg = lgn;
+    r.minT = lane_f32(r.minT, bsrc);
+    r.best = lane_u32(r.best, bsrc);
+    r.bu = lane_f32(r.bu, bsrc);
+    r.bv = lane_f32(r.bv, bsrc);
+    r.bound = lane_f32(r.bound, bsrc);
+    r.flags = lane_u32(r.flags, bsrc);
+    if (jn >= (1u << lg)) {
+        r.minT = r.bound = kMinTInit;
+        r.best = kInvalid;
+        r.flags &= kRayExact;
+    }
+    g.sp = n;
+    g.lg = lgn;
+    g.from = kInvalid;
     return own;
 }
 
@@ -583,32 +829,38 @@ __device__ __forceinline__ uint32_t group_log(uint32_t count) {
     return count <= 1u ? 6u : 5u - (31u - static_cast<uint32_t>(__builtin_clz(count - 1u)));
 }
 
-// Traces the wave's groups to their ends: `active` groups with stack size sp
-// (sp <= LDS << lg), the ray's index in `ray` (equal on all lanes of a
-// group).  Once half the groups have ended the rest are given their lanes.
-template <int LDS, int COLS, class Store>
+// Traces the wave's groups to their ends: `active` groups (stacks in LDS), the
+// ray's index in `ray` (equal on all lanes of a group).  Once half the groups
+// have ended the rest are given their lanes.
+template <int LDS, int COLS, class Load, class Store>
 __device__ __forceinline__ void group_trace(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                            RayState& r, uint32_t sp, uint32_t lg, bool active, uint32_t ray,
-                                            uint32_t (*s_stack)[COLS], uint32_t* spill, uint32_t* status,
+                                            RayState& r, Group& g, bool active, uint32_t ray,
+                                            uint32_t (*s_ray)[COLS], uint32_t* spill, uint32_t* status, Load load,
                                             Store store) {
     for (;;) {
-        const bool lead = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
+        const bool lead = (threadIdx.x & ((1u << g.lg) - 1u)) == 0u;
         const uint64_t act = __ballot(active && lead);
         if (act == 0ull) return;
         const uint32_t lgn = group_log(static_cast<uint32_t>(__popcll(act)));
-        if (lgn > lg && __ballot(active && sp > (static_cast<uint32_t>(LDS) << lg)) == 0ull) {
-            const uint32_t own = regroup<LDS>(r, sp, lg, lgn, act, s_stack);
+        if (lgn > g.lg && __ballot(active && !group_movable<LDS>(g)) == 0ull) {
+            const uint32_t own = regroup<LDS>(r, g, lgn, act, s_ray);
             ray = lane_u32(ray, own & 63u);
             active = own < 64u;
         }
-        group_round<LDS>(nodes, tris, r, sp, lg, s_stack, spill, status);
-        const bool ended = active && sp == 0u;
+        group_round<LDS>(nodes, tris, r, g, s_ray, spill, status);
+        const bool ended = active && g.sp == 0u;
         if (__ballot(ended) != 0ull) {
             RayState f = r;
-            group_best(f, lg);
+            const bool tie = group_best(f, g.lg);
             if (ended) {
-                if ((threadIdx.x & ((1u << lg) - 1u)) == 0u) store(ray, final_hit(f));
-                active = false;
+                if (tie) {
+                    V3 o, d;
+                    uint32_t single;
+                    group_start<LDS>(r, load(ray, o, d, single), kRayExact, g, s_ray);
+                } else {
+                    if ((threadIdx.x & ((1u << g.lg) - 1u)) == 0u) store(ray, final_hit(f));
+                    active = false;
+                }
             }
         }
     }
@@ -622,39 +874,40 @@ __device__ __forceinline__ void group_trace(const float4* __restrict__ nodes, co
 constexpr uint32_t kTailLanes = 32;
 static_assert(kTailLanes <= 32, "regroup takes at most 32 groups");
 
-template <int LDS, int COLS, class Store>
+template <int LDS, int COLS, class Load, class Store>
 __device__ __forceinline__ void group_tail(const float4* __restrict__ nodes, const float4* __restrict__ tris,
                                            RayState& r, uint32_t pend, bool active, uint32_t ray,
-                                           uint32_t (*s_stack)[COLS], uint32_t (*s_pend)[COLS], uint32_t* spill,
-                                           uint32_t* status, Store store) {
-    test_pending(tris, r, pend, s_pend);
+                                           uint32_t (*s_ray)[COLS], uint32_t* spill, uint32_t* status, Load load,
+                                           Store store) {
+    test_pending<LDS>(tris, r, pend, s_ray);
+    if (active && (r.flags & kRayTie)) {
+        V3 o, d;
+        uint32_t single;
+        init_ray(r, load(ray, o, d, single), kRayExact);
+    }
+    r.flags &= ~kRayTested;  // the group visits the node anew
     const bool walking = active && r.word != kInvalid;
-    if (walking) s_stack[r.sp][threadIdx.x] = r.word;
+    if (walking) s_ray[r.sp][threadIdx.x] = r.word;
     if (active && !walking) store(ray, final_hit(r));
-    group_trace<LDS>(nodes, tris, r, walking ? static_cast<uint32_t>(r.sp) + 1u : 0u, 0u, walking, ray, s_stack, spill,
-                     status, store);
+    Group g{walking ? static_cast<uint32_t>(r.sp) + 1u : 0u, 0u, kInvalid, kMinTInit};
+    group_trace<LDS>(nodes, tris, r, g, walking, ray, s_ray, spill, status, load, store);
 }
 
 // A launch of few rays: wave w traces rays [w << (6 - lg), ...) with 2^lg lanes
 // each from the start, without a queue.
 template <int LDS, int COLS, class Load, class Store>
 __device__ __forceinline__ void grouped_trace(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                              uint32_t nrays, uint32_t lg, uint32_t* status,
-                                              uint32_t (*s_stack)[COLS], Load load, Store store) {
-    uint32_t spill[kStackMax - LDS];
+                                              uint32_t nrays, uint32_t lg, uint32_t flags, uint32_t* status,
+                                              uint32_t (*s_ray)[COLS], Load load, Store store) {
+    uint32_t spill[kSpillMax<LDS>];
     keep_in_memory(spill);
     const uint32_t ray = (blockIdx.x * static_cast<uint32_t>(COLS) + threadIdx.x) >> lg;
     const bool lead = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
     RayState r;
-    r.o = r.d = r.dinv = v3(0.0f, 0.0f, 0.0f);
-    r.finite = true;
-    r.minT = kMinTInit;
-    r.best = kInvalid;
-    r.bu = r.bv = 0.0f;
-    r.word = 0u;
-    r.sp = 0;
+    r.o = r.d = v3(0.0f, 0.0f, 0.0f);
+    init_ray(r, 0u, 0u);
+    Group g{0u, lg, kInvalid, kMinTInit};
     bool active = false;
-    uint32_t sp = 0u;
     if (ray < nrays) {
         uint32_t single = kInvalid;
         const uint32_t root = load(ray, r.o, r.d, single);
@@ -663,11 +916,11 @@ __device__ __forceinline__ void grouped_trace(const float4* __restrict__ nodes, 
             const TraceHit h = trace_single<false>(tris, single, r.o, r.d, cnt);
             if (lead) store(ray, h);
         } else {
-            group_start<LDS>(r, root, sp, lg, s_stack);
+            group_start<LDS>(r, root, flags, g, s_ray);
             active = true;
         }
     }
-    group_trace<LDS>(nodes, tris, r, sp, lg, active, ray, s_stack, spill, status, store);
+    group_trace<LDS>(nodes, tris, r, g, active, ray, s_ray, spill, status, load, store);
 }
 
 // Lanes per ray (log2) of a launch of `nrays` rays on `lanes` lanes: as many as
@@ -753,9 +1006,8 @@ template <bool COUNT, int LDS, class Load, class Store>
 __device__ __forceinline__ void persistent_trace(const float4* __restrict__ nodes,
                                                  const float4* __restrict__ tris, uint32_t nrays,
                                                  uint32_t* __restrict__ queue, uint32_t* status,
-                                                 uint32_t refill, uint32_t pool_large,
-                                                 uint32_t (*s_stack)[kPersistThreads],
-                                                 uint32_t (*s_pend)[kPersistThreads], Load load, Store store,
+                                                 uint32_t refill, uint32_t pool_large, uint32_t flags,
+                                                 uint32_t (*s_ray)[kPersistThreads], Load load, Store store,
                                                  TraceCount& cnt) {
     // Waves past one per kRayPoolSmall rays leave at once: every wave that
     // stays drains the queue with the others, and on a short queue (a late
@@ -763,7 +1015,7 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
     // only add returning atomics on its few slice counters.
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     if (wave_id > 0u && static_cast<uint64_t>(wave_id) * kRayPoolSmall >= nrays) return;
-    uint32_t spill[kStackMax - LDS];
+    uint32_t spill[kSpillMax<LDS>];
     keep_in_memory(spill);
     const int lane = threadIdx.x & 63;
     const uint64_t lt = (1ull << lane) - 1ull;
@@ -818,7 +1070,7 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
                     if (root == kInvalid) {
                         store(ray, trace_single<COUNT>(tris, single, r.o, r.d, cnt));
                     } else {
-                        init_ray(r, root);
+                        init_ray(r, root, flags);
                         active = true;
                     }
                 }
@@ -857,20 +1109,26 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
             const uint64_t left = __ballot(active);
             if (left == 0ull) break;
             if (!COUNT && static_cast<uint32_t>(__popcll(left)) <= kTailLanes && __ballot(active && r.sp >= LDS) == 0ull) {
-                group_tail<LDS>(nodes, tris, r, pend, active, ray, s_stack, s_pend, spill, status, store);
+                group_tail<LDS>(nodes, tris, r, pend, active, ray, s_ray, spill, status, load, store);
                 break;
             }
         }
         bool ended;
         if constexpr (COUNT) {  // the reference's order of visits and tests, which the counts describe
-            ended = active && !(r.finite ? visit_step<true, LDS, true>(nodes, tris, r, s_stack, spill, cnt, status)
-                                         : visit_step<true, LDS, false>(nodes, tris, r, s_stack, spill, cnt, status));
+            ended = active && !(r.finite ? visit_step<true, LDS, true>(nodes, tris, r, s_ray, spill, cnt, status)
+                                         : visit_step<true, LDS, false>(nodes, tris, r, s_ray, spill, cnt, status));
         } else {
-            ended = walk_wave<LDS>(nodes, tris, r, pend, active, s_stack, s_pend, spill, status);
+            ended = walk_wave<LDS>(nodes, tris, r, pend, active, s_ray, spill, status);
         }
         if (ended) {
-            store(ray, final_hit(r));
-            active = false;
+            if (r.flags & kRayTie) {
+                V3 o, d;
+                uint32_t single;
+                init_ray(r, load(ray, o, d, single), kRayExact);
+            } else {
+                store(ray, final_hit(r));
+                active = false;
+            }
         }
     }
 }
@@ -919,13 +1177,12 @@ template <int LDS, class Load, class Store>
 __device__ __forceinline__ void persistent_trace_filtered(const float4* __restrict__ nodes,
                                                           const float4* __restrict__ tris, uint32_t nrays,
                                                           uint32_t* __restrict__ queue, uint32_t* status,
-                                                          uint32_t refill, uint32_t pool_large,
-                                                          uint32_t (*s_stack)[kPersistThreads],
-                                                          uint32_t (*s_pend)[kPersistThreads],
+                                                          uint32_t refill, uint32_t pool_large, uint32_t flags,
+                                                          uint32_t (*s_ray)[kPersistThreads],
                                                           uint32_t* __restrict__ s_surv, Load load, Store store) {
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u);
     if (wave_id > 0u && static_cast<uint64_t>(wave_id) * kRayPoolSmall >= nrays) return;
-    uint32_t spill[kStackMax - LDS];
+    uint32_t spill[kSpillMax<LDS>];
     keep_in_memory(spill);
     TraceCount cnt{0, 0, 0, 0};
     const int lane = threadIdx.x & 63;
@@ -992,7 +1249,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
                     if (root == kInvalid) {
                         store(fr, trace_single<false>(tris, single, f.o, f.d, cnt));
                     } else {
-                        init_ray(f, root);
+                        init_ray(f, root, flags);
                         surv = f.finite ? root_visit<true>(nodes, tris, f) : root_visit<false>(nodes, tris, f);
                         if (!surv) store(fr, final_hit(f));
                     }
@@ -1012,7 +1269,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
                 ray = s_surv[(qhead + rank) & (kSurvCap - 1u)];
                 uint32_t single = kInvalid;
                 const uint32_t root = load(ray, r.o, r.d, single);
-                init_ray(r, root);
+                init_ray(r, root, flags);
                 active = true;
             }
             qhead += min(static_cast<uint32_t>(__popcll(idle)), qn);
@@ -1021,13 +1278,19 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
             const uint64_t left = __ballot(active);
             if (left == 0ull) break;
             if (static_cast<uint32_t>(__popcll(left)) <= kTailLanes && __ballot(active && r.sp >= LDS) == 0ull) {
-                group_tail<LDS>(nodes, tris, r, pend, active, ray, s_stack, s_pend, spill, status, store);
+                group_tail<LDS>(nodes, tris, r, pend, active, ray, s_ray, spill, status, load, store);
                 break;
             }
         }
-        if (walk_wave<LDS>(nodes, tris, r, pend, active, s_stack, s_pend, spill, status)) {
-            store(ray, final_hit(r));
-            active = false;
+        if (walk_wave<LDS>(nodes, tris, r, pend, active, s_ray, spill, status)) {
+            if (r.flags & kRayTie) {
+                V3 o, d;
+                uint32_t single;
+                init_ray(r, load(ray, o, d, single), kRayExact);
+            } else {
+                store(ray, final_hit(r));
+                active = false;
+            }
         }
     }
 }
