@@ -668,10 +668,13 @@ __device__ __forceinline__ void answer_single(const FrameConst& fc, const PassPa
     r.flags = 0u;
 }
 
-// At most 96 VGPRs (5 waves per SIMD): the plain and the cache variants fit
+// Without lights at most 96 VGPRs (5 waves per SIMD), which these variants fit
 // without spilling.  At 80 (6 waves) they spill inside the visit, and a
 // 1,024 x 1,024 frame of the 871,200-triangle room took 7.2 ms for 2.9; at 4
-// waves it took the same as at 5.
+// waves it took the same as at 5.  With lights, whose shadow rays are walked
+// within the shading, at most 128 (4 waves): at 96 they spill 63-128 registers,
+// and a 16-pass 637 x 359 textured frame under two lights took 2.14 ms for 1.65, a
+// lit cache frame of 1,920 x 1,080 in a 20,000-triangle soup 2.29 for 1.89.
 // CACHE: a cache frame (one pass).  Its pixel paths (pixel = path) end in the
 // cache at their second hit (record_cache_vertex) with their throughput in
 // ps.ar/ag/ab, its training paths (path npix + key) after train_levels - 1
@@ -688,7 +691,7 @@ __device__ __forceinline__ void answer_single(const FrameConst& fc, const PassPa
 // go on as groups: a frame lasts as long as its longest path's chain of
 // visits, which the groups shorten (traverse.hpp).
 template <int LDS, bool LIGHTS, bool DETAIL, bool CACHE>
-__global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst fc, const PassParams* __restrict__ pp,
+__global__ __launch_bounds__(kPersistThreads, LIGHTS ? 4 : 5) void k_paths(const FrameConst fc, const PassParams* __restrict__ pp,
                                                            const pt_triangle_info* __restrict__ infos,
                                                            const float4* __restrict__ nodes,
                                                            const float4* __restrict__ tris,
@@ -850,7 +853,6 @@ __global__ __launch_bounds__(kPersistThreads, 5) void k_paths(const FrameConst f
                             answer_single<CACHE>(fc, pp, off, tris, path, r);
                         } else {
                             if (r.flags & kRayTie) init_ray(r, root, kRayExact);
-                            r.flags &= ~kRayTested;  // the group visits the node anew
                             if (r.word != kInvalid) {
                                 s_ray[r.sp][tid] = r.word;
                                 g.sp = static_cast<uint32_t>(r.sp) + 1u;

@@ -173,9 +173,8 @@ struct RayState {
     bool finite;
 };
 enum : uint32_t {
-    kRayExact = 1u,   // walks in the reference's order
-    kRayTested = 2u,  // ... and the current node's leaf children are tested
-    kRayTie = 4u,     // the hit may depend on the order: to be walked again with kRayExact
+    kRayExact = 1u,  // walks in the reference's order
+    kRayTie = 2u,    // the hit may depend on the order: to be walked again with kRayExact
 };
 
 __device__ __forceinline__ void init_ray(RayState& r, uint32_t root, uint32_t flags) {
@@ -223,18 +222,29 @@ __device__ __forceinline__ void init_ray(RayState& r, uint32_t root, uint32_t fl
 //    dinv component is a tie when one arises, and where a triangle's box is NaN
 //    (strict, from the build) every ray walks in the reference's order.
 
+// Minimum and maximum of distances that are no NaN and no less than zero (the
+// maximum also of -0 and, with another that is not, negative ones): of their
+// bits, without the canonicalizing instructions of fminf and fmaxf.
+__device__ __forceinline__ float near_of(float a, float b) {
+    return __int_as_float(min(__float_as_int(a), __float_as_int(b)));
+}
+__device__ __forceinline__ float far_of(float a, float b) {
+    return __int_as_float(max(__float_as_int(a), __float_as_int(b)));
+}
+
 // One tested triangle: its distance t (+inf: missed) and the h of its own box
 // (0 for kRayExact rays, whose bound is the best distance itself).  Returns
-// max(t, h).
+// max(t, h, 0) (t is no less than zero).
 __device__ __forceinline__ float take_hit(RayState& r, float t, uint32_t id, float u, float v, float h) {
-    const float c = __builtin_fmaxf(t, h);
-    const bool better = t < r.minT || (t == r.minT && id < r.best);
-    const float other = __builtin_fmaxf(t, r.minT);  // of the two, not the best
-    r.bound = better ? c : r.bound;  // lower, unless it is a tie
-    if (better) {
-        r.minT = t; r.best = id; r.bu = u; r.bv = v;
-    }
-    if (other < r.bound) r.flags |= kRayTie;
+    const float c = far_of(far_of(t, h), 0.0f);
+    const bool better = (t < r.minT) | ((t == r.minT) & (id < r.best));
+    const float other = far_of(t, r.minT);  // of the two, not the best
+    r.bound = better ? c : r.bound;         // lower, unless it is a tie
+    r.minT = better ? t : r.minT;
+    r.best = better ? id : r.best;
+    r.bu = better ? u : r.bu;
+    r.bv = better ? v : r.bv;
+    r.flags |= other < r.bound ? kRayTie : 0u;
     return c;
 }
 
@@ -286,7 +296,7 @@ __device__ __forceinline__ Children test_children(const float4* __restrict__ nod
     const uint32_t l = w >> 2;
     const float4* rec = nodes + 4 * static_cast<size_t>(l);
     const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
-    const uint2 cw = *reinterpret_cast<const uint2*>(rec + 3);
+    const float4 r3 = rec[3];
     // The first leaf child (the left one unless it is internal), and the
     // second of a node with two.
     TriRec ta, tb;
@@ -298,8 +308,8 @@ __device__ __forceinline__ Children test_children(const float4* __restrict__ nod
     Children c;
     c.h0 = child_box<COUNT, FINITE>(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
     c.h1 = child_box<COUNT, FINITE>(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
-    c.w0 = cw.x;
-    c.w1 = cw.y;
+    c.w0 = __float_as_uint(r3.x);
+    c.w1 = __float_as_uint(r3.y);
     if (COUNT) cnt.boxes += (w & 1u) + ((w >> 1) & 1u);
     if constexpr (!ORDERED && !FINITE) {
         if (!(r.flags & kRayExact) && (slab_nan(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y) ||
@@ -308,16 +318,18 @@ __device__ __forceinline__ Children test_children(const float4* __restrict__ nod
     }
     // An opaque copy of the word: with the same condition as above the
     // compiler would merge the two branches and issue the triangle loads
-    // only after the box tests, a second memory round trip.
+    // only after the box tests, a second memory round trip.  The record's unused
+    // words stay alive up to here too: as registers of a load on its way they
+    // would be taken for the triangles' addresses, which then wait for it.
     uint32_t wt = w;
-    asm volatile("" : "+v"(wt));
+    asm volatile("" : "+v"(wt) : "v"(r3.z), "v"(r3.w));
     if ((wt & 3u) != 3u) {
         float u, v;
         const float t = tri_test(ta, r.o, r.d, u, v);
         const uint32_t id = __float_as_uint(ta.p.w);
         if (COUNT) cnt.tris++;
         if constexpr (!ORDERED) {
-            *reach = __builtin_fminf(*reach, take_hit(r, t, id, u, v, (r.flags & kRayExact) ? 0.0f : ((wt & 1u) ? c.h1 : c.h0)));
+            *reach = near_of(*reach, take_hit(r, t, id, u, v, (r.flags & kRayExact) ? 0.0f : ((wt & 1u) ? c.h1 : c.h0)));
         } else if (t < r.minT || (t == r.minT && id < r.best)) {
             r.minT = t; r.best = id; r.bu = u; r.bv = v;
         }
@@ -327,7 +339,7 @@ __device__ __forceinline__ Children test_children(const float4* __restrict__ nod
             const uint32_t id2 = __float_as_uint(tb.p.w);
             if (COUNT) cnt.tris++;
             if constexpr (!ORDERED) {
-                *reach = __builtin_fminf(*reach, take_hit(r, t2, id2, u2, v2, (r.flags & kRayExact) ? 0.0f : c.h1));
+                *reach = near_of(*reach, take_hit(r, t2, id2, u2, v2, (r.flags & kRayExact) ? 0.0f : c.h1));
             } else if (t2 < r.minT || (t2 == r.minT && id2 < r.best)) {
                 r.minT = t2; r.best = id2; r.bu = u2; r.bv = v2;
             }
@@ -387,9 +399,8 @@ __device__ __forceinline__ bool visit_step(const float4* __restrict__ nodes,
 // walks on; the wave tests all noted triangles together (test_pending) once
 // kFlushLanes lanes cannot go on -- list full, or nothing left to walk -- or no
 // lane can.  The bound shrinks a few visits later, so a ray visits somewhat more
-// nodes; its hit is the reference's (see above).  A kRayExact lane cannot go on
-// while it has noted triangles, and culls the other child of their node only
-// after they are tested.
+// nodes; its hit is the reference's (see above).  A kRayExact lane tests leaf
+// children at once.
 // Measured (us; 16M shell rays on the 871,200-triangle mesh, 2M camera rays on
 // the 2.88M-triangle hair ball, two 1,024 x 1,024 room frames): tests at once
 // 897, 1,464, 5,790; four entries and 6 / 12 / 20 / 32 lanes 877 / 863 / 868 /
@@ -402,8 +413,9 @@ template <int LDS>
 constexpr int kRayRows = LDS + 2 * static_cast<int>(kPend);
 
 template <int LDS, bool FINITE, int COLS>
-__device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, RayState& r, uint32_t& pend,
-                                          uint32_t (*s_ray)[COLS], uint32_t* spill, uint32_t* status) {
+__device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, const float4* __restrict__ tris,
+                                          RayState& r, uint32_t& pend, uint32_t (*s_ray)[COLS], uint32_t* spill,
+                                          uint32_t* status) {
     const uint32_t w = r.word;
     const uint32_t l = w >> 2;
     const float4* rec = nodes + 4 * static_cast<size_t>(l);
@@ -417,27 +429,23 @@ __device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, RayS
             r.flags |= kRayTie;
     }
     if ((w & 3u) != 3u) {
-        uint32_t (*s_pend)[COLS] = s_ray + LDS;
-        const uint32_t one = (w & 1u) ? l + 1 : l;
-        if (!(r.flags & kRayExact)) {
-            s_pend[pend][threadIdx.x] = one;
+        if (r.flags & kRayExact) {
+#pragma unroll 1
+            for (uint32_t k = w & 1u; k <= (~w & 2u) >> 1; ++k) {
+                const TriRec c = load_tri(tris, l + k);
+                float u, v;
+                const float t = tri_test(c, r.o, r.d, u, v);
+                take_hit(r, t, __float_as_uint(c.p.w), u, v, 0.0f);
+            }
+        } else {
+            uint32_t (*s_pend)[COLS] = s_ray + LDS;
+            s_pend[pend][threadIdx.x] = (w & 1u) ? l + 1 : l;
             s_pend[kPend + pend][threadIdx.x] = __float_as_uint((w & 1u) ? h1 : h0);
             if ((w & 3u) == 0u) {
                 s_pend[pend + 1u][threadIdx.x] = l + 1;
                 s_pend[kPend + pend + 1u][threadIdx.x] = __float_as_uint(h1);
             }
             pend += (w & 3u) == 0u ? 2u : 1u;
-        } else if (!(r.flags & kRayTested)) {
-            // A full list, the triangles twice: the lane stops until they are tested.
-            for (uint32_t k = 0; k < kPend; ++k) {
-                s_pend[k][threadIdx.x] = (k & 1u) && (w & 3u) == 0u ? l + 1 : one;
-                s_pend[kPend + k][threadIdx.x] = 0u;
-            }
-            pend = kPend;
-            r.flags |= kRayTested;
-            return;
-        } else {
-            r.flags &= ~kRayTested;
         }
     }
     const bool g0 = (w & 1u) && h0 <= r.bound, g1 = (w & 2u) && h1 <= r.bound;
@@ -477,12 +485,14 @@ template <int LDS, int COLS>
 __device__ __forceinline__ void test_pending(const float4* __restrict__ tris, RayState& r, uint32_t& pend,
                                              uint32_t (*s_ray)[COLS]) {
     uint32_t (*s_pend)[COLS] = s_ray + LDS;
-    TriRec next;
-    if (pend > 0u) next = load_tri(tris, s_pend[0][threadIdx.x]);
-    for (uint32_t k = 0; __ballot(k < pend) != 0ull; ++k) {
-        const TriRec c = next;
-        if (k + 1u < pend) next = load_tri(tris, s_pend[k + 1u][threadIdx.x]);
+    TriRec rec[2];
+    if (pend > 0u) rec[0] = load_tri(tris, s_pend[0][threadIdx.x]);
+#pragma unroll
+    for (uint32_t k = 0; k < kPend; ++k) {
+        if (__ballot(k < pend) == 0ull) break;
+        if (k + 1u < pend) rec[(k + 1u) & 1u] = load_tri(tris, s_pend[k + 1u][threadIdx.x]);
         if (k < pend) {
+            const TriRec& c = rec[k & 1u];
             float u, v;
             const float t = tri_test(c, r.o, r.d, u, v);
             take_hit(r, t, __float_as_uint(c.p.w), u, v, __uint_as_float(s_pend[kPend + k][threadIdx.x]));
@@ -503,8 +513,8 @@ __device__ __forceinline__ bool walk_wave(const float4* __restrict__ nodes, cons
                                           RayState& r, uint32_t& pend, bool busy, uint32_t (*s_ray)[COLS],
                                           uint32_t* spill, uint32_t* status) {
     if (busy && r.word != kInvalid && pend <= kPend - 2u) {
-        if (r.finite) walk_step<LDS, true>(nodes, r, pend, s_ray, spill, status);
-        else walk_step<LDS, false>(nodes, r, pend, s_ray, spill, status);
+        if (r.finite) walk_step<LDS, true>(nodes, tris, r, pend, s_ray, spill, status);
+        else walk_step<LDS, false>(nodes, tris, r, pend, s_ray, spill, status);
     }
     const bool stuck = busy && ((r.word == kInvalid && pend > 0u) || pend > kPend - 2u);
     const uint64_t ns = __ballot(stuck);
@@ -612,7 +622,7 @@ __device__ __forceinline__ T group_min(T x, uint32_t lg, Min min2) {
 __device__ __forceinline__ float min_from_here(float x, uint32_t lg, uint32_t j) {
     const uint32_t G = 1u << lg, none = __float_as_uint(__builtin_huge_valf());
     auto with = [&](uint32_t up, uint32_t by) {
-        if (j + by < G) x = __builtin_fminf(x, __uint_as_float(up));
+        x = j + by < G ? near_of(x, __uint_as_float(up)) : x;
     };
     const uint32_t lane = threadIdx.x & 63u;
     with(dpp<0x101>(__float_as_uint(x), none), 1u);  // row_shl: from the lane above
@@ -624,9 +634,9 @@ __device__ __forceinline__ float min_from_here(float x, uint32_t lg, uint32_t j)
         float rows = __builtin_huge_valf();
         for (uint32_t k = 16u; k < G; k += 16u) {
             const float row = lane_f32(x, lane - j + k);
-            if (k > j) rows = __builtin_fminf(rows, row);
+            rows = k > j ? near_of(rows, row) : rows;
         }
-        x = __builtin_fminf(x, rows);
+        x = near_of(x, rows);
     }
     return x;
 }
@@ -685,9 +695,8 @@ __device__ __forceinline__ void group_round(const float4* __restrict__ nodes, co
     const bool hands_on = j == 0u && base > 0u && base <= cap;  // to the entry below, base - 1
     Children c{0.0f, 0.0f, 0u, 0u};
     TraceCount cnt{0, 0, 0, 0};
-    float bound = __builtin_huge_valf(), reach = __builtin_huge_valf(), below = 0.0f;
+    float bound = __builtin_huge_valf(), reach = __builtin_huge_valf();
     wave_fence();
-    if (hands_on) below = __uint_as_float(s_bound[(base - 1u) >> lg][first + ((base - 1u) & (G - 1u))]);
     if (mine) {
         const uint32_t e = base + j;
         const uint2 pair = get_entry<LDS>(s_ray, e < cap ? e >> lg : 0u, first + (e & (G - 1u)));
@@ -704,8 +713,8 @@ __device__ __forceinline__ void group_round(const float4* __restrict__ nodes, co
     }
     // Bounds of a round's nodes fall from the top down already unless one of them
     // found a hit or lies below the entry that the last round's minimum went to.
-    const bool scan = __ballot((mine && reach < bound) || (mine && base + 1u < gr.from)) != 0ull;
-    bound = __builtin_fminf(bound, reach);
+    const bool scan = __ballot(mine & ((reach < bound) | (base + 1u < gr.from))) != 0ull;
+    bound = near_of(bound, reach);
     if (scan) bound = min_from_here(bound, lg, j);
     const bool g0 = mine && (r.word & 1u) && c.h0 <= bound, g1 = mine && (r.word & 2u) && c.h1 <= bound;
     const uint64_t gm = group_mask(lg), lt = (1ull << (threadIdx.x & 63u)) - 1ull;
@@ -723,26 +732,25 @@ __device__ __forceinline__ void group_round(const float4* __restrict__ nodes, co
                 raise_status(status, kStatusStackOverflow);
             }
         };
-        if (g0 && g1) {
-            put(p, far_w);
-            put(p + 1u, near_w);
-        } else {
-            put(p, near_w);
-        }
+        put(p + (g0 && g1 ? 1u : 0u), near_w);
+        if (g0 && g1) put(p, far_w);
     }
-    if (hands_on && bound < below)
-        s_bound[(base - 1u) >> lg][first + ((base - 1u) & (G - 1u))] = __float_as_uint(bound);
+    if (hands_on) {  // near_of, in place
+        int* below = reinterpret_cast<int*>(&s_bound[(base - 1u) >> lg][first + ((base - 1u) & (G - 1u))]);
+        (void)__hip_atomic_fetch_min(below, __float_as_int(bound), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
     gr.sp = base + static_cast<uint32_t>(__popcll(any) + __popcll(both));
     gr.from = base;
     gr.run = bound;
     // A tie ends the group's walk (group_best reports it).
-    if (__ballot((r.flags & kRayTie) != 0u) & gm) gr.sp = 0u;
+    const uint64_t ties = __ballot((r.flags & kRayTie) != 0u);
+    if (ties != 0ull && (ties & gm) != 0ull) gr.sp = 0u;
 }
 
 // The group's hit on all its lanes (lowest id at the best distance).  Returns
 // whether it is a tie.
 __device__ __forceinline__ bool group_best(RayState& r, uint32_t lg) {
-    const float t = group_min(r.minT, lg, [](float a, float b) { return __builtin_fminf(a, b); });
+    const float t = group_min(r.minT, lg, [](float a, float b) { return near_of(a, b); });
     const uint32_t id = group_min(r.minT == t ? r.best : kInvalid, lg, [](uint32_t a, uint32_t b) { return min(a, b); });
     const uint64_t gm = group_mask(lg);
     const uint64_t who = __ballot(r.minT == t && r.best == id) & gm;
@@ -885,7 +893,6 @@ __device__ __forceinline__ void group_tail(const float4* __restrict__ nodes, con
         uint32_t single;
         init_ray(r, load(ray, o, d, single), kRayExact);
     }
-    r.flags &= ~kRayTested;  // the group visits the node anew
     const bool walking = active && r.word != kInvalid;
     if (walking) s_ray[r.sp][threadIdx.x] = r.word;
     if (active && !walking) store(ray, final_hit(r));
