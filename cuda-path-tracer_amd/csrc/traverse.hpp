@@ -268,7 +268,10 @@ __device__ __forceinline__ TraceHit final_hit(const RayState& r) {
 // Keeps a lane's private array of deferred nodes in scratch memory.  The
 // compiler would otherwise hold a short one (the 32 entries past a 32-entry
 // LDS stack) in vector registers: 31 of them in every lane for entries that
-// hardly any ray reaches, 4 waves per SIMD for 6.
+// hardly any ray reaches, 4 waves per SIMD for 6.  Not only for that: with the
+// array of a 32-entry LDS stack in registers (select chains over its elements)
+// the first form of the group code returned wrong hits.  Why is not known; every
+// user keeps its array in memory.
 __device__ __forceinline__ void keep_in_memory(uint32_t* spill) { asm volatile("" : : "v"(spill) : "memory"); }
 
 // What a visit finds about the node's two children: their box distances (of
@@ -425,8 +428,12 @@ __device__ __forceinline__ void walk_step(const float4* __restrict__ nodes, cons
     const float h1 = child_box<false, FINITE>(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w);
     if constexpr (!FINITE) {
         if (!(r.flags & kRayExact) && (slab_nan(r.o, r.dinv, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y) ||
-                                       slab_nan(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w)))
-            r.flags |= kRayTie;
+                                       slab_nan(r.o, r.dinv, r1.z, r1.w, r2.x, r2.y, r2.z, r2.w))) {
+            r.flags |= kRayTie;  // ends here
+            r.word = kInvalid;
+            pend = 0u;
+            return;
+        }
     }
     if ((w & 3u) != 3u) {
         if (r.flags & kRayExact) {
@@ -522,6 +529,18 @@ __device__ __forceinline__ bool walk_wave(const float4* __restrict__ nodes, cons
                        __ballot(busy && !stuck && r.word != kInvalid) == 0ull))
         test_pending<LDS>(tris, r, pend, s_ray);
     return busy && r.word == kInvalid && pend == 0u;
+}
+
+// Where many rays are ties, a wave goes over to walking all its further rays in
+// the reference's order: once kTieLimit of them were ties, counted with half the
+// weight for each pool before (64 rays or more).
+constexpr uint32_t kTieLimit = 16;
+__device__ __forceinline__ void note_ties(bool tie, uint32_t& ties, uint32_t& flags) {
+    const uint64_t tied = __ballot(tie);
+    if (tied != 0ull) {
+        ties += static_cast<uint32_t>(__popcll(tied));
+        if (ties >= kTieLimit) flags = kRayExact;
+    }
 }
 
 // ---- group traversal -------------------------------------------------------
@@ -1041,6 +1060,7 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
     // scalar registers (the compiler cannot tell that threadIdx.x / 64 is
     // uniform over a wave).
     uint32_t q = wave_id % nq;
+    uint32_t ties = 0;     // wave-uniform (note_ties)
     uint64_t seen = ~all;  // wave-uniform: slices this wave found used up
     bool used_up = false;  // wave-uniform: the refill loop found slice q used up
     for (;;) {
@@ -1065,6 +1085,7 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
                     }
                     pool_next = (base * nq + q) * pool;
                     pool_end = pool_next + min(pool, nrays - pool_next);
+                    ties >>= 1;
                 }
                 const uint32_t avail = pool_end - pool_next;
                 const uint32_t rank = static_cast<uint32_t>(__popcll(idle & lt));
@@ -1127,6 +1148,7 @@ __device__ __forceinline__ void persistent_trace(const float4* __restrict__ node
         } else {
             ended = walk_wave<LDS>(nodes, tris, r, pend, active, s_ray, spill, status);
         }
+        note_ties(ended && (r.flags & kRayTie), ties, flags);
         if (ended) {
             if (r.flags & kRayTie) {
                 V3 o, d;
@@ -1207,6 +1229,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
     const uint64_t all = nq == 64u ? ~0ull : (1ull << nq) - 1ull;
     uint64_t* mask = reinterpret_cast<uint64_t*>(queue + kQueueMask);
     uint32_t q = wave_id % nq;
+    uint32_t ties = 0;
     uint64_t seen = ~all;
     for (;;) {
         const uint32_t nbusy = static_cast<uint32_t>(__popcll(__ballot(active)));
@@ -1245,6 +1268,7 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
                     }
                     pool_next = (base * nq + q) * pool;
                     pool_end = pool_next + min(pool, nrays - pool_next);
+                    ties >>= 1;
                 }
                 const uint32_t avail = min(64u, pool_end - pool_next);
                 const uint32_t fr = pool_next + static_cast<uint32_t>(lane);
@@ -1289,7 +1313,9 @@ __device__ __forceinline__ void persistent_trace_filtered(const float4* __restri
                 break;
             }
         }
-        if (walk_wave<LDS>(nodes, tris, r, pend, active, s_ray, spill, status)) {
+        const bool ended = walk_wave<LDS>(nodes, tris, r, pend, active, s_ray, spill, status);
+        note_ties(ended && (r.flags & kRayTie), ties, flags);
+        if (ended) {
             if (r.flags & kRayTie) {
                 V3 o, d;
                 uint32_t single;
