@@ -175,7 +175,7 @@ def cache_leg(ctx, stream, args, seed_mesh):
         ctx.reset_frames()
         best, _ = autotune.tune_staged(lambda: cache_frame(0), stream,
                                        [{"render.paths": [1, 0]}, {"render.shade_min": [4, 8, 16]},
-                                        autotune.render_space(autotune.device_cus())], reps=3)
+                                        autotune.render_space(autotune.device_cus()), autotune.level_space()], reps=3)
         tuning["cache"] = best
     ctx.cache_init(7, bmin, bmax)
     cached = run(points, cache_frame, reset=lambda: ctx.cache_init(7, bmin, bmax), stop_mse=target,

@@ -1260,6 +1260,19 @@ auto cache_paths_kernel(const FrameConst& fc) {
                      : (fc.nlights ? k_paths<LDS, true, false, true> : k_paths<LDS, false, false, true>);
 }
 
+// The knobs that only one of the two frame structures reads, of a frame of that
+// one (the others stay 0, so that changing them captures no new graph).
+template <class Key>
+void set_structure_knobs(Key& key, bool path_persistent, const FrameConst& fc) {
+    if (path_persistent) {
+        key.shade_min = shade_batch(fc);
+        key.path_refill = render_tuning().refill;
+    } else {
+        key.refill = trace_tuning().refill;
+        key.pool = trace_tuning().pool;
+    }
+}
+
 // A path-persistent frame's paths, from primary rays to their radiance in ps.
 void launch_paths(const DeviceScene& scene, const FrameConst& fc, const PassParams* pp, const PathState& ps,
                   uint32_t* cnt, hipStream_t st) {
@@ -1582,13 +1595,10 @@ void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, cons
         key.counters = r.counters.as<void>();
         key.lights = scene.lights.as<void>();
         key.blocks = trace_tuning().blocks;
-        key.refill = trace_tuning().refill;
         key.lds = trace_tuning().lds;
-        key.pool = trace_tuning().pool;
         key.chains = nchains;
         key.paths = render_tuning().paths;
-        key.shade_min = shade_batch(fc);
-        key.path_refill = render_tuning().refill;
+        set_structure_knobs(key, nchains == 0, fc);
         key.stream = st;
         replay(r.graph_exec, r.graph_key, key, st,
                [&] { launch_frame(r, scene, fc, nchains, st); });
@@ -1765,12 +1775,9 @@ void render_cache_frame(Renderer& r, const DeviceScene& scene, RadianceCache& ca
         key.steps = cf.steps;
         key.train = cf.train;
         key.blocks = trace_tuning().blocks;
-        key.refill = trace_tuning().refill;
         key.lds = trace_tuning().lds;
-        key.pool = trace_tuning().pool;
         key.paths = render_tuning().paths;
-        key.shade_min = shade_batch(cf.fc);
-        key.path_refill = render_tuning().refill;
+        set_structure_knobs(key, render_tuning().paths != 0, cf.fc);
         const void* ptrs[13] = {scene.bvh.nodes.as<void>(), scene.bvh.tris.as<void>(), scene.infos.as<void>(),
                                 scene.off.as<void>(),       r.queues.as<void>(),     r.params.as<void>(),
                                 r.accum.as<void>(),         r.counters.as<void>(),   cache.master.as<void>(),

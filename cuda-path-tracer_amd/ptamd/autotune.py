@@ -55,12 +55,22 @@ def tune(run, stream, space, reps=3):
     return best, table
 
 
+class Stage(dict):
+    """A space of knobs that matter only where `when()` holds."""
+
+    def __init__(self, space, when):
+        super().__init__(space)
+        self.when = when
+
+
 def tune_staged(run, stream, stages, reps=3):
     """Coordinate search: grid-search each space of `stages` in turn, the
-    knobs of earlier stages held at their best.  Returns (best, table) over
-    all stages, like tune()."""
+    knobs of earlier stages held at their best; a Stage only where it applies.
+    Returns (best, table) over all stages, like tune()."""
     best, table = {}, []
     for space in stages:
+        if isinstance(space, Stage) and not space.when():
+            continue
         b, t = tune(run, stream, space, reps)
         best.update(b or {})
         table.extend(t)
@@ -86,22 +96,29 @@ def stack_space():
 def render_space(num_cus=256):
     """Traversal knobs for a progressive render, searched together on the
     render's own frames: its bounce rays traverse deeper than the closest-hit
-    microbench's shell rays and favour other lane and queue settings."""
+    microbench's shell rays and favour other launch shapes."""
     return {"trace.blocks": [num_cus * 6, num_cus * 8, num_cus * 12, num_cus * 16],
-            "trace.refill": [32, 48, 56, 64],
-            "trace.lds_stack": [8, 16],
-            "trace.pool": [128, 256]}
+            "trace.lds_stack": [8, 16]}
+
+
+def level_space():
+    """The closest-hit queue's knobs, which a render takes in bounce levels only
+    (path-persistent frames have render.refill and pools of their own)."""
+    return Stage({"trace.refill": [32, 48, 56, 64], "trace.pool": [128, 256]},
+                 when=lambda: tune_get("render.paths") == 0)
 
 
 def render_stages(num_cus=256):
     """Staged render search: the frame's structure first (path-persistent,
     or bounce levels in 1, 2 or 4 chains), then how many waiting lanes a
     path-persistent wave shades together and when its idle lanes take new
-    paths, then the traversal knobs, then the shade batch again."""
+    paths, then the traversal knobs (of bounce levels also the queue's), then
+    the shade batch again."""
     return [{"render.paths": [1, 0], "render.chains": [1, 2, 4]},
             {"render.shade_min": [8, 12, 16], "render.refill": [48, 60]},
             {"render.shade_lit": [32, 48, 64]},
             render_space(num_cus),
+            level_space(),
             {"render.shade_min": [4, 8, 12, 16, 24]}]
 
 

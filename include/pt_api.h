@@ -372,11 +372,15 @@ int pt_device_compute_units(int device, uint32_t* cus);
  *   "build.staged"  0 or 1: accepted, without effect (the tree's upper levels
  *                   are built one way)
  *   "trace.blocks"  persistent closest-hit workgroups (256 threads each)
- *   "trace.refill"  refill idle lanes when fewer than this many of 64 are busy
+ *   "trace.refill"  closest-hit queues and frames in bounce levels: a wave's idle
+ *                   lanes take new rays when fewer than this many of 64 are
+ *                   busy; with "trace.filter" 1 new filter rounds start below it,
+ *                   and rays that wait behind the filter already below 56.
+ *                   Launches of few rays, with several lanes each, do not read it
  *   "trace.lds_stack" traversal stack entries per lane kept in LDS (8, 16 or
  *                   32; deeper entries spill to scratch)
- *   "trace.pool"    rays a wave takes from the ray queue at a time on long
- *                   queues (64..4096)
+ *   "trace.pool"    rays a wave takes from such a queue at a time when it is long
+ *                   (64..4096)
  *   "trace.filter"  1: closest-hit batches run every ray's root visit in
  *                   converged 64-ray rounds and trace only the rays that go
  *                   deeper (fast when most rays miss the scene); 0: off
