@@ -596,8 +596,7 @@ int pt_render_pass(pt_context* ctx, int w, int h, uint64_t pass_seed) {
         hipStream_t st = ctx->stream;
         pt::render_resize(ctx->renderer, w, h, st);
         if (frames_allowed(ctx, 1) == 0) return;
-        PT_HIP(hipEventRecord(ctx->ev0, st));
-        pt::render_passes(ctx->renderer, ctx->scene, 1, nullptr, &pass_seed, nullptr, st);
+        pt::render_passes(ctx->renderer, ctx->scene, 1, nullptr, &pass_seed, nullptr, st, ctx->ev0);
         PT_HIP(hipEventRecord(ctx->ev1, st));
         ctx->renderer.timed = true;
         present(ctx);
@@ -613,8 +612,7 @@ int pt_render_passes(pt_context* ctx, int w, int h, uint32_t npasses, const floa
         pt::render_resize(ctx->renderer, w, h, st);
         const uint32_t run = npasses ? frames_allowed(ctx, npasses) : npasses;
         if (npasses && run == 0) return;
-        PT_HIP(hipEventRecord(ctx->ev0, st));
-        pt::render_passes(ctx->renderer, ctx->scene, run, dirs, seeds, scenes, st);
+        pt::render_passes(ctx->renderer, ctx->scene, run, dirs, seeds, scenes, st, ctx->ev0);
         PT_HIP(hipEventRecord(ctx->ev1, st));
         ctx->renderer.timed = true;
         present(ctx);
@@ -741,6 +739,10 @@ int pt_tune_set(const char* name, uint32_t value) {
 }
 
 int pt_tune_get(const char* name, uint32_t* value) {
+    if (name && value && std::string(name) == "render.beside") {
+        *value = pt::frames_beside();
+        return PT_OK;
+    }
     uint32_t* slot = tune_slot(name);
     if (!slot || !value) return PT_E_INVALID_ARG;
     *value = *slot;

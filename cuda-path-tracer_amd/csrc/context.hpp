@@ -303,9 +303,12 @@ RenderTuning& render_tuning();
 void render_resize(Renderer& r, int w, int h, hipStream_t stream);
 void render_reset(Renderer& r, hipStream_t stream);
 // npasses 1-spp passes in one frame; dirs = 12 floats per pass (NULL: the
-// renderer's corner rays for every pass); seeds[npasses].
+// renderer's corner rays for every pass); seeds[npasses].  `begin` is recorded
+// before the frame's first work, on the stream that does it.
 void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, const float* dirs,
-                   const uint64_t* seeds, const uint32_t* scenes, hipStream_t stream);
+                   const uint64_t* seeds, const uint32_t* scenes, hipStream_t stream, hipEvent_t begin);
+// Frames that were traced beside another so far (all renderers).
+uint32_t frames_beside();
 // Running-mean image (sum / spp as float, alpha 1) of the accumulator's
 // min(w, out_w) x min(h, out_h) corner into a device RGBA32F buffer whose rows
 // are `pitch` bytes apart.

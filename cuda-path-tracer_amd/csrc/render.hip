@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <string>
 #include <type_traits>
@@ -1485,6 +1486,8 @@ void replay(void*& exec, char (&key_store)[Cap], const Key& key, hipStream_t st,
 }  // namespace
 
 namespace {
+std::atomic<uint32_t> g_frames_beside{0};
+
 // Whether the last frame is still at work (or waits for its turn).
 bool frame_in_flight(Renderer& r) {
     if (!r.frame_sent) return false;
@@ -1513,6 +1516,8 @@ Renderer::FrameSlot* take_slot(Renderer& r, size_t npaths) {
 }
 }  // namespace
 
+uint32_t frames_beside() { return g_frames_beside.load(std::memory_order_relaxed); }
+
 // A frame's last paths leave most of the chip idle (a path is a chain of some
 // hundreds of dependent node visits: in a soup of 65,536 triangles 512 x 512
 // paths take 550 us and 1,024 x 1,024 no more than 1,130), so a frame that is
@@ -1524,7 +1529,7 @@ Renderer::FrameSlot* take_slot(Renderer& r, size_t npaths) {
 // 4,818 -> 3,978; a 16-pass 637 x 359 frame under two lights after another
 // 2,645 -> 1,862.  A frame that finds the last one done takes the graph as before.
 void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, const float* dirs,
-                   const uint64_t* seeds, const uint32_t* scenes, hipStream_t st) {
+                   const uint64_t* seeds, const uint32_t* scenes, hipStream_t st, hipEvent_t begin) {
     if (!scene.ready) throw Error(PT_E_NO_SCENE, "no scene uploaded");
     if (r.settings.bounces > 60) throw Error(PT_E_INVALID_ARG, "at most 60 bounces");
     if (npasses == 0 || npasses > kMaxPasses) throw Error(PT_E_INVALID_ARG, "1 .. 1024 passes per call");
@@ -1561,6 +1566,7 @@ void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, cons
     if (slot) {
         PT_HIP(hipStreamWaitEvent(slot->st, r.base_ev, 0));
         PT_HIP(hipStreamWaitEvent(slot->st, slot->added, 0));
+        PT_HIP(hipEventRecord(begin, slot->st));
         upload_pass_params(r, npasses, dirs, seeds, scenes, slot->params, slot->st);
         const PathState ps = carve_state(slot->state.as<char>(), npix * npasses);
         launch_paths(scene, fc, slot->params.as<PassParams>(), ps, slot->counters.as<uint32_t>(), slot->st);
@@ -1573,8 +1579,10 @@ void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, cons
         r.frame_sent = true;
         r.last_counters = slot->counters.as<uint32_t>();
         r.spp += npasses;
+        g_frames_beside.fetch_add(1, std::memory_order_relaxed);
         return;
     }
+    PT_HIP(hipEventRecord(begin, st));
     r.queues.reserve(slab_bytes(npix * npasses) * kQueueArrays);
     upload_pass_params(r, npasses, dirs, seeds, scenes, r.params, st);
     ensure_chain_streams(r, std::max(1u, nchains));

@@ -308,8 +308,10 @@ int pt_set_stop_frame(pt_context* ctx, uint32_t frames);
  * after the last reset to the render call that found the limit reached, or -1
  * while it has not been reached. */
 int pt_generation_time(pt_context* ctx, double* seconds);
-/* Wall time in ms of the last pt_render_pass (HIP events); of one sent while the
- * frame before was at work, the time the context's stream spent on it. */
+/* Wall time in ms of the last pt_render_pass(es) or pt_render_cache_frame, from
+ * the start of its work to its place in the accumulator (HIP events).  A frame
+ * that is traced beside the one before shares the GPU with it for that time, so
+ * the times of such frames add up to more than they take together. */
 int pt_last_render_ms(pt_context* ctx, float* ms);
 
 /* ---- learned radiance cache (no reference counterpart) -----------------------
@@ -403,7 +405,10 @@ int pt_device_compute_units(int device, uint32_t* cus);
  *                   into this many chains of bounce levels on streams of
  *                   their own (at most one per 16,384 paths), so one chain's
  *                   level tail overlaps the others' work
- * Unknown names and values outside a knob's range return PT_E_INVALID_ARG. */
+ * Unknown names and values outside a knob's range return PT_E_INVALID_ARG.
+ * Only to be read:
+ *   "render.beside" frames so far (of all contexts) that were traced beside
+ *                   another (see pt_render_pass) */
 int pt_tune_set(const char* name, uint32_t value);
 int pt_tune_get(const char* name, uint32_t* value);
 
