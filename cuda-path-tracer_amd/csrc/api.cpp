@@ -98,7 +98,7 @@ void check_status(pt_context* ctx) {
     if (f == 0u) return;
     std::string m = "device status:";
     if (f & PT_STATUS_STACK_OVERFLOW) m += " traversal stack deeper than 64 entries;";
-    if (f & PT_STATUS_REFIT_OVERFLOW) m += " refit level list overflow;";
+    if (f & PT_STATUS_REFIT_OVERFLOW) m += " a build level's open list over its capacity;";
     throw pt::Error(PT_E_INTERNAL, m + " results of the affected calls are incomplete");
 }
 

@@ -290,10 +290,10 @@ struct RenderTuning {
     uint32_t paths = 1;   // plain frames path-persistent (one launch, no bounce levels)
     // Path-persistent frames: lanes that shade together (1..64), the same in
     // scenes with directional lights, and how few busy lanes let the idle ones
-    // take new paths.  Two 1,024 x 1,024 room frames take 4.88 / 4.83 / 4.87 /
-    // 4.93 ms at shade_min 8 / 12 / 16 / 24 and refill 60, 5.03 / 4.90 / 4.91 at
+    // take new paths.  Two 1,024 x 1,024 room frames take 4.58 / 4.47 / 4.47 /
+    // 4.56 ms at shade_min 8 / 12 / 16 / 24 and refill 60, 4.65 / 4.52 / 4.53 at
     // 12 and refill 48 / 56 / 64; a 16-pass textured frame under two lights
-    // 4.90 / 3.31 / 2.94 at shade_lit 12 / 32 / 64.
+    // 3.91 / 2.55 / 2.05 at shade_lit 12 / 32 / 64.
     uint32_t shade_min = 12;
     uint32_t shade_lit = 64;
     uint32_t refill = 60;

@@ -600,10 +600,10 @@ struct Handout {
 enum : uint32_t { kLaneIdle = 0u, kLaneTrace = 1u, kLaneShade = 2u };
 
 // Groups whose segments have ended shade together once they are at least one
-// in group_shade of the wave's groups (1, 2, 4, 8: 5.98, 5.73, 5.73, 5.80 ms
-// for two 1,024 x 1,024 room frames, 2.04, 2.11, 2.09, 2.15 for eight 256 x 256
+// in group_shade of the wave's groups (1, 2, 4, 8: 4.50, 4.49, 4.48, 4.47 ms
+// for two 1,024 x 1,024 room frames, 1.53, 1.53, 1.52, 1.53 for eight 256 x 256
 // soup frames).  With lights, whose shadow rays make shading the longer part,
-// all of them (a 637 x 359 textured frame under two lights 1.06 -> 0.43 ms).
+// all of them (a 16-pass 637 x 359 textured frame under two lights 2.14 -> 2.03 ms).
 constexpr uint32_t group_shade(bool lights) { return lights ? 1u : 4u; }
 
 __global__ __launch_bounds__(64) void k_paths_setup(uint32_t* __restrict__ counters, uint32_t* __restrict__ queue,
@@ -1525,9 +1525,9 @@ uint32_t frames_beside() { return g_frames_beside.load(std::memory_order_relaxed
 // stream, beside that frame's end, into path state of its own.  Only the sum
 // into the accumulator is made on the frames' stream, in order, which waits for
 // the paths as if all had been done there.  Eight frames of 256 x 256 in the
-// soup and their image: 2,093 -> 1,196 us; two of 1,024 x 1,024 in a closed room
-// 4,818 -> 3,978; a 16-pass 637 x 359 frame under two lights after another
-// 2,645 -> 1,862.  A frame that finds the last one done takes the graph as before.
+// soup and their image: 2,310 -> 1,520 us; two of 1,024 x 1,024 in a closed room
+// 5,100 -> 4,470; a 16-pass 637 x 359 frame under two lights after another
+// 2,650 -> 2,030.  A frame that finds the last one done takes the graph as before.
 void render_passes(Renderer& r, const DeviceScene& scene, uint32_t npasses, const float* dirs,
                    const uint64_t* seeds, const uint32_t* scenes, hipStream_t st, hipEvent_t begin) {
     if (!scene.ready) throw Error(PT_E_NO_SCENE, "no scene uploaded");

@@ -219,8 +219,13 @@ __device__ __forceinline__ void init_ray(RayState& r, uint32_t root, uint32_t fl
 //    rays are in soups and rooms, 7 % at the edges of a wall of 3,200 triangles,
 //    9 % on two tessellations of one wall, 83 % on 4,000 overlapping decals.
 //  - The slab test is monotonic unless a product is NaN: a ray with an infinite
-//    dinv component is a tie when one arises, and where a triangle's box is NaN
-//    (strict, from the build) every ray walks in the reference's order.
+//    or zero dinv component is a tie when one arises, and where a triangle's box is
+//    NaN (strict, from the build) every ray walks in the reference's order.
+// Against culling by the best distance alone, with the visiting order deciding:
+// 16M shell rays 868 us for 869, 2M hair ball rays 1,216 for 1,189, 2,000 rays in a
+// soup 20.7 for 18.9, two room frames 4,229 for 4,047.  Where many rays are ties
+// (2M rays on 1,500 decals in one plane 1,231 us) it is slower than one lane per
+// ray in the reference's order (950).
 
 // Minimum and maximum of distances that are no NaN and no less than zero (the
 // maximum also of -0 and, with another that is not, negative ones): of their
@@ -405,10 +410,11 @@ __device__ __forceinline__ bool visit_step(const float4* __restrict__ nodes,
 // nodes; its hit is the reference's (see above).  A kRayExact lane tests leaf
 // children at once.
 // Measured (us; 16M shell rays on the 871,200-triangle mesh, 2M camera rays on
-// the 2.88M-triangle hair ball, two 1,024 x 1,024 room frames): tests at once
-// 897, 1,464, 5,790; four entries and 6 / 12 / 20 / 32 lanes 877 / 863 / 868 /
-// 996, 1,356 / 1,364 / 1,414 / 1,681, 5,630 / 5,490 / 5,505 / 6,630; six entries
-// and 12 lanes 883, 1,366, 5,460.
+// the 2.88M-triangle hair ball, two 1,024 x 1,024 room frames): four entries and
+// 6 / 12 / 20 / 32 lanes 879 / 862 / 885 / 1,044, 1,220 / 1,217 / 1,260 / 1,452,
+// 4,650 / 4,550 / 4,475 / 4,800; six entries and 12 lanes 869, 1,218, 5,035.  When
+// the list came in (tests at once -> four entries, 12 lanes): 897 -> 863, 1,464 ->
+// 1,364, 5,790 -> 5,490.
 constexpr uint32_t kPend = 4;  // list entries per lane
 constexpr uint32_t kFlushLanes = 12;
 // LDS words per lane: its stack, then its list (triangles, then distances).
@@ -895,9 +901,9 @@ __device__ __forceinline__ void group_trace(const float4* __restrict__ nodes, co
 
 // The end of a persistent loop: the wave's active lanes (at most kTailLanes,
 // each with fewer than LDS deferred nodes) go on as groups.  16M shell rays on
-// the 871,200-triangle mesh: 1,236 us without, 932 / 901 / 897 us from 8 / 16 /
-// 32 lanes on; 2M camera rays on the 2.88M-triangle hair ball 1,655 us
-// without, 1,645 / 1,505 / 1,460.
+// the 871,200-triangle mesh: 870 us without, 921 / 866 / 862 us from 8 / 16 /
+// 32 lanes on; 2M camera rays on the 2.88M-triangle hair ball 1,219 us
+// without, 1,407 / 1,279 / 1,217.
 constexpr uint32_t kTailLanes = 32;
 static_assert(kTailLanes <= 32, "regroup takes at most 32 groups");
 
@@ -951,10 +957,10 @@ __device__ __forceinline__ void grouped_trace(const float4* __restrict__ nodes, 
 
 // Lanes per ray (log2) of a launch of `nrays` rays on `lanes` lanes: as many as
 // there are lanes for, at most 2^kGroupMax; 0: one lane per ray, persistent.
-// Measured: 2,000 rays in a 4,096-triangle soup 89 us with one lane per ray,
-// 23 with up to 8, 19 with up to 16, 18 with up to 32; 131,072 rays (4 lanes)
-// after a rebuild of 2^20 triangles 565 -> 306 us; 65,536-path frames 1,040 ->
-// 260 us.  At 16 the wider rounds already find too few nodes to go further.
+// Measured: 2,000 rays in a 4,096-triangle soup 58 us with one lane per ray, 26
+// with up to 8, 23 with up to 16, 22 with up to 32; 131,072 rays (4 lanes) after a
+// rebuild of 2^20 triangles 448 -> 291 us; eight 65,536-path frames in a row 3,650
+// -> 1,520 us.  At 16 the wider rounds already find too few nodes to go further.
 constexpr uint32_t kGroupMax = 4;
 inline uint32_t launch_group(uint64_t nrays, uint64_t lanes) {
     uint32_t lg = 0;
@@ -984,7 +990,8 @@ inline uint32_t grouped_blocks(uint64_t nrays, uint32_t lg) {
 // contiguous rays, 64 places of an image at a time, 10^6 camera rays on the
 // 871,200-triangle mesh took 365 us (234), 700,000 on a hair ball of 50,000
 // triangles 162 (117), 2,073,600 on one of 2.88M 1,215 (1,170), 4M in a soup 920
-// (858); 16M shell rays in no order 865 (857).
+// (858); 16M shell rays in no order 865 (857).  (Both sides measured with culling
+// by the best distance alone, which camera rays walk 2-3 % faster.)
 constexpr uint32_t kQueueSlices = 64;
 constexpr uint32_t kQueueStride = 64;  // words between counters (256 bytes)
 constexpr uint32_t kQueueMask = kQueueSlices * kQueueStride;  // word offset of the mask
@@ -1181,9 +1188,8 @@ constexpr uint32_t kSurvCap = 128;  // survivor ring entries per wave
 // with a survivor ready for every idle lane, or no more rays to filter, that
 // costs no filter round.  (Filter rounds wait for the launch's `refill`: with 48
 // for both, 16M shell rays, which mostly end in the filter, took 1 % longer.)
-// 2.88M-triangle hair ball, 2,073,600 camera rays: 1,344 us without, 1,275 / 1,245
-// / 1,220 at 40 / 48 / 56, 10^6 rays 930 and 770 / 764 / 760; 4M camera rays on
-// the 871,200-triangle mesh 654 and 640 / 628 / 613; 16M shell rays 867 each.
+// 2.88M-triangle hair ball, 2,073,600 camera rays: 1,393 us without, 1,262 at 48,
+// 1,217 at 56; 16M shell rays on the 871,200-triangle mesh 854, 867 and 862.
 constexpr uint32_t kReadyRefill = 56;
 
 // The root visit alone (visit_step's decisions without the stack): leaf

@@ -242,10 +242,12 @@ int pt_trace_closest_device_noalloc(pt_context* ctx, const float* d_rays, uint32
 int pt_trace_closest_scenes_device(pt_context* ctx, const float* d_rays, const uint32_t* d_scene,
                                    uint32_t n, uint32_t* d_id, float* d_t, float* d_uv,
                                    void* stream);
-/* Measurement variant (no reference counterpart): the same traversal, also
- * counting inner-loop iterations, box tests and triangle tests into
- * counters[0..2] (host, uint64, totals) and the deepest deferred-node stack
- * any ray reached into counters[3].  Host-synchronous. */
+/* Measurement variant (no reference counterpart): the same hits by a walk in the
+ * reference's order (every leaf tested as its node is visited), counting
+ * inner-loop iterations, box tests and triangle tests into counters[0..2] (host,
+ * uint64, totals) and the deepest deferred-node stack any ray reached into
+ * counters[3].  The other entry points test leaves later or several nodes at once
+ * and visit a few more nodes than it counts.  Host-synchronous. */
 int pt_trace_closest_counted(pt_context* ctx, const float* d_rays, uint32_t n,
                              uint32_t* d_id, float* d_t, float* d_uv,
                              uint64_t* counters, void* stream);
