@@ -298,8 +298,8 @@ __device__ __forceinline__ half8 join_relu(floatx4 a, floatx4 b) { return join(r
 // blocks at a time so each weight fragment read from LDS feeds kInferBlocks
 // MFMAs.  2,073,600 samples take 81 us (152 with inputs indexed through
 // scratch, MFMA results in accumulation registers and 16 lanes finishing one
-// block's outputs): of a SIMD's 197,000 cycles its matrix core is busy 77,000,
-// its vector instructions issue for 96,000, and 25,000 of these coincide.
+// block's outputs): of a SIMD's 181,000 cycles its matrix core is busy 77,000,
+// its vector instructions issue for 95,000, and 34,000 of these coincide.
 // Prefetching the next samples (142 registers, three waves) changed nothing;
 // what memory and staging alone take is 31 us.
 constexpr int kInferBlocks = 4;
