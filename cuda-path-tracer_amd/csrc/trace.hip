@@ -176,6 +176,14 @@ uint32_t launch_grouped(const DeviceScene& s, uint32_t first, const float* d_ray
     return lg;
 }
 
+// The filtered kernel's stack at trace.lds_stack 32: with two entries fewer it and
+// the survivor rings take 40,960 bytes of LDS, so that four workgroups share a CU
+// as they do without the filter.  With all 32 three do: 16M shell rays on the
+// 871,200-triangle mesh 1,060 us for 887, 2M hair ball rays 1,496 for 1,264.
+constexpr int kFilterStack = 30;
+static_assert(sizeof(uint32_t) * (kRayRows<kFilterStack> * kPersistThreads + kPersistThreads / 64 * kSurvCap) * 4 <= 160 * 1024,
+              "four workgroups");
+
 __global__ __launch_bounds__(64) void k_zero_queue(uint32_t* queue) { zero_queue(queue, 1u); }
 
 template <bool COUNT>
@@ -205,7 +213,7 @@ void launch_trace(const DeviceScene& s, uint32_t* queue, const float* d_rays, ui
     const bool filter = !COUNT && tune.filter != 0;
     auto kern = filter ? (tune.lds <= 8 ? k_trace_persistent<false, 8, true>
                                         : (tune.lds <= 16 ? k_trace_persistent<false, 16, true>
-                                                          : k_trace_persistent<false, 32, true>))
+                                                          : k_trace_persistent<false, kFilterStack, true>))
                        : (tune.lds <= 8 ? k_trace_persistent<COUNT, 8, false>
                                         : (tune.lds <= 16 ? k_trace_persistent<COUNT, 16, false>
                                                           : k_trace_persistent<COUNT, 32, false>));

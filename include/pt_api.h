@@ -382,7 +382,9 @@ int pt_device_compute_units(int device, uint32_t* cus);
  *                   and rays that wait behind the filter already below 56.
  *                   Launches of few rays, with several lanes each, do not read it
  *   "trace.lds_stack" traversal stack entries per lane kept in LDS (8, 16 or
- *                   32; deeper entries spill to scratch)
+ *                   32, of which the root filter takes 2; deeper entries spill to
+ *                   scratch).  Launches of few rays and path-persistent frames
+ *                   keep at most 16
  *   "trace.pool"    rays a wave takes from such a queue at a time when it is long
  *                   (64..4096)
  *   "trace.filter"  1: closest-hit batches run every ray's root visit in
